@@ -52,6 +52,10 @@ constexpr int kT3Words = 2 * kT3Reps;
 // minus signs, a type-1 code +-4s on two positions.
 constexpr int kT2Octads = 759;
 constexpr int kT2Tiles = 48;  // 768 octad slots
+// NN-T and NN-P resolve an exact tie between type-1/2 codes by the group of 256 that holds the code's pair in
+// the sweep order, then by row (the order in which a sweep of the table meets them); NN-B by row alone.
+constexpr int kRowBits = 18;
+constexpr int kTieGroup = 256;
 constexpr int kT2Subsets5 = 42504;  // C(24, 5): each in exactly one octad
 constexpr int kT3DecWords = 4096 + 12 + 24;  // Golay decoder: leaders by syndrome, basis, position syndromes
 
@@ -65,7 +69,6 @@ constexpr uint32_t kSqrt12Bits = 0x405DB3D7u;      // fp32(sqrt 12)
 struct DeviceTables {
   int device = -1;
   uint8_t *sw_bf16_tiles = nullptr;  // [kSweepTiles][3][16][8] bf16 bits of the sweep codes (MFMA A operands)
-  uint8_t *sw_raw_tiles = nullptr;   // the same layout, bf16 bits of the raw integers (NN-P)
   uint32_t *sw_dq = nullptr;         // [kSweepTiles*16][3] value-id words of the sweep codes (rescans)
   uint32_t *sw_idx = nullptr;        // [kSweepTiles*16] codebook row of each sweep code, 0 for padding
   uint32_t *sw_anti = nullptr;       // [(kSweepTiles-kType3Tiles)*16] antipode rows, from the pair region's start
@@ -82,8 +85,8 @@ struct DeviceTables {
   uint32_t *t3_rows = nullptr;       // [4096][24] codebook row of the type-3 code (word of id, -3 at position p)
   uint8_t *t2_tiles = nullptr;       // [kT2Tiles][3][16][8] bf16 octad indicators times 2s
   uint2 *t2_pos = nullptr;           // [kT2Tiles*16] the 8 positions of each octad, one byte each
-  uint32_t *t2_rows = nullptr;       // [759][128] codebook row of the octad code with sign pattern p
-  uint32_t *t1_rows = nullptr;       // [24][24][4] codebook row of the type-1 code at i < j, minus bits
+  uint32_t *t2_rows = nullptr;       // [759][128] row | tie group << 18 of the octad code with sign pattern p
+  uint32_t *t1_rows = nullptr;       // [24][24][4] row | tie group << 18 of the type-1 code at i < j, minus bits
   uint16_t *t2_steiner = nullptr;    // [kT2Subsets5] the octad holding each 5-subset (colex rank)
   uint32_t *t3_dec = nullptr;        // [kT3DecWords] Golay coset leaders by syndrome, basis words, position syndromes
 };

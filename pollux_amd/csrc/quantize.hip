@@ -26,40 +26,34 @@
 // Selection semantics (per atom, codes in ascending index order).
 //   NN-B (castor.py:549-557): bucket(s) = bf16_rne(s); winner = lowest code
 //     with the maximal bucket M; origin iff 2*M < 0x407FFFFF, i.e. M < 2.0.
-//   NN-T (castor.py:419-460): winner = lowest code with the maximal fp32
-//     score S; origin iff 2*S < 0x407FFFFF.
+//   NN-T (castor.py:419-460): bf16 operands, winner = lowest code with the
+//     maximal fp32 score S; origin iff 2*S < 0x407FFFFF.
 //   NN-P (pack.py:167-177): fp32 atom against the fp32 codebook, winner =
-//     lowest code with the maximal score; origin iff |x|_2 < 1e-8.  The atom
-//     is split exactly into three bf16 parts (x = h + m + l up to 2^-27|x|)
-//     and scored against the raw integer codes (exact in bf16) by three
-//     chained MFMAs per tile; the fp32 codebook is the raw table times
-//     fp32(1/sqrt 8) (3s rounded), so these scores order the codes like the
-//     fp32 ones up to 2^-21 * sum|x_i c_i|, inside the near-tie envelope.
-//   Both are tracked with one integer threshold R per (atom, lane): a group of
-//   kG tiles (4 kG codes per lane) improves when its max score, as an int bit
-//   pattern, exceeds R (positive floats order like ints; negative scores can
-//   only lose to the origin threshold R starts at).  NN-B raises R to the
-//   largest fp32 that still rounds to the new bucket, so later codes in the
-//   same bucket never displace the earlier group; NN-T raises R to the score.
-//   Each (atom, slice) ends as one atomic max into the atom's key word:
-//   (best bucket or score, 1023 - earliest group reaching it, mask of the
-//   atom's four lanes whose earliest group that is), 32 bits for NN-B
-//   (bucket << 16 | (1023 - g) << 6 | mask << 2), 64 bits for NN-T / NN-P
-//   (score << 32 | (1023 - g) << 4 | mask).  Slices own disjoint groups, so
-//   the maximum over slices is the highest bucket / score, then the earliest
-//   group holding it -- the group of the lowest code the selection rule
-//   wants -- and no two slices write the same (score, group).  prep_kernel
-//   (NN-P: clear_keys_kernel) zeroes the keys; 0 means the origin threshold
+//     lowest code with the maximal score; origin iff |x|_2 < 1e-8.
+//   (NN-T / NN-P: an exact tie between type-1/2 codes -- a near-tie, which the
+//   parity oracle leaves open -- goes to the code whose pair comes first in
+//   groups of 256, then to the lowest row: kTieGroup.)
+// All three run the structured scorers (t12_kernel, t3_kernel, pick_kernel),
+// which differ by mode only in how two scores are compared (Sel) and, NN-P, in
+// the atoms they score.  nn_kernel and resolve_kernel are NN-B scored densely
+// (PLX_NN_DENSE_TYPE3), the baseline of the structured path:
+//   a group of kG tiles (4 kG codes per lane) is tracked by one integer key per
+//   (atom, lane) (group_key, pair_key); each (atom, slice) ends as one atomic
+//   max into the atom's key word: bucket << 16 | (1023 - earliest group
+//   reaching it) << 6 | mask of the atom's four lanes whose earliest group that
+//   is << 2.  Slices own disjoint groups, so the maximum over slices is the
+//   highest bucket, then the earliest group holding it -- the group of the
+//   lowest code the selection rule wants -- and no two slices write the same
+//   (bucket, group).  prep_kernel zeroes the keys; 0 means the origin threshold
 //   was never beaten.
 //
 // resolve_kernel -- per atom its key, then an exact-product rescan
-//   (v_dot2_f32_bf16; NN-P: fp64 dot products of the fp32 atom and the fp32
-//   codebook rows, exact up to 2^-48) of the key's group in the lanes of its
-//   mask to find the lowest code, 4 lanes per (group, lane) with coalesced
-//   table reads, then the index and the packed 9-byte groups.  Both fp32 sums
-//   (MFMA, dot2) lie within 24 * 2^-24 * sum|x_i c_i| of the exact score
-//   (MFMA measured at < 2^-22), so the result equals the exact-score answer
-//   on every atom that is not a near-tie within that envelope.
+//   (v_dot2_f32_bf16) of the key's group in the lanes of its mask to find the
+//   lowest code, 4 lanes per (group, lane) with coalesced table reads, then the
+//   index and the packed 9-byte groups.  Both fp32 sums (MFMA, dot2) lie within
+//   24 * 2^-24 * sum|x_i c_i| of the exact score (MFMA measured at < 2^-22), so
+//   the result equals the exact-score answer on every atom that is not a
+//   near-tie within that envelope.
 
 #include <mutex>
 #include <type_traits>
@@ -89,33 +83,9 @@ static_assert(kST % kG == 0 && kG >= 8 && kG <= 64 && (kG & (kG - 1)) == 0, "who
 constexpr int kModeB = PLX_NN_BF16_SCORES;
 constexpr int kModeP = PLX_NN_PACK_FP32;
 
-// bf16 parts per atom coordinate: NN-P carries the fp32 value as h + m + l.
-template <int MODE>
-constexpr int n_splits() {
-  return MODE == kModeP ? 3 : 1;
-}
-
-template <int MODE>
-__device__ __forceinline__ int initial_threshold() {
-  // NN-B: the largest group key of bucket 0x3FFF (bf16 max below 2.0); any
-  //       group reaching bucket 0x4000 has a larger key (group_key).
-  // NN-T: largest fp32 s with 2*s < 0x407FFFFF.
-  // NN-P: +0.0 -- no score threshold (every nonzero atom has a positive
-  //       maximum: the best +-4 pair scores 4s(|x_i| + |x_j|)).
-  return MODE == kModeB ? 0x3FFFFFFF : MODE == kModeP ? 0 : 0x3FFFFFFE;
-}
-
-// New threshold after a group whose maximum is gm.  NN-T: gm itself.  NN-B:
-// the largest fp32 bit pattern in gm's bf16 bucket, with the bucket taken by
-// round-half-up ((gm + 0x8000) >> 16) -- two VALU ops instead of five.  It
-// differs from round-to-nearest-even only when gm's low 16 bits are exactly
-// 0x8000, a score sitting exactly on a bf16 rounding midpoint, which the
-// parity oracle classifies as a near-tie.
-template <int MODE>
-__device__ __forceinline__ int raised_threshold(int gm) {
-  if (MODE != kModeB) return gm;
-  return static_cast<int>(((static_cast<uint32_t>(gm) + 0x8000u) & 0xFFFF0000u) | 0x7FFFu);
-}
+// The largest group key of bucket 0x3FFF (bf16 max below 2.0); any group
+// reaching bucket 0x4000 has a larger key (group_key).
+constexpr int kInitialThreshold = 0x3FFFFFFF;
 
 // Lattice coordinates 8q..8q+7 of atom a (zeros past the end / for q == 3).
 // FUSED: x = (w / max(sigma[row], 1e-8)) / fp32(1/sqrt 2) (castor.py:332-333,
@@ -143,7 +113,8 @@ __device__ __forceinline__ void load_coords8(const float *__restrict__ src, cons
 // bf16 lattice coordinates of every atom, row-major [n_atoms][24] (one
 // 16-byte plane of 8 per thread), written once per launch so the scoring
 // blocks of all slices load ready-made MFMA B operands instead of each
-// repeating the row-scale divisions.  NN-B / NN-T only.
+// repeating the row-scale divisions (the batched requantize: for all its
+// latents, before t12_kernel).
 // Also clears the atoms' 16-byte key slots before nn_kernel merges its
 // slices into them.
 template <bool FUSED>
@@ -164,14 +135,10 @@ __global__ __launch_bounds__(256) void prep_kernel(const float *__restrict__ src
   xb[i] = w;
 }
 
-// NN-P has no prep pass: its key slots are cleared here.
-__global__ __launch_bounds__(256) void clear_keys_kernel(uint4 *__restrict__ keys, int64_t n) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i < n) keys[i] = make_uint4(0u, 0u, 0u, 0u);
-}
-
-// NN-B tracking key of a type-3 group: bucket (round-half-up, see
-// raised_threshold) in the high half, 0xFFFF - group in the low half, so one
+// Tracking key of a type-3 group: bucket (by round-half-up, (gm + 0x8000) >>
+// 16: two VALU ops instead of five.  It differs from round-to-nearest-even
+// only when gm's low 16 bits are exactly 0x8000, a score on a bf16 rounding
+// midpoint, which the parity oracle classifies as a near-tie) in the high half, 0xFFFF - group in the low half, so one
 // signed max keeps the highest bucket and, within it, the earliest group.
 // v_perm_b32 takes bytes 2-3 of the rounded score and bytes 0-1 of the
 // (uniform) group field in one instruction.
@@ -206,20 +173,16 @@ __device__ __forceinline__ uint32_t atom_lanes(uint64_t bal, int j) {
                                ((bal >> (j + 45)) & 8u));
 }
 
-// src: NN-P: the fp32 atoms; NN-B / NN-T: xb, the bf16 planes of prep_kernel.
+// xb: the bf16 planes of prep_kernel.
 // tiles: the sweep-order tiles (type-3 codes, then pair representatives).
-// recs (NN-B): one record per (atom, slice >= s0, the slices holding pair
-// tiles), [slice - s0][n_atoms].
-// NN-B: at most 168 VGPRs (3 waves per SIMD; the MFMA issue rate needs the
-// third wave), which costs two 8-byte spills outside the scoring loops;
-// NN-T / NN-P keep 2 waves per SIMD (their wider keys and split operands
-// would spill inside the loops at 168).
-template <int MODE>
-__global__ __launch_bounds__(kThreads, MODE == kModeB ? 3 : 2) void nn_kernel(const void *__restrict__ src,
-                                                                             int64_t n_atoms,
-                                                          const uint8_t *__restrict__ tiles, int n_slices,
-                                                          int tiles_per_slice, uint4 *__restrict__ keys,
-                                                          uint64_t *__restrict__ recs, int s0) {
+// recs: one record per (atom, slice >= s0, the slices holding pair tiles),
+// [slice - s0][n_atoms].
+// At most 168 VGPRs (3 waves per SIMD; the MFMA issue rate needs the third
+// wave), which costs two 8-byte spills outside the scoring loops.
+__global__ __launch_bounds__(kThreads, 3) void nn_kernel(const uint4 *__restrict__ xb, int64_t n_atoms,
+                                                         const uint8_t *__restrict__ tiles, int n_slices,
+                                                         int tiles_per_slice, uint4 *__restrict__ keys,
+                                                         uint64_t *__restrict__ recs, int s0) {
   __shared__ __align__(16) uint8_t lds[2][kStageBytes];
 
   const int slice = static_cast<int>(blockIdx.x % static_cast<unsigned>(n_slices));
@@ -229,32 +192,13 @@ __global__ __launch_bounds__(kThreads, MODE == kModeB ? 3 : 2) void nn_kernel(co
   const int64_t wave_atom0 = ablock * kAtomsPerBlock + static_cast<int64_t>(wave) * (kAT * 16);
 
   // B operands: kAT atom tiles, lane holds coordinates 8q..8q+7 of atom j
-  // (NN-P: as three bf16 parts, b[0] + b[1] + b[2]).
-  constexpr int NS = n_splits<MODE>();
-  bf16x8 b[NS][kAT];
+  bf16x8 b[kAT];
 #pragma unroll
   for (int at = 0; at < kAT; ++at) {
     const int64_t a = wave_atom0 + at * 16 + j;
-    if constexpr (NS == 1) {
-      uint4 w = make_uint4(0u, 0u, 0u, 0u);
-      if (a < n_atoms && q < 3) w = static_cast<const uint4 *>(src)[a * 3 + q];
-      b[0][at] = __builtin_bit_cast(bf16x8, w);
-      continue;
-    }
-    float v[8];
-    load_coords8<false>(static_cast<const float *>(src), nullptr, 1, n_atoms, a, q, v);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t h = bf16_rne_bits(v[e]);
-      b[0][at][e] = __builtin_bit_cast(__bf16, static_cast<uint16_t>(h));
-      if constexpr (NS == 3) {
-        const float r1 = v[e] - bf16_bits_to_float(h);  // exact
-        const uint32_t m = bf16_rne_bits(r1);
-        const float r2 = r1 - bf16_bits_to_float(m);    // exact
-        b[1][at][e] = __builtin_bit_cast(__bf16, static_cast<uint16_t>(m));
-        b[2][at][e] = __builtin_bit_cast(__bf16, static_cast<uint16_t>(bf16_rne_bits(r2)));
-      }
-    }
+    uint4 w = make_uint4(0u, 0u, 0u, 0u);
+    if (a < n_atoms && q < 3) w = xb[a * 3 + q];
+    b[at] = __builtin_bit_cast(bf16x8, w);
   }
 
   const int t0 = slice * tiles_per_slice;
@@ -279,27 +223,25 @@ __global__ __launch_bounds__(kThreads, MODE == kModeB ? 3 : 2) void nn_kernel(co
   __syncthreads();
 
   const int a_off = (q < 3 ? q : 0) * 256 + j * 16;
-  int R[kAT], best[kAT];
+  int R[kAT];
 
   // Stages [st0, st1) of one region.  PAIR: the fold takes max |score| (the
-  // antipode of each representative scores exactly its negation), and NN-B
+  // antipode of each representative scores exactly its negation) and
   // tracks the first and last group at the best bucket (pair_key).
   // Software pipeline: the MFMA result of tile k for atom tile `at` is folded
   // into the group maximum while tile k+1's MFMAs issue, and tile k+1's A
   // operand is read from LDS right after tile k's first MFMA.  A group of kG
-  // tiles is compared against the threshold once its last tile has been
-  // folded, i.e. during the next group's first tile (NN-B: the next group's
-  // tile at % 8); the region's last tile is folded after its loop.
+  // tiles enters its key once its last tile has been folded, i.e. during the
+  // next group's tile at % 8; the region's last tile is folded after its loop.
   auto run = [&](auto pair_tag, int st0, int st1) {
     constexpr bool PAIR = decltype(pair_tag)::value;
     const int g_base = (t0 + st0 * kST) / kG;  // global group of the region's first group in this slice
 #pragma unroll
     for (int at = 0; at < kAT; ++at) {
-      R[at] = PAIR && MODE == kModeB ? static_cast<int>(kPairInit) : initial_threshold<MODE>();
-      best[at] = -1;
+      R[at] = PAIR ? static_cast<int>(kPairInit) : kInitialThreshold;
     }
     int gm[kAT];
-    f32x4 acc[kAT], part[kAT];
+    f32x4 acc[kAT];
 #pragma unroll
     for (int at = 0; at < kAT; ++at) {
       gm[at] = INT_MIN;
@@ -311,7 +253,6 @@ __global__ __launch_bounds__(kThreads, MODE == kModeB ? 3 : 2) void nn_kernel(co
       if (st + 1 < n_stages) stage_copy(st + 1, buf ^ 1);
       const uint8_t *L = lds[buf] + a_off;
       bf16x8 a = *reinterpret_cast<const bf16x8 *>(L);
-      bool up[kAT];
       int gdone[kAT];
       // One group of kG tiles: tile 0 closes the previous group, tile 1 starts
       // this group's maximum.
@@ -322,7 +263,7 @@ __global__ __launch_bounds__(kThreads, MODE == kModeB ? 3 : 2) void nn_kernel(co
           bf16x8 an;
 #pragma unroll
           for (int at = 0; at < kAT; ++at) {
-            const f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[0][at], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            const f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[at], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
             if (at == 0) {
               // the LDS wait that guards `a` must not also wait for this read
               __builtin_amdgcn_sched_barrier(0);
@@ -356,33 +297,19 @@ __global__ __launch_bounds__(kThreads, MODE == kModeB ? 3 : 2) void nn_kernel(co
             // stops the machine scheduler from hoisting every MFMA, so the
             // matrix pipe and the VALU work in parallel.
             asm volatile("" : "+v"(m));
-            if (t == 0) {
-              gdone[at] = m;
-              if constexpr (MODE != kModeB) up[at] = m > R[at];
-            }
-            // NN-B: the closed group's key enters R in tile at % 8 of the next
+            if (t == 0) gdone[at] = m;
+            // the closed group's key enters R in tile at % 8 of the next
             // group, one atom tile per code tile, so the key's VALU work is
             // spread evenly under the MFMAs instead of piling up in tile 0.
-            if (MODE == kModeB && at % 8 == t) {
+            if (at % 8 == t) {
               if constexpr (PAIR)
                 R[at] = static_cast<int>(pair_key(static_cast<uint32_t>(R[at]), gdone[at], group_prev - g_base));
               else
                 R[at] = max(R[at], group_key(gdone[at], group_prev));
             }
             gm[at] = m;
-            if constexpr (NS == 1)
-              acc[at] = c;
-            else
-              part[at] = c;
+            acc[at] = c;
             __builtin_amdgcn_sched_barrier(0);
-          }
-          if constexpr (NS == 3) {
-#pragma unroll
-            for (int at = 0; at < kAT; ++at)
-              part[at] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[1][at], part[at], 0, 0, 0);
-#pragma unroll
-            for (int at = 0; at < kAT; ++at)
-              acc[at] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[2][at], part[at], 0, 0, 0);
           }
           a = an;
         }
@@ -390,15 +317,6 @@ __global__ __launch_bounds__(kThreads, MODE == kModeB ? 3 : 2) void nn_kernel(co
 #pragma unroll 1
       for (int k0 = 0; k0 < kST; k0 += kG) {
         group_tiles(k0);
-        if constexpr (MODE != kModeB) {
-#pragma unroll
-          for (int at = 0; at < kAT; ++at) {
-            if (up[at]) {
-              R[at] = raised_threshold<MODE>(gdone[at]);
-              best[at] = group_prev;
-            }
-          }
-        }
         group_prev = (t0 + st * kST + k0) / kG;
       }
       __syncthreads();
@@ -416,15 +334,10 @@ __global__ __launch_bounds__(kThreads, MODE == kModeB ? 3 : 2) void nn_kernel(co
         m = max(max(gm[at], __float_as_int(acc[at][0])), __float_as_int(acc[at][1]));
         m = max(max(m, __float_as_int(acc[at][2])), __float_as_int(acc[at][3]));
       }
-      if constexpr (MODE == kModeB) {
-        if constexpr (PAIR)
-          R[at] = static_cast<int>(pair_key(static_cast<uint32_t>(R[at]), m, group_prev - g_base));
-        else
-          R[at] = max(R[at], group_key(m, group_prev));
-      } else if (m > R[at]) {
-        R[at] = raised_threshold<MODE>(m);
-        best[at] = group_prev;
-      }
+      if constexpr (PAIR)
+        R[at] = static_cast<int>(pair_key(static_cast<uint32_t>(R[at]), m, group_prev - g_base));
+      else
+        R[at] = max(R[at], group_key(m, group_prev));
     }
 
     // ---- merge this region of the slice into the atom's keys ----
@@ -437,17 +350,17 @@ __global__ __launch_bounds__(kThreads, MODE == kModeB ? 3 : 2) void nn_kernel(co
     for (int at = 0; at < kAT; ++at) {
       const int64_t a = wave_atom0 + at * 16 + j;
       const bool mine = q == 0 && a < n_atoms;
-      if constexpr (MODE == kModeB && !PAIR) {
+      if constexpr (!PAIR) {
         int Rm = R[at];
         Rm = max(Rm, __shfl_xor(Rm, 16, 64));
         Rm = max(Rm, __shfl_xor(Rm, 32, 64));
         const uint32_t mask = atom_lanes(__ballot(R[at] == Rm), j);
         const uint32_t g = 0xFFFFu - (static_cast<uint32_t>(Rm) & 0xFFFFu);
-        const uint32_t key = Rm != initial_threshold<MODE>()
+        const uint32_t key = Rm != kInitialThreshold
                                  ? (static_cast<uint32_t>(Rm) & 0xFFFF0000u) | ((0x3FFu - g) << 6) | (mask << 2)
                                  : 0u;
         if (mine) atomicMax(&keys[a].x, key);
-      } else if constexpr (MODE == kModeB) {
+      } else {
         // This slice's record: the best bucket Bm over the atom's lanes; among
         // the lanes at Bm, the earliest first group F and the latest last
         // group L (pair-region indices), the lanes with a hit in F and in L,
@@ -473,24 +386,6 @@ __global__ __launch_bounds__(kThreads, MODE == kModeB ? 3 : 2) void nn_kernel(co
                                             ((pb + F) << 32) | ((pb + Lg) << 24) | (mf << 4) | ml
                                       : 0ull;
         if (mine) recs[static_cast<int64_t>(slice - s0) * n_atoms + a] = rec;
-      } else {
-        // (score, 1023 - group) as one 64-bit value (pair groups counted from
-        // the pair region's start), lanes that never beat the threshold 0
-        const bool hit = best[at] >= 0;
-        const uint32_t g = static_cast<uint32_t>(best[at] - (PAIR ? kType3Tiles / kG : 0));
-        const uint64_t v = hit ? (static_cast<uint64_t>(static_cast<uint32_t>(R[at])) << 32) |
-                                     (static_cast<uint64_t>(0x3FFu - g) << 4)
-                               : 0ull;
-        uint64_t vm = v;
-        uint64_t o = static_cast<uint64_t>(__shfl_xor(static_cast<long long>(vm), 16, 64));
-        vm = o > vm ? o : vm;
-        o = static_cast<uint64_t>(__shfl_xor(static_cast<long long>(vm), 32, 64));
-        vm = o > vm ? o : vm;
-        const uint64_t mask = atom_lanes(__ballot(v == vm), j);
-        const uint64_t key = vm != 0ull ? vm | mask : 0ull;
-        if (mine)
-          atomicMax(reinterpret_cast<unsigned long long *>(&keys[a]) + (PAIR ? 1 : 0),
-                    static_cast<unsigned long long>(key));
       }
     }
   };
@@ -561,10 +456,71 @@ constexpr int kT3Surv = 384;                       // survivor words per wave (4
 constexpr float kT3Alpha = 1.416015625f;           // bf16(3s) + bf16(s)
 constexpr float kT3Beta = 0.708984375f;            // bf16(3s) - bf16(s)
 constexpr float kT3S = 0.353515625f;               // bf16(s)
+constexpr float kP3Alpha = 4.f * kT3S;             // NN-P: 3s + s
+constexpr float kP3Beta = 2.f * kT3S;              // NN-P: 3s - s
 static_assert(kT3StageVecs % 64 == 0, "type-3 stage splits into whole wave loads");
 static_assert(kT3Tiles % kT3ST == 0, "whole type-3 stages");
 
 __device__ __forceinline__ uint32_t t3_bucket(float v) { return (__float_as_uint(v) + 0x8000u) >> 16; }
+
+// What the structured scorers compare, per mode.  key(v): a positive score's order key -- NN-B its bf16
+// bucket, NN-T / NN-P its fp32 bits; kMin: the lowest key that is not the origin's; lo(M): a score that can
+// still give or tie key M is at least this; load / store: the key in a 32-bit word of the atom's key slot.
+// NN-P scores are fp32 sums of fp32 products, so its lo lies 2^-14 below: both sums of two codes that tie
+// in exact arithmetic lie within 24 * 2^-24 * sum|x_i c_i| <= 24 * 2^-24 * |x| |c| of it, and the best code
+// scores at least 0.28 |x| |c| (the two largest |x| of any atom, type 1), so the two differ by less than
+// 2^-16.6 of the best; every code at or above lo is then compared in fp64.
+template <int MODE>
+struct Sel {
+  static constexpr uint32_t kMin = MODE == kModeB ? 0x4000u : MODE == kModeP ? 1u : 0x3FFFFFFFu;
+  static __device__ __forceinline__ uint32_t key(float v) {
+    if constexpr (MODE == kModeB) return t3_bucket(v);
+    return __float_as_uint(v);
+  }
+  static __device__ __forceinline__ float lo(uint32_t M) {
+    if constexpr (MODE == kModeB) return __uint_as_float((M << 16) - 0x8000u);
+    if constexpr (MODE == kModeP) return M == 0u ? __builtin_inff() : __uint_as_float(M) * (1.f - 0x1p-14f);
+    return __uint_as_float(M);
+  }
+  static __device__ __forceinline__ uint32_t store(uint32_t M) { return MODE == kModeB ? M << 16 : M; }
+  static __device__ __forceinline__ uint32_t load(uint32_t w) { return MODE == kModeB ? w >> 16 : w; }
+  // a positive score's key, 0 below kMin
+  static __device__ __forceinline__ uint32_t key_or_0(float v) {
+    const uint32_t k = v > 0.f ? key(v) : 0u;
+    return k >= kMin ? k : 0u;
+  }
+  // whether a code of score v, key k can be the best where the best found so far is M
+  static __device__ __forceinline__ bool reaches(float v, uint32_t k, uint32_t M) {
+    if constexpr (MODE == kModeP) return M == 0u || v >= lo(M);
+    return k >= M;
+  }
+  // whether a code of score v is at the final best M (NN-P: close enough to be compared in fp64)
+  static __device__ __forceinline__ bool at(float v, uint32_t M) {
+    if constexpr (MODE == kModeP) return v >= lo(M);
+    return v > 0.f && key(v) == M;
+  }
+};
+
+// The fp32 codebook's exact score in fp64 (NN-P), products summed in coordinate order as the pack-time
+// rescan always has: x.c for c given as raw integers through coef(i).
+template <typename F>
+__device__ __forceinline__ double exact_score(const float *__restrict__ x, F coef) {
+  double d = 0.0;
+#pragma unroll 4
+  for (int i = 0; i < kDim; ++i) d = fma(static_cast<double>(x[i]), static_cast<double>(raw_value_f32(coef(i))), d);
+  return d;
+}
+
+// NN-P: a coordinate's part that its bf16 rounding drops.
+__device__ __forceinline__ float bf16_loss(float x) { return fabsf(x - bf16_bits_to_float(bf16_rne_bits(x))); }
+
+// S of representative word wb from fp32 coordinates (NN-P): as t3_dot below.
+__device__ __forceinline__ float t3_dot(const float *__restrict__ x, uint32_t wb) {
+  float S = 0.f;
+#pragma unroll
+  for (int d = 0; d < kDim; ++d) S = fmaf(__uint_as_float(__float_as_uint(x[d]) ^ ((wb >> d) & 1u) << 31), kT3S, S);
+  return S;
+}
 
 // S of representative word wb: sum over the 24 coordinates of (-s where wb has a 1, else +s) * x,
 // in coordinate order (exact products, fp32 sums); xr: the atom's 12 words of bf16 pairs.
@@ -594,12 +550,19 @@ __device__ __forceinline__ float t3_dot(const uint32_t *xr, uint32_t wb) {
 // roundings.  Record: ra = (h1 | h2 << 16, p1 | p2 << 8 | mg's bf16 bits rounded up << 16) in the type-3
 // half of the atom's key (t3_kernel reads it, then writes its result there), rb = (m3, eb + dl).
 // add() takes the coordinates in ascending order, record() gives the record.
+// NN-P: the same from the fp32 coordinates with the raw codebook's ratios (alpha = 4s, beta = 2s; scores in
+// units of s = bf16(s) instead of fp32(1/sqrt 8), which orders codes alike; fp32(3s) differs from 3 fp32(s)
+// by 2^-25, inside every margin); mg also covers what rounding x to the MFMA's bf16 operand drops.
+template <int MODE>
 struct T3Setup {
+  static constexpr float kA = MODE == kModeP ? kP3Alpha : kT3Alpha, kB = MODE == kModeP ? kP3Beta : kT3Beta;
+  float loss = 0.f;
   float m1 = -__builtin_inff(), m2 = -__builtin_inff(), m3 = -__builtin_inff(), x1 = 0.f, x2 = 0.f, ax = 0.f;
   uint32_t p1 = 0u, p2 = 1u;
   // coordinate i (ascending) of the atom
   __device__ __forceinline__ void add(float x, uint32_t i) {
-    const float t = fmaxf(-x * kT3Alpha, -x * kT3Beta);
+    const float t = fmaxf(-x * kA, -x * kB);
+    if constexpr (MODE == kModeP) loss += bf16_loss(x);
     const bool a1 = t > m1, a2 = t > m2;
     m3 = a2 ? m2 : fmaxf(m3, t);
     m2 = a1 ? m1 : (a2 ? t : m2);
@@ -611,7 +574,7 @@ struct T3Setup {
     ax += fabsf(x);
   }
   __device__ __forceinline__ void record(uint2 &ra, uint2 &rb) const {
-    const float a1 = -x1 * kT3Alpha, b1 = -x1 * kT3Beta, a2 = -x2 * kT3Alpha, b2 = -x2 * kT3Beta;
+    const float a1 = -x1 * kA, b1 = -x1 * kB, a2 = -x2 * kA, b2 = -x2 * kB;
     const float e00 = fmaxf(fmaxf(a1, a2), m3), e11 = fmaxf(fmaxf(b1, b2), m3);
     const float e01 = fmaxf(fmaxf(a1, b2), m3), e10 = fmaxf(fmaxf(b1, a2), m3);
     const float ebar = fmaxf((e00 + e11) * 0.5f, (e01 + e10) * 0.5f);
@@ -620,26 +583,31 @@ struct T3Setup {
     const uint32_t h1 = bf16_rne_bits(x1 + k1 / kT3S), h2 = bf16_rne_bits(x2 + k2 / kT3S);
     const float dl =
         fabsf((bf16_bits_to_float(h1) - x1) * kT3S - k1) + fabsf((bf16_bits_to_float(h2) - x2) * kT3S - k2);
-    const float mg = (ax * kT3S + fabsf(m1)) * 0x1p-14f;
+    float mg = (ax * kT3S + fabsf(m1)) * 0x1p-14f;
+    if constexpr (MODE == kModeP) mg += loss * kT3S;
     const uint32_t mgb = (__float_as_uint(mg) + 0xFFFFu) >> 16;  // (mg >= 0: rounded up)
     ra = make_uint2(h1 | h2 << 16, p1 | p2 << 8 | mgb << 16);
     rb = make_uint2(__float_as_uint(m3), __float_as_uint(ebar + dl));
   }
 };
 
-template <int AT>
-__global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict__ xb, int64_t n_atoms,
+template <int AT, int MODE>
+__global__ __launch_bounds__(kThreads, MODE == kModeP ? 3 : 4) void t3_kernel(const uint4 *__restrict__ xb,
+                                                         const float *__restrict__ xf, int64_t n_atoms,
                                                          const uint8_t *__restrict__ t3_tiles,
                                                          const uint32_t *__restrict__ t3_words,
                                                          const uint32_t *__restrict__ t3_rows,
                                                          uint4 *__restrict__ keys, const uint2 *__restrict__ rec,
                                                          int rows_by_sweep) {
+  typedef Sel<MODE> sel;
+  constexpr bool P = MODE == kModeP;
+  constexpr float kA = P ? kP3Alpha : kT3Alpha, kB = P ? kP3Beta : kT3Beta;
   constexpr int NA = AT * 16;  // atoms per wave
   static_assert(NA <= 128, "entry layout: 7 bits of atom");
   __shared__ __align__(16) uint8_t stg[2][kT3StageBytes];
   __shared__ uint32_t cand[kWaves][kT3Cap];  // atom | tile << 7 | quarter << 14 | output mask << 16 | done << 20
   __shared__ uint32_t surv[kWaves][kT3Surv];  // atom | pattern id << 7: words at or above the atom's running best
-  __shared__ uint32_t st_x[kWaves][NA];  // x at p1 | x at p2 << 16 (bf16 bits)
+  __shared__ uint32_t st_x[P ? 1 : kWaves][P ? 1 : NA];  // x at p1 | x at p2 << 16 (bf16 bits; NN-P reads the atom)
   __shared__ uint32_t st_m[kWaves][NA], st_r[kWaves][NA];
   __shared__ float st_t[kWaves][NA];    // lo(floor) less twice the margin: which signs of a word to evaluate
   __shared__ float st_m3[kWaves][NA];   // the third largest position term (the largest off p1, p2)
@@ -647,12 +615,15 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
   __shared__ uint8_t st_p[kWaves][NA][2];  // p1, p2: the positions of the two largest position terms
   __shared__ uint32_t surv_n[kWaves];
   __shared__ uint32_t st_ovf[kWaves][2];   // atoms (bits) whose survivor list lost an entry: rows by pass 2
+  __shared__ unsigned long long st_d[P ? kWaves : 1][P ? NA : 1];  // NN-P: bits of the best fp64 score
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, j = lane & 15;
   const int64_t wave_atom0 = static_cast<int64_t>(blockIdx.x) * (kWaves * NA) + static_cast<int64_t>(wave) * NA;
 
   if (lane < 2) st_ovf[wave][lane] = 0u;
   if (lane == 0) surv_n[wave] = 0u;
+  if constexpr (P)
+    for (int i = lane; i < NA; i += 64) st_d[wave][i] = 0ull;
   bf16x8 b[AT];
   float offs[AT];  // eb, the raised coordinate's rounding and the margin: thr = lo(floor) - offs
 #pragma unroll
@@ -678,8 +649,9 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
 #pragma unroll
         for (int k = 0; k < 4; ++k)
           if (static_cast<uint32_t>(k) == (e >> 1)) {
-            reinterpret_cast<uint16_t *>(&st_x[wave][at * 16 + j])[r] =
-                static_cast<uint16_t>((e & 1u) ? ww[k] >> 16 : ww[k] & 0xFFFFu);
+            if constexpr (!P)
+              reinterpret_cast<uint16_t *>(&st_x[wave][at * 16 + j])[r] =
+                  static_cast<uint16_t>((e & 1u) ? ww[k] >> 16 : ww[k] & 0xFFFFu);
             ww[k] = (e & 1u) ? (ww[k] & 0xFFFFu) | (h << 16) : (ww[k] & 0xFFFF0000u) | h;
           }
       }
@@ -702,7 +674,7 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
   for (int at = 0; at < AT; ++at) {
     const int64_t a = wave_atom0 + at * 16 + j;
     uint32_t m = 0u;
-    if (q == 0 && a < n_atoms) m = keys[a].z >> 16;
+    if (q == 0 && a < n_atoms) m = sel::load(keys[a].z);
     if (q == 0) {
       st_m[wave][at * 16 + j] = m;
       st_r[wave][at * 16 + j] = 0xFFFFFFFFu;
@@ -725,15 +697,57 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
     }
   };
 
+  // An atom's coordinates, read from global memory (L1 / L2) when its words are scored: the bf16 planes,
+  // NN-P the fp32 atom (an entry's atom is in range).
+  typedef typename std::conditional<P, const float *, const uint32_t *>::type atom_t;
+  auto atom_of = [&](int al) {
+    const int64_t a = min(wave_atom0 + al, n_atoms - 1);
+    if constexpr (P)
+      return static_cast<atom_t>(xf + a * kDim);
+    else
+      return reinterpret_cast<atom_t>(xb + a * 3);
+  };
   // The scores of word wr (sg: its complement) of atom al at its 24 positions, through f(p, t).
-  auto word_scores = [&](const uint32_t *xr, uint32_t wr, int sg, float D, auto f) {
+  auto word_scores = [&](atom_t xr, uint32_t wr, int sg, float D, auto f) {
     const uint32_t wb = sg ? wr ^ 0xFFFFFFu : wr;
     const float S = sg ? -D : D;
+    if constexpr (P) {
 #pragma unroll
-    for (int d = 0; d < 12; ++d) {
-      const uint32_t xx = xr[d];
-      f(2 * d, fmaf(-__uint_as_float(xx << 16), ((wb >> (2 * d)) & 1u) ? kT3Beta : kT3Alpha, S));
-      f(2 * d + 1, fmaf(-__uint_as_float(xx & 0xFFFF0000u), ((wb >> (2 * d + 1)) & 1u) ? kT3Beta : kT3Alpha, S));
+      for (int d = 0; d < kDim; ++d) f(d, fmaf(-xr[d], ((wb >> d) & 1u) ? kB : kA, S));
+    } else {
+#pragma unroll
+      for (int d = 0; d < 12; ++d) {
+        const uint32_t xx = xr[d];
+        f(2 * d, fmaf(-__uint_as_float(xx << 16), ((wb >> (2 * d)) & 1u) ? kB : kA, S));
+        f(2 * d + 1, fmaf(-__uint_as_float(xx & 0xFFFF0000u), ((wb >> (2 * d + 1)) & 1u) ? kB : kA, S));
+      }
+    }
+  };
+  // The rows of word wid (pattern id) of atom al at its final best M: the lowest into st_r.  NN-P takes two
+  // calls, the first (rows = false) for the best fp64 score of the positions that are close to M.
+  auto word_rows = [&](int al, atom_t xr, uint32_t wid, float D, uint32_t wr, bool rows) {
+    const uint32_t M = st_m[wave][al];
+    const int sg = wid >= static_cast<uint32_t>(kT3Reps) ? 1 : 0;
+    if constexpr (P) {
+      uint32_t near = 0u;
+      word_scores(xr, wr, sg, D, [&](int p, float t) { near |= (sel::at(t, M) ? 1u : 0u) << p; });
+      const uint32_t wb = sg ? wr ^ 0xFFFFFFu : wr;
+      for (; near != 0u; near &= near - 1u) {
+        const int p = __builtin_ctz(near);
+        const double d = exact_score(xr, [&](int i) { return i == p ? -3 : ((wb >> i) & 1u) ? -1 : 1; });
+        const unsigned long long db = static_cast<unsigned long long>(__double_as_longlong(d));
+        if (!rows) {
+          if (d > 0.0) atomicMax(&st_d[wave][al], db);
+        } else if (db == st_d[wave][al]) {
+          atomicMin(&st_r[wave][al], t3_rows[wid * kDim + p]);
+        }
+      }
+    } else {
+      uint32_t rmin = 0xFFFFFFFFu;
+      word_scores(xr, wr, sg, D, [&](int p, float t) {
+        if (sel::at(t, M)) rmin = min(rmin, t3_rows[wid * kDim + p]);
+      });
+      if (rmin != 0xFFFFFFFFu) atomicMin(&st_r[wave][al], rmin);
     }
   };
 
@@ -756,22 +770,27 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
         const int al = static_cast<int>(ce & 0x7Fu);
         const uint32_t rep = ((ce >> 7) & 0x7Fu) * kTileCodes + 4 * ((ce >> 14) & 3u) +
                              static_cast<uint32_t>(__builtin_ctz(mask));
-        // (the atom's coordinates from its bf16 planes in global memory; an entry's atom is in range)
-        const uint32_t *xr = reinterpret_cast<const uint32_t *>(xb + min(wave_atom0 + al, n_atoms - 1) * 3);
+        const atom_t xr = atom_of(al);
         const float tlo = st_t[wave][al];
         // the bound on the bonus of a word by its bits at p1, p2 (as at set-up)
         const uint32_t pa = st_p[wave][al][0], pb = st_p[wave][al][1];
         const float m3v = st_m3[wave][al];
-        const uint32_t xab = st_x[wave][al];
-        const float xa1 = __uint_as_float(xab << 16);
-        const float xa2 = __uint_as_float(xab & 0xFFFF0000u);
+        float xa1, xa2;
+        if constexpr (P) {
+          xa1 = xr[pa];
+          xa2 = xr[pb];
+        } else {
+          const uint32_t xab = st_x[wave][al];
+          xa1 = __uint_as_float(xab << 16);
+          xa2 = __uint_as_float(xab & 0xFFFF0000u);
+        }
         const uint32_t wr = t3_words[rep];
         const float D = t3_dot(xr, wr);
         const uint32_t ba = (wr >> pa) & 1u, bb = (wr >> pb) & 1u;
         // the representative (S = D) and its complement (S = -D, the other bits at p1, p2), each when its
         // S + e(word) can reach the floor; one of them per round (bit 20: the representative is done)
-        const float ew0 = fmaxf(fmaxf(-xa1 * (ba ? kT3Beta : kT3Alpha), -xa2 * (bb ? kT3Beta : kT3Alpha)), m3v);
-        const float ew1 = fmaxf(fmaxf(-xa1 * (ba ? kT3Alpha : kT3Beta), -xa2 * (bb ? kT3Alpha : kT3Beta)), m3v);
+        const float ew0 = fmaxf(fmaxf(-xa1 * (ba ? kB : kA), -xa2 * (bb ? kB : kA)), m3v);
+        const float ew1 = fmaxf(fmaxf(-xa1 * (ba ? kA : kB), -xa2 * (bb ? kA : kB)), m3v);
         const bool q0 = ((ce >> 20) & 1u) == 0u && D + ew0 >= tlo, q1 = -D + ew1 >= tlo;
         const uint32_t rest = mask & (mask - 1u);
         back = q0 && q1 ? ce | 1u << 20 : rest != 0u ? (ce & ~0x1F0000u) | rest << 16 : 0u;
@@ -781,10 +800,10 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
           if (pass == 1) {
             float best = -__builtin_inff();
             word_scores(xr, wr, sg, D, [&](int, float t) { best = fmaxf(best, t); });
-            const uint32_t bk = best > 0.f ? t3_bucket(best) : 0u;
-            if (bk >= 0x4000u) {
+            const uint32_t bk = sel::key_or_0(best);
+            if (bk != 0u) {
               const uint32_t old = atomicMax(&st_m[wave][al], bk);
-              if (bk >= old) {
+              if (sel::reaches(best, bk, old)) {
                 const uint32_t slot = atomicAdd(&surv_n[wave], 1u);
                 if (slot < static_cast<uint32_t>(kT3Surv))
                   surv[wave][slot] = static_cast<uint32_t>(al) | wid << 7;
@@ -793,12 +812,7 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
               }
             }
           } else {
-            const uint32_t M = st_m[wave][al];
-            uint32_t rmin = 0xFFFFFFFFu;
-            word_scores(xr, wr, sg, D, [&](int p, float t) {
-              if (t > 0.f && t3_bucket(t) == M) rmin = min(rmin, t3_rows[wid * kDim + p]);
-            });
-            if (rmin != 0xFFFFFFFFu) atomicMin(&st_r[wave][al], rmin);
+            word_rows(al, xr, wid, D, wr, !P || pass == 3);
           }
         }
       }
@@ -817,8 +831,9 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
   // bucket found so far.
   float thr[AT];
   auto set_thr = [&](int at, uint32_t mlow) {
-    mlow = max(mlow, max(mp[at], 0x4000u));
-    const float lo = __uint_as_float((mlow << 16) - 0x8000u);
+    mlow = max(mlow, mp[at]);
+    if constexpr (!P) mlow = max(mlow, sel::kMin);
+    const float lo = sel::lo(mlow);  // (NN-P: an atom without a pair key, as past the end, has no candidates)
     thr[at] = lo - offs[at];
     if (q == 0) st_t[wave][at * 16 + j] = lo - 2.f * st_mg[wave][at * 16 + j];
   };
@@ -841,7 +856,7 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
         const int al = at * 16 + j;
         const bool redo = rows_by_sweep != 0 || ((st_ovf[wave][al >> 5] >> (al & 31)) & 1u) != 0u;
         const uint32_t M = st_m[wave][al];
-        const float lo = redo && M >= 0x4000u ? __uint_as_float((M << 16) - 0x8000u) : __builtin_inff();
+        const float lo = redo && M >= sel::kMin ? sel::lo(M) : __builtin_inff();
         thr[at] = lo - offs[at];
         if (q == 0) st_t[wave][at * 16 + j] = lo - 2.f * st_mg[wave][at * 16 + j];
       }
@@ -884,7 +899,7 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
     // floor from the pair key leaves little for rising thresholds to gain, and fuller rounds keep the
     // lanes busy and the block's waves in step at the barriers (4.93 -> 4.64 ms against a flush at
     // every stage end holding 64 entries, config 4)
-    if (g == kT3Stages - 1 || g == 2 * kT3Stages - 1) flush(pass);
+    if (g % kT3Stages == kT3Stages - 1) flush(pass);
     if (pass == 1 && flushed) {
       // the thresholds rise with the best buckets found so far (this wave's own atoms: no barrier needed);
       // the buckets change only in a flush
@@ -896,7 +911,7 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
       // pass 1 done: pass 2 only if a survivor list lost entries (all waves agree), for those atoms
       // (rows_by_sweep: pass 2 for every atom -- the path an overflow takes, for its tests)
       if (__syncthreads_or(rows_by_sweep != 0 || (st_ovf[wave][0] | st_ovf[wave][1]) != 0u)) {
-        g_end = 2 * kT3Stages;
+        g_end = (P ? 3 : 2) * kT3Stages;  // (NN-P: the best fp64 score, then the rows)
         stage_copy(g + 1, buf ^ 1);  // buffer buf ^ 1 was last read in stage g - 1, before the barrier
         __syncthreads();
       }
@@ -908,22 +923,17 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
     // the lowest row at each atom's best bucket, from its survivors (every word that reached the final
     // best bucket was at or above the running best when it was evaluated); pass 2 gave the others'
     const int ns = static_cast<int>(min(surv_n[wave], static_cast<uint32_t>(kT3Surv)));
-    for (int i = lane; i < ns; i += 64) {
-      const uint32_t se = surv[wave][i];
-      const int al = static_cast<int>(se & 0x7Fu);
-      if (rows_by_sweep != 0 || ((st_ovf[wave][al >> 5] >> (al & 31)) & 1u) != 0u) continue;
-      const uint32_t wid = se >> 7;
-      const uint32_t M = st_m[wave][al];
-      const uint32_t *xr = reinterpret_cast<const uint32_t *>(xb + min(wave_atom0 + al, n_atoms - 1) * 3);
-      const uint32_t wr = t3_words[wid & (kT3Reps - 1)];
-      const int sg = wid >= static_cast<uint32_t>(kT3Reps) ? 1 : 0;
-      const float D = t3_dot(xr, wr);
-      uint32_t rmin = 0xFFFFFFFFu;
-      word_scores(xr, wr, sg, D, [&](int p, float t) {
-        if (t > 0.f && t3_bucket(t) == M) rmin = min(rmin, t3_rows[wid * kDim + p]);
-      });
-      if (rmin != 0xFFFFFFFFu) atomicMin(&st_r[wave][al], rmin);
-    }
+#pragma unroll 1
+    for (int r = P ? 0 : 1; r < 2; ++r)  // (NN-P: the best fp64 scores first; a wave's lists are its own)
+      for (int i = lane; i < ns; i += 64) {
+        const uint32_t se = surv[wave][i];
+        const int al = static_cast<int>(se & 0x7Fu);
+        if (rows_by_sweep != 0 || ((st_ovf[wave][al >> 5] >> (al & 31)) & 1u) != 0u) continue;
+        const uint32_t wid = se >> 7;
+        const atom_t xr = atom_of(al);
+        const uint32_t wr = t3_words[wid & (kT3Reps - 1)];
+        word_rows(al, xr, wid, t3_dot(xr, wr), wr, r == 1);
+      }
   }
   __syncthreads();
   if (q == 0) {
@@ -932,7 +942,8 @@ __global__ __launch_bounds__(kThreads, 4) void t3_kernel(const uint4 *__restrict
       const int64_t a = wave_atom0 + at * 16 + j;
       if (a >= n_atoms) continue;
       const uint32_t M = st_m[wave][at * 16 + j], r = st_r[wave][at * 16 + j];
-      *reinterpret_cast<uint2 *>(&keys[a]) = M >= 0x4000u && r != 0xFFFFFFFFu ? make_uint2(M << 16, r) : make_uint2(0u, 0u);
+      *reinterpret_cast<uint2 *>(&keys[a]) =
+          M >= sel::kMin && r != 0xFFFFFFFFu ? make_uint2(sel::store(M), r) : make_uint2(0u, 0u);
     }
   }
 }
@@ -990,6 +1001,7 @@ constexpr int kT2StageVecs = kT2StageBytes / 16;   // 384
 constexpr int kT2Cap = 384;                        // candidate entries per wave (4 bytes each)
 constexpr int kT2Surv = 256;                       // survivor entries per wave (4 bytes each)
 constexpr uint32_t kNonFinite = 0xFFFFFFFFu;       // pair key of an atom with a NaN or infinite coordinate
+constexpr uint32_t kRowMask = (1u << kRowBits) - 1u;
 constexpr float kC1 = 1.4140625f;                  // bf16(4s)
 constexpr float kC2 = 0.70703125f;                 // bf16(2s)
 static_assert(kT2StageVecs % 64 == 0, "octad stage splits into whole wave loads");
@@ -1006,6 +1018,18 @@ __device__ __forceinline__ uint32_t t2_load(const uint32_t *xr, uint2 pp, float 
     const uint32_t h = xh[p];
     xa[k] = __uint_as_float((h & 0x7FFFu) << 16);
     sg |= (h >> 15) << k;
+  }
+  return sg;
+}
+
+// The same from fp32 coordinates (NN-P).
+__device__ __forceinline__ uint32_t t2_load(const float *x, uint2 pp, float *xa) {
+  uint32_t sg = 0u;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float v = x[((k < 4 ? pp.x : pp.y) >> (8 * (k & 3))) & 0xFFu];
+    xa[k] = fabsf(v);
+    sg |= (__float_as_uint(v) >> 31) << k;
   }
   return sg;
 }
@@ -1039,62 +1063,74 @@ __device__ __forceinline__ uint32_t subset5_rank(const uint32_t *p) {
          p[4] * (p[4] - 1u) * (p[4] - 2u) * (p[4] - 3u) * (p[4] - 4u) / 120u;
 }
 
-// The lowest row among octad o's codes at bucket M: every flip set of the parity of sg whose flipped |x|
-// can fit in U - lo(M) is scored.
-__device__ __forceinline__ uint32_t t2_rows_at(const float *xa, uint32_t sg, uint32_t o, uint32_t M,
-                                               const uint32_t *__restrict__ t2_rows) {
+// The rows of octad o's codes at the best M, each through f(row, fp64 score of the fp32 codebook -- NN-P
+// only): every flip set of the parity of sg whose flipped |x| can fit in U - lo(M) is scored.
+template <int MODE, typename Fn>
+__device__ __forceinline__ void t2_rows_at(const float *xa, uint32_t sg, uint32_t o, uint32_t M,
+                                           const uint32_t *__restrict__ t2_rows, Fn f) {
+  typedef Sel<MODE> sel;
   float U = 0.f;
 #pragma unroll
   for (int k = 0; k < 8; ++k) U = fmaf(xa[k], kC2, U);
-  const float room = (U - __uint_as_float((M << 16) - 0x8000u)) + U * 0x1p-14f;
+  const float room = (U - sel::lo(M)) + U * 0x1p-14f;
   uint32_t C = 0u;
 #pragma unroll
   for (int k = 0; k < 8; ++k) C |= (xa[k] * (2.f * kC2) <= room ? 1u : 0u) << k;
   const uint32_t par = static_cast<uint32_t>(__popc(sg)) & 1u;
-  uint32_t rmin = 0xFFFFFFFFu;
   for (uint32_t F = C;; F = (F - 1u) & C) {  // every subset of C, the empty one last
     if ((static_cast<uint32_t>(__popc(F)) & 1u) == par) {
       const float S = t2_score(xa, F);
-      if (S > 0.f && t3_bucket(S) == M) rmin = min(rmin, t2_rows[o * 128u + ((sg ^ F) & 0x7Fu)]);
+      if (sel::at(S, M)) {
+        double d = 0.0;
+        if constexpr (MODE == kModeP) {
+          const double c = static_cast<double>(raw_value_f32(2));
+#pragma unroll
+          for (int k = 0; k < 8; ++k) d = fma(static_cast<double>(xa[k]), ((F >> k) & 1u) ? -c : c, d);
+        }
+        f(t2_rows[o * 128u + ((sg ^ F) & 0x7Fu)], d);
+      }
     }
     if (F == 0u) break;
   }
-  return rmin;
 }
 
-// The lowest row among the type-1 codes at bucket M of the atom whose bf16 coordinates are xr (v1: its
-// largest |x|): the positions i with c1 (|x_i| + v1) >= lo(M) - margin, every pair of them, all four signs.
-__device__ uint32_t t1_rows_at(const uint32_t *xr, float v1, uint32_t M, const uint32_t *__restrict__ t1_rows) {
-  const uint16_t *xh = reinterpret_cast<const uint16_t *>(xr);
-  const float lo = __uint_as_float((M << 16) - 0x8000u);
+// The rows of the type-1 codes at the best M of an atom (x(i): its coordinates; v1: its largest |x|), through
+// f as above: the positions i with c1 (|x_i| + v1) >= lo(M) - margin, every pair of them, all four signs.
+template <int MODE, typename X, typename F>
+__device__ void t1_rows_at(X x, float v1, uint32_t M, const uint32_t *__restrict__ t1_rows, F f) {
+  typedef Sel<MODE> sel;
   const float top = v1 * kC1;
-  const float need = lo - top - top * 0x1p-13f;
+  const float need = sel::lo(M) - top - top * 0x1p-13f;
   uint32_t C = 0u;
-  for (int i = 0; i < kDim; ++i) {
-    const float a = __uint_as_float((static_cast<uint32_t>(xh[i]) & 0x7FFFu) << 16);
-    C |= (a * kC1 >= need ? 1u : 0u) << i;
-  }
-  uint32_t rmin = 0xFFFFFFFFu;
+  for (int i = 0; i < kDim; ++i) C |= (fabsf(x(i)) * kC1 >= need ? 1u : 0u) << i;
   for (uint32_t ci = C; ci != 0u; ci &= ci - 1u) {
     const int i = __builtin_ctz(ci);
-    const float xi = __uint_as_float(static_cast<uint32_t>(xh[i]) << 16) * kC1;
+    const float xi = x(i) * kC1;
     for (uint32_t cj = ci & (ci - 1u); cj != 0u; cj &= cj - 1u) {
       const int j = __builtin_ctz(cj);
-      const float xj = __uint_as_float(static_cast<uint32_t>(xh[j]) << 16) * kC1;
+      const float xj = x(j) * kC1;
 #pragma unroll
       for (uint32_t e = 0; e < 4; ++e) {
         const float S = ((e & 1u) ? -xi : xi) + ((e & 2u) ? -xj : xj);
-        if (S > 0.f && t3_bucket(S) == M) rmin = min(rmin, t1_rows[(static_cast<uint32_t>(i) * kDim + j) * 4u + e]);
+        if (sel::at(S, M)) {
+          double d = 0.0;
+          if constexpr (MODE == kModeP) {
+            const double c = static_cast<double>(raw_value_f32(4));
+            d = fma(static_cast<double>(x(j)), (e & 2u) ? -c : c, static_cast<double>(x(i)) * ((e & 1u) ? -c : c));
+          }
+          f(t1_rows[(static_cast<uint32_t>(i) * kDim + j) * 4u + e], d);
+        }
       }
     }
   }
-  return rmin;
 }
 
 // LOAD: 0 the bf16 planes from prep_kernel (xb); 1 the fp32 atoms (src), rounded here and written to xb
 // for t3_kernel; 2 the same with the row scale applied first (src / sigma, as prep_kernel<true>).
-template <int AT, int LOAD>
-__global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb, const float *__restrict__ src,
+// NN-P (LOAD 1): the fp32 atoms are kept in LDS and every candidate is scored from them; only the MFMA's bound
+// on U uses the rounded ones (its margin covers what the rounding drops).
+template <int AT, int LOAD, int MODE>
+__global__ __launch_bounds__(kThreads, MODE == kModeP ? 3 : 4) void t12_kernel(uint4 *__restrict__ xb, const float *__restrict__ src,
                                                           const float *__restrict__ sigma, int64_t atoms_per_row,
                                                           int64_t n_atoms,
                                                           const uint8_t *__restrict__ t2_tiles,
@@ -1105,18 +1141,25 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
                                                           const uint32_t *__restrict__ t3_dec,
                                                           uint4 *__restrict__ keys, uint2 *__restrict__ rec,
                                                           int rows_by_sweep) {
+  typedef Sel<MODE> sel;
+  constexpr bool P = MODE == kModeP;
+  static_assert(!P || LOAD == 1, "NN-P scores fp32 atoms as they are");
   constexpr int NA = AT * 16;  // atoms per wave
   static_assert(NA <= 128 && NA <= 64, "entry layout: 7 bits of atom; one lane per atom at set-up");
   __shared__ __align__(16) uint8_t stg[2][kT2StageBytes];
-  __shared__ uint32_t cand[kWaves][kT2Cap];   // atom | tile << 7 | quarter << 13 | output mask << 16
-  __shared__ uint32_t surv[kWaves][kT2Surv];  // atom | octad << 7 | (bucket - 0x4000) << 17
-  __shared__ __align__(16) uint32_t xw[kWaves][NA][12];  // the atoms' bf16 coordinates (pairs)
+  constexpr int kCap = P ? 256 : kT2Cap;  // (NN-P: 53.6 KB in all, so that 3 blocks share a CU)
+  __shared__ uint32_t cand[kWaves][kCap];     // atom | tile << 7 | quarter << 13 | output mask << 16
+  __shared__ uint32_t surv[kWaves][kT2Surv];  // atom | octad << 7 | upper 15 bits of its key << 17
+  // the atoms' coordinates: bf16 pairs; NN-P: fp32 (25 words apart: a lane per atom, no bank conflicts)
+  constexpr int kXW = P ? 25 : 12;
+  __shared__ __align__(16) uint32_t xw[kWaves][NA][kXW];
   __shared__ uint32_t st_m[kWaves][NA], st_r[kWaves][NA];
   __shared__ uint32_t st_o[kWaves][NA];  // the octad of the atom's 5 largest |x| (scored at set-up)
   __shared__ uint32_t st_o2[kWaves][NA];  // the octad of its 4 largest and its 6th largest |x| (set-up)
   __shared__ uint32_t st_f[kWaves][NA];   // the type-3 floor: bucket of the best decoded type-3 code (or 0)
   __shared__ uint32_t surv_n[kWaves];
   __shared__ uint32_t st_ovf[kWaves][2];  // atoms (bits) whose survivor list lost an entry: rows by pass 2
+  __shared__ unsigned long long st_d[P ? kWaves : 1][P ? NA : 1];  // NN-P: bits of the best fp64 score
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, j = lane & 15;
   const int64_t wave_atom0 = static_cast<int64_t>(blockIdx.x) * (kWaves * NA) + static_cast<int64_t>(wave) * NA;
@@ -1125,16 +1168,21 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
   if (lane == 0) surv_n[wave] = 0u;
   bf16x8 b[AT];
   float mg[AT], v1[AT];
-  uint32_t m1b[AT];  // the best type-1 bucket (0 below 2.0)
+  uint32_t m1b[AT];  // the best type-1 key (0: below the origin's bound)
+  float s1v[P ? AT : 1];    // NN-P: its score
   uint32_t nonfinite = 0u;  // bit at: the atom has a NaN or infinite coordinate, or sum |x| overflows fp32
+                            // (NN-P: or sum |x| >= 2^96; pick_kernel scans every code for such an atom)
+  uint32_t snap = 0u;       // NN-P, bit at: |x| < 1e-8, the origin whatever the scores
+  typedef typename std::conditional<P, const float *, const uint32_t *>::type atom_t;
+  auto atom_of = [&](int al) { return reinterpret_cast<atom_t>(xw[wave][al]); };
 #pragma unroll
   for (int at = 0; at < AT; ++at) {
     const int64_t a = wave_atom0 + at * 16 + j;
     uint4 w = make_uint4(0u, 0u, 0u, 0u);
+    float v[8];
     if constexpr (LOAD == 0) {
       if (a < n_atoms && q < 3) w = xb[a * 3 + q];
     } else {
-      float v[8];
       load_coords8<LOAD == 2>(src, sigma, atoms_per_row, n_atoms, a, q, v);  // (zeros past the end, q == 3)
       w.x = bf16_rne_bits(v[0]) | (bf16_rne_bits(v[1]) << 16);
       w.y = bf16_rne_bits(v[2]) | (bf16_rne_bits(v[3]) << 16);
@@ -1142,18 +1190,25 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
       w.w = bf16_rne_bits(v[6]) | (bf16_rne_bits(v[7]) << 16);
       if (a < n_atoms && q < 3) xb[a * 3 + q] = w;
     }
-    if (q < 3) *reinterpret_cast<uint4 *>(&xw[wave][at * 16 + j][4 * q]) = w;
+    if constexpr (P) {
+      if (q < 3)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xw[wave][at * 16 + j][8 * q + e] = __float_as_uint(v[e]);
+    } else {
+      if (q < 3) *reinterpret_cast<uint4 *>(&xw[wave][at * 16 + j][4 * q]) = w;
+    }
     const uint4 wa = make_uint4(w.x & 0x7FFF7FFFu, w.y & 0x7FFF7FFFu, w.z & 0x7FFF7FFFu, w.w & 0x7FFF7FFFu);
     b[at] = __builtin_bit_cast(bf16x8, wa);
     // the two largest |x| and sum |x| over this lane's 8 coordinates, then over the atom's lanes
-    float t1 = 0.f, t2 = 0.f, ax = 0.f;
+    float t1 = 0.f, t2 = 0.f, ax = 0.f, loss = 0.f;
     const uint32_t ww[4] = {wa.x, wa.y, wa.z, wa.w};
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float v = __uint_as_float(e & 1 ? ww[e / 2] & 0xFFFF0000u : ww[e / 2] << 16);
-      t2 = fmaxf(t2, fminf(t1, v));
-      t1 = fmaxf(t1, v);
-      ax += v;
+      const float va = P ? fabsf(v[e]) : __uint_as_float(e & 1 ? ww[e / 2] & 0xFFFF0000u : ww[e / 2] << 16);
+      t2 = fmaxf(t2, fminf(t1, va));
+      t1 = fmaxf(t1, va);
+      ax += va;
+      if constexpr (P) loss += bf16_loss(va);
     }
 #pragma unroll
     for (int sh = 16; sh <= 32; sh <<= 1) {
@@ -1161,18 +1216,50 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
       t2 = fmaxf(fmaxf(t2, o2), fminf(t1, o1));
       t1 = fmaxf(t1, o1);
       ax += __shfl_xor(ax, sh, 64);
+      if constexpr (P) loss += __shfl_xor(loss, sh, 64);
+    }
+    if constexpr (P) {
+      // the origin rule (pack.py:174): |x|_2 < fp32(1e-8), in fp64 (only tiny atoms can meet it)
+      if (__ballot(ax < 1e-6f) != 0ull) {
+        double n2 = 0.0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) n2 = fma(static_cast<double>(v[e]), static_cast<double>(v[e]), n2);
+        n2 += __shfl_xor(n2, 16, 64);
+        n2 += __shfl_xor(n2, 32, 64);
+        snap |= (sqrt(n2) < static_cast<double>(__uint_as_float(kEpsBits)) ? 1u : 0u) << at;
+      }
     }
     // sum |x| is NaN or infinite exactly when a coordinate is (or the sum overflows fp32): such an atom
     // goes to the origin
-    nonfinite |= (ax <= 3.402823466e38f ? 0u : 1u) << at;
-    const float s1 = t1 * kC1 + t2 * kC1;  // exact products, one rounding
-    const uint32_t bk = s1 > 0.f ? t3_bucket(s1) : 0u;
-    m1b[at] = bk >= 0x4000u ? bk : 0u;
+    nonfinite |= (ax <= (P ? 0x1p96f : 3.402823466e38f) ? 0u : 1u) << at;
+    const float s1 = t1 * kC1 + t2 * kC1;  // (NN-B / NN-T: exact products, one rounding)
+    m1b[at] = sel::key_or_0(s1);
+    if constexpr (P) {
+      s1v[at] = s1;
+      if ((snap | nonfinite) >> at & 1u) m1b[at] = 0u;  // (such an atom has no candidates)
+    }
     v1[at] = t1;
-    // the margin for the MFMA's fp32 summation order of U
-    mg[at] = ax * kC2 * 0x1p-14f;
+    // the margin for the MFMA's fp32 summation order of U (NN-P: and for the rounding of its operand)
+    mg[at] = ax * kC2 * 0x1p-14f + (P ? loss * kC2 : 0.f);
   }
   for (int i = lane; i < NA; i += 64) st_r[wave][i] = 0xFFFFFFFFu;
+  if constexpr (P)
+    for (int i = lane; i < NA; i += 64) st_d[wave][i] = 0ull;
+  // a code of the atom at its final best, from the row walks below: its row into st_r, with its tie group above
+  // it in NN-T / NN-P (NN-P: first, with rows false, its fp64 score into st_d, then the row if that score is
+  // the best)
+  auto take = [&](int al, uint32_t row, double d, bool rows) {
+    if constexpr (P) {
+      const unsigned long long db = static_cast<unsigned long long>(__double_as_longlong(d));
+      if (!rows) {
+        if (d > 0.0) atomicMax(&st_d[wave][al], db);
+      } else if (db == st_d[wave][al]) {
+        atomicMin(&st_r[wave][al], row);
+      }
+    } else {
+      atomicMin(&st_r[wave][al], MODE == kModeB ? row & kRowMask : row);
+    }
+  };
 #pragma unroll
   for (int at = 0; at < AT; ++at)
     if (q == 0) st_m[wave][at * 16 + j] = m1b[at];
@@ -1190,6 +1277,9 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
     }
   };
 
+  // a key's upper 15 bits for the survivor entries (keys of positive scores stay below 0x7F80'0000; NN-B: the
+  // whole bucket)
+  auto upper15 = [](uint32_t k) { return MODE == kModeB ? k : k >> 16; };
   int cnt = 0;  // entries in this wave's candidate list (wave-uniform)
   // One flagged octad per lane per round (the list is worked as a stack: an entry with flagged octads left
   // goes back on it).  pass 1: the octad's best code -> st_m (atomic max), and the octad onto the survivor
@@ -1209,25 +1299,25 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
         const uint32_t o = ((ce >> 7) & 0x3Fu) * kTileCodes + 4u * ((ce >> 13) & 3u) +
                            static_cast<uint32_t>(__builtin_ctz(mask));
         // (padding slots: U = 0 unless the margin is not finite; the set-up octads: scored already)
-        if (o < static_cast<uint32_t>(kT2Octads) && (pass == 2 || (o != st_o[wave][al] && o != st_o2[wave][al]))) {
+        if (o < static_cast<uint32_t>(kT2Octads) && (pass != 1 || (o != st_o[wave][al] && o != st_o2[wave][al]))) {
           float xa[8];
-          const uint32_t sg = t2_load(xw[wave][al], t2_pos[o], xa);
+          const uint32_t sg = t2_load(atom_of(al), t2_pos[o], xa);
           if (pass == 1) {
             const float S = t2_best(xa, sg);
-            const uint32_t bk = S > 0.f ? t3_bucket(S) : 0u;
-            if (bk >= 0x4000u) {
+            const uint32_t bk = sel::key_or_0(S);
+            if (bk != 0u) {
               const uint32_t old = atomicMax(&st_m[wave][al], bk);
-              if (bk >= old) {
+              if (sel::reaches(S, bk, old)) {
                 const uint32_t slot = atomicAdd(&surv_n[wave], 1u);
                 if (slot < static_cast<uint32_t>(kT2Surv))
-                  surv[wave][slot] = static_cast<uint32_t>(al) | o << 7 | (bk - 0x4000u) << 17;
+                  surv[wave][slot] = static_cast<uint32_t>(al) | o << 7 | upper15(bk) << 17;
                 else
                   atomicOr(&st_ovf[wave][al >> 5], 1u << (al & 31));
               }
             }
           } else {
-            const uint32_t r = t2_rows_at(xa, sg, o, st_m[wave][al], t2_rows);
-            if (r != 0xFFFFFFFFu) atomicMin(&st_r[wave][al], r);
+            t2_rows_at<MODE>(xa, sg, o, st_m[wave][al], t2_rows,
+                             [&](uint32_t row, double d) { take(al, row, d, !P || pass == 3); });
           }
         }
       }
@@ -1252,7 +1342,11 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
       bool keep = false;
       if (i < n) {
         e = surv[wave][i];
-        keep = (e >> 17) + 0x4000u == st_m[wave][e & 0x7Fu];
+        const uint32_t M = st_m[wave][e & 0x7Fu];
+        if constexpr (P)
+          keep = (e >> 17) >= upper15(__float_as_uint(sel::lo(M)));  // (maybe a few more than can be the best)
+        else
+          keep = (e >> 17) == upper15(M);
       }
       const uint64_t msk = __ballot(keep);
       // (in place: every lane read its entry before any writes, and w + rank <= i)
@@ -1268,8 +1362,8 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
   // floor (2.0, the best type-1 bucket, the best octad bucket found so far) can win.
   float thr[AT];
   auto set_thr = [&](int at, uint32_t mlow) {
-    mlow = max(mlow, 0x4000u);
-    thr[at] = __uint_as_float((mlow << 16) - 0x8000u) - mg[at];
+    if constexpr (!P) mlow = max(mlow, sel::kMin);
+    thr[at] = sel::lo(mlow) - mg[at];  // (NN-P: an atom without a type-1 key has no candidates)
   };
 
   const int a_off = (q < 3 ? q : 0) * 256 + j * 16;
@@ -1283,14 +1377,19 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
   if (lane < NA) {
     const int al = lane;
     const uint16_t *xh = reinterpret_cast<const uint16_t *>(xw[wave][al]);
+    // coordinate i as the scores take it, and its bf16 bits (the floors need no more to order by)
+    auto coord = [&](int i) {
+      return P ? __uint_as_float(xw[wave][al][i]) : __uint_as_float(static_cast<uint32_t>(xh[i]) << 16);
+    };
+    auto half_bits = [&](int i) { return P ? xw[wave][al][i] >> 16 : static_cast<uint32_t>(xh[i]); };
     // the 6 largest keys |x| bits << 5 | position (bf16 magnitudes order as integers; distinct keys), kept
     // descending by a max / min pair per slot
     uint32_t tk[6] = {0u, 0u, 0u, 0u, 0u, 0u};
     uint32_t ysg = 0u, lk0 = 0xFFFFFFFFu, lk1 = 0xFFFFFFFFu;  // sign bits; the two smallest keys
-    T3Setup t3s;  // t3_kernel's set-up record
+    T3Setup<MODE> t3s;  // t3_kernel's set-up record
     for (int i = 0; i < kDim; ++i) {
-      const uint32_t h = xh[i];
-      t3s.add(__uint_as_float(h << 16), static_cast<uint32_t>(i));
+      const uint32_t h = half_bits(i);
+      t3s.add(coord(i), static_cast<uint32_t>(i));
       uint32_t k = (h & 0x7FFFu) << 5 | static_cast<uint32_t>(i);
       ysg |= (h >> 15) << i;
       lk1 = min(lk1, max(lk0, k));
@@ -1310,9 +1409,14 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
     // simulated: 0.58 -> 0.40 of the atom-tile x octad-tile steps hold a candidate), and t3_kernel
     // starts from it (0.24 -> 0.19 of its steps).
     {
-      uint32_t xr[12];
+      typename std::conditional<P, float, uint32_t>::type xr[P ? kDim : 12];
 #pragma unroll
-      for (int d = 0; d < 12; ++d) xr[d] = xw[wave][al][d];
+      for (int d = 0; d < (P ? kDim : 12); ++d) {
+        if constexpr (P)
+          xr[d] = coord(d);
+        else
+          xr[d] = xw[wave][al][d];
+      }
       uint32_t syn = 0u;
 #pragma unroll
       for (int jj = 0; jj < 12; ++jj) syn |= static_cast<uint32_t>(__popc(ysg & t3_dec[4096 + jj]) & 1) << jj;
@@ -1323,7 +1427,7 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
 #pragma unroll
       for (int c = 0; c < 6; ++c) {
         tpos[c] = tk[c] & 31u;
-        xp[c] = __uint_as_float(static_cast<uint32_t>(xh[tpos[c]]) << 16);
+        xp[c] = coord(static_cast<int>(tpos[c]));
       }
       float best = -__builtin_inff();
 #pragma unroll
@@ -1335,10 +1439,10 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
         const float D = t3_dot(xr, sg ? w ^ 0xFFFFFFu : w);
         const float S = sg ? -D : D;
 #pragma unroll
-        for (int c = 0; c < 6; ++c) best = fmaxf(best, fmaf(-xp[c], ((w >> tpos[c]) & 1u) ? kT3Beta : kT3Alpha, S));
+        for (int c = 0; c < 6; ++c)
+          best = fmaxf(best, fmaf(-xp[c], ((w >> tpos[c]) & 1u) ? T3Setup<MODE>::kB : T3Setup<MODE>::kA, S));
       }
-      const uint32_t f3 = best > 0.f ? t3_bucket(best) : 0u;
-      st_f[wave][al] = f3 >= 0x4000u ? f3 : 0u;
+      st_f[wave][al] = P && st_m[wave][al] == 0u ? 0u : sel::key_or_0(best);
     }
     {
       uint2 ra, rb;
@@ -1376,14 +1480,15 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
       const uint32_t o = r ? o2 : o1;
       if (r == 1 && o2 == o1) break;
       float xa[8];
-      const uint32_t sg = t2_load(xw[wave][al], t2_pos[o], xa);
+      const uint32_t sg = t2_load(atom_of(al), t2_pos[o], xa);
       const float S = t2_best(xa, sg);
-      const uint32_t bk = S > 0.f ? t3_bucket(S) : 0u;
-      if (bk >= 0x4000u && bk >= st_m[wave][al]) {
-        st_m[wave][al] = bk;
+      const uint32_t bk = sel::key_or_0(S), m = st_m[wave][al];
+      if (P && m == 0u) break;  // (no candidates: an atom past the end, the origin's, or pick_kernel's)
+      if (bk != 0u && sel::reaches(S, bk, m)) {
+        st_m[wave][al] = max(m, bk);
         const uint32_t slot = atomicAdd(&surv_n[wave], 1u);
         if (slot < static_cast<uint32_t>(kT2Surv))
-          surv[wave][slot] = static_cast<uint32_t>(al) | o << 7 | (bk - 0x4000u) << 17;
+          surv[wave][slot] = static_cast<uint32_t>(al) | o << 7 | upper15(bk) << 17;
         else
           atomicOr(&st_ovf[wave][al >> 5], 1u << (al & 31));
       }
@@ -1391,6 +1496,35 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
   }
 #pragma unroll
   for (int at = 0; at < AT; ++at) set_thr(at, max(st_m[wave][at * 16 + j], st_f[wave][at * 16 + j]));
+  // whether pair codes at M can be the answer beside the type-3 floor F
+  auto pair_can_win = [](uint32_t M, uint32_t F) {
+    if constexpr (P) return F == 0u || __uint_as_float(M) >= sel::lo(F);
+    return M >= F;
+  };
+  // the type-1 codes of each atom at its best (NN-B / NN-T: at exactly the best key), through take
+  auto type1 = [&](bool rows) {
+    if (q != 0) return;
+#pragma unroll
+    for (int at = 0; at < AT; ++at) {
+      const int al = at * 16 + j;
+      const uint32_t M = st_m[wave][al];
+      bool t1 = M >= sel::kMin && pair_can_win(M, st_f[wave][al]);
+      if constexpr (P)
+        t1 = t1 && s1v[at] >= sel::lo(M);
+      else
+        t1 = t1 && m1b[at] == M;
+      if (t1)
+        t1_rows_at<MODE>(
+            [&](int i) {
+              if constexpr (P)
+                return __uint_as_float(xw[wave][al][i]);
+              else
+                return __uint_as_float(static_cast<uint32_t>(reinterpret_cast<const uint16_t *>(xw[wave][al])[i])
+                                       << 16);
+            },
+            v1[at], M, t1_rows, [&](uint32_t row, double d) { take(al, row, d, rows); });
+    }
+  };
   int g_end = kT2Stages;
   for (int g = 0; g < g_end; ++g) {
     const int pass = 1 + g / kT2Stages, buf = g & 1;
@@ -1403,9 +1537,9 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
         const bool redo = rows_by_sweep != 0 || ((st_ovf[wave][al >> 5] >> (al & 31)) & 1u) != 0u;
         const uint32_t M = st_m[wave][al];
         // (an atom below its type-3 floor needs no pair rows)
-        thr[at] = redo && M >= 0x4000u && M >= st_f[wave][al] ? __uint_as_float((M << 16) - 0x8000u) - mg[at]
-                                                              : __builtin_inff();
+        thr[at] = redo && M >= sel::kMin && pair_can_win(M, st_f[wave][al]) ? sel::lo(M) - mg[at] : __builtin_inff();
       }
+      if constexpr (P) type1(false);  // (their fp64 scores, before pass 3 compares rows with the best)
     }
     const uint8_t *L = stg[buf] + a_off;
     const int tile0 = (g % kT2Stages) * kT2ST;
@@ -1427,7 +1561,7 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
         const bool hit = mx >= thr[at];
         const uint64_t msk = __ballot(hit);
         if (msk == 0ull) continue;
-        if (cnt > kT2Cap - 64) flush(pass);
+        if (cnt > kCap - 64) flush(pass);
         if (hit) {
           const bool h0 = c[at][0] >= thr[at], h1 = c[at][1] >= thr[at];
           const bool h2 = c[at][2] >= thr[at], h3 = c[at][3] >= thr[at];
@@ -1443,7 +1577,7 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
     // the list is evaluated when it is nearly full (in the tile loop) and at the end of each pass (with the
     // type-3 floor, evaluating at stage ends once 64 entries were listed measured 4% slower); the best
     // buckets change only then, so the survivors are compacted and the thresholds raised only after one
-    if (g == kT2Stages - 1 || g == 2 * kT2Stages - 1) flush(pass);
+    if (g % kT2Stages == kT2Stages - 1) flush(pass);
     if (pass == 1 && flushed) {
       compact();
       flushed = false;
@@ -1452,7 +1586,7 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
     }
     if (g == kT2Stages - 1) {
       if (__syncthreads_or(rows_by_sweep != 0 || (st_ovf[wave][0] | st_ovf[wave][1]) != 0u)) {
-        g_end = 2 * kT2Stages;
+        g_end = (P ? 3 : 2) * kT2Stages;  // (NN-P: the best fp64 score, then the rows)
         stage_copy(g + 1, buf ^ 1);  // buffer buf ^ 1 was last read in stage g - 1, before the barrier
         __syncthreads();
       }
@@ -1465,16 +1599,20 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
     // set-up octad left below it has no code at the final bucket, so it gives no row);
     // pass 2 gave the rows of the atoms whose list lost entries
     const int ns = static_cast<int>(min(surv_n[wave], static_cast<uint32_t>(kT2Surv)));
-    for (int i = lane; i < ns; i += 64) {
-      const uint32_t se = surv[wave][i];
-      const int al = static_cast<int>(se & 0x7Fu);
-      if (rows_by_sweep != 0 || ((st_ovf[wave][al >> 5] >> (al & 31)) & 1u) != 0u) continue;
-      if (st_m[wave][al] < st_f[wave][al]) continue;  // (below the type-3 floor: no pair rows needed)
-      const uint32_t o = (se >> 7) & 0x3FFu;
-      float xa[8];
-      const uint32_t sg = t2_load(xw[wave][al], t2_pos[o], xa);
-      const uint32_t r = t2_rows_at(xa, sg, o, st_m[wave][al], t2_rows);
-      if (r != 0xFFFFFFFFu) atomicMin(&st_r[wave][al], r);
+#pragma unroll 1
+    for (int r = P ? 0 : 1; r < 2; ++r) {  // (NN-P: the best fp64 scores first; a wave's lists are its own)
+      for (int i = lane; i < ns; i += 64) {
+        const uint32_t se = surv[wave][i];
+        const int al = static_cast<int>(se & 0x7Fu);
+        if (rows_by_sweep != 0 || ((st_ovf[wave][al >> 5] >> (al & 31)) & 1u) != 0u) continue;
+        if (!pair_can_win(st_m[wave][al], st_f[wave][al])) continue;  // (below the type-3 floor: no pair rows needed)
+        const uint32_t o = (se >> 7) & 0x3FFu;
+        float xa[8];
+        const uint32_t sg = t2_load(atom_of(al), t2_pos[o], xa);
+        t2_rows_at<MODE>(xa, sg, o, st_m[wave][al], t2_rows,
+                         [&](uint32_t row, double d) { take(al, row, d, r == 1); });
+      }
+      type1(r == 1);
     }
   }
   __syncthreads();
@@ -1483,37 +1621,33 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
     for (int at = 0; at < AT; ++at) {
       const int64_t a = wave_atom0 + at * 16 + j;
       if (a >= n_atoms) continue;
-      const uint32_t M = st_m[wave][at * 16 + j], F = st_f[wave][at * 16 + j];
-      uint32_t r = st_r[wave][at * 16 + j];
-      if (M >= 0x4000u && M >= F && m1b[at] == M) r = min(r, t1_rows_at(xw[wave][at * 16 + j], v1[at], M, t1_rows));
+      const uint32_t M = st_m[wave][at * 16 + j], F = st_f[wave][at * 16 + j], r = st_r[wave][at * 16 + j];
       // (a non-finite atom: the marker kNonFinite, which pick_kernel maps to the origin as the dense sweep
-      // does; as a pair bucket it gives t3_kernel a NaN threshold, hence no candidates.  An atom whose
-      // type-3 floor is above its best pair bucket: the floor without a row, as t3_kernel's starting best,
-      // which its type-3 best reaches, so pick_kernel takes t3_kernel's row)
+      // does; as a pair key it gives t3_kernel a NaN threshold, hence no candidates.  An atom whose
+      // type-3 floor is above its best pair key: the floor without a row, as t3_kernel's starting best,
+      // which its type-3 best reaches, so pick_kernel takes t3_kernel's row.  NN-P: the marker's second word
+      // is 0 for the origin, 1 for an atom that pick_kernel scans)
       reinterpret_cast<uint2 *>(&keys[a])[1] =
-          (nonfinite >> at) & 1u ? make_uint2(kNonFinite, 0u)
-          : F > M               ? make_uint2(F << 16, 0xFFFFFFFFu)
-          : M >= 0x4000u && r != 0xFFFFFFFFu ? make_uint2(M << 16, r)
-                                             : make_uint2(0u, 0u);
+          ((nonfinite | snap) >> at) & 1u ? make_uint2(kNonFinite, P && ((snap >> at) & 1u) == 0u ? 1u : 0u)
+          : !pair_can_win(M, F)           ? make_uint2(sel::store(F), 0xFFFFFFFFu)
+          : M >= sel::kMin && r != 0xFFFFFFFFu ? make_uint2(sel::store(M), r & kRowMask)
+                                               : make_uint2(0u, 0u);
     }
   }
 }
 
-// Resolve: per block 256 atoms.
-//   scan     thread per atom: its keys (type-3 region; pair region: NN-B the
-//            first and the last group at the best bucket, NN-T / NN-P the
-//            first group at the best |score|), the atom's coordinates into LDS
-//            (bf16 pairs; NN-P: fp32), and its candidates: (group, lane) of
-//            the keys' masks in the regions holding the overall best;
+// Resolve (the dense sweep): per block 256 atoms.
+//   scan     thread per atom: its keys (type-3 region; pair region: the first
+//            and the last group at the best bucket), the atom's coordinates
+//            into LDS (bf16 pairs), and its candidates: (group, lane) of the
+//            keys' masks in the regions holding the overall best;
 //   rounds   up to kRsPerRound candidates per atom per round, compacted into
 //            one LDS list by a block prefix sum and rescanned kRL = 4 lanes
 //            per candidate, lane t scoring the 4 codes of its quarter in
-//            tiles t, t+4, t+8, t+12 of the group (NN-B/T: value ids from
-//            sw_dq expanded to bf16 pairs, v_dot2_f32_bf16 = exact bf16
-//            products, fp32 sums; NN-P: the rows' raw int8 coordinates, fp64
-//            dot products of the fp32 atom with the fp32 codebook values,
-//            exact to 2^-48), combined by DPP quad moves and merged per atom;
-//   span     NN-B atoms whose best pair bucket is reached in a group that is
+//            tiles t, t+4, t+8, t+12 of the group (value ids from sw_dq
+//            expanded to bf16 pairs, v_dot2_f32_bf16 = exact bf16 products,
+//            fp32 sums), combined by DPP quad moves and merged per atom;
+//   span     atoms whose best pair bucket is reached in a group that is
 //            neither a first nor a last group of any lane (a lane with three or
 //            more such groups, or three or more pair slices at that bucket) and
 //            whose earliest such group holds no positive hit: the pair groups
@@ -1530,9 +1664,7 @@ __global__ __launch_bounds__(kThreads, 4) void t12_kernel(uint4 *__restrict__ xb
 //   the best bucket when that group has one, else somewhere up to the last --
 //   and otherwise the antipode of the highest negative hit, which lies in the
 //   last group.  The answer is the lower of that and the type-3 winner.
-// NN-T / NN-P compare exact scores, where two codes reach the same maximum
-// only on an exact fp32 tie (a near-tie); the first group's winner is taken.
-// NN-B falls back to the best rounded score, lowest row on ties, if the fp32
+// It falls back to the best rounded score, lowest row on ties, if the fp32
 // sums disagree with the sweep's bucket.  Then the int32 index and,
 // optionally, the packed 9-byte groups.
 constexpr int kRsPerRound = 4;
@@ -1540,11 +1672,6 @@ constexpr int kRsCap = 256 * kRsPerRound;
 constexpr int kRL = 4;         // rescan lanes per candidate (one quad)
 constexpr int kRT = kG / kRL;  // tiles per rescan lane
 constexpr uint32_t kNone = 0xFFFFFFFFu;
-
-template <int MODE>
-struct RsScore {  // per-candidate / per-atom running result
-  typedef typename std::conditional<MODE == kModeP, double, float>::type T;
-};
 
 // Sweep position (global, code granularity) of lane qq's code e in tile t of group g.
 __device__ __forceinline__ int sweep_pos(int g, int t, int qq, int e) { return (g * kG + t) * kTileCodes + 4 * qq + e; }
@@ -1570,38 +1697,32 @@ __device__ __forceinline__ void store_packed_block(const int32_t *ids, uint8_t *
   }
 }
 
-template <int MODE, bool FUSED>
 __global__ __launch_bounds__(256) void resolve_kernel(const uint4 *__restrict__ keys, int64_t n_atoms,
-                                                      const float *__restrict__ src,
-                                                      const float *__restrict__ sigma, int64_t atoms_per_row,
                                                       const uint4 *__restrict__ xb,
                                                       const uint32_t *__restrict__ sw_dq,
                                                       const uint32_t *__restrict__ sw_idx,
                                                       const uint32_t *__restrict__ sw_anti,
-                                                      const int8_t *__restrict__ cb_raw,
                                                       const uint8_t *__restrict__ sw_tiles,
                                                       const uint64_t *__restrict__ recs, int n_recs,
                                                       int64_t rec_stride,
                                                       int32_t *__restrict__ idx_out, uint8_t *__restrict__ packed_out) {
-  typedef typename RsScore<MODE>::T score_t;
-  constexpr bool B = MODE == kModeB;
-  constexpr int XW = MODE == kModeP ? kDim : 12;  // words of one atom's coordinates in LDS
-  constexpr int kP0 = kType3Tiles / kG;           // first global group of the pair region
+  constexpr int XW = 12;                 // words of one atom's coordinates in LDS
+  constexpr int kP0 = kType3Tiles / kG;  // first global group of the pair region
   __shared__ __align__(16) uint32_t xs[256 * XW];
   __shared__ uint32_t tmp[kRsPerRound * 256];     // per-thread candidates before compaction
   __shared__ uint32_t cand[kRsCap];               // atom | lane << 8 | pair << 10 | global group << 11
-  __shared__ score_t res_v[kRsCap];
+  __shared__ float res_v[kRsCap];
   __shared__ uint32_t res_c[kRsCap];              // row of the best (rounded) score
-  __shared__ uint32_t res_f0[B ? kRsCap : 1];     // NN-B: lowest row at bucket M (pair: positive hits)
-  __shared__ uint32_t res_f1[B ? kRsCap : 1];     // NN-B pair: lowest antipode row of negative hits
-  __shared__ uint32_t Ms[256];                    // per atom: the best bucket (NN-B)
+  __shared__ uint32_t res_f0[kRsCap];             // lowest row at bucket M (pair: positive hits)
+  __shared__ uint32_t res_f1[kRsCap];             // pair: lowest antipode row of negative hits
+  __shared__ uint32_t Ms[256];                    // per atom: the best bucket
   __shared__ int wave_sum[4];
   __shared__ int32_t ids[256];
   __shared__ __align__(16) uint8_t bytes[64 * 9];
-  __shared__ uint32_t span_list[B ? 256 : 1];      // NN-B: atoms needing the span rescan, their first code,
-  __shared__ uint32_t span_lo[B ? 256 : 1];        // code count, running offset and lowest positive-hit row
-  __shared__ uint32_t span_cnt[B ? 256 : 1];
-  __shared__ uint32_t span_min[B ? 256 : 1];
+  __shared__ uint32_t span_list[256];             // atoms needing the span rescan, their first code,
+  __shared__ uint32_t span_lo[256];        // code count, running offset and lowest positive-hit row
+  __shared__ uint32_t span_cnt[256];
+  __shared__ uint32_t span_min[256];
   __shared__ uint32_t span_n;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1611,17 +1732,16 @@ __global__ __launch_bounds__(256) void resolve_kernel(const uint4 *__restrict__ 
 
   // ---- scan: keys, coordinates, origin rules ----
   // candidate groups (global) and lane masks: [0] type-3; [1..4] pair groups:
-  // NN-B the first and last group of the pair record with the earliest first
+  // the first and last group of the pair record with the earliest first
   // group and of the one with the latest last group (the records of the pair
-  // slices at the best pair bucket, in slice = group order); NN-T / NN-P the
-  // first group at the best |score| in [1]
+  // slices at the best pair bucket, in slice = group order)
   uint32_t M = 0, grp[5] = {0u, 0u, 0u, 0u, 0u}, lanes[5] = {0u, 0u, 0u, 0u, 0u};
-  uint32_t span_g0 = 0, span_g1 = 0;  // NN-B: pair groups (span_g0, span_g1] to rescan for positive hits
+  uint32_t span_g0 = 0, span_g1 = 0;  // pair groups (span_g0, span_g1] to rescan for positive hits
   bool many = false;
   bool active = false;
   if (a < n_atoms) {
     const uint4 k = keys[a];
-    if constexpr (B) {
+    {
       const uint32_t MT = k.x >> 16;
       uint32_t MP = 0u;
       uint64_t rF = 0ull, rL = 0ull;
@@ -1667,50 +1787,25 @@ __global__ __launch_bounds__(256) void resolve_kernel(const uint4 *__restrict__ 
       } else {
         many = false;
       }
-    } else {
-      const uint64_t kt = (static_cast<uint64_t>(k.y) << 32) | k.x, kp = (static_cast<uint64_t>(k.w) << 32) | k.z;
-      const uint32_t MT = static_cast<uint32_t>(kt >> 32), MP = static_cast<uint32_t>(kp >> 32);
-      M = max(MT, MP);
-      if (kt != 0ull && MT == M) {
-        grp[0] = 0x3FFu - static_cast<uint32_t>((kt >> 4) & 0x3FFu);
-        lanes[0] = static_cast<uint32_t>(kt & 0xFu);
-      }
-      if (kp != 0ull && MP == M) {
-        grp[1] = kP0 + 0x3FFu - static_cast<uint32_t>((kp >> 4) & 0x3FFu);
-        lanes[1] = static_cast<uint32_t>(kp & 0xFu);
-      }
     }
-    double nrm2 = 0.0;
-    bool nonfinite = false;  // NN-B / NN-T: a NaN or infinite coordinate (its index is the origin)
+    bool nonfinite = false;  // a NaN or infinite coordinate (its index is the origin)
 #pragma unroll
     for (int qq = 0; qq < 3; ++qq) {
-      if constexpr (MODE == kModeP) {
-        float v[8];
-        load_coords8<FUSED>(src, sigma, atoms_per_row, n_atoms, a, qq, v);
+      const uint4 w = xb[a * 3 + qq];  // bf16 pairs from prep_kernel
+      *reinterpret_cast<uint4 *>(xs + tid * XW + 4 * qq) = w;
+      const uint32_t wv[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          xs[tid * XW + 8 * qq + e] = __float_as_uint(v[e]);
-          nrm2 = fma(static_cast<double>(v[e]), static_cast<double>(v[e]), nrm2);
-        }
-      } else {
-        const uint4 w = xb[a * 3 + qq];  // bf16 pairs from prep_kernel
-        *reinterpret_cast<uint4 *>(xs + tid * XW + 4 * qq) = w;
-        const uint32_t wv[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          nonfinite |= (wv[k] & 0x7F80u) == 0x7F80u || (wv[k] & 0x7F800000u) == 0x7F800000u;
-      }
+      for (int k = 0; k < 4; ++k)
+        nonfinite |= (wv[k] & 0x7F80u) == 0x7F80u || (wv[k] & 0x7F800000u) == 0x7F800000u;
     }
-    // NN-P's origin rule (pack.py:174): |x|_2 < fp32(1e-8); no scan needed
-    const bool p_snap = MODE == kModeP && sqrt(nrm2) < static_cast<double>(__uint_as_float(kEpsBits));
-    active = M != 0u && (lanes[0] | lanes[1] | lanes[2] | lanes[3] | lanes[4]) != 0u && !p_snap && !nonfinite;
+    active = M != 0u && (lanes[0] | lanes[1] | lanes[2] | lanes[3] | lanes[4]) != 0u && !nonfinite;
   }
   Ms[tid] = M;
 
   // per-atom merge state
-  uint32_t fT = kNone, fPpos = kNone, fPneg = kNone;  // NN-B
-  bool pos_first = false;  // NN-B: a positive hit in the earliest pair group (then the lowest pair row is known)
-  score_t best_v = -__builtin_inf();
+  uint32_t fT = kNone, fPpos = kNone, fPneg = kNone;
+  bool pos_first = false;  // a positive hit in the earliest pair group (then the lowest pair row is known)
+  float best_v = -__builtin_inff();
   uint32_t best_code = kNone;
   int next = 0;  // next candidate slot: 4 * kind + lane
   const uint4 bt = bf16_value_table();
@@ -1757,9 +1852,9 @@ __global__ __launch_bounds__(256) void resolve_kernel(const uint4 *__restrict__ 
     // (rising for type-3 codes and representatives, falling for antipodes,
     // and every representative row is below every antipode row), so a lane
     // tracks positions and the candidate looks its rows up once, after the
-    // reduction: NN-B the lowest position at bucket M (type-3: any score;
+    // reduction: the lowest position at bucket M (type-3: any score;
     // pair: positive) and the highest pair position at bucket M with a
-    // negative score; all modes the best value and a preference that orders
+    // negative score; and the best value and a preference that orders
     // equal values the way their rows order and encodes the position
     // (type-3: kPrefBase - pos; pair, positive: 2^31 + kPrefBase - pos; pair,
     // negative: pos; 0: nothing compared).
@@ -1774,32 +1869,8 @@ __global__ __launch_bounds__(256) void resolve_kernel(const uint4 *__restrict__ 
       int pos0[kRT];
 #pragma unroll
       for (int j = 0; j < kRT; ++j) pos0[j] = sweep_pos(g, t + kRL * j, qq, 0);
-      score_t sc[kRT][4];
-      if constexpr (MODE == kModeP) {
-        uint32_t rows[kRT][4];
-#pragma unroll
-        for (int j = 0; j < kRT; ++j)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) rows[j][e] = sw_idx[pos0[j] + e];
-        double xd[kDim];
-#pragma unroll
-        for (int k = 0; k < kDim; ++k) xd[k] = static_cast<double>(__uint_as_float(xs[al * XW + k]));
-#pragma unroll
-        for (int j = 0; j < kRT; ++j)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const uint2 *cr = reinterpret_cast<const uint2 *>(cb_raw + static_cast<size_t>(rows[j][e]) * kDim);
-            const uint2 r0 = cr[0], r1 = cr[1], r2 = cr[2];
-            const uint32_t w6[6] = {r0.x, r0.y, r1.x, r1.y, r2.x, r2.y};
-            double sv = 0.0;
-#pragma unroll
-            for (int k = 0; k < kDim; ++k) {
-              const int r = static_cast<int32_t>(w6[k / 4] << (24 - 8 * (k % 4))) >> 24;
-              sv = fma(xd[k], static_cast<double>(raw_value_f32(r)), sv);
-            }
-            sc[j][e] = sv;
-          }
-      } else {
+      float sc[kRT][4];
+      {
         uint32_t idw[kRT][12];
 #pragma unroll
         for (int j = 0; j < kRT; ++j) {
@@ -1835,21 +1906,19 @@ __global__ __launch_bounds__(256) void resolve_kernel(const uint4 *__restrict__ 
       }
       const uint32_t Mk = Ms[al];
       uint32_t p_lo = kNone, bpref = 0u, p_hi = 0u;  // p_hi: highest negative-hit position + 1
-      score_t bv = -__builtin_inf();
+      float bv = -__builtin_inff();
 #pragma unroll
       for (int j = 0; j < kRT; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const uint32_t pos = static_cast<uint32_t>(pos0[j] + e);
-          const bool neg = pair && sc[j][e] < static_cast<score_t>(0);
-          score_t v = neg ? -sc[j][e] : sc[j][e];
+          const bool neg = pair && sc[j][e] < 0.f;
+          float v = neg ? -sc[j][e] : sc[j][e];
           const uint32_t pref = !pair ? kPrefBase - pos : neg ? pos : 0x80000000u + kPrefBase - pos;
-          if constexpr (B) {
-            const uint32_t bk = bf16_rne_bits(static_cast<float>(sc[j][e]));
-            if (bk == Mk) p_lo = min(p_lo, pos);
-            if (pair && bk == (Mk | 0x8000u)) p_hi = max(p_hi, pos + 1u);
-            v = bf16_bits_to_float(bf16_rne_bits(static_cast<float>(v)));
-          }
+          const uint32_t bk = bf16_rne_bits(sc[j][e]);
+          if (bk == Mk) p_lo = min(p_lo, pos);
+          if (pair && bk == (Mk | 0x8000u)) p_hi = max(p_hi, pos + 1u);
+          v = bf16_bits_to_float(bf16_rne_bits(v));
           if (v > bv || (v == bv && pref > bpref)) {
             bv = v;
             bpref = pref;
@@ -1859,23 +1928,13 @@ __global__ __launch_bounds__(256) void resolve_kernel(const uint4 *__restrict__ 
       auto step = [&](auto ctrl) {
         constexpr int C = decltype(ctrl)::value;
         const uint32_t opref = dpp_u32<C>(bpref);
-        score_t ov;
-        if constexpr (MODE == kModeP) {
-          const uint64_t b = static_cast<uint64_t>(__double_as_longlong(bv));
-          const uint64_t o = static_cast<uint64_t>(dpp_u32<C>(static_cast<uint32_t>(b))) |
-                             static_cast<uint64_t>(dpp_u32<C>(static_cast<uint32_t>(b >> 32))) << 32;
-          ov = __longlong_as_double(static_cast<long long>(o));
-        } else {
-          ov = dpp_f32<C>(bv);
-        }
+        const float ov = dpp_f32<C>(bv);
         if (ov > bv || (ov == bv && opref > bpref)) {
           bv = ov;
           bpref = opref;
         }
-        if constexpr (B) {
-          p_lo = min(p_lo, dpp_u32<C>(p_lo));
-          p_hi = max(p_hi, dpp_u32<C>(p_hi));
-        }
+        p_lo = min(p_lo, dpp_u32<C>(p_lo));
+        p_hi = max(p_hi, dpp_u32<C>(p_hi));
       };
       step(std::integral_constant<int, 0xB1>{});
       step(std::integral_constant<int, 0x4E>{});
@@ -1883,37 +1942,33 @@ __global__ __launch_bounds__(256) void resolve_kernel(const uint4 *__restrict__ 
         const uint32_t bpos = !pair ? kPrefBase - bpref : bpref < 0x80000000u ? bpref : 0x80000000u + kPrefBase - bpref;
         res_v[c] = bv;
         res_c[c] = bpref == 0u ? kNone : pair && bpref < 0x80000000u ? sw_anti[bpos - kType3Codes] : sw_idx[bpos];
-        if constexpr (B) {
-          res_f0[c] = p_lo == kNone ? kNone : sw_idx[p_lo];
-          res_f1[c] = p_hi == 0u ? kNone : sw_anti[p_hi - 1u - kType3Codes];
-        }
+        res_f0[c] = p_lo == kNone ? kNone : sw_idx[p_lo];
+        res_f1[c] = p_hi == 0u ? kNone : sw_anti[p_hi - 1u - kType3Codes];
       }
     }
     __syncthreads();
 
     // ---- merge this thread's candidates ----
     for (int i = 0; i < nm; ++i) {
-      const score_t v = res_v[off + i];
+      const float v = res_v[off + i];
       const uint32_t code = res_c[off + i];
       if (v > best_v || (v == best_v && code < best_code)) {
         best_v = v;
         best_code = code;
       }
-      if constexpr (B) {
-        if (((cand[off + i] >> 10) & 1u) == 0u) {
-          fT = min(fT, res_f0[off + i]);
-        } else {
-          fPpos = min(fPpos, res_f0[off + i]);
-          fPneg = min(fPneg, res_f1[off + i]);
-          pos_first |= (cand[off + i] >> 11) == span_g0 && res_f0[off + i] != kNone;
-        }
+      if (((cand[off + i] >> 10) & 1u) == 0u) {
+        fT = min(fT, res_f0[off + i]);
+      } else {
+        fPpos = min(fPpos, res_f0[off + i]);
+        fPneg = min(fPneg, res_f1[off + i]);
+        pos_first |= (cand[off + i] >> 11) == span_g0 && res_f0[off + i] != kNone;
       }
     }
     if (!__syncthreads_or(more)) break;
   }
 
-  uint32_t fS = kNone;  // NN-B: the lowest winning pair-code row
-  if constexpr (B) {
+  uint32_t fS = kNone;  // the lowest winning pair-code row
+  {
     // ---- span rescan for atoms whose first pair group has only negative hits ----
     // (rare: some group at the best pair bucket is not among the candidates)
     // The block steps through the span in ascending chunks of kSpanChunk
@@ -1976,21 +2031,11 @@ __global__ __launch_bounds__(256) void resolve_kernel(const uint4 *__restrict__ 
 
   int32_t id = 0;
   if (active) {
-    bool snap;
-    uint32_t row;
-    if (MODE == kModeP) {
-      row = best_code;
-      snap = best_code == kNone;  // non-finite atom: no score compared
-    } else if (B) {
-      const uint32_t found = min(fT, fS);
-      const uint32_t bucket = found != kNone ? M : (__float_as_uint(static_cast<float>(best_v)) >> 16);
-      row = found != kNone ? found : best_code;
-      // bf16 max below 2.0
-      snap = (found == kNone && !(best_v > 0.f)) || bucket < 0x4000u;
-    } else {
-      row = best_code;
-      snap = !(2.0f * static_cast<float>(best_v) >= __uint_as_float(kCSqNormBits));
-    }
+    const uint32_t found = min(fT, fS);
+    const uint32_t bucket = found != kNone ? M : (__float_as_uint(best_v) >> 16);
+    const uint32_t row = found != kNone ? found : best_code;
+    // bf16 max below 2.0
+    const bool snap = (found == kNone && !(best_v > 0.f)) || bucket < 0x4000u;
     id = snap || row == kNone ? 0 : static_cast<int32_t>(row);
   }
   if (idx_out && a < n_atoms) idx_out[a] = id;
@@ -2000,29 +2045,94 @@ __global__ __launch_bounds__(256) void resolve_kernel(const uint4 *__restrict__ 
   store_packed_block(ids, bytes, a0, n_atoms, packed_out, tid);
 }
 
-// NN-B with the structured scorers: the higher of the pair key (t12_kernel)
-// and the type-3 key (t3_kernel), the lower row on equal buckets, the origin
-// when neither reaches 2.0 or the atom has a NaN or infinite coordinate; then
+// The fp32 codebook row's exact score of fp32 atom x (fp64, as exact_score).
+__device__ __forceinline__ double row_score(const float *__restrict__ x, const int8_t *__restrict__ cb_raw,
+                                            uint32_t row) {
+  const int8_t *c = cb_raw + static_cast<size_t>(row) * kDim;
+  return exact_score(x, [&](int i) { return static_cast<int>(c[i]); });
+}
+
+// The structured scorers' answer: the higher of the pair key (t12_kernel) and
+// the type-3 key (t3_kernel), the lower row on equal keys, the origin when
+// neither reaches its bound or the atom has a NaN or infinite coordinate; then
 // the int32 index and, optionally, the packed 9-byte groups.
+// NN-P (x: the atoms): two keys closer than their fp32 sums can be trusted are
+// compared by the rows' fp64 scores, and the block scans all codes in fp64 for
+// an atom that the scorers left out (an infinite or NaN coordinate, or one so
+// large that an fp32 score could overflow): the lowest row of the highest
+// score that is a number, else the origin.
+template <int MODE>
 __global__ __launch_bounds__(256) void pick_kernel(const uint4 *__restrict__ keys, int64_t n_atoms,
+                                                   const float *__restrict__ x, const int8_t *__restrict__ cb_raw,
                                                    int32_t *__restrict__ idx_out, uint8_t *__restrict__ packed_out) {
+  typedef Sel<MODE> sel;
+  constexpr bool P = MODE == kModeP;
   __shared__ int32_t ids[256];
   __shared__ __align__(16) uint8_t bytes[64 * 9];
   const int tid = threadIdx.x;
   const int64_t a0 = static_cast<int64_t>(blockIdx.x) * 256;
   const int64_t a = a0 + tid;
   int32_t id = 0;
+  bool scan = false;
   if (a < n_atoms) {
     const uint4 k = keys[a];
-    const uint32_t M3 = k.x >> 16, M2 = k.z >> 16, M = max(M2, M3);
+    const uint32_t M3 = sel::load(k.x), M2 = sel::load(k.z), M = max(M2, M3);
     uint32_t row = kNone;
-    if (M >= 0x4000u && k.z != kNonFinite) {  // (a non-finite atom: the origin)
-      if (M3 == M) row = k.y;
-      if (M2 == M) row = min(row, k.w);
+    if (M >= sel::kMin && k.z != kNonFinite) {  // (a non-finite atom: the origin)
+      bool t3 = M3 == M, t2 = M2 == M;
+      if constexpr (P) {
+        // (a pair key without a row is a type-3 score that t3_kernel reached too)
+        if (M3 != 0u && M2 != 0u && k.w != kNone && sel::at(__uint_as_float(min(M2, M3)), M)) {
+          const double d3 = row_score(x + a * kDim, cb_raw, k.y), d2 = row_score(x + a * kDim, cb_raw, k.w);
+          t3 = d3 >= d2;
+          t2 = d2 >= d3;
+        }
+      }
+      if (t3) row = k.y;
+      if (t2) row = min(row, k.w);
     }
     id = row == kNone ? 0 : static_cast<int32_t>(row);
-    if (idx_out) idx_out[a] = id;
+    if constexpr (P) scan = k.z == kNonFinite && k.w == 1u;
   }
+  if constexpr (P) {
+    if (__syncthreads_or(scan)) {
+      __shared__ double best_d[256];
+      __shared__ uint32_t best_r[256];
+      ids[tid] = scan ? 1 : 0;
+      __syncthreads();
+      for (int al = 0; al < 256; ++al) {
+        if (ids[al] == 0) continue;  // (block-uniform)
+        const float *xa = x + (a0 + al) * kDim;
+        double bd = -__builtin_inf();
+        uint32_t br = 0u;
+        for (uint32_t r = 1u + static_cast<uint32_t>(tid); r <= static_cast<uint32_t>(kKissing); r += 256u) {
+          const double d = row_score(xa, cb_raw, r);
+          if (d > bd) {
+            bd = d;
+            br = r;
+          }
+        }
+        best_d[tid] = bd;
+        best_r[tid] = br;
+        __syncthreads();
+        for (int w = 128; w > 0; w >>= 1) {
+          if (tid < w) {
+            const double od = best_d[tid + w];
+            const uint32_t orow = best_r[tid + w];
+            if (od > best_d[tid] || (od == best_d[tid] && orow < best_r[tid])) {
+              best_d[tid] = od;
+              best_r[tid] = orow;
+            }
+          }
+          __syncthreads();
+        }
+        if (tid == al) id = static_cast<int32_t>(best_r[0]);
+        __syncthreads();
+      }
+      __syncthreads();  // (ids is written again below)
+    }
+  }
+  if (idx_out && a < n_atoms) idx_out[a] = id;
   if (!packed_out) return;
   ids[tid] = id;
   __syncthreads();
@@ -2093,114 +2203,134 @@ size_t recs_bytes(int64_t n_atoms) {
   return (static_cast<size_t>(n_atoms) * static_cast<size_t>(n_slices) * 8 + 255) & ~static_cast<size_t>(255);
 }
 
-// t3_kernel: atom tiles per wave by launch size, so small launches still fill the chip.
-int t3_launch(const uint4 *xb, int64_t n_atoms, const DeviceTables *tab, uint4 *keys, const uint2 *rec,
-              hipStream_t s, int rows_by_sweep) {
-  // 4 atom tiles per wave from 131,072 atoms, 2 from 98,304, else 1 (measured per launch size: 55,296
-  // atoms take 35 + 42 us in t12 + t3 at 1 tile, 39 + 47 at 2; from 165,888 atoms 4 tiles are fastest).
-  // At 4 tiles: 40 KB of LDS (16-tile stages) and 128 VGPRs, 4 blocks (16 waves) per CU, which the
-  // kernel's stalls need (8 tiles per wave at 2 blocks per CU was 30% slower); the representative words
-  // and, when a list is worked, the atoms' coordinates are read from global memory (L1 / L2) to leave
-  // the LDS to the stages and lists.
-  const int AT = n_atoms >= 131072 ? 4 : n_atoms >= 98304 ? 2 : 1;
+// Atom tiles per wave of the structured scorers by launch size, so small launches still fill the chip: 4
+// from 131,072 atoms, 2 from 98,304, else 1 (measured per launch size, NN-B: 55,296 atoms take 35 + 42 us in
+// t12 + t3 at 1 tile, 39 + 47 at 2; from 165,888 atoms 4 tiles are fastest).
+// At 4 tiles: 40 KB of LDS (t3: 16-tile stages; t12 38 KB) and 128 VGPRs, 4 blocks (16 waves) per CU, which
+// the kernels' stalls need (8 tiles per wave at 2 blocks per CU was 30% slower); the representative words
+// and, when a list is worked, the atoms' coordinates are read from global memory (L1 / L2) to leave
+// the LDS to the stages and lists.  (NN-P's t12_kernel: 53 KB, 3 blocks.)
+int scorer_tiles(int64_t n_atoms) { return n_atoms >= 131072 ? 4 : n_atoms >= 98304 ? 2 : 1; }
+
+int scorer_grid(int64_t n_atoms, int AT, dim3 *g) {
   const int64_t per_block = static_cast<int64_t>(kWaves) * AT * 16;
   const int64_t blocks = (n_atoms + per_block - 1) / per_block;
   if (blocks > 0x7FFFFFFFll) return fail(PLX_EINVAL, "quantize: %lld atoms exceed one launch", static_cast<long long>(n_atoms));
-  const dim3 g(static_cast<unsigned>(blocks));
+  *g = dim3(static_cast<unsigned>(blocks));
+  return PLX_OK;
+}
+
+template <int MODE>
+int t3_launch(const uint4 *xb, const float *xf, int64_t n_atoms, const DeviceTables *tab, uint4 *keys,
+              const uint2 *rec, hipStream_t s, int rows_by_sweep) {
+  const int AT = scorer_tiles(n_atoms);
+  dim3 g;
+  const int st = scorer_grid(n_atoms, AT, &g);
+  if (st != PLX_OK) return st;
   profile_before(s, PLX_PROF_T3);
+  auto go = [&](auto at) {
+    hipLaunchKernelGGL((t3_kernel<decltype(at)::value, MODE>), g, dim3(kThreads), 0, s, xb, xf, n_atoms, tab->t3_tiles,
+                       tab->t3_words, tab->t3_rows, keys, rec, rows_by_sweep);
+  };
   if (AT == 4)
-    hipLaunchKernelGGL(t3_kernel<4>, g, dim3(kThreads), 0, s, xb, n_atoms, tab->t3_tiles, tab->t3_words, tab->t3_rows,
-                       keys, rec, rows_by_sweep);
+    go(std::integral_constant<int, 4>{});
   else if (AT == 2)
-    hipLaunchKernelGGL(t3_kernel<2>, g, dim3(kThreads), 0, s, xb, n_atoms, tab->t3_tiles, tab->t3_words, tab->t3_rows,
-                       keys, rec, rows_by_sweep);
+    go(std::integral_constant<int, 2>{});
   else
-    hipLaunchKernelGGL(t3_kernel<1>, g, dim3(kThreads), 0, s, xb, n_atoms, tab->t3_tiles, tab->t3_words, tab->t3_rows,
-                       keys, rec, rows_by_sweep);
+    go(std::integral_constant<int, 1>{});
   profile_after(s, PLX_PROF_T3);
   return check_launch("t3_kernel");
 }
 
-// t12_kernel: atom tiles per wave by launch size, as t3_kernel (38 KB of LDS at 4 tiles per wave).
-template <int LOAD>
+template <int LOAD, int MODE>
 int t12_launch_load(uint4 *xb, const float *src, const float *sigma, int64_t apr, int64_t n_atoms,
                     const DeviceTables *tab, uint4 *keys, uint2 *rec, hipStream_t s, int rows_by_sweep) {
-  const int AT = n_atoms >= 131072 ? 4 : n_atoms >= 98304 ? 2 : 1;
-  const int64_t per_block = static_cast<int64_t>(kWaves) * AT * 16;
-  const int64_t blocks = (n_atoms + per_block - 1) / per_block;
-  if (blocks > 0x7FFFFFFFll) return fail(PLX_EINVAL, "quantize: %lld atoms exceed one launch", static_cast<long long>(n_atoms));
-  const dim3 g(static_cast<unsigned>(blocks));
+  const int AT = scorer_tiles(n_atoms);
+  dim3 g;
+  const int st = scorer_grid(n_atoms, AT, &g);
+  if (st != PLX_OK) return st;
   profile_before(s, PLX_PROF_T12);
+  auto go = [&](auto at) {
+    hipLaunchKernelGGL((t12_kernel<decltype(at)::value, LOAD, MODE>), g, dim3(kThreads), 0, s, xb, src, sigma, apr,
+                       n_atoms, tab->t2_tiles, tab->t2_pos, tab->t2_rows, tab->t1_rows, tab->t2_steiner, tab->t3_dec,
+                       keys, rec, rows_by_sweep);
+  };
   if (AT == 4)
-    hipLaunchKernelGGL((t12_kernel<4, LOAD>), g, dim3(kThreads), 0, s, xb, src, sigma, apr, n_atoms, tab->t2_tiles,
-                       tab->t2_pos, tab->t2_rows, tab->t1_rows, tab->t2_steiner, tab->t3_dec, keys, rec, rows_by_sweep);
+    go(std::integral_constant<int, 4>{});
   else if (AT == 2)
-    hipLaunchKernelGGL((t12_kernel<2, LOAD>), g, dim3(kThreads), 0, s, xb, src, sigma, apr, n_atoms, tab->t2_tiles,
-                       tab->t2_pos, tab->t2_rows, tab->t1_rows, tab->t2_steiner, tab->t3_dec, keys, rec, rows_by_sweep);
+    go(std::integral_constant<int, 2>{});
   else
-    hipLaunchKernelGGL((t12_kernel<1, LOAD>), g, dim3(kThreads), 0, s, xb, src, sigma, apr, n_atoms, tab->t2_tiles,
-                       tab->t2_pos, tab->t2_rows, tab->t1_rows, tab->t2_steiner, tab->t3_dec, keys, rec, rows_by_sweep);
+    go(std::integral_constant<int, 1>{});
   profile_after(s, PLX_PROF_T12);
   return check_launch("t12_kernel");
 }
 
-// The structured NN-B path: t12_kernel (types 1-2; LOAD 1 / 2: it also rounds the atoms into xb, so no
+int resolve_launch(const uint4 *keys, int64_t n_atoms, const uint4 *xb, const DeviceTables *tab, const uint64_t *recs,
+                   int n_recs, int64_t rec_stride, int32_t *idx_out, uint8_t *packed_out, hipStream_t s) {
+  hipLaunchKernelGGL(resolve_kernel, dim3(static_cast<unsigned>((n_atoms + 255) / 256)), dim3(256), 0, s, keys, n_atoms,
+                     xb, tab->sw_dq, tab->sw_idx, tab->sw_anti, tab->sw_bf16_tiles, recs, n_recs, rec_stride, idx_out,
+                     packed_out);
+  return check_launch("resolve_kernel");
+}
+
+template <int MODE>
+int pick_launch(const uint4 *keys, int64_t n_atoms, const float *x, const DeviceTables *tab, int32_t *idx_out,
+                uint8_t *packed_out, hipStream_t s) {
+  hipLaunchKernelGGL(pick_kernel<MODE>, dim3(static_cast<unsigned>((n_atoms + 255) / 256)), dim3(256), 0, s, keys,
+                     n_atoms, x, tab->cb_raw, idx_out, packed_out);
+  return check_launch("pick_kernel");
+}
+
+// The structured path: t12_kernel (types 1-2; LOAD 1 / 2: it also rounds the atoms into xb, so no
 // prep_kernel runs), t3_kernel (type 3), pick_kernel.  Every atom's key halves are written by the two
 // scorers, so the keys need no clearing.
-template <int LOAD>
+template <int LOAD, int MODE>
 int structured_launch(uint4 *xb, const float *src, const float *sigma, int64_t apr, int64_t n_atoms,
                       const DeviceTables *tab, uint4 *keys, uint2 *rec, int32_t *idx_out, uint8_t *packed_out,
                       hipStream_t s, int rows_by_sweep) {
   int st;
-  if ((st = t12_launch_load<LOAD>(xb, src, sigma, apr, n_atoms, tab, keys, rec, s, rows_by_sweep)) != PLX_OK)
+  if ((st = t12_launch_load<LOAD, MODE>(xb, src, sigma, apr, n_atoms, tab, keys, rec, s, rows_by_sweep)) != PLX_OK)
     return st;
-  if ((st = t3_launch(xb, n_atoms, tab, keys, rec, s, rows_by_sweep)) != PLX_OK) return st;
-  hipLaunchKernelGGL(pick_kernel, dim3(static_cast<unsigned>((n_atoms + 255) / 256)), dim3(256), 0, s, keys, n_atoms,
-                     idx_out, packed_out);
-  return check_launch("pick_kernel");
+  if ((st = t3_launch<MODE>(xb, src, n_atoms, tab, keys, rec, s, rows_by_sweep)) != PLX_OK) return st;
+  return pick_launch<MODE>(keys, n_atoms, src, tab, idx_out, packed_out, s);
 }
 
-// workspace = per-atom keys, the NN-B pair records, then (NN-B / NN-T) the bf16 planes.
-// STRUCT (NN-B): the structured scorers (t12_kernel, t3_kernel, pick_kernel);
-// otherwise every sweep code is scored densely (nn_kernel, resolve_kernel).
-template <int MODE, bool FUSED, bool STRUCT = false>
+// workspace = per-atom keys, the dense sweep's pair records (the structured scorers: t3_kernel's set-up
+// records), then the bf16 planes.
+// Every mode runs the structured scorers (t12_kernel, t3_kernel, pick_kernel): against the dense sweep that
+// NN-T and NN-P had before, 614,400 atoms take 3.07 -> 0.28 ms under NN-T and 7.92 -> 0.38 ms under NN-P (there
+// three MFMAs per tile; same box), 700 atoms 56 -> 44 us under NN-T, so no size is left to the sweep.
+// DENSE (NN-B): every sweep code is scored densely instead (nn_kernel, resolve_kernel), the baseline the scorers
+// are measured against.
+template <int MODE, bool FUSED, bool DENSE = false>
 int launch_mode(const float *x, const float *sigma, int64_t apr, int64_t n_atoms, const DeviceTables *tab,
                 int32_t *idx_out, uint8_t *packed_out, uint8_t *workspace, hipStream_t s, int rows_by_sweep = 0) {
-  static_assert(!STRUCT || MODE == kModeB, "the structured scorers have NN-B semantics");
-  const int64_t ablocks = (n_atoms + kAtomsPerBlock - 1) / kAtomsPerBlock;
-  const int n_slices = choose_slices(ablocks);
-  const int tiles_per_slice = kSweepTiles / n_slices;
-  const int64_t grid = ablocks * n_slices;
-  if (grid > 0x7FFFFFFFll) return fail(PLX_EINVAL, "quantize: %lld atoms exceed one launch", static_cast<long long>(n_atoms));
+  static_assert(!DENSE || MODE == kModeB, "the dense sweep has NN-B semantics");
   uint4 *keys = reinterpret_cast<uint4 *>(workspace);
   uint64_t *recs = reinterpret_cast<uint64_t *>(workspace + keys_bytes(n_atoms));
   uint4 *xb = reinterpret_cast<uint4 *>(workspace + keys_bytes(n_atoms) + recs_bytes(n_atoms));
-  const int s0 = first_pair_slice(n_slices);
-  if constexpr (STRUCT)
-    return structured_launch<FUSED ? 2 : 1>(xb, x, sigma, apr, n_atoms, tab, keys, reinterpret_cast<uint2 *>(recs),
-                                            idx_out, packed_out, s, rows_by_sweep);
-  int st;
-  if (MODE != kModeP) {
+  if constexpr (!DENSE) {
+    return structured_launch<FUSED ? 2 : 1, MODE>(xb, x, sigma, apr, n_atoms, tab, keys,
+                                                  reinterpret_cast<uint2 *>(recs), idx_out, packed_out, s,
+                                                  rows_by_sweep);
+  } else {
+    const int64_t ablocks = (n_atoms + kAtomsPerBlock - 1) / kAtomsPerBlock;
+    const int n_slices = choose_slices(ablocks);
+    const int tiles_per_slice = kSweepTiles / n_slices;
+    const int64_t grid = ablocks * n_slices;
+    if (grid > 0x7FFFFFFFll) return fail(PLX_EINVAL, "quantize: %lld atoms exceed one launch", static_cast<long long>(n_atoms));
+    const int s0 = first_pair_slice(n_slices);
+    int st;
     hipLaunchKernelGGL((prep_kernel<FUSED>), dim3(static_cast<unsigned>((n_atoms * 3 + 255) / 256)), dim3(256), 0, s, x,
                        sigma, apr, n_atoms, xb, keys);
     if ((st = check_launch("prep_kernel")) != PLX_OK) return st;
-  } else {
-    hipLaunchKernelGGL(clear_keys_kernel, dim3(static_cast<unsigned>((n_atoms + 255) / 256)), dim3(256), 0, s, keys,
-                       n_atoms);
-    if ((st = check_launch("clear_keys_kernel")) != PLX_OK) return st;
+    profile_before(s);
+    hipLaunchKernelGGL(nn_kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), 0, s, xb, n_atoms,
+                       tab->sw_bf16_tiles, n_slices, tiles_per_slice, keys, recs, s0);
+    if ((st = check_launch("nn_kernel")) != PLX_OK) return st;
+    profile_after(s);
+    return resolve_launch(keys, n_atoms, xb, tab, recs, n_slices - s0, n_atoms, idx_out, packed_out, s);
   }
-  profile_before(s);
-  const uint8_t *tiles = MODE == kModeP ? tab->sw_raw_tiles : tab->sw_bf16_tiles;
-  const void *operand = MODE == kModeP ? static_cast<const void *>(x) : static_cast<const void *>(xb);
-  hipLaunchKernelGGL((nn_kernel<MODE>), dim3(static_cast<unsigned>(grid)), dim3(kThreads), 0, s, operand, n_atoms, tiles,
-                     n_slices, tiles_per_slice, keys, recs, s0);
-  if ((st = check_launch("nn_kernel")) != PLX_OK) return st;
-  profile_after(s);
-  hipLaunchKernelGGL((resolve_kernel<MODE, FUSED>), dim3(static_cast<unsigned>((n_atoms + 255) / 256)), dim3(256), 0, s,
-                     keys, n_atoms, x, sigma, apr, xb, tab->sw_dq, tab->sw_idx, tab->sw_anti, tab->cb_raw,
-                     tab->sw_bf16_tiles, static_cast<const uint64_t *>(recs), n_slices - s0, n_atoms, idx_out,
-                     packed_out);
-  return check_launch("resolve_kernel");
 }
 
 }  // namespace
@@ -2242,13 +2372,13 @@ int launch_quantize(const float *x, const float *sigma, int64_t rows, int64_t co
   if (mode == PLX_NN_PACK_FP32)
     st = launch_mode<PLX_NN_PACK_FP32, false>(x, nullptr, apr, n_atoms, tab, idx_out, packed_out, ws, s);
   else if (mode == PLX_NN_BF16_SCORES && !dense)
-    st = fused ? launch_mode<PLX_NN_BF16_SCORES, true, true>(x, sigma, apr, n_atoms, tab, idx_out, packed_out, ws, s,
-                                                             rows_by_sweep)
-               : launch_mode<PLX_NN_BF16_SCORES, false, true>(x, sigma, apr, n_atoms, tab, idx_out, packed_out, ws, s,
-                                                              rows_by_sweep);
+    st = fused ? launch_mode<PLX_NN_BF16_SCORES, true>(x, sigma, apr, n_atoms, tab, idx_out, packed_out, ws, s,
+                                                       rows_by_sweep)
+               : launch_mode<PLX_NN_BF16_SCORES, false>(x, sigma, apr, n_atoms, tab, idx_out, packed_out, ws, s,
+                                                        rows_by_sweep);
   else if (mode == PLX_NN_BF16_SCORES)
-    st = fused ? launch_mode<PLX_NN_BF16_SCORES, true>(x, sigma, apr, n_atoms, tab, idx_out, packed_out, ws, s)
-               : launch_mode<PLX_NN_BF16_SCORES, false>(x, sigma, apr, n_atoms, tab, idx_out, packed_out, ws, s);
+    st = fused ? launch_mode<PLX_NN_BF16_SCORES, true, true>(x, sigma, apr, n_atoms, tab, idx_out, packed_out, ws, s)
+               : launch_mode<PLX_NN_BF16_SCORES, false, true>(x, sigma, apr, n_atoms, tab, idx_out, packed_out, ws, s);
   else
     st = fused ? launch_mode<PLX_NN_FP32_SCORES, true>(x, sigma, apr, n_atoms, tab, idx_out, packed_out, ws, s)
                : launch_mode<PLX_NN_FP32_SCORES, false>(x, sigma, apr, n_atoms, tab, idx_out, packed_out, ws, s);
@@ -2265,15 +2395,15 @@ int launch_quantize(const float *x, const float *sigma, int64_t rows, int64_t co
 namespace {
 
 // Several latents in one scoring pass: row scale and operand planes per
-// matrix, one launch of the scorers over all their atoms (STRUCT: t12_kernel
-// and t3_kernel; otherwise nn_kernel with fewer codebook slices per atom
-// block; no per-matrix tail of the grid either way), then per matrix the
-// index + pack (pick_kernel / resolve_kernel) and the scaled gather of the
-// reconstructed weight.
-template <int MODE, bool STRUCT = false>
+// matrix, one launch of the scorers over all their atoms (t12_kernel and
+// t3_kernel; DENSE: nn_kernel with fewer codebook slices per atom block; no
+// per-matrix tail of the grid either way), then per matrix the index + pack
+// (pick_kernel / resolve_kernel) and the scaled gather of the reconstructed
+// weight.
+template <int MODE, bool DENSE = false>
 int launch_batch_mode(const RequantItem *items, int n_items, const DeviceTables *tab, uint8_t *workspace,
                       hipStream_t s) {
-  static_assert(!STRUCT || MODE == kModeB, "the structured scorers have NN-B semantics");
+  static_assert(!DENSE || MODE == kModeB, "the dense sweep has NN-B semantics");
   int64_t total = 0;
   for (int i = 0; i < n_items; ++i) total += items[i].rows * (items[i].cols / kDim);
   if (total == 0) return PLX_OK;
@@ -2298,16 +2428,16 @@ int launch_batch_mode(const RequantItem *items, int n_items, const DeviceTables 
     if ((st = check_launch("prep_kernel")) != PLX_OK) return st;
     off += n;
   }
-  if constexpr (STRUCT) {
-    if ((st = t12_launch_load<0>(xb, nullptr, nullptr, 1, total, tab, keys, reinterpret_cast<uint2 *>(recs), s, 0)) !=
-        PLX_OK)
+  if constexpr (!DENSE) {
+    if ((st = t12_launch_load<0, MODE>(xb, nullptr, nullptr, 1, total, tab, keys, reinterpret_cast<uint2 *>(recs), s,
+                                       0)) != PLX_OK)
       return st;
-    if ((st = t3_launch(xb, total, tab, keys, reinterpret_cast<const uint2 *>(recs), s, 0)) != PLX_OK) return st;
+    if ((st = t3_launch<MODE>(xb, nullptr, total, tab, keys, reinterpret_cast<const uint2 *>(recs), s, 0)) != PLX_OK)
+      return st;
   } else {
     profile_before(s);
-    hipLaunchKernelGGL((nn_kernel<MODE>), dim3(static_cast<unsigned>(grid)), dim3(kThreads), 0, s,
-                       static_cast<const void *>(xb), total, tab->sw_bf16_tiles, n_slices, tiles_per_slice, keys, recs,
-                       s0);
+    hipLaunchKernelGGL(nn_kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), 0, s, xb, total,
+                       tab->sw_bf16_tiles, n_slices, tiles_per_slice, keys, recs, s0);
     if ((st = check_launch("nn_kernel")) != PLX_OK) return st;
     profile_after(s);
   }
@@ -2316,17 +2446,11 @@ int launch_batch_mode(const RequantItem *items, int n_items, const DeviceTables 
     const RequantItem &it = items[i];
     const int64_t apr = it.cols / kDim, n = it.rows * apr;
     if (n == 0) continue;
-    if constexpr (STRUCT) {
-      hipLaunchKernelGGL(pick_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, keys + off, n,
-                         it.idx, it.packed);
-      if ((st = check_launch("pick_kernel")) != PLX_OK) return st;
-    } else {
-      hipLaunchKernelGGL((resolve_kernel<MODE, true>), dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s,
-                         keys + off, n, it.latent, it.sigma, apr, xb + off * 3, tab->sw_dq, tab->sw_idx, tab->sw_anti,
-                         tab->cb_raw, tab->sw_bf16_tiles, static_cast<const uint64_t *>(recs + off), n_slices - s0,
-                         total, it.idx, it.packed);
-      if ((st = check_launch("resolve_kernel")) != PLX_OK) return st;
-    }
+    if constexpr (!DENSE)
+      st = pick_launch<MODE>(keys + off, n, nullptr, tab, it.idx, it.packed, s);
+    else
+      st = resolve_launch(keys + off, n, xb + off * 3, tab, recs + off, n_slices - s0, total, it.idx, it.packed, s);
+    if (st != PLX_OK) return st;
     if (it.weight) {
       hipLaunchKernelGGL((gather_kernel<0, true>), dim3(static_cast<unsigned>((n * 6 + 255) / 256)), dim3(256), 0, s,
                          it.idx, n, tab->cb_raw, it.sigma, apr, static_cast<void *>(it.weight));
@@ -2358,8 +2482,8 @@ int launch_requantize_batch(const RequantItem *items, int n_items, int mode, voi
   const bool dense = (mode & PLX_NN_DENSE_TYPE3) != 0;
   mode &= ~(PLX_NN_DENSE_TYPE3 | PLX_NN_T3_ROWS_BY_SWEEP);
   if (mode == PLX_NN_BF16_SCORES)
-    return dense ? launch_batch_mode<PLX_NN_BF16_SCORES>(items, n_items, tab, ws, s)
-                 : launch_batch_mode<PLX_NN_BF16_SCORES, true>(items, n_items, tab, ws, s);
+    return dense ? launch_batch_mode<PLX_NN_BF16_SCORES, true>(items, n_items, tab, ws, s)
+                 : launch_batch_mode<PLX_NN_BF16_SCORES>(items, n_items, tab, ws, s);
   return launch_batch_mode<PLX_NN_FP32_SCORES>(items, n_items, tab, ws, s);
 }
 

@@ -6,8 +6,6 @@
 //                bf16 casts round them (castor.py:437, autocast at
 //                castor.py:552), in the MFMA tile layout of quantize.hip;
 //                9216 tiles x 768 B = 7,077,888 B.
-// sw_raw_tiles   the same codes' raw integers (exact in bf16), same layout,
-//                for the fp32-exact NN-P scoring (7,077,888 B).
 // sw_dq          the sweep codes' value-id words (kp_dq's format, below) in
 //                sweep order, for the quantizer's rescans (1,769,472 B).
 // sw_idx         the codebook row of every sweep code (0 for padding) and
@@ -54,10 +52,12 @@
 // t2_pos         each octad's 8 positions, ascending, one byte each (6,144 B);
 // t2_rows        the codebook row of the type-2 code on octad o whose minus
 //                signs on the octad's positions k = 0..6 (ascending) are the
-//                bits of p (the eighth sign: even parity), [759][128]
-//                (388,608 B);
+//                bits of p (the eighth sign: even parity), [759][128], each
+//                with the code's tie group << 18: the sweep group (of 256)
+//                of its pair's representative (388,608 B);
 // t1_rows        the codebook row of the type-1 code with +-4 at positions
-//                i < j, [24][24][4] by minus at i | minus at j << 1 (9,216 B);
+//                i < j, [24][24][4] by minus at i | minus at j << 1, with its
+//                tie group as in t2_rows (9,216 B);
 // t2_steiner     the octad holding each 5-subset of the 24 positions (every
 //                5 positions lie in exactly one octad), by the subset's colex
 //                rank C(p0,1) + C(p1,2) + ... + C(p4,5), p0 < ... < p4
@@ -169,7 +169,6 @@ int build(int dev, DeviceTables *t) {
   anti.resize(static_cast<size_t>(kSweepTiles - kType3Tiles) * kTileCodes, 0);  // every pair-region position
 
   std::vector<uint16_t> tiles(static_cast<size_t>(kSweepTiles) * (kTileBytes / 2), 0);
-  std::vector<uint16_t> raw_tiles(tiles.size(), 0);
   for (int tile = 0; tile < kSweepTiles; ++tile)
     for (int i = 0; i < kTileCodes; ++i) {
       const int code = sweep[static_cast<size_t>(tile) * kTileCodes + i];
@@ -177,9 +176,7 @@ int build(int dev, DeviceTables *t) {
       for (int p = 0; p < 3; ++p)
         for (int e = 0; e < 8; ++e) {
           const int k = raw[static_cast<size_t>(code) * kDim + 8 * p + e];
-          const size_t at = static_cast<size_t>(tile) * 384 + p * 128 + i * 8 + e;
-          tiles[at] = bf_of[k + 4];
-          raw_tiles[at] = f32_to_bf16_rne(static_cast<float>(k));
+          tiles[static_cast<size_t>(tile) * 384 + p * 128 + i * 8 + e] = bf_of[k + 4];
         }
     }
 
@@ -340,18 +337,21 @@ int build(int dev, DeviceTables *t) {
         hi = c;
         ++nz;
       }
+    // codes come in row order, so the pairs' members are counted in theirs; the k-th from either end is a pair
+    const int rank = n_t2 + n_t1, pair = rank < kPairCodes ? rank : 2 * kPairCodes - 1 - rank;
+    const uint32_t slot_value = static_cast<uint32_t>(code) | static_cast<uint32_t>(pair / kTieGroup) << kRowBits;
     if (nz == 8) {
       const int o = static_cast<int>(std::lower_bound(oct_masks.begin(), oct_masks.end(), m) - oct_masks.begin());
       if (o >= kT2Octads || oct_masks[o] != m || (__builtin_popcount(minus) & 1) != 0)
         return fail(PLX_EINVAL, "codebook row %d is no even-sign octad code", code);
       uint32_t &slot = t2_rows[static_cast<size_t>(o) * 128 + (minus & 0x7Fu)];
       if (slot != 0) return fail(PLX_EINVAL, "two octad codes share a sign pattern (row %d)", code);
-      slot = static_cast<uint32_t>(code);
+      slot = slot_value;
       ++n_t2;
     } else if (nz == 2) {
       uint32_t &slot = t1_rows[(static_cast<size_t>(lo) * kDim + hi) * 4 + minus];
       if (slot != 0) return fail(PLX_EINVAL, "two type-1 codes share positions and signs (row %d)", code);
-      slot = static_cast<uint32_t>(code);
+      slot = slot_value;
       ++n_t1;
     }
   }
@@ -413,7 +413,7 @@ int build(int dev, DeviceTables *t) {
   for (size_t i = 0; i < sweep.size(); ++i)
     for (int p = 0; p < 3; ++p) sw_dq[i * 3 + p] = dq[static_cast<size_t>(sweep[i]) * 3 + p];
 
-  void *dt = nullptr, *drt = nullptr, *dsq = nullptr, *dsi = nullptr, *dsa = nullptr, *dr = nullptr, *dg = nullptr,
+  void *dt = nullptr, *dsq = nullptr, *dsi = nullptr, *dsa = nullptr, *dr = nullptr, *dg = nullptr,
        *dd = nullptr, *dk = nullptr, *dpi = nullptr, *dcp = nullptr, *dpn = nullptr, *d3t = nullptr, *d3w = nullptr,
        *d3r = nullptr, *dgv = nullptr, *d2t = nullptr, *d2p = nullptr, *d2r = nullptr, *d1r = nullptr,
        *d2s = nullptr, *d3d = nullptr;
@@ -441,7 +441,6 @@ int build(int dev, DeviceTables *t) {
   }
   const Upload ups[] = {
       {tiles.data(), tiles.size() * 2, &dt},
-      {raw_tiles.data(), raw_tiles.size() * 2, &drt},
       {sw_dq.data(), sw_dq.size() * 4, &dsq},
       {sweep.data(), sweep.size() * 4, &dsi},
       {anti.data(), anti.size() * 4, &dsa},
@@ -479,7 +478,6 @@ int build(int dev, DeviceTables *t) {
     return st;
   }
   t->sw_bf16_tiles = static_cast<uint8_t *>(dt);
-  t->sw_raw_tiles = static_cast<uint8_t *>(drt);
   t->sw_dq = static_cast<uint32_t *>(dsq);
   t->sw_idx = static_cast<uint32_t *>(dsi);
   t->sw_anti = static_cast<uint32_t *>(dsa);
