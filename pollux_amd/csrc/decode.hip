@@ -17,15 +17,10 @@
 //   step while the position advances on the device; a position outside the
 //   cache writes nothing and yields NaN outputs.
 //
-// prefill_attention_kernel: the same for a chunk of up to 256 new positions
-//   p .. p+tc-1 of every sequence (the prompt of a prefill, pollux.py:615-626
-//   with is_causal over the cached prefix): one block per (head, sequence)
-//   normalises the chunk's q and k rows (a thread per row), writes k and v
-//   into the caches and keeps all three in LDS; then 16 lanes per query i
-//   (keys j = lane, lane + 16, ... <= p + i; cached ones from the caches, the
-//   chunk's from LDS) run an online softmax each and combine by DPP within
-//   their row of 16 lanes.  Chunks of a longer prompt are consecutive launches,
-//   so each one reads the previous chunks' rows from the caches.
+// prefill_attention_kernel: the same for t new positions p .. p+t-1 of every
+//   sequence (the prompt of a prefill, pollux.py:615-626 with is_causal over
+//   the cached prefix) on fp32 MFMA, in one launch: a block takes 64 queries of
+//   one (head, sequence) and walks the keys up to its last query 64 at a time.
 
 #include "plx_device.h"
 
@@ -269,121 +264,215 @@ __global__ __launch_bounds__(kAttnThreads, 5) void decode_attention_kernel(
   }
 }
 
-constexpr int kPrefillChunk = 256;  // new positions per launch (q, k, v rows of the chunk in LDS: 72 KB)
+// q, k, v, out: [b, t, H, 24] (rows of the prompt, at cache positions p0 .. p0+t-1); caches
+// [b, H, max_len, 24].  One block of 4 waves per 64 queries (16 a wave) of one (head, sequence), the blocks
+// with the most keys first.  Keys come in tiles of 64: the cached prefix from the caches, the prompt's from
+// k and v, their norm (k_ln) taken here by every block that needs them (4 lanes a key; a few percent of the
+// tile's products), so no block waits for another; the block whose queries are the tile's positions writes
+// its rows into the caches.
+//   Contractions: v_mfma_f32_16x16x4_f32, fp32 throughout.  S^T = K Q^T per 16 keys: lane l holds query l % 16
+// and keys 4 (l / 16) + r, r = 0..3; the contraction index is dim 6 g + c for lane group g and step c, so a
+// lane reads its 6 dims of a key as 3 8-byte pieces.  P^T is then, register r, the B operand of a step over
+// keys 4 g + r without any exchange between lanes; its A operand is V^T from LDS (one 16-byte read per lane
+// for 4 steps), in two tiles of dims (0-15; 16-23, then a row of ones that sums the probabilities).
+// Online softmax per query: the maximum over the tile's 64 keys, exchanged between the four lanes of a query
+// once per tile; the accumulators are rescaled only in tiles where some maximum of the wave rose.
+//   A V row that is not finite must not reach the queries before it (0 * inf): the tile that holds both
+// (the block's own) then adds its keys one by one, each to the queries at or after it.
+//   What bounds it: the fp32 matrix rate (56 MFMAs of 32 cycles per 16 queries x 64 keys; 25% of the second
+// dims tile is padding).  1,024 tokens x 80 heads: 889 -> 119 us against a thread row of 16 lanes per query on the
+// VALU in four launches of 256 positions.
+constexpr int kPfTile = 64;               // queries per block, keys per tile
+constexpr int kPfK = 26;                  // floats between keys in LDS (K)
+constexpr int kPfV = 68;                  // floats between dims in LDS (V^T)
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// q, k, v, out: [b, t, H, 24] (rows of the whole prompt; this launch takes rows
-// c0 .. c0+tc-1 of each sequence at cache positions p .. p+tc-1); caches
-// [b, H, max_len, 24].
-__global__ __launch_bounds__(kAttnThreads) void prefill_attention_kernel(
+__global__ __launch_bounds__(kAttnThreads, 4) void prefill_attention_kernel(
     const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v,
     const float *__restrict__ q_w, const float *__restrict__ k_w, float eps, float *__restrict__ k_cache,
-    float *__restrict__ v_cache, int64_t heads, int64_t in_stride, int64_t t_total, int64_t c0, int tc, int64_t p,
-    int64_t max_len, float scale, float *__restrict__ out) {
-  __shared__ __align__(16) float qs[kPrefillChunk][kDim];
-  __shared__ __align__(16) float ks[kPrefillChunk][kDim];
-  __shared__ __align__(16) float vs[kPrefillChunk][kDim];
-  const int tid = threadIdx.x;
-  const int64_t h = blockIdx.x, bb = blockIdx.y;
-  const int64_t row_stride = heads * kDim;                           // out: between positions of one sequence
-  const int64_t in0 = (bb * t_total + c0) * in_stride + h * kDim;    // q, k, v: row c0 of this (sequence, head)
-  const int64_t out0 = (bb * t_total + c0) * row_stride + h * kDim;
-  float *kc = k_cache + (bb * heads + h) * max_len * kDim;
-  float *vc = v_cache + (bb * heads + h) * max_len * kDim;
+    float *__restrict__ v_cache, int64_t heads, int64_t in_stride, int t_total, int p0, int64_t max_len,
+    float scale_log2, float *__restrict__ out) {
+  constexpr int kSub = kDim / 4;  // dims per lane
+  __shared__ __align__(16) float ks[2][kPfTile * kPfK];
+  __shared__ __align__(16) float vt[2][(kDim + 1) * kPfV];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int64_t bh = blockIdx.y;  // sequence * heads + head
+  const int64_t bb = bh / heads, h = bh % heads;
+  const int qt = static_cast<int>(gridDim.x - 1 - blockIdx.x);  // query tile: the longest first
+  const float *kin = k + bb * t_total * in_stride + h * kDim, *vin = v + bb * t_total * in_stride + h * kDim;
+  float *kc = k_cache + bh * max_len * kDim, *vc = v_cache + bh * max_len * kDim;
+  const int n_pre = (p0 + kPfTile - 1) / kPfTile;  // tiles of the cached prefix
+  const int n_tiles = n_pre + qt + 1;
 
-  // the chunk's rows: RMS norms of q and k (q_ln / k_ln), k and v into the caches
-  for (int r = tid; r < tc; r += kAttnThreads) {
-    const float4 *q4 = reinterpret_cast<const float4 *>(q + in0 + r * in_stride);
-    const float4 *k4 = reinterpret_cast<const float4 *>(k + in0 + r * in_stride);
-    const float4 *v4 = reinterpret_cast<const float4 *>(v + in0 + r * in_stride);
-    float qv[kDim], kv[kDim], vv[kDim];
+  // a tile's rows: 4 lanes a key, 6 dims each; rows past the prefix / the prompt: zeros
+  const int key = tid >> 2, d0 = (tid & 3) * kSub;
+  float kr[kSub], vr[kSub];
+  auto load = [&](int tile) {
+    const bool pre = tile < n_pre;
+    const int r = (pre ? tile : tile - n_pre) * kPfTile + key, lim = pre ? p0 : t_total;
+    const int64_t rc = r < lim ? r : lim - 1;
+    const float2 *a = reinterpret_cast<const float2 *>((pre ? kc + rc * kDim : kin + rc * in_stride) + d0);
+    const float2 *b = reinterpret_cast<const float2 *>((pre ? vc + rc * kDim : vin + rc * in_stride) + d0);
 #pragma unroll
-    for (int i = 0; i < kDim / 4; ++i) {
-      const float4 a = q4[i], b = k4[i], c = v4[i];
-      qv[4 * i] = a.x; qv[4 * i + 1] = a.y; qv[4 * i + 2] = a.z; qv[4 * i + 3] = a.w;
-      kv[4 * i] = b.x; kv[4 * i + 1] = b.y; kv[4 * i + 2] = b.z; kv[4 * i + 3] = b.w;
-      vv[4 * i] = c.x; vv[4 * i + 1] = c.y; vv[4 * i + 2] = c.z; vv[4 * i + 3] = c.w;
+    for (int i = 0; i < kSub / 2; ++i) {
+      const float2 x = a[i], y = b[i];
+      kr[2 * i] = x.x; kr[2 * i + 1] = x.y;
+      vr[2 * i] = y.x; vr[2 * i + 1] = y.y;
     }
-    float sq = 0.f, sk = 0.f;
+  };
+  // the loaded rows into LDS (the prompt's keys normalised; the block's own also into the caches); returns
+  // whether this thread's part of V is finite
+  float kw[kSub];
 #pragma unroll
-    for (int i = 0; i < kDim; ++i) {
-      sq = fmaf(qv[i], qv[i], sq);
-      sk = fmaf(kv[i], kv[i], sk);
-    }
-    const float rq = 1.0f / sqrtf(sq / static_cast<float>(kDim) + eps);
-    const float rk = 1.0f / sqrtf(sk / static_cast<float>(kDim) + eps);
-    float4 *kd = reinterpret_cast<float4 *>(kc + (p + r) * kDim);
-    float4 *vd = reinterpret_cast<float4 *>(vc + (p + r) * kDim);
+  for (int i = 0; i < kSub; ++i) kw[i] = k_w[d0 + i];
+  auto store = [&](int tile, int buf) {
+    const bool pre = tile < n_pre;
+    const int r = (pre ? tile : tile - n_pre) * kPfTile + key;
+    const bool valid = r < (pre ? p0 : t_total);
+    if (!pre) {
+      float sq = 0.f;
 #pragma unroll
-    for (int i = 0; i < kDim / 4; ++i) {
-      const float4 qn = make_float4(qv[4 * i] * rq * q_w[4 * i], qv[4 * i + 1] * rq * q_w[4 * i + 1],
-                                    qv[4 * i + 2] * rq * q_w[4 * i + 2], qv[4 * i + 3] * rq * q_w[4 * i + 3]);
-      const float4 kn = make_float4(kv[4 * i] * rk * k_w[4 * i], kv[4 * i + 1] * rk * k_w[4 * i + 1],
-                                    kv[4 * i + 2] * rk * k_w[4 * i + 2], kv[4 * i + 3] * rk * k_w[4 * i + 3]);
-      const float4 vn = make_float4(vv[4 * i], vv[4 * i + 1], vv[4 * i + 2], vv[4 * i + 3]);
-      reinterpret_cast<float4 *>(qs[r])[i] = qn;
-      reinterpret_cast<float4 *>(ks[r])[i] = kn;
-      reinterpret_cast<float4 *>(vs[r])[i] = vn;
-      kd[i] = kn;
-      vd[i] = vn;
-    }
-  }
-  __syncthreads();
-
-  // 16 lanes (one DPP row) per query; a row whose query is past the chunk
-  // skips the round as a whole, so every DPP exchange sees its full row
-  const int grp = tid >> 4, l16 = tid & 15;
-  for (int i = grp; i < tc; i += kAttnThreads / 16) {
-    const int64_t last = p + i;  // the query's own position: keys 0 .. last
-    float qr[kDim];
+      for (int i = 0; i < kSub; ++i) sq = fmaf(kr[i], kr[i], sq);
+      sq += dpp_f32<0xB1>(sq);
+      sq += dpp_f32<0x4E>(sq);
+      const float rk = 1.0f / sqrtf(sq / static_cast<float>(kDim) + eps);
 #pragma unroll
-    for (int c = 0; c < kDim; ++c) qr[c] = qs[i][c];
-    float m = -INFINITY, l = 0.f, acc[kDim];
+      for (int i = 0; i < kSub; ++i) kr[i] = kr[i] * rk * kw[i];
+      if (tile == n_tiles - 1 && valid) {
 #pragma unroll
-    for (int c = 0; c < kDim; ++c) acc[c] = 0.f;
-    auto step = [&](const float4 *k4, const float4 *v4) {
-      float kr[kDim], vr[kDim];
-#pragma unroll
-      for (int c = 0; c < kDim / 4; ++c) {
-        const float4 a = k4[c], b = v4[c];
-        kr[4 * c] = a.x; kr[4 * c + 1] = a.y; kr[4 * c + 2] = a.z; kr[4 * c + 3] = a.w;
-        vr[4 * c] = b.x; vr[4 * c + 1] = b.y; vr[4 * c + 2] = b.z; vr[4 * c + 3] = b.w;
+        for (int i = 0; i < kSub / 2; ++i) {
+          reinterpret_cast<float2 *>(kc + static_cast<int64_t>(p0 + r) * kDim + d0)[i] = make_float2(kr[2 * i], kr[2 * i + 1]);
+          reinterpret_cast<float2 *>(vc + static_cast<int64_t>(p0 + r) * kDim + d0)[i] = make_float2(vr[2 * i], vr[2 * i + 1]);
+        }
       }
-      float sc = 0.f;
+    }
+    bool finite = true;
 #pragma unroll
-      for (int c = 0; c < kDim; ++c) sc = fmaf(qr[c], kr[c], sc);
-      sc *= scale;
-      const float mn = fmaxf(m, sc);
-      const float a = expf(m - mn), pr = expf(sc - mn);  // m = -inf at a lane's first key: a = 0
-      l = fmaf(l, a, pr);
+    for (int i = 0; i < kSub; ++i) {
+      if (!valid) kr[i] = vr[i] = 0.f;
+      finite &= (__float_as_uint(vr[i]) & 0x7F800000u) != 0x7F800000u;
+      vt[buf][(d0 + i) * kPfV + key] = vr[i];
+    }
 #pragma unroll
-      for (int c = 0; c < kDim; ++c) acc[c] = fmaf(acc[c], a, pr * vr[c]);
+    for (int i = 0; i < kSub / 2; ++i)
+      *reinterpret_cast<float2 *>(&ks[buf][key * kPfK + d0 + 2 * i]) = make_float2(kr[2 * i], kr[2 * i + 1]);
+    return finite;
+  };
+  load(0);
+  if (tid < 2 * kPfTile) vt[tid >> 6][kDim * kPfV + (tid & 63)] = 1.f;  // the probabilities' sum
+
+  // this wave's 16 queries: lane (n, g) holds dims 6g .. 6g+5 of query n, normalised (q_ln) and scaled
+  const int qrow = qt * kPfTile + wave * 16 + n;
+  float qv[kSub];
+  {
+    const int64_t rc = qrow < t_total ? qrow : t_total - 1;
+    const float2 *a = reinterpret_cast<const float2 *>(q + (bb * t_total + rc) * in_stride + h * kDim + g * kSub);
+    float sq = 0.f;
+#pragma unroll
+    for (int i = 0; i < kSub / 2; ++i) {
+      const float2 x = a[i];
+      qv[2 * i] = x.x; qv[2 * i + 1] = x.y;
+      sq = fmaf(x.y, x.y, fmaf(x.x, x.x, sq));
+    }
+    sq += __shfl_xor(sq, 16, 64);
+    sq += __shfl_xor(sq, 32, 64);
+    const float rq = 1.0f / sqrtf(sq / static_cast<float>(kDim) + eps);
+#pragma unroll
+    for (int i = 0; i < kSub; ++i) qv[i] = qv[i] * rq * q_w[g * kSub + i] * scale_log2;
+  }
+
+  f32x4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};  // dims 4g + r; 16 + 4g + r (24: the sum)
+  float m = -INFINITY;
+  const int vrow0 = n * kPfV + 4 * g, vrow1 = min(16 + n, kDim) * kPfV + 4 * g;
+  bool finite = store(0, 0);
+  for (int tile = 0; tile < n_tiles; ++tile) {
+    const int buf = tile & 1;
+    const bool own = tile == n_tiles - 1;
+    const bool all_finite = __syncthreads_and(finite) != 0;  // (tile's rows are in LDS; the other buffer is free)
+    if (!own) load(tile + 1);
+    const int live = own ? wave + 1 : kPfTile / 16;  // 16-key parts with a key at or before some query of the wave
+    f32x4 sc[4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+      sc[kt] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if (kt >= live) continue;  // (wave-uniform)
+      const float2 *a = reinterpret_cast<const float2 *>(&ks[buf][(16 * kt + n) * kPfK + g * kSub]);
+      f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < kSub / 2; ++i) {
+        const float2 x = a[i];
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, qv[2 * i], c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, qv[2 * i + 1], c, 0, 0, 0);
+      }
+      sc[kt] = c;
+    }
+    // keys past the query (own tile) or past the prefix (its last tile)
+    if (own || tile == n_pre - 1) {
+      const int last = own ? wave * 16 + n : p0 - 1 - tile * kPfTile;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * kt + 4 * g + r > last) sc[kt][r] = -INFINITY;
+    }
+    float mx = sc[0][0];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[kt][r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (__any(mx > m)) {
+      const float mn = fmaxf(m, mx);
+      const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        o0[r] *= f;
+        o1[r] *= f;
+      }
       m = mn;
-    };
-    // keys j = l16 + 16n in increasing order: the cached ones, then the chunk's
-    int64_t j = l16;
-    for (; j < p; j += 16)
-      step(reinterpret_cast<const float4 *>(kc + j * kDim), reinterpret_cast<const float4 *>(vc + j * kDim));
-    for (; j <= last; j += 16)
-      step(reinterpret_cast<const float4 *>(ks[j - p]), reinterpret_cast<const float4 *>(vs[j - p]));
-    // the row's maximum, every lane's state rescaled to it, then the sums
-    float bmv[1] = {m};
-    group_reduce<16, true>(bmv);
-    const float f = m == -INFINITY ? 0.f : expf(m - bmv[0]);
-    float part[kDim + 1];
+    }
 #pragma unroll
-    for (int c = 0; c < kDim; ++c) part[c] = acc[c] * f;
-    part[kDim] = l * f;
-    group_reduce<16>(part);
-    float *o = out + out0 + static_cast<int64_t>(i) * row_stride;
-    const float inv = part[kDim];
-    // lane c writes coordinate c, lanes 0..7 also c + 16 (static indices: no scratch)
-    float v0 = part[0], v1 = part[16];
+    for (int kt = 0; kt < 4; ++kt) {
+      if (kt >= live) continue;  // (wave-uniform)
 #pragma unroll
-    for (int c = 1; c < 16; ++c) v0 = l16 == c ? part[c] : v0;
+      for (int r = 0; r < 4; ++r)
+        sc[kt][r] = __builtin_amdgcn_exp2f(sc[kt][r] - m);  // (a masked key: 2^-inf = 0)
+      if (!own || all_finite) {
+        const float4 a = *reinterpret_cast<const float4 *>(&vt[buf][vrow0 + 16 * kt]);
+        const float4 b = *reinterpret_cast<const float4 *>(&vt[buf][vrow1 + 16 * kt]);
+        o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, sc[kt][0], o0, 0, 0, 0);
+        o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, sc[kt][0], o1, 0, 0, 0);
+        o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, sc[kt][1], o0, 0, 0, 0);
+        o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, sc[kt][1], o1, 0, 0, 0);
+        o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, sc[kt][2], o0, 0, 0, 0);
+        o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(b.z, sc[kt][2], o1, 0, 0, 0);
+        o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, sc[kt][3], o0, 0, 0, 0);
+        o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(b.w, sc[kt][3], o1, 0, 0, 0);
+      } else {
+        float *ps = &ks[buf ^ 1][wave * 256];  // (the last tile: the other buffer is done with)
 #pragma unroll
-    for (int c = 17; c < kDim; ++c) v1 = l16 == c - 16 ? part[c] : v1;
-    o[l16] = v0 / inv;
-    if (l16 < kDim - 16) o[16 + l16] = v1 / inv;
+        for (int r = 0; r < 4; ++r) ps[(4 * g + r) * 16 + n] = sc[kt][r];
+#pragma unroll 1
+        for (int kk = 0; kk < 16; ++kk) {
+          const float pr = ps[kk * 16 + n];
+          if (16 * kt + kk > wave * 16 + n) continue;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            o0[e] = fmaf(pr, vt[buf][(4 * g + e) * kPfV + 16 * kt + kk], o0[e]);
+            o1[e] = fmaf(pr, vt[buf][min(16 + 4 * g + e, kDim) * kPfV + 16 * kt + kk], o1[e]);
+          }
+        }
+      }
+    }
+    if (!own) finite = store(tile + 1, buf ^ 1);
+  }
+  const float sum = __shfl(o1[0], 32 + n, 64);  // dim 24: lanes of g = 2, register 0
+  if (qrow < t_total) {
+    float *o = out + (bb * t_total + qrow) * heads * kDim + h * kDim + 4 * g;
+    *reinterpret_cast<float4 *>(o) = make_float4(o0[0] / sum, o0[1] / sum, o0[2] / sum, o0[3] / sum);
+    if (g < 2)
+      *reinterpret_cast<float4 *>(o + 16) = make_float4(o1[0] / sum, o1[1] / sum, o1[2] / sum, o1[3] / sum);
   }
 }
 
@@ -534,12 +623,17 @@ int launch_prefill_attention(const float *q, const float *k, const float *v, int
   if (qkv_stride < heads * kDim || qkv_stride % 4 != 0)
     return fail(PLX_EINVAL, "prefill_attention: q, k, v rows %lld floats apart (at least %lld, a multiple of 4)",
                 static_cast<long long>(qkv_stride), static_cast<long long>(heads * kDim));
-  const float scale = 1.0f / sqrtf(static_cast<float>(kDim));
-  for (int64_t c0 = 0; c0 < t; c0 += kPrefillChunk) {
-    const int tc = static_cast<int>(t - c0 < kPrefillChunk ? t - c0 : kPrefillChunk);
-    hipLaunchKernelGGL(prefill_attention_kernel, dim3(static_cast<unsigned>(heads), static_cast<unsigned>(b)),
-                       dim3(kAttnThreads), 0, s, q, k, v, q_w, k_w, eps, k_cache, v_cache, heads, qkv_stride, t, c0, tc,
-                       p0 + c0, max_len, scale, out);
+  const int64_t q_tiles = (t + kPfTile - 1) / kPfTile;
+  // scores in units of log2: the softmax takes powers of two
+  const float scale_log2 = static_cast<float>(1.4426950408889634 / sqrt(static_cast<double>(kDim)));
+  // the grid's y dimension holds 65,535 (sequence, head) pairs: more go in several launches
+  const int64_t seqs = 0xFFFFll / heads;
+  for (int64_t s0 = 0; s0 < b; s0 += seqs) {
+    const int64_t nb = b - s0 < seqs ? b - s0 : seqs;
+    const int64_t in = s0 * t * qkv_stride, cache = s0 * heads * max_len * kDim;
+    hipLaunchKernelGGL(prefill_attention_kernel, dim3(static_cast<unsigned>(q_tiles), static_cast<unsigned>(nb * heads)),
+                       dim3(kAttnThreads), 0, s, q + in, k + in, v + in, q_w, k_w, eps, k_cache + cache, v_cache + cache,
+                       heads, qkv_stride, static_cast<int>(t), static_cast<int>(p0), max_len, scale_log2, out + s0 * t * heads * kDim);
     const int st = check_launch("prefill_attention_kernel");
     if (st != PLX_OK) return st;
   }
