@@ -956,7 +956,7 @@ int launch_dql(DqlTargets t, int64_t apr, const void *x, int64_t m, const uint4 
 //             quads of 4 (= 3 K steps of 32) and reads its activation
 //             fragments (up to 32 bf16 tokens: from x in place; otherwise
 //             from a fragment-order copy that a small kernel writes first,
-//             fp32 x as three bf16 parts; L2-resident either way: every block
+//             fp32 x as two fp16 parts; L2-resident either way: every block
 //             reads all of it), PD quads ahead in registers; per K step a
 //             lane decodes its B fragments (8 weights of one row = one plane
 //             of one atom) from one LDS word with v_perm_b32 byte lookups and
@@ -979,6 +979,7 @@ int launch_dql(DqlTargets t, int64_t apr, const void *x, int64_t m, const uint4 
 // ---------------------------------------------------------------------------
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kMmRows = 32;             // output rows per block
@@ -1037,20 +1038,46 @@ __device__ __forceinline__ void group_codes(uint32_t d0, uint32_t d1, uint32_t d
   c[3] = static_cast<int32_t>(((lo & 0x3FFu) << 8) | b8);
 }
 
-// Fragment-order copy of the activations for dqmm_kernel (fp32 x, and bf16 x
-// above 32 tokens).  One thread per 16-byte fragment position (slab, quad Q,
-// K step s, token tile t, lane): x[64 slab + 16t + (lane & 15)][96Q + 32s +
-// 8(lane >> 4) .. +8), zero for tokens >= m and columns >= cols (token tiles
-// t >= `tiles`, which the GEMM does not read, are not written), stored at
-// xf[slab][Q][part][s][t][lane].  bf16 x is one part.  fp32 x is split
-// exactly into three bf16 parts, x = h + m + l (h = bf16(x), m = bf16(x - h),
-// l = x - h - m, exact while the parts stay normal, |x| >= ~2^-110; inf / nan
-// go to h alone), so that bf16 MFMAs form the products of the fp32
-// activations.
-template <bool XF32>
-__global__ __launch_bounds__(256) void xfrag_kernel(const void *__restrict__ x, int64_t m_total, int64_t cols,
+// Fragment-order copies of the activations for the MFMA kernels.  A 16-byte fragment position (slab, quad Q,
+// K step s, token tile t, lane) holds x[64 slab + 16t + (lane & 15)][96Q + 32s + 8(lane >> 4) .. +8), zero for
+// tokens >= m and columns >= cols, stored at xf[slab][Q][part][s][t][lane] (token tiles t >= `tiles`, which the
+// GEMM does not read, are not written).
+//
+// bf16 x is one part, as it is (above 32 tokens): xfrag_kernel, one thread per position.
+//
+// fp32 x is two fp16 parts: the token's row is scaled by a power of two (its largest finite |x| into
+// [2^14, 2^15)), then h = fp16(x'), m = fp16(2^11 (x' - h)).  x' - h is exact and has at most 13 significant
+// bits, so h + 2^-11 m is x' up to its last fp32 bit, i.e. 2^-23 |x| (0.5 * 2^-23 |x| rms), where |x| is at
+// least 2^-28 of the row's largest; smaller elements keep 2^-52 of that largest.  fp16 weights need no split,
+// so the GEMM takes two MFMAs per tile where three bf16 parts against hi + lo took six; with a third of the
+// fp32 roundings its results are closer to float64 than the exact split's (a
+// decoder block's keys at 1,024 tokens: 2.3e-7 -> 1.8e-7 relative), its time a third less (183 -> 123 us for 1,024
+// tokens, 7680x1920 and its like).
+// inf / nan go to h alone, as they are.  The scale's inverse per token goes to tscale.
+__device__ __forceinline__ float pow2f(int e) { return __uint_as_float(static_cast<uint32_t>(e + 127) << 23); }
+
+// exponent e such that |v| 2^e is in [2^14, 2^15) for the largest finite |v| of a row (|e| <= 126)
+__device__ __forceinline__ int row_exponent(float mx) {
+  const int e = static_cast<int>(__float_as_uint(mx) >> 23);  // biased (0: zero or subnormal)
+  return mx == 0.f ? 0 : min(14 - (e - 127), 126);
+}
+
+__device__ __forceinline__ float finite_abs(float v) {
+  const float a = fabsf(v);
+  return a <= 3.402823466e38f ? a : 0.f;
+}
+
+// fp16 bits of the two parts of v (scaled by sc), h | m << 16
+__device__ __forceinline__ uint32_t split_f16(float v, float sc) {
+  const float x = v * sc;
+  const __half h = __float2half_rn(x);
+  const float r = x - __half2float(h);
+  const uint32_t mb = fabsf(v) <= 3.402823466e38f ? __half_as_ushort(__float2half_rn(r * 2048.f)) : 0u;
+  return __half_as_ushort(h) | mb << 16;
+}
+
+__global__ __launch_bounds__(256) void xfrag_kernel(const uint16_t *__restrict__ x, int64_t m_total, int64_t cols,
                                                     int64_t n_quads_row, int tiles, uint4 *__restrict__ xf) {
-  constexpr int XP = XF32 ? 3 : 1;
   constexpr int kQuadFrags = kXfQuadBytes / 16;  // 768 per part
   const int64_t per_slab = n_quads_row * kQuadFrags;
   const int64_t f = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;  // fragment position within the slab
@@ -1060,60 +1087,91 @@ __global__ __launch_bounds__(256) void xfrag_kernel(const void *__restrict__ x, 
   const int t = static_cast<int>(rest & 3);
   if (t >= tiles) return;  // a token tile the GEMM does not read (it reads `tiles` per slab)
   const int64_t qs = rest >> 2;  // 3Q + s
-  const int64_t quad = qs / 3, within = f - quad * kQuadFrags;
   const int64_t tok = static_cast<int64_t>(blockIdx.y) * 64 + 16 * t + (lane & 15);
   const int64_t col = 32 * qs + 8 * (lane >> 4);
-  uint4 *dst = xf + static_cast<int64_t>(blockIdx.y) * per_slab * XP + quad * XP * kQuadFrags + within;
-  const bool live = tok < m_total && col < cols;
-  if constexpr (!XF32) {
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (live) v = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(x) + tok * cols + col);
-    dst[0] = v;
+  uint4 v = make_uint4(0u, 0u, 0u, 0u);
+  if (tok < m_total && col < cols) v = *reinterpret_cast<const uint4 *>(x + tok * cols + col);
+  xf[static_cast<int64_t>(blockIdx.y) * per_slab + f] = v;
+}
+
+// the two fp16 parts of columns 4i .. 4i+3 of token (slab, t, tl) into the copy
+__device__ __forceinline__ void store_parts(uint2 *__restrict__ xf, int64_t slab, int64_t n_quads_row, int t, int tl,
+                                            int64_t i, const float *v, float sc) {
+  constexpr int kQuadFrags = kXfQuadBytes / 16;
+  const int64_t qs = i >> 3, quad = qs / 3;  // K step of the row, its quad
+  const int c8 = static_cast<int>(i >> 1) & 3;
+  uint32_t p[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) p[e] = split_f16(v[e], sc);
+  const int64_t within = ((qs - 3 * quad) * 4 + t) * 64 + tl + 16 * c8;
+  uint2 *d = xf + 2 * ((slab * n_quads_row + quad) * 2 * kQuadFrags + within) + (i & 1);
+  d[0] = make_uint2((p[0] & 0xFFFFu) | p[1] << 16, (p[2] & 0xFFFFu) | p[3] << 16);
+  d[2 * kQuadFrags] = make_uint2(p[0] >> 16 | (p[1] & 0xFFFF0000u), p[2] >> 16 | (p[3] & 0xFFFF0000u));
+}
+
+// fp32 x, one block per token row of each slab's `tiles` token tiles; REG: rows of up to 8,192 columns are read
+// once, into registers.
+constexpr int kXsVec = 8;
+template <bool REG>
+__global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x, int64_t m_total, int64_t cols,
+                                                     int64_t n_quads_row, int tiles, uint2 *__restrict__ xf,
+                                                     float *__restrict__ tscale) {
+  __shared__ float red[4];
+  const int tid = threadIdx.x;
+  const int per_slab = 16 * tiles;
+  const int64_t slab = blockIdx.x / static_cast<unsigned>(per_slab);
+  const int t = static_cast<int>(blockIdx.x % static_cast<unsigned>(per_slab)) >> 4, tl = blockIdx.x & 15;
+  const int64_t tok = slab * 64 + 16 * t + tl;
+  const bool live = tok < m_total;
+  const int64_t n4 = live ? cols >> 2 : 0, n_pad = n_quads_row * 24;  // float4s of the row, with the last quad's padding
+  const float4 *xr = reinterpret_cast<const float4 *>(x + (live ? tok : 0) * cols);
+  float4 v[REG ? kXsVec : 1];
+  float mx[1] = {0.f};
+  auto top = [&](float4 a) {
+    mx[0] = fmaxf(fmaxf(fmaxf(mx[0], finite_abs(a.x)), finite_abs(a.y)), fmaxf(finite_abs(a.z), finite_abs(a.w)));
+  };
+  if constexpr (REG) {
+#pragma unroll
+    for (int k = 0; k < kXsVec; ++k) {
+      const int64_t i = tid + 256 * k;
+      v[k] = i < n4 ? xr[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int k = 0; k < kXsVec; ++k) top(v[k]);
   } else {
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (live) {
-      const float4 *src = reinterpret_cast<const float4 *>(static_cast<const float *>(x) + tok * cols + col);
-      const float4 a = src[0], b = src[1];
-      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    for (int64_t i = tid; i < n4; i += 256) top(xr[i]);
+  }
+  group_reduce<64, true>(mx);
+  if ((tid & 63) == 0) red[tid >> 6] = mx[0];
+  __syncthreads();
+  const int e = row_exponent(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+  const float sc = pow2f(e);
+  if (tid == 0) tscale[tok] = pow2f(-e);
+  if constexpr (REG) {
+#pragma unroll
+    for (int k = 0; k < kXsVec; ++k) {
+      const int64_t i = tid + 256 * k;
+      const float a[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+      if (i < n_pad) store_parts(xf, slab, n_quads_row, t, tl, i, a, sc);
     }
-    uint32_t part[3][4];
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-      uint32_t hb[2], mb[2], lb[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const float xv = v[e + u];
-        hb[u] = bf16_rne_bits(xv);
-        mb[u] = lb[u] = 0u;
-        if (fabsf(xv) <= 3.0e38f) {
-          const float r1 = xv - __uint_as_float(hb[u] << 16);
-          mb[u] = bf16_rne_bits(r1);
-          lb[u] = bf16_rne_bits(r1 - __uint_as_float(mb[u] << 16));
-        }
-      }
-      part[0][e / 2] = hb[0] | (hb[1] << 16);
-      part[1][e / 2] = mb[0] | (mb[1] << 16);
-      part[2][e / 2] = lb[0] | (lb[1] << 16);
+  } else {
+    for (int64_t i = tid; i < n_pad; i += 256) {
+      const float4 u = i < n4 ? xr[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float a[4] = {u.x, u.y, u.z, u.w};
+      store_parts(xf, slab, n_quads_row, t, tl, i, a, sc);
     }
-#pragma unroll
-    for (int pp = 0; pp < 3; ++pp) dst[pp * kQuadFrags] = make_uint4(part[pp][0], part[pp][1], part[pp][2], part[pp][3]);
   }
 }
 
-// RMS norm of fp32 token rows written straight into the fragment-order copy:
-// rmsnorm_kernel (decode.hip) and xfrag_kernel<true> in one launch, with the
-// same values (the sum of squares in rmsnorm_kernel's order: lane l holds
-// float4 l + 64k of the row, fmaf over k and the four components, then the
-// wave sum).  One wave per token row of each 64-token slab; rows >= m write
-// zeros, rows of token tiles the GEMM does not read (t >= tiles) nothing.  Fragment 32k + j holds the row's columns 8(32k + j) .. +8, i.e.
-// float4s 64k + 2j and 64k + 2j + 1: lanes 2j and 2j + 1 each write their
-// 8-byte half of the fragment in every part.  Rows of up to 32 * kNfVec
-// fragments (kNfVec * 256 columns, padding of the last quad included).
+// RMS norm of fp32 token rows written straight into the fragment-order copy: rmsnorm_kernel (decode.hip) and
+// xsplit_kernel in one launch, with the same values (the sum of squares in rmsnorm_kernel's order: lane l holds
+// float4 l + 64k of the row, fmaf over k and the four components, then the wave sum).  One wave per token row of
+// each 64-token slab; rows >= m write zeros, rows of token tiles the GEMM does not read (t >= tiles) nothing.
+// Rows of up to 64 * kNfVec float4s (padding of the last quad included).
 constexpr int kNfVec = 8;
 __global__ __launch_bounds__(256) void normfrag_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                        int64_t m_total, int cols, int64_t n_quads_row, int tiles,
-                                                       float eps, uint2 *__restrict__ xf) {
-  constexpr int kQuadFrags = kXfQuadBytes / 16;
+                                                       float eps, uint2 *__restrict__ xf, float *__restrict__ tscale) {
   const int lane = threadIdx.x & 63;
   const int64_t tok = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   const int64_t slab = tok >> 6;
@@ -1140,32 +1198,23 @@ __global__ __launch_bounds__(256) void normfrag_kernel(const float *__restrict__
   }
   ss = wave_reduce_sum(ss);
   const float r = 1.0f / sqrtf(ss / static_cast<float>(cols) + eps);
-  const int64_t n_frag = n_quads_row * 12;
-  const int64_t per_slab = n_quads_row * kQuadFrags;
-  uint2 *dst = xf + 2 * slab * per_slab * 3 + (lane & 1);
+  float mx[1] = {0.f};
 #pragma unroll
   for (int k = 0; k < kNfVec; ++k) {
-    const int fg = 32 * k + (lane >> 1);
-    if (fg >= n_frag) continue;
-    const int qs = fg >> 2, c8 = fg & 3, quad = qs / 3;
-    const int64_t within = static_cast<int64_t>(qs * 4 + t) * 64 + tl + 16 * c8 - static_cast<int64_t>(quad) * kQuadFrags;
-    const float y[4] = {v[k].x * r * g[k].x, v[k].y * r * g[k].y, v[k].z * r * g[k].z, v[k].w * r * g[k].w};
-    uint32_t hb[4], mb[4], lb[4];
+    v[k] = live ? make_float4(v[k].x * r * g[k].x, v[k].y * r * g[k].y, v[k].z * r * g[k].z, v[k].w * r * g[k].w)
+                : make_float4(0.f, 0.f, 0.f, 0.f);
+    mx[0] = fmaxf(fmaxf(fmaxf(mx[0], finite_abs(v[k].x)), finite_abs(v[k].y)),
+                  fmaxf(finite_abs(v[k].z), finite_abs(v[k].w)));
+  }
+  group_reduce<64, true>(mx);
+  const int e = row_exponent(mx[0]);
+  const float sc = pow2f(e);
+  if (lane == 0) tscale[tok] = pow2f(-e);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float xv = live ? y[e] : 0.f;
-      hb[e] = bf16_rne_bits(xv);
-      mb[e] = lb[e] = 0u;
-      if (fabsf(xv) <= 3.0e38f) {
-        const float r1 = xv - __uint_as_float(hb[e] << 16);
-        mb[e] = bf16_rne_bits(r1);
-        lb[e] = bf16_rne_bits(r1 - __uint_as_float(mb[e] << 16));
-      }
-    }
-    uint2 *d = dst + 2 * (static_cast<int64_t>(quad) * 3 * kQuadFrags + within);
-    d[0] = make_uint2(hb[0] | (hb[1] << 16), hb[2] | (hb[3] << 16));
-    d[2 * kQuadFrags] = make_uint2(mb[0] | (mb[1] << 16), mb[2] | (mb[3] << 16));
-    d[4 * kQuadFrags] = make_uint2(lb[0] | (lb[1] << 16), lb[2] | (lb[3] << 16));
+  for (int k = 0; k < kNfVec; ++k) {
+    const int i = lane + 64 * k;
+    const float a[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+    if (i < n_quads_row * 24) store_parts(xf, slab, n_quads_row, t, tl, i, a, sc);
   }
 }
 
@@ -1176,8 +1225,59 @@ __device__ __forceinline__ uint32_t hi_lo_pack(float v) {
   return hb | (bf16_rne_bits(v - __uint_as_float(hb << 16)) << 16);
 }
 
+// The byte tables (ids_to_pairs' order) of a row's 8 weight values by value id, from its fp16 row scale: F16:
+// the fp16 values times the power of two that brings the largest into [2^13, 2^14) (lo is not written; returns
+// its inverse; 1 and the values as they are where the largest is 0, inf or nan), else bf16 hi and lo (hi + lo
+// exactly the fp16 value).
+template <bool F16>
+__device__ __forceinline__ float row_value_tables(float sig, uint4 *hi, uint4 *lo) {
+  const float sl = __uint_as_float(kSLatticeBits);
+  const uint32_t v0 = dq_value(0, sig, sl), v1 = dq_value(1, sig, sl), v2 = dq_value(2, sig, sl);
+  const uint32_t v3 = dq_value(3, sig, sl), v4 = dq_value(4, sig, sl);
+  const uint32_t h[8] = {v0, v1, v2, v4, v4 ^ 0x8000u, v3 ^ 0x8000u, v2 ^ 0x8000u, v1 ^ 0x8000u};
+  float inv = 1.f, up = 1.f;
+  if constexpr (F16) {
+    const float top = fabsf(__half2float(__ushort_as_half(static_cast<uint16_t>(v4))));
+    if (top > 0.f && top <= 65504.f) {
+      const int e = 13 - (static_cast<int>(__float_as_uint(top) >> 23) - 127);
+      up = pow2f(e);
+      inv = pow2f(-e);
+    }
+  }
+  uint32_t hl[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float v = __half2float(__ushort_as_half(static_cast<uint16_t>(h[e])));
+    if constexpr (F16)
+      hl[e] = __half_as_ushort(__float2half_rn(v * up));  // (exact: a power of two)
+    else
+      hl[e] = hi_lo_pack(v);
+  }
+#pragma unroll
+  for (int half = 0; half < (F16 ? 1 : 2); ++half) {
+    uint32_t lb0 = 0, lb1 = 0, hb0 = 0, hb1 = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t b0 = hl[e] >> (16 * half), b1 = hl[e + 4] >> (16 * half);
+      lb0 |= (b0 & 0xFFu) << (8 * e);
+      lb1 |= (b1 & 0xFFu) << (8 * e);
+      hb0 |= ((b0 >> 8) & 0xFFu) << (8 * e);
+      hb1 |= ((b1 >> 8) & 0xFFu) << (8 * e);
+    }
+    *(half ? lo : hi) = make_uint4(lb0, lb1, hb0, hb1);
+  }
+  return inv;
+}
+
+// a fragment of scaled fp16 weights times 2^-11 (exact), against the activations' second part
+__device__ __forceinline__ f16x8_t times_2m11(f16x8_t w) {
+  constexpr _Float16 c = static_cast<_Float16>(0x1p-11f);
+  return w * f16x8_t{c, c, c, c, c, c, c, c};
+}
+
 // token tiles of 16; waves per block; quads of x in flight per wave; exact fp16 weights (hi + lo);
-// bf16 parts per activation (1: bf16 x; 3: fp32 x, see xfrag_kernel)
+// parts per activation (1: bf16 x; 2: fp32 x as two fp16 parts against the scaled fp16 weights and them times
+// 2^-11, see xsplit_kernel)
 // PLN: `packed` is the plane layout (3 uint16 records per atom); the value-id
 // words come from the plane table, staged in LDS, instead of kp_dq gathers.
 template <int MT, int WV, int PD, bool EXACT, int XP, bool XD, bool PLN>
@@ -1185,8 +1285,10 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
     const uint8_t *__restrict__ packed, int64_t packed_bytes, const uint16_t *__restrict__ sigma16, int64_t rows,
     int64_t atoms_per_row, const uint4 *__restrict__ xf, int64_t n_quads_row, int64_t m_total, int splits, int apb,
     const uint32_t *__restrict__ kp_dq, const uint32_t *__restrict__ pl_ids, int pl_vecs, float *__restrict__ y,
-    float *__restrict__ partial, const float *__restrict__ residual, int gelu) {
+    float *__restrict__ partial, const float *__restrict__ residual, const float *__restrict__ tscale, int gelu) {
   extern __shared__ __align__(16) uint8_t smem[];
+  constexpr bool F16 = XP == 2;
+  static_assert(!F16 || (EXACT && !XD), "fp32 x: exact weights, from the copy");
   constexpr int NT = 64 * WV;
   constexpr int TOK = 16 * MT;
   const int ws = mm_row_words(apb);
@@ -1195,6 +1297,7 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
   uint32_t *wt = reinterpret_cast<uint32_t *>(smem);          // [32][ws] kp_dq words
   float *red = reinterpret_cast<float *>(smem);               // after the k loop: [WV][TOK][kMmRedStride]
   uint4 *rtab = reinterpret_cast<uint4 *>(smem + region);     // [EXACT ? 2 : 1][32] row byte tables
+  float *rscale = reinterpret_cast<float *>(rtab + kMmRows);  // F16 (one table): the rows' scales, inverted
   // PLN: the plane table, after the kp_dq words (read in the prologue only; the cross-wave sum may reuse it)
   uint32_t *ptab = wt + kMmRows * ws;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, q = lane >> 4;
@@ -1258,31 +1361,14 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
 #pragma unroll
   for (int u = 0; u < PD; ++u) load_quad(xa[u], u);  // in flight during the prologue
 
-  // ---- per-row byte tables (threads 0..31, one row each): low / high bytes of hi (and lo) ----
+  // ---- per-row byte tables (threads 0..31, one row each) ----
   auto build_row_tables = [&]() {
     if (tid >= kMmRows) return;
     const int64_t row = row0 + tid;
-    const float sl = __uint_as_float(kSLatticeBits);
     const float sig = row < rows ? __half2float(__ushort_as_half(sigma16[row])) : 0.f;
-    const uint32_t v0 = dq_value(0, sig, sl), v1 = dq_value(1, sig, sl), v2 = dq_value(2, sig, sl);
-    const uint32_t v3 = dq_value(3, sig, sl), v4 = dq_value(4, sig, sl);
-    const uint32_t h[8] = {v0, v1, v2, v4, v4 ^ 0x8000u, v3 ^ 0x8000u, v2 ^ 0x8000u, v1 ^ 0x8000u};
-    uint32_t hl[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) hl[e] = hi_lo_pack(__half2float(__ushort_as_half(static_cast<uint16_t>(h[e]))));
-#pragma unroll
-    for (int half = 0; half < (EXACT ? 2 : 1); ++half) {
-      uint32_t lb0 = 0, lb1 = 0, hb0 = 0, hb1 = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t b0 = hl[e] >> (16 * half), b1 = hl[e + 4] >> (16 * half);
-        lb0 |= (b0 & 0xFFu) << (8 * e);
-        lb1 |= (b1 & 0xFFu) << (8 * e);
-        hb0 |= ((b0 >> 8) & 0xFFu) << (8 * e);
-        hb1 |= ((b1 >> 8) & 0xFFu) << (8 * e);
-      }
-      rtab[half * kMmRows + tid] = make_uint4(lb0, lb1, hb0, hb1);
-    }
+    uint4 lo;
+    const float inv = row_value_tables<F16>(sig, &rtab[tid], EXACT && !F16 ? &rtab[kMmRows + tid] : &lo);
+    if constexpr (F16) rscale[tid] = inv;
   };
 
   // ---- codes -> kp_dq words in LDS ----
@@ -1412,7 +1498,7 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) acc[t][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const uint4 ta0 = rtab[j], ta1 = rtab[16 + j];
-  const uint4 tb0 = rtab[EXACT ? kMmRows + j : j], tb1 = rtab[EXACT ? kMmRows + 16 + j : 16 + j];
+  const uint4 tb0 = rtab[EXACT && !F16 ? kMmRows + j : j], tb1 = rtab[EXACT && !F16 ? kMmRows + 16 + j : 16 + j];
   // word of (row, block atom a, plane p) = 3a + p; K step s of quad Q, lane group q: 12Q + 4s + q
   const uint32_t *wrow0 = wt + j * ws + 12 * wq0 + q;
   const uint32_t *wrow1 = wt + (16 + j) * ws + 12 * wq0 + q;
@@ -1422,6 +1508,23 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
       const uint32_t w0 = wrow0[12 * qd + 4 * s], w1 = wrow1[12 * qd + 4 * s];
       const bf16x8_t b0 = perm_decode(w0, ta0.x, ta0.y, ta0.z, ta0.w);
       const bf16x8_t b1 = perm_decode(w1, ta1.x, ta1.y, ta1.z, ta1.w);
+      if constexpr (F16) {
+        const f16x8_t h0 = __builtin_bit_cast(f16x8_t, b0), h1 = __builtin_bit_cast(f16x8_t, b1);
+        const f16x8_t m0 = times_2m11(h0), m1 = times_2m11(h1);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          const f16x8_t av = __builtin_bit_cast(f16x8_t, xa_q[s][0][t]);
+          acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, h0, acc[t][0], 0, 0, 0);
+          acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, h1, acc[t][1], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          const f16x8_t av = __builtin_bit_cast(f16x8_t, xa_q[s][XP - 1][t]);
+          acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, m0, acc[t][0], 0, 0, 0);
+          acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, m1, acc[t][1], 0, 0, 0);
+        }
+        continue;
+      }
 #pragma unroll
       for (int pp = 0; pp < XP; ++pp)
 #pragma unroll
@@ -1495,6 +1598,11 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
     for (int w = 1; w < WV; ++w) sum += *reinterpret_cast<const f32x4_t *>(red + (w * TOK + tl) * kMmRedStride + 4 * g);
     const int64_t row = row0 + 4 * g;
     if (tok0 + tl >= m_total || row >= rows) continue;
+    if constexpr (F16) {  // the scales back (powers of two)
+      const float ts = tscale[tok0 + tl];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) sum[c] = sum[c] * rscale[4 * g + c] * ts;
+    }
     float *d = dst + (tok_base + tl) * rows + row;
     if (splits == 1) {  // the final output: epilogue here (with a K split, in dqmm_reduce_kernel)
 #pragma unroll
@@ -1562,7 +1670,8 @@ MmPlan mm_plan(int64_t rows, int64_t apr) {
 template <int MT, int WV, int PD, bool EXACT, int XP, bool XD>
 int launch_dqmm_t(const uint8_t *packed, int64_t pb, const uint16_t *sigma16, int64_t rows, int64_t apr,
                   const uint4 *xf, int64_t m, float *y, float *partial, const MmPlan &pl, const uint32_t *kp_dq,
-                  const uint32_t *pl_ids, int pl_vecs, const float *residual, int gelu, hipStream_t s) {
+                  const uint32_t *pl_ids, int pl_vecs, const float *residual, const float *tscale, int gelu,
+                  hipStream_t s) {
   const int64_t row_blocks = (rows + kMmRows - 1) / kMmRows;
   const int64_t slabs = (m + 63) / 64;
   const int64_t nq = (apr + 3) / 4;
@@ -1575,41 +1684,41 @@ int launch_dqmm_t(const uint8_t *packed, int64_t pb, const uint16_t *sigma16, in
   const dim3 g(static_cast<unsigned>(row_blocks * pl.splits), static_cast<unsigned>(slabs));
   if (pl_ids)
     hipLaunchKernelGGL((dqmm_kernel<MT, WV, PD, EXACT, XP, XD, true>), g, dim3(64 * WV), shm, s, packed, pb, sigma16,
-                       rows, apr, xf, nq, m, pl.splits, pl.apb, kp_dq, pl_ids, pl_vecs, y, partial, residual, gelu);
+                       rows, apr, xf, nq, m, pl.splits, pl.apb, kp_dq, pl_ids, pl_vecs, y, partial, residual, tscale,
+                       gelu);
   else
     hipLaunchKernelGGL((dqmm_kernel<MT, WV, PD, EXACT, XP, XD, false>), g, dim3(64 * WV), shm, s, packed, pb, sigma16,
-                       rows, apr, xf, nq, m, pl.splits, pl.apb, kp_dq, pl_ids, pl_vecs, y, partial, residual, gelu);
+                       rows, apr, xf, nq, m, pl.splits, pl.apb, kp_dq, pl_ids, pl_vecs, y, partial, residual, tscale,
+                       gelu);
   return check_launch("dqmm_kernel");
 }
 
 template <int MT>
 int launch_dqmm(const uint8_t *packed, int64_t pb, const uint16_t *sigma16, int64_t rows, int64_t apr,
-                const uint4 *xf, int64_t m, float *y, float *partial, const MmPlan &pl, const uint32_t *kp_dq,
-                const uint32_t *pl_ids, int pl_vecs, bool exact, bool x_f32, bool direct, const float *residual,
-                int gelu, hipStream_t s) {
+                const uint4 *xf, const float *tscale, int64_t m, float *y, float *partial, const MmPlan &pl,
+                const uint32_t *kp_dq, const uint32_t *pl_ids, int pl_vecs, bool exact, bool x_f32, bool direct,
+                const float *residual, int gelu, hipStream_t s) {
   // 8 waves (two per SIMD cover each other's load latency), one quad of x in
   // flight per wave; 4 waves with 2 quads in flight measured within 3%.
   // `direct`: bf16 x read in place (xf = x), else the fragment-order copy.
-  if (x_f32)
-    return launch_dqmm_t<MT, 8, 1, true, 3, false>(packed, pb, sigma16, rows, apr, xf, m, y, partial, pl, kp_dq, pl_ids, pl_vecs,
-                                                   residual, gelu, s);
+  auto go = [&](auto exact_, auto parts, auto direct_) {
+    return launch_dqmm_t<MT, 8, 1, decltype(exact_)::value, decltype(parts)::value, decltype(direct_)::value>(
+        packed, pb, sigma16, rows, apr, xf, m, y, partial, pl, kp_dq, pl_ids, pl_vecs, residual, tscale, gelu, s);
+  };
+  using T = std::true_type;
+  using F = std::false_type;
+  using One = std::integral_constant<int, 1>;
+  if (x_f32) return go(T{}, std::integral_constant<int, 2>{}, F{});
   if constexpr (MT <= 2)  // direct is only chosen up to 32 tokens
-    if (direct)
-      return exact ? launch_dqmm_t<MT, 8, 1, true, 1, true>(packed, pb, sigma16, rows, apr, xf, m, y, partial, pl, kp_dq, pl_ids, pl_vecs,
-                                                            residual, gelu, s)
-                   : launch_dqmm_t<MT, 8, 1, false, 1, true>(packed, pb, sigma16, rows, apr, xf, m, y, partial, pl,
-                                                             kp_dq, pl_ids, pl_vecs, residual, gelu, s);
-  return exact ? launch_dqmm_t<MT, 8, 1, true, 1, false>(packed, pb, sigma16, rows, apr, xf, m, y, partial, pl, kp_dq, pl_ids, pl_vecs,
-                                                         residual, gelu, s)
-               : launch_dqmm_t<MT, 8, 1, false, 1, false>(packed, pb, sigma16, rows, apr, xf, m, y, partial, pl,
-                                                          kp_dq, pl_ids, pl_vecs, residual, gelu, s);
+    if (direct) return exact ? go(T{}, One{}, T{}) : go(F{}, One{}, T{});
+  return exact ? go(T{}, One{}, F{}) : go(F{}, One{}, F{});
 }
 
-// Workspace of the batched path: the fragment-order x copy (a multiple of 256
-// bytes), then, with a K split, the split partial tiles [slab][split][64][rows] fp32.
+// Workspace of the batched path: the fragment-order x copy, for fp32 x followed by the tokens' scales (256 bytes
+// a slab), then, with a K split, the split partial tiles [slab][split][64][rows] fp32.
 struct MmWorkspace {
-  size_t xf = 0, partial = 0;
-  size_t total() const { return xf + partial; }
+  size_t xf = 0, tscale = 0, partial = 0;
+  size_t x_bytes() const { return xf + tscale; }
 };
 
 // bf16 x of up to 32 tokens is read in place by dqmm_kernel; larger batches
@@ -1619,7 +1728,8 @@ bool mm_x_copy(bool x_f32, int64_t m) { return x_f32 || m > 32; }
 MmWorkspace mm_workspace(int64_t rows, int64_t cols, int64_t m, const MmPlan &pl, bool x_f32) {
   MmWorkspace w;
   const size_t slabs = static_cast<size_t>((m + 63) / 64);
-  if (mm_x_copy(x_f32, m)) w.xf = slabs * static_cast<size_t>((cols / kDim + 3) / 4) * kXfQuadBytes * (x_f32 ? 3 : 1);
+  if (mm_x_copy(x_f32, m)) w.xf = slabs * static_cast<size_t>((cols / kDim + 3) / 4) * kXfQuadBytes * (x_f32 ? 2 : 1);
+  if (x_f32) w.tscale = slabs * 64 * sizeof(float);
   if (pl.splits > 1) w.partial = slabs * pl.splits * 64 * static_cast<size_t>(rows) * sizeof(float);
   return w;
 }
@@ -1642,7 +1752,7 @@ size_t mm_workspace_bytes_multi(const int64_t *rows, int n, int64_t cols, int64_
   for (int i = 0; i < n; ++i) {
     if (rows[i] <= 0) continue;
     const MmWorkspace w = mm_workspace(rows[i], cols, m, mm_plan(rows[i], cols / kDim), (flags & PLX_DQL_X_F32) != 0);
-    xf = w.xf;
+    xf = w.x_bytes();
     partial = partial > w.partial ? partial : w.partial;
   }
   return xf + partial;
@@ -1701,15 +1811,16 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
     uint8_t *wsb = static_cast<uint8_t *>(workspace);
     const uint4 *xf = reinterpret_cast<const uint4 *>(wsb);
     const int64_t slabs = (m + 63) / 64, nq = (apr + 3) / 4;
-    const dim3 gx(static_cast<unsigned>(nq * 3), static_cast<unsigned>(slabs));
     const bool copy = mm_x_copy(x_is_f32 != 0, m);
+    const size_t xf_bytes = mm_workspace(1, cols, m, MmPlan{}, x_is_f32 != 0).xf;
+    float *tscale = reinterpret_cast<float *>(wsb + xf_bytes);  // fp32 x only
     // token tiles per slab the GEMM reads (its MT below): the copies write only these
     const int tiles = m > 32 ? 4 : m > 16 ? 2 : 1;
-    if (norm && copy && nq * 12 <= 32 * kNfVec) {
+    if (norm && nq * 24 <= 64 * kNfVec) {
       // the norm writes the fragment-order copy itself (rows that fit normfrag_kernel's registers)
       hipLaunchKernelGGL(normfrag_kernel, dim3(static_cast<unsigned>(slabs * 16)), dim3(256), 0, s,
                          static_cast<const float *>(x), norm_w, m, static_cast<int>(cols), nq, tiles, norm_eps,
-                         reinterpret_cast<uint2 *>(wsb));
+                         reinterpret_cast<uint2 *>(wsb), tscale);
       st = check_launch("normfrag_kernel");
     } else {
       if (norm) {
@@ -1717,13 +1828,18 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
         if (st != PLX_OK) return st;
         x = xnorm;
       }
-      if (copy) {
-        if (x_is_f32)
-          hipLaunchKernelGGL((xfrag_kernel<true>), gx, dim3(256), 0, s, x, m, cols, nq, tiles,
-                             reinterpret_cast<uint4 *>(wsb));
+      if (x_is_f32) {
+        const dim3 gs(static_cast<unsigned>(slabs * 16 * tiles));
+        if (nq * 24 <= 256 * kXsVec)
+          hipLaunchKernelGGL(xsplit_kernel<true>, gs, dim3(256), 0, s, static_cast<const float *>(x), m, cols, nq, tiles,
+                             reinterpret_cast<uint2 *>(wsb), tscale);
         else
-          hipLaunchKernelGGL((xfrag_kernel<false>), gx, dim3(256), 0, s, x, m, cols, nq, tiles,
-                             reinterpret_cast<uint4 *>(wsb));
+          hipLaunchKernelGGL(xsplit_kernel<false>, gs, dim3(256), 0, s, static_cast<const float *>(x), m, cols, nq, tiles,
+                             reinterpret_cast<uint2 *>(wsb), tscale);
+        st = check_launch("xsplit_kernel");
+      } else if (copy) {
+        hipLaunchKernelGGL(xfrag_kernel, dim3(static_cast<unsigned>(nq * 3), static_cast<unsigned>(slabs)), dim3(256), 0,
+                           s, static_cast<const uint16_t *>(x), m, cols, nq, tiles, reinterpret_cast<uint4 *>(wsb));
         st = check_launch("xfrag_kernel");
       } else {
         xf = static_cast<const uint4 *>(x);  // read in place by dqmm_kernel
@@ -1733,15 +1849,15 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
       const DqlTarget &t = targets[i];
       if (t.rows <= 0) continue;
       const MmPlan pl = mm_plan(t.rows, apr);
-      float *part = reinterpret_cast<float *>(wsb + mm_workspace(t.rows, cols, m, pl, x_is_f32 != 0).xf);
+      float *part = reinterpret_cast<float *>(wsb + mm_workspace(t.rows, cols, m, pl, x_is_f32 != 0).x_bytes());
       const int64_t pb = ((t.rows * apr + 3) / 4) * 9;  // packed stream length
-      st = m > 32 ? launch_dqmm<4>(t.packed, planes ? 6 * t.rows * apr : pb, t.sigma16, t.rows, apr, xf, m, t.y,
+      st = m > 32 ? launch_dqmm<4>(t.packed, planes ? 6 * t.rows * apr : pb, t.sigma16, t.rows, apr, xf, tscale, m, t.y,
                                    part, pl, tab->kp_dq, planes ? tab->pl_ids : nullptr, pl_vecs, !round_w, x_is_f32,
                                    !copy, t.residual, gelu, s)
-                  : m > 16 ? launch_dqmm<2>(t.packed, planes ? 6 * t.rows * apr : pb, t.sigma16, t.rows, apr, xf, m,
+                  : m > 16 ? launch_dqmm<2>(t.packed, planes ? 6 * t.rows * apr : pb, t.sigma16, t.rows, apr, xf, tscale, m,
                                             t.y, part, pl, tab->kp_dq, planes ? tab->pl_ids : nullptr, pl_vecs,
                                             !round_w, x_is_f32, !copy, t.residual, gelu, s)
-                           : launch_dqmm<1>(t.packed, planes ? 6 * t.rows * apr : pb, t.sigma16, t.rows, apr, xf, m,
+                           : launch_dqmm<1>(t.packed, planes ? 6 * t.rows * apr : pb, t.sigma16, t.rows, apr, xf, tscale, m,
                                             t.y, part, pl, tab->kp_dq, planes ? tab->pl_ids : nullptr, pl_vecs,
                                             !round_w, x_is_f32, !copy, t.residual, gelu, s);
       if (st != PLX_OK || pl.splits == 1) continue;
