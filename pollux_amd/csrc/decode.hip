@@ -277,6 +277,8 @@ __global__ __launch_bounds__(kAttnThreads, 5) void decode_attention_kernel(
 // for 4 steps), in two tiles of dims (0-15; 16-23, then a row of ones that sums the probabilities).
 // Online softmax per query: the maximum over the tile's 64 keys, exchanged between the four lanes of a query
 // once per tile; the accumulators are rescaled only in tiles where some maximum of the wave rose.
+//   Error: scores in two chains of three MFMAs, a tile's sums from zero and then added: 1.9e-7 from float64 at 1,024
+// positions (one chain through the running sums 3.4e-7; the VALU form 1.9e-7).
 //   A V row that is not finite must not reach the queries before it (0 * inf): the tile that holds both
 // (the block's own) then adds its keys one by one, each to the queries at or after it.
 //   What bounds it: the fp32 matrix rate (56 MFMAs of 32 cycles per 16 queries x 64 keys; 25% of the second
@@ -361,7 +363,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void prefill_attention_kernel(
   load(0);
   if (tid < 2 * kPfTile) vt[tid >> 6][kDim * kPfV + (tid & 63)] = 1.f;  // the probabilities' sum
 
-  // this wave's 16 queries: lane (n, g) holds dims 6g .. 6g+5 of query n, normalised (q_ln) and scaled
+  // this wave's 16 queries: lane (n, g) holds dims 6g .. 6g+5 of query n, normalised (q_ln)
   const int qrow = qt * kPfTile + wave * 16 + n;
   float qv[kSub];
   {
@@ -378,7 +380,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void prefill_attention_kernel(
     sq += __shfl_xor(sq, 32, 64);
     const float rq = 1.0f / sqrtf(sq / static_cast<float>(kDim) + eps);
 #pragma unroll
-    for (int i = 0; i < kSub; ++i) qv[i] = qv[i] * rq * q_w[g * kSub + i] * scale_log2;
+    for (int i = 0; i < kSub; ++i) qv[i] = qv[i] * rq * q_w[g * kSub + i];
   }
 
   f32x4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};  // dims 4g + r; 16 + 4g + r (24: the sum)
@@ -397,14 +399,14 @@ __global__ __launch_bounds__(kAttnThreads, 4) void prefill_attention_kernel(
       sc[kt] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
       if (kt >= live) continue;  // (wave-uniform)
       const float2 *a = reinterpret_cast<const float2 *>(&ks[buf][(16 * kt + n) * kPfK + g * kSub]);
-      f32x4 c = {0.f, 0.f, 0.f, 0.f};
+      f32x4 c = {0.f, 0.f, 0.f, 0.f}, d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < kSub / 2; ++i) {
         const float2 x = a[i];
         c = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, qv[2 * i], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, qv[2 * i + 1], c, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, qv[2 * i + 1], d, 0, 0, 0);
       }
-      sc[kt] = c;
+      sc[kt] = c + d;
     }
     // keys past the query (own tile) or past the prefix (its last tile)
     if (own || tile == n_pre - 1) {
@@ -424,7 +426,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void prefill_attention_kernel(
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     if (__any(mx > m)) {
       const float mn = fmaxf(m, mx);
-      const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+      const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mn) * scale_log2);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         o0[r] *= f;
@@ -432,23 +434,26 @@ __global__ __launch_bounds__(kAttnThreads, 4) void prefill_attention_kernel(
       }
       m = mn;
     }
+    const float mc = m * scale_log2;
+    // the tile's sums from zero, added to the running ones on the VALU: one rounding of those per tile
+    f32x4 t0 = {0.f, 0.f, 0.f, 0.f}, t1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
       if (kt >= live) continue;  // (wave-uniform)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        sc[kt][r] = __builtin_amdgcn_exp2f(sc[kt][r] - m);  // (a masked key: 2^-inf = 0)
+        sc[kt][r] = __builtin_amdgcn_exp2f(fmaf(sc[kt][r], scale_log2, -mc));  // (a masked key: 2^-inf = 0)
       if (!own || all_finite) {
         const float4 a = *reinterpret_cast<const float4 *>(&vt[buf][vrow0 + 16 * kt]);
         const float4 b = *reinterpret_cast<const float4 *>(&vt[buf][vrow1 + 16 * kt]);
-        o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, sc[kt][0], o0, 0, 0, 0);
-        o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, sc[kt][0], o1, 0, 0, 0);
-        o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, sc[kt][1], o0, 0, 0, 0);
-        o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, sc[kt][1], o1, 0, 0, 0);
-        o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, sc[kt][2], o0, 0, 0, 0);
-        o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(b.z, sc[kt][2], o1, 0, 0, 0);
-        o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, sc[kt][3], o0, 0, 0, 0);
-        o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(b.w, sc[kt][3], o1, 0, 0, 0);
+        t0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, sc[kt][0], t0, 0, 0, 0);
+        t1 = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, sc[kt][0], t1, 0, 0, 0);
+        t0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, sc[kt][1], t0, 0, 0, 0);
+        t1 = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, sc[kt][1], t1, 0, 0, 0);
+        t0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, sc[kt][2], t0, 0, 0, 0);
+        t1 = __builtin_amdgcn_mfma_f32_16x16x4f32(b.z, sc[kt][2], t1, 0, 0, 0);
+        t0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, sc[kt][3], t0, 0, 0, 0);
+        t1 = __builtin_amdgcn_mfma_f32_16x16x4f32(b.w, sc[kt][3], t1, 0, 0, 0);
       } else {
         float *ps = &ks[buf ^ 1][wave * 256];  // (the last tile: the other buffer is done with)
 #pragma unroll
@@ -459,12 +464,14 @@ __global__ __launch_bounds__(kAttnThreads, 4) void prefill_attention_kernel(
           if (16 * kt + kk > wave * 16 + n) continue;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            o0[e] = fmaf(pr, vt[buf][(4 * g + e) * kPfV + 16 * kt + kk], o0[e]);
-            o1[e] = fmaf(pr, vt[buf][min(16 + 4 * g + e, kDim) * kPfV + 16 * kt + kk], o1[e]);
+            t0[e] = fmaf(pr, vt[buf][(4 * g + e) * kPfV + 16 * kt + kk], t0[e]);
+            t1[e] = fmaf(pr, vt[buf][min(16 + 4 * g + e, kDim) * kPfV + 16 * kt + kk], t1[e]);
           }
         }
       }
     }
+    o0 += t0;
+    o1 += t1;
     if (!own) finite = store(tile + 1, buf ^ 1);
   }
   const float sum = __shfl(o1[0], 32 + n, 64);  // dim 24: lanes of g = 2, register 0
@@ -624,7 +631,7 @@ int launch_prefill_attention(const float *q, const float *k, const float *v, int
     return fail(PLX_EINVAL, "prefill_attention: q, k, v rows %lld floats apart (at least %lld, a multiple of 4)",
                 static_cast<long long>(qkv_stride), static_cast<long long>(heads * kDim));
   const int64_t q_tiles = (t + kPfTile - 1) / kPfTile;
-  // scores in units of log2: the softmax takes powers of two
+  // the softmax takes powers of two
   const float scale_log2 = static_cast<float>(1.4426950408889634 / sqrt(static_cast<double>(kDim)));
   // the grid's y dimension holds 65,535 (sequence, head) pairs: more go in several launches
   const int64_t seqs = 0xFFFFll / heads;
