@@ -1714,6 +1714,345 @@ int launch_dqmm(const uint8_t *packed, int64_t pb, const uint16_t *sigma16, int6
   return exact ? go(T{}, One{}, F{}) : go(F{}, One{}, F{});
 }
 
+// ---------------------------------------------------------------------------
+// dequant-GEMM for large batches of fp32 x: the weights are decoded once per call into a fragment-order copy
+// (wfrag_kernel, a chunk of rows at a time) and a dense GEMM runs on the two copies (dgemm_kernel).
+// dqmm_kernel decodes its rows again for every 64 tokens and reads every x fragment for 32 rows: more than the
+// copy costs (2 bytes a weight, written and read: 11 us for 7680x1920) above 320 tokens.  Per call, us,
+// dqmm_kernel / this path: 7680x1920 58 / 59 at 257 tokens, 85 / 65 at 512, 152 / 96 at 1,024; 1920x7680 63 / 63,
+// 96 / 74, 176 / 117; 1920x1920 39 / 33, 59 / 37, 100 / 46; 5760x1920 47 / 48, 67 / 60, 124 / 88.  (bf16 x stays
+// with dqmm_kernel, where it is one part and not scaled: 7680x1920 48 us at 512 tokens, here 59; 5760x1920 at
+// 1,024 70, here 90.)
+// wf[row tile of 16][K step of 32][lane]: lane (j, q) holds columns 8q .. 8q+7 of the step of row j as scaled fp16
+// (zero past the weight), 16 bytes.
+// ---------------------------------------------------------------------------
+constexpr int kBgRows = 128, kBgTok = 128;          // block tile
+constexpr int64_t kBigTokens = 321;
+constexpr int64_t kBgChunkWeights = 24 << 20;       // weights decoded per launch: a copy of 48 MB
+constexpr int64_t kBgMaxCols = 1 << 16;             // longer rows stay with dqmm_kernel (a chunk of 128 rows)
+
+// One block: 16 rows x 16 K steps (wave w: steps w, w + 4, ...: their 4 code loads in flight together).
+template <bool PLN>
+__global__ __launch_bounds__(256) void wfrag_kernel(const uint8_t *__restrict__ packed, int64_t packed_bytes,
+                                                    const uint16_t *__restrict__ sigma16, int64_t row_base, int64_t rows,
+                                                    int64_t atoms_per_row, int ksteps,
+                                                    const uint32_t *__restrict__ kp_dq,
+                                                    const uint32_t *__restrict__ pl_ids, int n_planes,
+                                                    uint4 *__restrict__ wf, float *__restrict__ rscale) {
+  __shared__ uint4 rtab[16];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, q = lane >> 4;
+  const int64_t row = row_base + static_cast<int64_t>(blockIdx.x) * 16 + j;
+  uint32_t w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int ks = static_cast<int>(blockIdx.y) * 16 + wave + 4 * i;
+    const int plane = 4 * ks + q, atom = plane / 3, p = plane - 3 * atom;
+    w[i] = 0u;
+    if (row < rows && atom < atoms_per_row) {
+      const int64_t n = row * atoms_per_row + atom;
+      if constexpr (PLN) {
+        const uint32_t rec = reinterpret_cast<const uint16_t *>(packed)[3 * n + p] & 0x1FFFu;
+        w[i] = pl_ids[min(rec, static_cast<uint32_t>(n_planes - 1))];
+      } else {
+        const int32_t code = packed_index_dw(packed, packed_bytes, n);
+        w[i] = kp_dq[static_cast<int64_t>(code > kKissing ? 0 : code) * 3 + p];
+      }
+    }
+  }
+  if (tid < 16) {  // (j = tid)
+    const float inv =
+        row_value_tables<true>(row < rows ? __half2float(__ushort_as_half(sigma16[row])) : 0.f, &rtab[j], nullptr);
+    if (blockIdx.y == 0) rscale[blockIdx.x * 16 + j] = inv;
+  }
+  __syncthreads();
+  const uint4 t = rtab[j];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int ks = static_cast<int>(blockIdx.y) * 16 + wave + 4 * i;
+    if (ks < ksteps) {
+      uint4 v = __builtin_bit_cast(uint4, perm_decode(w[i], t.x, t.y, t.z, t.w));
+      const uint32_t neg = (ks & 1) ? 0x80008000u : 0u;  // odd steps negated (dgemm_kernel)
+      v.x ^= neg;
+      v.y ^= neg;
+      v.z ^= neg;
+      v.w ^= neg;
+      wf[(static_cast<int64_t>(blockIdx.x) * ksteps + ks) * 64 + lane] = v;
+    }
+  }
+}
+
+// y[tok, row] for 128 tokens (two slabs of the x copy) x 128 rows of the decoded chunk.  4 waves, each 64 tokens
+// x 64 rows as 4 x 4 MFMA tiles of 16 (weights as the A operand, so a lane ends with 4 consecutive rows of one
+// token; per tile the activations' second part against the weights times 2^-11, then the first against the weights,
+// from zero, then added to the running sums on the VALU: a chain of MFMAs through the running sums took 10% less
+// time and left the results 4.0e-7 from float64 where this leaves 1.7e-7 and dqmm_kernel, whose waves split K,
+// 1.8e-7).  The MFMA rounds its sums down, whatever their sign (measured); a common error of all outputs would be
+// multiplied by the mean of the next layer's weights, so the weights of odd steps are stored negated and their
+// sums subtracted: the outputs' mean error goes from -6e-8 of their size to below 1e-9 (dqmm_kernel -1e-8), a
+// decoder block's output from 1.2e-6 to 2.5e-7.  Per K step the block's fragments (24 KB) go global -> registers (two steps ahead) -> LDS (three
+// buffers) -> registers (one step ahead); every fragment is a contiguous KiB, conflict-free; LDS traffic and loads
+// are spread between the MFMAs.  Two blocks share a CU (72 KB of LDS, 228 VGPRs).  K is split over blockIdx.x
+// where the tiles alone leave CUs idle (partial tiles in dqmm_kernel's layout, summed by dqmm_reduce_kernel).
+// What bounds it: matrix and VALU issue together; 7680x1920 at 1,024 tokens runs its 60 GFLOP of MFMA work at
+// 850 TFLOP/s, 70% of what a large bf16 product of the library reaches on the card.
+__global__ __launch_bounds__(256, 2) void dgemm_kernel(const uint4 *__restrict__ xf, const uint4 *__restrict__ wf,
+                                                       const float *__restrict__ tscale,
+                                                       const float *__restrict__ rscale, int64_t m_total, int64_t slabs,
+                                                       int n_quads_row, int64_t row_base, int64_t rows, int splits,
+                                                       int steps_per_split, float *__restrict__ y,
+                                                       float *__restrict__ partial, const float *__restrict__ residual,
+                                                       int gelu) {
+  constexpr int UA = 2 * 4 * 2, UB = 8, NU = UA + UB, UPW = NU / 4;  // KiB units per K step; per wave
+  __shared__ uint4 lds[3][NU * 64];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, j = lane & 15, q = lane >> 4;
+  const int64_t rb = blockIdx.x / static_cast<unsigned>(splits);  // row block of the chunk
+  const int split = static_cast<int>(blockIdx.x % static_cast<unsigned>(splits));
+  const int64_t slab0 = static_cast<int64_t>(blockIdx.y) * 2;
+  const int ksteps = 3 * n_quads_row;
+  const int k0 = split * steps_per_split, k1 = min(k0 + steps_per_split, ksteps);
+  // A step's units of 1 KiB: x fragments (slab, part, token tile), then weights (row tile); wave w loads token tile
+  // w of every slab and part, and row tiles w, w + 4.
+  // Raw buffer loads: the compiler moves plain loads of read-only memory down to where their values are stored.
+  const int64_t slab_bytes = static_cast<int64_t>(n_quads_row) * 2 * kXfQuadBytes;
+  const int64_t tile_bytes = static_cast<int64_t>(ksteps) * 1024;  // one row tile's weights
+  auto rsrc = [](const void *p, int64_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), static_cast<short>(0), static_cast<int>(bytes),
+                                             kBufferFlags);
+  };
+  const uint8_t *xb = reinterpret_cast<const uint8_t *>(xf);
+  const __amdgpu_buffer_rsrc_t xr0 = rsrc(xb + slab0 * slab_bytes, slab_bytes);
+  // (a block's second slab may lie past the batch: the first again)
+  const __amdgpu_buffer_rsrc_t xr1 = rsrc(xb + min(slab0 + 1, slabs - 1) * slab_bytes, slab_bytes);
+  const __amdgpu_buffer_rsrc_t wsr = rsrc(reinterpret_cast<const uint8_t *>(wf) + rb * 8 * tile_bytes, 8 * tile_bytes);
+  constexpr int XU = UA / 4, WU = UB / 4;
+  constexpr int kAhead = 2;  // steps whose loads are in flight (register slots)
+  u32x4_t st[kAhead][UPW];
+  auto load = [&](int ks, u32x4_t (&r)[UPW]) {
+    ks = min(ks, k1 - 1);  // (past the end: the last step again, never computed)
+    const int quad = ks / 3, s = ks - 3 * quad;
+#pragma unroll
+    for (int i = 0; i < XU; ++i)
+      r[i] = __builtin_amdgcn_raw_buffer_load_b128(i < 2 ? xr0 : xr1, 16 * lane,
+                                                   (quad * 2 + i % 2) * kXfQuadBytes + s * 4096 + wave * 1024, 0);
+#pragma unroll
+    for (int i = 0; i < WU; ++i)
+      r[XU + i] = __builtin_amdgcn_raw_buffer_load_b128(
+          wsr, 16 * lane, (wave + 4 * i) * static_cast<int>(tile_bytes) + ks * 1024, 0);
+  };
+  auto store = [&](int buf, const u32x4_t (&r)[UPW]) {
+#pragma unroll
+    for (int i = 0; i < UPW; ++i) lds[buf][(wave + 4 * i) * 64 + lane] = __builtin_bit_cast(uint4, r[i]);
+  };
+  f32x4_t acc[4][4];  // [row tile][token tile]
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int ws = wave & 1, wr = wave >> 1;  // this wave's slab and half of the rows
+  const int64_t slab = slab0 + ws;
+  const int64_t local0 = rb * kBgRows + wr * 64;  // this wave's first row within the chunk
+  struct Frags {
+    uint4 xa[2][4], wb[4];
+  };
+  auto fetch = [&](int buf, Frags &f) {
+    const uint4 *L = lds[buf] + lane;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) f.wb[r] = L[(UA + wr * 4 + r) * 64];
+#pragma unroll
+    for (int pa = 0; pa < 2; ++pa)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) f.xa[pa][t] = L[((ws * 2 + pa) * 4 + t) * 64];
+  };
+  auto compute = [&](const Frags &f, auto odd) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const f16x8_t h = __builtin_bit_cast(f16x8_t, f.wb[r]), m = times_2m11(h);
+      f32x4_t d[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(m, __builtin_bit_cast(f16x8_t, f.xa[1][t]),
+                                                      f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(h, __builtin_bit_cast(f16x8_t, f.xa[0][t]), d[t], 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[r][t] = decltype(odd)::value ? acc[r][t] - d[t] : acc[r][t] + d[t];
+    }
+  };
+  // Step k is in LDS buffer k % 3 one barrier before its fragments are read, its fragments in registers one step
+  // before its MFMAs.
+  constexpr int kReads = 12;  // LDS reads of a step's fragments
+  Frags fr[2];
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) load(k0 + u, st[u]);
+  store(0, st[0]);
+  load(k0 + 2, st[0]);
+  store(1, st[1]);
+  load(k0 + 3, st[1]);
+  __syncthreads();
+  fetch(0, fr[0]);
+  int b1 = 1, b2 = 2;  // the buffers of steps ks + 1, ks + 2
+  int ks = k0;
+  for (; ks + 1 < k1; ks += 2) {  // (no branch inside: the waits then count the loads in flight exactly)
+    auto step = [&](auto odd) {
+      constexpr int u = decltype(odd)::value ? 1 : 0;
+      fetch(b1, fr[u ^ 1]);
+      compute(fr[u], odd);
+      store(b2, st[u]);  // (last read as step ks - 1, before the last barrier)
+      load(ks + u + 4, st[u]);
+      // LDS reads, writes and loads spread between the MFMAs: the block's waves run in step, so phases of their
+      // own would leave the matrix cores idle meanwhile
+#pragma unroll
+      for (int i = 0; i < kReads; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+      }
+#pragma unroll
+      for (int i = 0; i < UPW; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // load
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      __syncthreads();
+      b1 = b2;
+      b2 = b2 == 2 ? 0 : b2 + 1;
+    };
+    step(std::false_type{});
+    step(std::true_type{});
+  }
+  if (ks < k1) compute(fr[0], std::false_type{});  // an odd number of steps
+
+  // lane (j, q): token 16t + j, rows 16r + 4q .. +3
+  // the scales back (powers of two), requested together
+  float ts[4];
+  float4 rs[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    ts[i] = tscale[min(slab * 64 + 16 * i + j, m_total - 1)];
+    rs[i] = *reinterpret_cast<const float4 *>(rscale + local0 + 16 * i + 4 * q);
+  }
+  float *dst = splits == 1 ? y : partial + (slab * splits + split) * 64 * rows;
+  const bool fin = splits == 1;  // the final output (with a K split the epilogue runs in dqmm_reduce_kernel)
+  const bool vec = (rows & 3) == 0 && ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(residual)) & 15u) == 0;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int tl = 16 * t + j;
+    const int64_t tok = slab * 64 + tl;
+    float4 res[4];  // (requested together, from clamped addresses: no load waits for another)
+    if (fin && vec && residual) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        res[r] = *reinterpret_cast<const float4 *>(residual + min(tok, m_total - 1) * rows +
+                                                   min(row_base + local0 + 16 * r + 4 * q, rows - 4));
+    }
+    if (tok >= m_total) continue;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t row = row_base + local0 + 16 * r + 4 * q;
+      if (row >= rows) continue;
+      f32x4_t v = acc[r][t];
+      v[0] = v[0] * rs[r].x * ts[t];
+      v[1] = v[1] * rs[r].y * ts[t];
+      v[2] = v[2] * rs[r].z * ts[t];
+      v[3] = v[3] * rs[r].w * ts[t];
+      float *d = dst + (fin ? tok : tl) * rows + row;
+      if (vec) {
+        if (fin) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] = dql_epilogue(v[c], nullptr, 0, gelu);
+          if (residual) v += f32x4_t{res[r].x, res[r].y, res[r].z, res[r].w};
+        }
+        *reinterpret_cast<f32x4_t *>(d) = v;
+      } else {
+        for (int c = 0; c < 4 && row + c < rows; ++c)
+          d[c] = fin ? dql_epilogue(v[c], residual, tok * rows + row + c, gelu) : v[c];
+      }
+    }
+  }
+}
+
+// The large-batch plan of one weight: rows decoded per launch (whole blocks), K splits and steps per split.
+struct BgPlan {
+  int64_t chunk = 0;
+  int splits = 1, steps = 0;
+};
+
+BgPlan bg_plan(int64_t rows, int64_t cols, int64_t m) {
+  BgPlan p;
+  const int64_t nq = (cols / kDim + 3) / 4;
+  const int64_t blocks_rows = (rows + kBgRows - 1) / kBgRows;
+  const int64_t fit = max(static_cast<int64_t>(1), kBgChunkWeights / (nq * 96) / kBgRows);
+  // even chunks
+  const int64_t n_chunks = (blocks_rows + fit - 1) / fit;
+  const int64_t per = (blocks_rows + n_chunks - 1) / n_chunks;
+  p.chunk = per * kBgRows;
+  // K splits: about 1 us a step with two blocks on each of 256 CUs, and the split sum's bytes (written, read and
+  // summed) at 4 TB/s
+  const int64_t tiles = per * ((m + kBgTok - 1) / kBgTok), steps = 3 * nq;
+  double best = 0;
+  for (int64_t sp = 1; sp <= max(static_cast<int64_t>(1), min(static_cast<int64_t>(16), steps / 8)); ++sp) {
+    const int64_t per_split = ((steps + sp - 1) / sp + 1) & ~static_cast<int64_t>(1);  // (even: a split starts at an even step)
+    const double cost = static_cast<double>((tiles * sp + 511) / 512) * static_cast<double>(per_split) +
+                        (sp > 1 ? 3.0 + static_cast<double>(2 * sp + 1) * static_cast<double>(m * rows) * 1e-6 / n_chunks : 0.0);
+    if (sp == 1 || cost < best) {
+      best = cost;
+      p.steps = static_cast<int>(per_split);
+      p.splits = static_cast<int>((steps + per_split - 1) / per_split);
+    }
+  }
+  return p;
+}
+
+bool uses_big(int64_t cols, int64_t m, bool x_f32) { return x_f32 && m >= kBigTokens && cols <= kBgMaxCols; }
+
+size_t bg_w_bytes(const BgPlan &p, int64_t cols) {  // the decoded chunk, then its row scales
+  return static_cast<size_t>(p.chunk) * (static_cast<size_t>((cols / kDim + 3) / 4) * 96 * 2 + sizeof(float));
+}
+size_t bg_partial_bytes(const BgPlan &p, int64_t rows, int64_t m) {
+  return p.splits > 1 ? static_cast<size_t>((m + 63) / 64) * p.splits * 64 * static_cast<size_t>(rows) * sizeof(float) : 0;
+}
+
+int launch_reduce(const float *partial, int splits, int64_t rows, int64_t m, float *y, const float *residual, int gelu,
+                  hipStream_t s) {
+  const int64_t cnt = m * rows;
+  if (rows % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0)
+    hipLaunchKernelGGL((dqmm_reduce_kernel<true>), dim3(static_cast<unsigned>((cnt / 4 + 255) / 256)), dim3(256), 0, s,
+                       partial, splits, rows, m, y, residual, gelu);
+  else
+    hipLaunchKernelGGL((dqmm_reduce_kernel<false>), dim3(static_cast<unsigned>((cnt + 255) / 256)), dim3(256), 0, s,
+                       partial, splits, rows, m, y, residual, gelu);
+  return check_launch("dqmm_reduce_kernel");
+}
+
+// One weight of a large batch; ws: bg_w_bytes, then the split partials.
+int launch_big(const DqlTarget &t, int64_t cols, int64_t m, const uint4 *xf, const float *tscale, const DeviceTables *tab,
+               bool planes, uint8_t *ws, int gelu, hipStream_t s) {
+  const BgPlan p = bg_plan(t.rows, cols, m);
+  const int64_t apr = cols / kDim;
+  const int nq = static_cast<int>((apr + 3) / 4);
+  uint4 *wf = reinterpret_cast<uint4 *>(ws);
+  float *rscale = reinterpret_cast<float *>(ws + static_cast<size_t>(p.chunk) * nq * 96 * 2);
+  float *partial = reinterpret_cast<float *>(ws + bg_w_bytes(p, cols));
+  const int64_t pb = ((t.rows * apr + 3) / 4) * 9, slabs = (m + 63) / 64;
+  const int n_planes = static_cast<int>(plane_tables_host()->ids.size());
+  auto wfrag = planes ? wfrag_kernel<true> : wfrag_kernel<false>;
+  int st = PLX_OK;
+  for (int64_t r0 = 0; r0 < t.rows; r0 += p.chunk) {
+    const int64_t blocks = (min(p.chunk, t.rows - r0) + kBgRows - 1) / kBgRows;
+    hipLaunchKernelGGL(wfrag, dim3(static_cast<unsigned>(blocks * (kBgRows / 16)), static_cast<unsigned>((3 * nq + 15) / 16)),
+                       dim3(256), 0, s, t.packed, pb, t.sigma16, r0, t.rows, apr, 3 * nq, tab->kp_dq, tab->pl_ids,
+                       n_planes, wf, rscale);
+    if ((st = check_launch("wfrag_kernel")) != PLX_OK) return st;
+    hipLaunchKernelGGL(dgemm_kernel, dim3(static_cast<unsigned>(blocks * p.splits), static_cast<unsigned>((slabs + 1) / 2)),
+                       dim3(256), 0, s, xf, wf, tscale, rscale, m, slabs, nq, r0, t.rows, p.splits, p.steps, t.y, partial,
+                       t.residual, gelu);
+    if ((st = check_launch("dgemm_kernel")) != PLX_OK) return st;
+  }
+  if (p.splits == 1) return PLX_OK;
+  return launch_reduce(partial, p.splits, t.rows, m, t.y, t.residual, gelu, s);
+}
+
 // Workspace of the batched path: the fragment-order x copy, for fp32 x followed by the tokens' scales (256 bytes
 // a slab), then, with a K split, the split partial tiles [slab][split][64][rows] fp32.
 struct MmWorkspace {
@@ -1752,8 +2091,13 @@ size_t mm_workspace_bytes_multi(const int64_t *rows, int n, int64_t cols, int64_
   for (int i = 0; i < n; ++i) {
     if (rows[i] <= 0) continue;
     const MmWorkspace w = mm_workspace(rows[i], cols, m, mm_plan(rows[i], cols / kDim), (flags & PLX_DQL_X_F32) != 0);
+    size_t rest = w.partial;
+    if (uses_big(cols, m, (flags & PLX_DQL_X_F32) != 0)) {
+      const BgPlan p = bg_plan(rows[i], cols, m);
+      rest = bg_w_bytes(p, cols) + bg_partial_bytes(p, rows[i], m);
+    }
     xf = w.x_bytes();
-    partial = partial > w.partial ? partial : w.partial;
+    partial = partial > rest ? partial : rest;
   }
   return xf + partial;
 }
@@ -1848,6 +2192,11 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
     for (int i = 0; i < n && st == PLX_OK; ++i) {
       const DqlTarget &t = targets[i];
       if (t.rows <= 0) continue;
+      if (uses_big(cols, m, x_is_f32 != 0)) {
+        st = launch_big(t, cols, m, xf, tscale, tab, planes,
+                        wsb + mm_workspace(t.rows, cols, m, MmPlan{}, true).x_bytes(), gelu, s);
+        continue;
+      }
       const MmPlan pl = mm_plan(t.rows, apr);
       float *part = reinterpret_cast<float *>(wsb + mm_workspace(t.rows, cols, m, pl, x_is_f32 != 0).x_bytes());
       const int64_t pb = ((t.rows * apr + 3) / 4) * 9;  // packed stream length
@@ -1861,14 +2210,7 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
                                             t.y, part, pl, tab->kp_dq, planes ? tab->pl_ids : nullptr, pl_vecs,
                                             !round_w, x_is_f32, !copy, t.residual, gelu, s);
       if (st != PLX_OK || pl.splits == 1) continue;
-      const int64_t cnt = m * t.rows;
-      if (t.rows % 4 == 0 && (reinterpret_cast<uintptr_t>(t.y) & 15u) == 0)
-        hipLaunchKernelGGL((dqmm_reduce_kernel<true>), dim3(static_cast<unsigned>((cnt / 4 + 255) / 256)), dim3(256), 0,
-                           s, part, pl.splits, t.rows, m, t.y, t.residual, gelu);
-      else
-        hipLaunchKernelGGL((dqmm_reduce_kernel<false>), dim3(static_cast<unsigned>((cnt + 255) / 256)), dim3(256), 0, s,
-                           part, pl.splits, t.rows, m, t.y, t.residual, gelu);
-      st = check_launch("dqmm_reduce_kernel");
+      st = launch_reduce(part, pl.splits, t.rows, m, t.y, t.residual, gelu, s);
     }
     return st;
   }

@@ -36,7 +36,7 @@ def _bar(x, w, cols):
 @pytest.mark.parametrize("rows,cols,m", [
     (32, 24, 5), (48, 96, 16), (33, 120, 17), (130, 480, 33), (257, 1920, 64), (127, 984, 65), (129, 1920, 128),
     (384, 504, 129), (1921, 960, 160), (1920, 1920, 192), (640, 7680, 200), (61, 2424, 257), (2000, 336, 513),
-    (5760, 1920, 300), (1, 48, 300), (24, 9624, 200)])
+    (5760, 1920, 300), (1, 48, 300), (24, 9624, 200), (2000, 1920, 1024), (300, 7680, 384), (129, 120, 321), (24, 9624, 350)])
 def test_against_float64(dev, rows, cols, m, dtype, planes):
     pk, sg = _weight(dev, rows, cols, rows + cols)
     g = torch.Generator(device=dev).manual_seed(m)
@@ -51,7 +51,7 @@ def test_against_float64(dev, rows, cols, m, dtype, planes):
     assert worst <= 1.0
 
 
-@pytest.mark.parametrize("m", [7, 64, 200])
+@pytest.mark.parametrize("m", [7, 64, 200, 330])
 @pytest.mark.parametrize("what", ["tiny", "huge", "outliers", "subnormal", "mixed"])
 def test_activation_ranges(dev, m, what):
     rows, cols = 200, 960
@@ -78,7 +78,7 @@ def test_activation_ranges(dev, m, what):
     assert ((y.double() - xd @ w.T).abs() <= bar).all()
 
 
-@pytest.mark.parametrize("m", [7, 200])
+@pytest.mark.parametrize("m", [7, 200, 330])
 def test_row_scale_ranges(dev, m):
     # fp16 row scales from subnormal (weights of a few bits, or none) to where the largest weights overflow
     sg = torch.tensor([0.0, 6e-8, 1e-7, 3e-6, 1e-4, 1.0, 300.0, 40_000.0], device=dev).half().repeat(8)
@@ -93,7 +93,7 @@ def test_row_scale_ranges(dev, m):
     assert not torch.isfinite(y[:, ~fine]).any()
 
 
-@pytest.mark.parametrize("m", [7, 200])
+@pytest.mark.parametrize("m", [7, 200, 330])
 def test_bad_tokens_stay_alone(dev, m):
     rows, cols = 160, 480
     pk, sg = _weight(dev, rows, cols, 5)
@@ -107,7 +107,7 @@ def test_bad_tokens_stay_alone(dev, m):
     assert torch.equal(y[keep], ref[keep]) and not torch.isfinite(y[[1, 3]]).any()
 
 
-@pytest.mark.parametrize("m", [16, 150, 260])
+@pytest.mark.parametrize("m", [16, 150, 330])
 def test_epilogues_and_targets(dev, m):
     # the norm prologue, GELU and residuals over several weights: the same as separate calls
     cols, shapes = 960, (130, 960, 64)
