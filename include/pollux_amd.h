@@ -404,11 +404,20 @@ int plx_dequant_int8_rows(const int8_t *q, const uint16_t *mu16, int64_t rows, i
  * cols % 16 == 0 and <= 4,096; q, x, norm_weight 16-byte aligned.  Up to 4
  * tokens a GEMV streams the INT8 rows once per 4 tokens; from 5 tokens an MFMA
  * kernel reads them once per 64 tokens (both exact products, fp32 sums; with a
- * norm the MFMA kernel scales each token's sums by the rsqrt at the end). */
+ * norm the MFMA kernel scales each token's sums by the rsqrt at the end).
+ * plx_int8_linear_ws: the same with a workspace (the size below, 16-byte
+ * aligned; nothing needs clearing; null: as plx_int8_linear).  From 5 tokens x
+ * is then normalised and split once, into two fp16 parts per row scaled by a
+ * power of two (x to its last fp32 bit; elements below 2^-28 of their row's
+ * largest to 2^-52 of that), and the products are exact. */
 int plx_int8_linear(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x,
                     int64_t m_rows, const float *norm_weight, float norm_eps, float *y, void *stream);
+size_t plx_int8_linear_workspace_bytes(int64_t rows, int64_t cols, int64_t m_rows);
+int plx_int8_linear_ws(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x,
+                       int64_t m_rows, const float *norm_weight, float norm_eps, float *y, void *workspace,
+                       size_t workspace_bytes, void *stream);
 
-/* plx_int8_linear with greedy decoding's token choice fused in: y as above,
+/* plx_int8_linear_ws with greedy decoding's token choice fused in: y as above,
  * then ids[t] = the index of the maximum of y[t, :] (int64 [m_rows]) by
  * torch.argmax's rule (the first index among equal maxima; a NaN counts as
  * the maximum) -- generate.py:313-320 with top_k = 1 after the head

@@ -476,13 +476,24 @@ int64_t plx_plane_table(uint32_t *ids, int64_t capacity) {
   return n;
 }
 
-int plx_int8_linear(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x, int64_t m_rows,
-                    const float *norm_weight, float norm_eps, float *y, void *stream) {
+int plx_int8_linear_ws(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x, int64_t m_rows,
+                       const float *norm_weight, float norm_eps, float *y, void *workspace, size_t workspace_bytes,
+                       void *stream) {
   PLX_REQUIRE(rows >= 0 && cols > 0 && m_rows >= 0, "plx_int8_linear: bad shape (%lld, %lld) x %lld tokens",
               static_cast<long long>(rows), static_cast<long long>(cols), static_cast<long long>(m_rows));
   if (rows == 0 || m_rows == 0) return PLX_OK;
   PLX_REQUIRE(q != nullptr && mu16 != nullptr && x != nullptr && y != nullptr, "plx_int8_linear: null pointer");
-  return launch_int8_linear(q, mu16, rows, cols, x, m_rows, norm_weight, norm_eps, y, nullptr, as_stream(stream));
+  return launch_int8_linear(q, mu16, rows, cols, x, m_rows, norm_weight, norm_eps, y, workspace, workspace_bytes,
+                            as_stream(stream));
+}
+
+int plx_int8_linear(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x, int64_t m_rows,
+                    const float *norm_weight, float norm_eps, float *y, void *stream) {
+  return plx_int8_linear_ws(q, mu16, rows, cols, x, m_rows, norm_weight, norm_eps, y, nullptr, 0, stream);
+}
+
+size_t plx_int8_linear_workspace_bytes(int64_t rows, int64_t cols, int64_t m_rows) {
+  return int8_linear_workspace_bytes(rows, cols, m_rows);
 }
 
 size_t plx_int8_linear_argmax_workspace_bytes(int64_t rows, int64_t m_rows) {

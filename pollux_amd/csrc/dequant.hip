@@ -2067,7 +2067,7 @@ bool mm_x_copy(bool x_f32, int64_t m) { return x_f32 || m > 32; }
 MmWorkspace mm_workspace(int64_t rows, int64_t cols, int64_t m, const MmPlan &pl, bool x_f32) {
   MmWorkspace w;
   const size_t slabs = static_cast<size_t>((m + 63) / 64);
-  if (mm_x_copy(x_f32, m)) w.xf = slabs * static_cast<size_t>((cols / kDim + 3) / 4) * kXfQuadBytes * (x_f32 ? 2 : 1);
+  if (mm_x_copy(x_f32, m)) w.xf = slabs * static_cast<size_t>((cols + 95) / 96) * kXfQuadBytes * (x_f32 ? 2 : 1);
   if (x_f32) w.tscale = slabs * 64 * sizeof(float);
   if (pl.splits > 1) w.partial = slabs * pl.splits * 64 * static_cast<size_t>(rows) * sizeof(float);
   return w;
@@ -2114,6 +2114,38 @@ size_t dequant_linear_workspace_bytes(int64_t rows, int64_t cols, int64_t m, int
   return dequant_linear_workspace_bytes_multi(&rows, 1, cols, m, flags);
 }
 
+size_t x_parts_bytes(int64_t cols, int64_t m) {
+  const MmWorkspace w = mm_workspace(1, cols, m, MmPlan{}, true);
+  return w.x_bytes();
+}
+
+bool x_parts_fuses_norm(int64_t cols) { return (cols + 95) / 96 * 24 <= 64 * kNfVec; }
+
+int launch_x_parts(const float *x, const float *norm_w, float norm_eps, int64_t m, int64_t cols, float *xnorm, void *ws,
+                   hipStream_t s) {
+  const int64_t slabs = (m + 63) / 64, nq = (cols + 95) / 96;
+  const int tiles = x_parts_tiles(m);
+  float *tscale = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + mm_workspace(1, cols, m, MmPlan{}, true).xf);
+  uint2 *xf = static_cast<uint2 *>(ws);
+  if (norm_w && x_parts_fuses_norm(cols)) {
+    // the norm writes the fragment-order copy itself (rows that fit normfrag_kernel's registers)
+    hipLaunchKernelGGL(normfrag_kernel, dim3(static_cast<unsigned>(slabs * 16)), dim3(256), 0, s, x, norm_w, m,
+                       static_cast<int>(cols), nq, tiles, norm_eps, xf, tscale);
+    return check_launch("normfrag_kernel");
+  }
+  if (norm_w) {
+    const int st = launch_rms_norm(x, norm_w, xnorm, m, cols, norm_eps, s);
+    if (st != PLX_OK) return st;
+    x = xnorm;
+  }
+  const dim3 gs(static_cast<unsigned>(slabs * 16 * tiles));
+  if (nq * 24 <= 256 * kXsVec)
+    hipLaunchKernelGGL(xsplit_kernel<true>, gs, dim3(256), 0, s, x, m, cols, nq, tiles, xf, tscale);
+  else
+    hipLaunchKernelGGL(xsplit_kernel<false>, gs, dim3(256), 0, s, x, m, cols, nq, tiles, xf, tscale);
+  return check_launch("xsplit_kernel");
+}
+
 int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, const void *x, int flags, int64_t m,
                                 const float *norm_w, float norm_eps, void *workspace, size_t workspace_bytes,
                                 hipStream_t s) {
@@ -2158,36 +2190,15 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
     const bool copy = mm_x_copy(x_is_f32 != 0, m);
     const size_t xf_bytes = mm_workspace(1, cols, m, MmPlan{}, x_is_f32 != 0).xf;
     float *tscale = reinterpret_cast<float *>(wsb + xf_bytes);  // fp32 x only
-    // token tiles per slab the GEMM reads (its MT below): the copies write only these
-    const int tiles = m > 32 ? 4 : m > 16 ? 2 : 1;
-    if (norm && nq * 24 <= 64 * kNfVec) {
-      // the norm writes the fragment-order copy itself (rows that fit normfrag_kernel's registers)
-      hipLaunchKernelGGL(normfrag_kernel, dim3(static_cast<unsigned>(slabs * 16)), dim3(256), 0, s,
-                         static_cast<const float *>(x), norm_w, m, static_cast<int>(cols), nq, tiles, norm_eps,
-                         reinterpret_cast<uint2 *>(wsb), tscale);
-      st = check_launch("normfrag_kernel");
+    if (x_is_f32) {
+      st = launch_x_parts(static_cast<const float *>(x), norm_w, norm_eps, m, cols, xnorm, wsb, s);
+    } else if (copy) {
+      const int tiles = m > 32 ? 4 : 2;  // token tiles per slab the GEMM reads (its MT below): the copy writes only these
+      hipLaunchKernelGGL(xfrag_kernel, dim3(static_cast<unsigned>(nq * 3), static_cast<unsigned>(slabs)), dim3(256), 0, s,
+                         static_cast<const uint16_t *>(x), m, cols, nq, tiles, reinterpret_cast<uint4 *>(wsb));
+      st = check_launch("xfrag_kernel");
     } else {
-      if (norm) {
-        st = launch_rms_norm(static_cast<const float *>(x), norm_w, xnorm, m, cols, norm_eps, s);
-        if (st != PLX_OK) return st;
-        x = xnorm;
-      }
-      if (x_is_f32) {
-        const dim3 gs(static_cast<unsigned>(slabs * 16 * tiles));
-        if (nq * 24 <= 256 * kXsVec)
-          hipLaunchKernelGGL(xsplit_kernel<true>, gs, dim3(256), 0, s, static_cast<const float *>(x), m, cols, nq, tiles,
-                             reinterpret_cast<uint2 *>(wsb), tscale);
-        else
-          hipLaunchKernelGGL(xsplit_kernel<false>, gs, dim3(256), 0, s, static_cast<const float *>(x), m, cols, nq, tiles,
-                             reinterpret_cast<uint2 *>(wsb), tscale);
-        st = check_launch("xsplit_kernel");
-      } else if (copy) {
-        hipLaunchKernelGGL(xfrag_kernel, dim3(static_cast<unsigned>(nq * 3), static_cast<unsigned>(slabs)), dim3(256), 0,
-                           s, static_cast<const uint16_t *>(x), m, cols, nq, tiles, reinterpret_cast<uint4 *>(wsb));
-        st = check_launch("xfrag_kernel");
-      } else {
-        xf = static_cast<const uint4 *>(x);  // read in place by dqmm_kernel
-      }
+      xf = static_cast<const uint4 *>(x);  // read in place by dqmm_kernel
     }
     for (int i = 0; i < n && st == PLX_OK; ++i) {
       const DqlTarget &t = targets[i];

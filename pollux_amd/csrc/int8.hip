@@ -302,6 +302,7 @@ __global__ __launch_bounds__(64 * kLinWaves) void int8_linear_kernel(
 typedef __bf16 bf16x8_i8 __attribute__((ext_vector_type(8)));
 typedef float f32x4_i8 __attribute__((ext_vector_type(4)));
 
+constexpr int64_t kI8MaxCols = 64 * 16 * 4;
 constexpr int kI8mmRows = 64;     // output rows per block (four MFMA row tiles)
 constexpr int kI8mmWaves = 4;     // waves per block, splitting K
 constexpr int kI8mmRedStride = 68; // floats per token row of the cross-wave sum (64 rows + pad)
@@ -354,11 +355,11 @@ __device__ __forceinline__ void int8x8_hilo(uint32_t d0, uint32_t d1, __half2 s2
   lo = __builtin_bit_cast(bf16x8_i8, u4{pl[0], pl[1], pl[2], pl[3]});
 }
 
-template <int MT, bool NORM, bool ARG>
+// x split by every block (no workspace): the form of a call without one.
+template <int MT, bool NORM>
 __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8mm_kernel(
     const int8_t *__restrict__ q, const uint16_t *__restrict__ mu16, int64_t rows, int cols,
-    const float *__restrict__ x, int64_t m_total, const float *__restrict__ norm_w, float eps, float *__restrict__ y,
-    uint64_t *__restrict__ keys) {
+    const float *__restrict__ x, int64_t m_total, const float *__restrict__ norm_w, float eps, float *__restrict__ y) {
   constexpr int TOK = 16 * MT;
   __shared__ __align__(16) float red[kI8mmWaves][TOK][kI8mmRedStride];
   __shared__ float sq[kI8mmWaves][TOK];
@@ -517,7 +518,6 @@ __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8mm_kernel(
     for (int w = 1; w < kI8mmWaves; ++w) t2 += sq[w][tl];
     rs = 1.0f / sqrtf(t2 / static_cast<float>(cols) + eps);
   }
-  uint64_t kb = 0;
 #pragma unroll
   for (int i = 0; i < kRpt; ++i) {
     const int rr = part + kTpt * i;
@@ -525,6 +525,159 @@ __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8mm_kernel(
 #pragma unroll
     for (int w = 1; w < kI8mmWaves; ++w) sum += red[w][tl][rr];
     if constexpr (NORM) sum *= rs;
+    const int64_t row = row0 + rr;
+    if (tok < m_total && row < rows) y[tok * rows + row] = sum;
+  }
+}
+
+// int8parts_kernel: the same product from the activations' two scaled fp16 parts (launch_x_parts), split once per
+// call instead of once per block.  The fp16 weights are decoded from their bytes, scaled by a power of two per row
+// (exact) and need no split: two v_mfma_f32_16x16x32_f16 per tile (the parts against the weights and against them
+// times 2^-11) where three bf16 parts against hi + lo took six, no split arithmetic, and a third of the fp32
+// roundings.  A block owns 64 rows x 16 MT tokens, its 4 waves split K; blocks of one XCD take the token slabs of a
+// row block in turn, so its bytes come from that XCD's L2 after the first.
+// A lane loads 16 bytes of a row, the pieces 2 qd and 2 qd + 1 of 8 columns of a double step of 64; the MFMA's K
+// order is free, so the fragments of x are read in the order that fits (256 contiguous bytes per lane group).
+//   What bounds it, from counting: reads of x from L2 (each of 792 row blocks reads all of it: 1.5 GB at 256 tokens;
+// the MFMAs take about 40 us of the 141), at up to 16 tokens the weights' 97 MB.  50,688 x 1,920 with the norm, split
+// launch included, against int8mm_kernel: 5-16 tokens 56 -> 31 us, 32 73 -> 39, 64 112 -> 52, 128 194 -> 81, 256
+// 361 -> 141; error against float64 at 256 tokens 3.2e-7 -> 2.1e-7.
+typedef _Float16 f16x8_i8 __attribute__((ext_vector_type(8)));
+
+template <int MT, bool ARG>
+__global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8parts_kernel(
+    const int8_t *__restrict__ q, const uint16_t *__restrict__ mu16, int64_t rows, int cols,
+    const uint8_t *__restrict__ xf, const float *__restrict__ tscale, int64_t m_total, int row_blocks, int slabs,
+    float *__restrict__ y, uint64_t *__restrict__ keys) {
+  constexpr int TOK = 16 * MT;
+  constexpr int kPart = 3 * 4 * 1024, kQuad = 2 * kPart;  // bytes of the copy per part and per 96 columns
+  __shared__ __align__(16) float red[kI8mmWaves][TOK][kI8mmRedStride];
+  __shared__ float rinv[kI8mmRows];
+  const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, qd = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // blocks go to the XCDs in turn: block 8 i + c is the i-th of XCD c
+  const int xcd = static_cast<int>(blockIdx.x & 7u), turn = static_cast<int>(blockIdx.x >> 3);
+  const int slab = turn % slabs, rb = (turn / slabs) * 8 + xcd;
+  if (rb >= row_blocks) return;  // (the whole block)
+  const int64_t row0 = static_cast<int64_t>(rb) * kI8mmRows;
+  const int64_t tok0 = static_cast<int64_t>(slab) * TOK;  // (more than one slab only with MT = 4)
+  const int nsteps = (cols + 63) / 64;                    // double steps of 64 columns
+  const int sb = nsteps / kI8mmWaves, sx = nsteps % kI8mmWaves;
+  const int s0 = wave * sb + min(wave, sx), sn = sb + (wave < sx ? 1 : 0);
+
+  // per row tile: the lane's row scale, and the power of two that brings 127 times it to 2^13 .. 2^14 (at most
+  // 2^15; 1 where it is 0, inf or nan), and that times 2^-11: all products with them are exact
+  __half2 s2[4], up2[4], um2[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int64_t row = row0 + 16 * r + j < rows ? row0 + 16 * r + j : rows - 1;
+    const float s16 = int8_row_scale(mu16[row]), top = fabsf(127.0f * s16);
+    int e = 0;
+    if (top > 0.f && top <= 1.0e6f) e = min(15, 13 - (static_cast<int>(__float_as_uint(top) >> 23) - 127));
+    s2[r] = __float2half2_rn(s16);  // exact: an fp16 value
+    up2[r] = __float2half2_rn(__uint_as_float(static_cast<uint32_t>(127 + e) << 23));
+    um2[r] = __float2half2_rn(__uint_as_float(static_cast<uint32_t>(116 + e) << 23));
+    if (wave == 0 && qd == 0) rinv[16 * r + j] = __uint_as_float(static_cast<uint32_t>(127 - e) << 23);
+  }
+  // Raw buffer loads: rows past the end, columns past the row and steps past the wave's share read as zeros (no
+  // load sits under a branch).
+  const int nq = (cols + 95) / 96;
+  const int64_t rows_b = rows - row0 < kI8mmRows ? rows - row0 : kI8mmRows;
+  const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<int8_t *>(q + row0 * cols), static_cast<short>(0), static_cast<int>(rows_b * cols), kBufferFlags);
+  const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t *>(xf + static_cast<int64_t>(slab) * nq * kQuad), static_cast<short>(0), nq * kQuad,
+      kBufferFlags);
+
+  f32x4_i8 acc[MT][4];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[t][r] = f32x4_i8{0.f, 0.f, 0.f, 0.f};
+
+  uint4 wv[2][4], xv[2][2][MT];  // weights of two double steps, x (part, token tile) of two halves of one
+  auto load_w = [&](int step, uint4 (&w)[4]) {
+    const int k = 64 * step + 16 * qd;
+    const bool ok = k < cols && step < s0 + sn;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      int off = ok ? (16 * r + j) * cols + k : kBufferOutOfRange;
+      asm("" : "+v"(off));
+      w[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wrs, off, 0, 0));
+    }
+  };
+  auto load_x = [&](int step, int half, uint4 (&x)[2][MT]) {
+    const int s32 = 2 * step + (qd >> 1);  // the 32 columns of the lane's piece, its quarter of them
+    const int quad = s32 / 3;
+    int off = step < s0 + sn ? quad * kQuad + (s32 - 3 * quad) * 4096 + 16 * (j + 16 * ((2 * qd + half) & 3))
+                             : kBufferOutOfRange;
+    asm("" : "+v"(off));
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        x[p][t] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, p * kPart + t * 1024, 0));
+  };
+  auto compute = [&](const uint4 (&w)[4], int half, const uint4 (&x)[2][MT]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      __half2 v[4], h[4], m[4];
+      int8x4_weights(half ? w[r].z : w[r].x, s2[r], v[0], v[1]);
+      int8x4_weights(half ? w[r].w : w[r].y, s2[r], v[2], v[3]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        h[i] = __hmul2(v[i], up2[r]);
+        m[i] = __hmul2(v[i], um2[r]);
+      }
+      struct Four { __half2 v[4]; };
+      const f16x8_i8 wh = __builtin_bit_cast(f16x8_i8, Four{{h[0], h[1], h[2], h[3]}});
+      const f16x8_i8 wm = __builtin_bit_cast(f16x8_i8, Four{{m[0], m[1], m[2], m[3]}});
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        acc[t][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_i8, x[1][t]), wm, acc[t][r], 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        acc[t][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_i8, x[0][t]), wh, acc[t][r], 0, 0, 0);
+    }
+  };
+  load_w(s0, wv[0]);
+  load_x(s0, 0, xv[0]);
+  load_w(s0 + 1, wv[1]);
+  for (int i = 0; i < sn; i += 2) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int st = s0 + i + u;
+      if (i + u < sn) {  // wave-uniform
+        load_x(st, 1, xv[1]);
+        compute(wv[u], 0, xv[0]);
+        load_x(st + 1, 0, xv[0]);
+        compute(wv[u], 1, xv[1]);
+        load_w(st + 2, wv[u]);
+      }
+    }
+  }
+
+  // C[token 16t + 4qd + e][row 16r + j] of every wave into LDS, summed in wave order, the scales taken back
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) red[wave][16 * t + 4 * qd + e][16 * r + j] = acc[t][r][e];
+  __syncthreads();
+  constexpr int kTpt = 64 * kI8mmWaves / TOK;  // threads per token
+  constexpr int kRpt = kI8mmRows / kTpt;       // rows per thread
+  const int tl = tid / kTpt, part = tid % kTpt;
+  const int64_t tok = tok0 + tl;
+  const float ts = tscale[tok < m_total ? tok : m_total - 1];
+  uint64_t kb = 0;
+#pragma unroll
+  for (int i = 0; i < kRpt; ++i) {
+    const int rr = part + kTpt * i;
+    float sum = red[0][tl][rr];
+#pragma unroll
+    for (int w = 1; w < kI8mmWaves; ++w) sum += red[w][tl][rr];
+    sum = sum * rinv[rr] * ts;
     const int64_t row = row0 + rr;
     if (tok < m_total && row < rows) {
       y[tok * rows + row] = sum;
@@ -540,7 +693,7 @@ __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8mm_kernel(
       const uint64_t o = shfl_xor_u64(kb, d);
       kb = o > kb ? o : kb;
     }
-    if (part == 0 && tok < m_total) keys[tok * gridDim.x + blockIdx.x] = kb;
+    if (part == 0 && tok < m_total) keys[tok * row_blocks + rb] = kb;
   }
 }
 
@@ -669,47 +822,49 @@ int int8_linear_blocks(int64_t rows, int64_t *rows_per_wave) {
   return static_cast<int>(std::min<int64_t>((waves + kLinWaves - 1) / kLinWaves, 0x7FFFFFFFll));
 }
 
-// From this many tokens the MFMA kernel runs: it reads the weights once for up
-// to 64 tokens, the GEMV once per 4 tokens.  Measured on the Pollux head
-// (50,688 x 1,920): GEMV 20.8 / 25.8 / 47.4 / 79.2 us at 1 / 2 / 4 / 5 tokens;
-// MFMA 52-54 us at 5..16 tokens (VALU-bound by the weight decode and the exact
-// bf16 splits: ~10 VALU instructions per weight), 67 at 17, 99 at 33, 170 at
-// 65, 373 at 256 (torch F.linear on the cached fp32 cast: 70-73, 76, 95, 162,
-// 392).
+// From this many tokens the MFMA kernels run: they read the weights once for up to 64 tokens, the GEMV once per 4
+// tokens.  Measured on the Pollux head (50,688 x 1,920): GEMV 20.8 / 25.8 / 47.4 / 79.2 us at 1 / 2 / 4 / 5 tokens,
+// int8parts_kernel 31 at 5..16 (the lower edge stays at 5: the graph prefill's padded lengths count on it).  With a
+// workspace int8parts_kernel runs, always the faster; int8mm_kernel is left for calls without one.
 constexpr int64_t kI8mmMinTokens = 5;
 
 int64_t int8mm_row_blocks(int64_t rows) { return (rows + kI8mmRows - 1) / kI8mmRows; }
 
 int launch_int8mm(const int8_t *q, const uint16_t *mu16, int64_t rows, int cols, const float *x, int64_t m,
-                  const float *norm_w, float eps, float *y, uint64_t *keys, hipStream_t s) {
-  const int mt = m <= 16 ? 1 : m <= 32 ? 2 : 4;
+                  const float *norm_w, float eps, float *y, hipStream_t s) {
+  const int mt = x_parts_tiles(m);
   const int64_t slabs = (m + 16 * mt - 1) / (16 * mt);
   if (slabs > 0xFFFFll) return fail(PLX_EINVAL, "int8_linear: %lld tokens", static_cast<long long>(m));
   const dim3 g(static_cast<unsigned>(int8mm_row_blocks(rows)), static_cast<unsigned>(slabs)), b(64 * kI8mmWaves);
-#define PLX_I8MM_K(MT, NORM)                                                                                        \
-  do {                                                                                                              \
-    if (keys)                                                                                                       \
-      hipLaunchKernelGGL((int8mm_kernel<MT, NORM, true>), g, b, 0, s, q, mu16, rows, cols, x, m, norm_w, eps, y, keys); \
-    else                                                                                                            \
-      hipLaunchKernelGGL((int8mm_kernel<MT, NORM, false>), g, b, 0, s, q, mu16, rows, cols, x, m, norm_w, eps, y,    \
-                         keys);                                                                                     \
-  } while (0)
-#define PLX_I8MM(MT)              \
-  do {                            \
-    if (norm_w)                   \
-      PLX_I8MM_K(MT, true);       \
-    else                          \
-      PLX_I8MM_K(MT, false);      \
-  } while (0)
-  if (mt == 1)
-    PLX_I8MM(1);
-  else if (mt == 2)
-    PLX_I8MM(2);
-  else
-    PLX_I8MM(4);
-#undef PLX_I8MM
-#undef PLX_I8MM_K
+  auto k = norm_w ? (mt == 1 ? int8mm_kernel<1, true> : mt == 2 ? int8mm_kernel<2, true> : int8mm_kernel<4, true>)
+                  : (mt == 1 ? int8mm_kernel<1, false> : mt == 2 ? int8mm_kernel<2, false> : int8mm_kernel<4, false>);
+  hipLaunchKernelGGL(k, g, b, 0, s, q, mu16, rows, cols, x, m, norm_w, eps, y);
   return check_launch("int8mm_kernel");
+}
+
+// Workspace of the MFMA path from `ws` (16-byte aligned): the split x, then the normalised x where the norm is a
+// launch of its own (rows longer than the split kernel's registers).
+size_t int8parts_bytes(int64_t cols, int64_t m) {
+  const size_t x = (x_parts_bytes(cols, m) + 255) & ~static_cast<size_t>(255);
+  return x + (x_parts_fuses_norm(cols) ? 0 : static_cast<size_t>(m * cols) * sizeof(float));
+}
+
+int launch_int8parts(const int8_t *q, const uint16_t *mu16, int64_t rows, int cols, const float *x, int64_t m,
+                     const float *norm_w, float eps, float *y, uint64_t *keys, uint8_t *ws, hipStream_t s) {
+  const int mt = x_parts_tiles(m);
+  const int64_t slabs = (m + 63) / 64, rbs = int8mm_row_blocks(rows);
+  const int64_t blocks = (rbs + 7) / 8 * 8 * slabs;
+  if (slabs > 0xFFFFll || blocks > 0x7FFFFFFFll)
+    return fail(PLX_EINVAL, "int8_linear: %lld tokens", static_cast<long long>(m));
+  const size_t x_bytes = x_parts_bytes(cols, m), xf_bytes = x_bytes - static_cast<size_t>(slabs) * 64 * sizeof(float);
+  float *xnorm = reinterpret_cast<float *>(ws + ((x_bytes + 255) & ~static_cast<size_t>(255)));
+  const int st = launch_x_parts(x, norm_w, eps, m, cols, xnorm, ws, s);
+  if (st != PLX_OK) return st;
+  auto k = keys ? (mt == 1 ? int8parts_kernel<1, true> : mt == 2 ? int8parts_kernel<2, true> : int8parts_kernel<4, true>)
+                : (mt == 1 ? int8parts_kernel<1, false> : mt == 2 ? int8parts_kernel<2, false> : int8parts_kernel<4, false>);
+  hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(blocks)), dim3(64 * kI8mmWaves), 0, s, q, mu16, rows, cols, ws,
+                     reinterpret_cast<const float *>(ws + xf_bytes), m, static_cast<int>(rbs), static_cast<int>(slabs), y, keys);
+  return check_launch("int8parts_kernel");
 }
 
 // blocks of the kernel a call at m tokens launches (the argmax keys' parts)
@@ -717,16 +872,22 @@ int64_t int8_linear_parts(int64_t rows, int64_t m) {
   return m >= kI8mmMinTokens ? int8mm_row_blocks(rows) : int8_linear_blocks(rows, nullptr);
 }
 
-int launch_int8_linear(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x, int64_t m,
-                       const float *norm_w, float eps, float *y, uint64_t *keys, hipStream_t s) {
+namespace {
+
+int int8_linear(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x, int64_t m,
+                const float *norm_w, float eps, float *y, uint64_t *keys, uint8_t *ws, hipStream_t s) {
   if (rows == 0 || m == 0) return PLX_OK;
-  if (cols <= 0 || cols % 16 != 0 || cols > 64 * 16 * 4)
+  if (cols <= 0 || cols % 16 != 0 || cols > kI8MaxCols)
     return fail(PLX_EINVAL, "int8_linear: %lld columns (a multiple of 16 up to 4,096)", static_cast<long long>(cols));
   const uintptr_t al = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(x) |
                        reinterpret_cast<uintptr_t>(norm_w);
   if ((al & 15u) != 0) return fail(PLX_EINVAL, "int8_linear: q, x and the norm weight must be 16-byte aligned");
   if (rows > 0x7FFFFFFFll) return fail(PLX_EINVAL, "int8_linear: too many rows");
-  if (m >= kI8mmMinTokens) return launch_int8mm(q, mu16, rows, static_cast<int>(cols), x, m, norm_w, eps, y, keys, s);
+  if (m >= kI8mmMinTokens) {
+    const int ci = static_cast<int>(cols);
+    return ws ? launch_int8parts(q, mu16, rows, ci, x, m, norm_w, eps, y, keys, ws, s)
+              : launch_int8mm(q, mu16, rows, ci, x, m, norm_w, eps, y, s);
+  }
   int64_t rpw = 0;
   const int blocks = int8_linear_blocks(rows, &rpw);
   const int cpl = static_cast<int>((cols / 16 + 63) / 64);
@@ -771,17 +932,41 @@ int launch_int8_linear(const int8_t *q, const uint16_t *mu16, int64_t rows, int6
   return check_launch("int8_linear_kernel");
 }
 
+// bytes of the argmax keys ahead of the MFMA path's part, with room to align that
+size_t int8_keys_bytes(int64_t rows, int64_t m) {
+  const size_t k = static_cast<size_t>(m) * static_cast<size_t>(int8_linear_parts(rows, m)) * sizeof(uint64_t);
+  return m >= kI8mmMinTokens ? k + 16 : k;
+}
+
+uint8_t *align16(uint8_t *p) { return reinterpret_cast<uint8_t *>((reinterpret_cast<uintptr_t>(p) + 15) & ~uintptr_t{15}); }
+
+}  // namespace
+
+size_t int8_linear_workspace_bytes(int64_t rows, int64_t cols, int64_t m) {
+  if (rows <= 0 || m < kI8mmMinTokens || cols <= 0 || cols > kI8MaxCols) return 0;
+  return int8parts_bytes(cols, m);
+}
+
+int launch_int8_linear(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x, int64_t m,
+                       const float *norm_w, float eps, float *y, void *workspace, size_t workspace_bytes, hipStream_t s) {
+  const size_t need = int8_linear_workspace_bytes(rows, cols, m);
+  if (workspace && (workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0))
+    return fail(PLX_EINVAL, "int8_linear: workspace of %zu bytes (16-byte aligned) needed", need);
+  return int8_linear(q, mu16, rows, cols, x, m, norm_w, eps, y, nullptr, static_cast<uint8_t *>(workspace), s);
+}
+
 int launch_int8_linear_argmax(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x,
                               int64_t m, const float *norm_w, float eps, float *y, int64_t *ids, int64_t *history,
                               int64_t hist_len, int64_t *pos, void *workspace, size_t workspace_bytes, hipStream_t s) {
   if (m == 0) return PLX_OK;
   if (rows <= 0 || rows > 0x7FFFFFFFll) return fail(PLX_EINVAL, "int8_linear_argmax: %lld rows", static_cast<long long>(rows));
   const int64_t parts = int8_linear_parts(rows, m);
-  const size_t need = static_cast<size_t>(m) * static_cast<size_t>(parts) * sizeof(uint64_t);
+  const size_t keys_bytes = int8_keys_bytes(rows, m), need = keys_bytes + int8_linear_workspace_bytes(rows, cols, m);
   if (workspace == nullptr || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 7u) != 0)
     return fail(PLX_EINVAL, "int8_linear_argmax: workspace of %zu bytes (8-byte aligned) needed", need);
   uint64_t *keys = static_cast<uint64_t *>(workspace);
-  const int st = launch_int8_linear(q, mu16, rows, cols, x, m, norm_w, eps, y, keys, s);
+  uint8_t *ws = align16(static_cast<uint8_t *>(workspace) + static_cast<size_t>(m) * static_cast<size_t>(parts) * 8);
+  const int st = int8_linear(q, mu16, rows, cols, x, m, norm_w, eps, y, keys, ws, s);
   if (st != PLX_OK) return st;
   int rsh = 0;
   while ((int64_t{1} << rsh) < m && rsh < 4) ++rsh;
@@ -792,7 +977,7 @@ int launch_int8_linear_argmax(const int8_t *q, const uint16_t *mu16, int64_t row
 
 size_t int8_linear_argmax_workspace_bytes(int64_t rows, int64_t m) {
   if (rows <= 0 || m <= 0 || rows > 0x7FFFFFFFll) return 0;
-  return static_cast<size_t>(m) * static_cast<size_t>(int8_linear_parts(rows, m)) * sizeof(uint64_t);
+  return int8_keys_bytes(rows, m) + int8_linear_workspace_bytes(rows, kI8MaxCols, m);  // (any row length)
 }
 
 int launch_int8_embed(const int8_t *q, const uint16_t *mu16, int64_t vocab, int64_t cols, const int64_t *idx,

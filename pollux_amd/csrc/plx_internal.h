@@ -166,8 +166,19 @@ int launch_requantize_batch(const RequantItem *items, int n_items, int mode, voi
 int launch_gather(const int32_t *idx, int64_t n, int out_dtype, void *out, hipStream_t s);
 int launch_dequant_f16(const uint8_t *packed, const uint16_t *sigma16, int64_t rows, int64_t cols,
                        uint16_t *w16, hipStream_t s);
+// fp32 x (normalised first when norm_w is given) as two scaled fp16 parts per row in MFMA fragment order, followed
+// by the rows' inverse scales (dequant.hip, xsplit_kernel): slab of 64 tokens, 96 columns (zero-padded), part,
+// 32 columns, token tile of 16, lane: 16 bytes.  Only the first x_parts_tiles(m) token tiles of a slab are written.
+// xnorm: [m, cols] scratch, used when the norm is not fused into the copy.  cols % 4 == 0, x 16-byte aligned.
+constexpr int x_parts_tiles(int64_t m) { return m > 32 ? 4 : m > 16 ? 2 : 1; }
+size_t x_parts_bytes(int64_t cols, int64_t m);
+bool x_parts_fuses_norm(int64_t cols);
+int launch_x_parts(const float *x, const float *norm_w, float norm_eps, int64_t m, int64_t cols, float *xnorm, void *ws,
+                   hipStream_t s);
+// workspace may be null: the MFMA kernel that splits x itself
 int launch_int8_linear(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x, int64_t m,
-                       const float *norm_w, float eps, float *y, uint64_t *keys, hipStream_t s);
+                       const float *norm_w, float eps, float *y, void *workspace, size_t workspace_bytes, hipStream_t s);
+size_t int8_linear_workspace_bytes(int64_t rows, int64_t cols, int64_t m);
 int launch_int8_linear_argmax(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x,
                               int64_t m, const float *norm_w, float eps, float *y, int64_t *ids, int64_t *history,
                               int64_t hist_len, int64_t *pos, void *workspace, size_t workspace_bytes, hipStream_t s);

@@ -408,7 +408,7 @@ def dequantize_int8_rows(q: torch.Tensor, mu16: torch.Tensor) -> torch.Tensor:
 
 def int8_linear(q: torch.Tensor, mu16: torch.Tensor, x: torch.Tensor, *,
                 norm: tuple[torch.Tensor, float] | None = None) -> torch.Tensor:
-    """fp32 [..., rows] = n(x) @ W.T with W = q * (mu / 127) in fp16 (never stored), one HIP kernel (plx_int8_linear).
+    """fp32 [..., rows] = n(x) @ W.T with W = q * (mu / 127) in fp16 (never stored) (plx_int8_linear_ws).
 
     Exact products, fp32 sums: F.linear(x, W.float()) up to summation order
     (PackedInt8Linear.forward, pollux.py:562-563).  ``norm``: (weight, eps) of
@@ -432,10 +432,14 @@ def int8_linear(q: torch.Tensor, mu16: torch.Tensor, x: torch.Tensor, *,
             raise ValueError(f"int8_linear: the norm weight must be fp32 with {cols} values")
         if nw.data_ptr() % 16:
             nw = nw.clone()
-    y = torch.empty((xx.shape[0], rows), dtype=torch.float32, device=x.device)
+    m = xx.shape[0]
+    y = torch.empty((m, rows), dtype=torch.float32, device=x.device)
+    n = int(_lib.lib().plx_int8_linear_workspace_bytes(rows, cols, m))
+    ws = torch.empty(n, dtype=torch.uint8, device=x.device) if n else None
     with torch.cuda.device(x.device):
-        st = _lib.lib().plx_int8_linear(_lib.ptr(qq), _lib.ptr(mu16.contiguous()), rows, cols, _lib.ptr(xx),
-                                        xx.shape[0], _lib.ptr(nw), eps, _lib.ptr(y), _lib.stream_of(x.device))
+        st = _lib.lib().plx_int8_linear_ws(_lib.ptr(qq), _lib.ptr(mu16.contiguous()), rows, cols, _lib.ptr(xx), m,
+                                           _lib.ptr(nw), eps, _lib.ptr(y), _lib.ptr(ws), n,
+                                           _lib.stream_of(x.device))
     _lib.check(st, "int8_linear")
     return y.reshape(*x.shape[:-1], rows)
 
