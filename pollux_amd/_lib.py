@@ -7,6 +7,7 @@ compute entry point.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import threading
 from pathlib import Path
@@ -137,8 +138,20 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+_ON_CURRENT = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """``torch.cuda.device(device)``, or nothing to enter and leave where that device is the current one already."""
+    if device.index is None or device.index == torch.cuda.current_device():
+        return _ON_CURRENT
+    return torch.cuda.device(device)
+
+
 def stream_of(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The handle of the device's current stream (no Stream object made: it costs more than the launch)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def require_device(t: torch.Tensor, name: str) -> None:

@@ -166,7 +166,7 @@ def pack_indices(indices: torch.Tensor) -> torch.Tensor:
         flat = flat.to(torch.int64)
     flat = flat.contiguous()
     out = torch.empty(((n + 3) // 4) * BYTES_PER_CHUNK, dtype=torch.uint8, device=flat.device)
-    with torch.cuda.device(flat.device):
+    with _lib.on_device(flat.device):
         st = _lib.lib().plx_pack_indices(
             _lib.ptr(flat), int(flat.dtype == torch.int64), n, _lib.ptr(out), _lib.stream_of(flat.device)
         )
@@ -189,7 +189,7 @@ def unpack_indices(packed: torch.Tensor, num_indices: int) -> torch.Tensor:
         num_indices = max(total + num_indices, 0)
     num_indices = min(num_indices, total)
     out = torch.empty(num_indices, dtype=torch.int64, device=flat.device)
-    with torch.cuda.device(flat.device):
+    with _lib.on_device(flat.device):
         st = _lib.lib().plx_unpack_indices(
             _lib.ptr(flat), flat.numel(), num_indices, _lib.ptr(out), _lib.stream_of(flat.device)
         )
@@ -209,7 +209,7 @@ def row_rms_from_matrix(weight: torch.Tensor) -> torch.Tensor:
     _lib.require_device(weight, "row_rms_from_matrix input")
     w = weight.detach().float().contiguous()
     out = torch.empty(w.shape[0], dtype=torch.float32, device=w.device)
-    with torch.cuda.device(w.device):
+    with _lib.on_device(w.device):
         st = _lib.lib().plx_row_rms(_lib.ptr(w), w.shape[0], w.shape[1], _lib.ptr(out), _lib.stream_of(w.device))
     _lib.check(st, "row_rms_from_matrix")
     return out
@@ -314,7 +314,7 @@ def quantize_indices(x: torch.Tensor, mode: str | None = None) -> torch.Tensor:
         raise ValueError(f"nn mode must be one of {sorted(_INDEX_MODES)}, got {m!r}")
     code = _INDEX_MODES[m]
     ws = _workspace(n, xf.device)
-    with torch.cuda.device(xf.device):
+    with _lib.on_device(xf.device):
         st = _lib.lib().plx_quantize(
             _lib.ptr(xf), n, code, _lib.ptr(idx), _lib.ptr(ws), ws.numel(), _lib.stream_of(xf.device)
         )
@@ -330,7 +330,7 @@ def gather_codebook(idx: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     gdt = dtype if dtype in _GATHER_DTYPES else torch.float32
     out = torch.empty((n, H24_DIM), dtype=gdt, device=idx.device)
     if n:
-        with torch.cuda.device(idx.device):
+        with _lib.on_device(idx.device):
             st = _lib.lib().plx_gather_codebook(
                 _lib.ptr(idx), n, _GATHER_DTYPES[gdt], _lib.ptr(out), _lib.stream_of(idx.device)
             )
@@ -402,7 +402,7 @@ def requantize_h24(latent: torch.Tensor, *, mode: str | None = None, pack: bool 
     packed = torch.empty(((n + 3) // 4) * BYTES_PER_CHUNK, dtype=torch.uint8, device=dev) if pack else None
     w = torch.empty_like(lat) if weight else None
     ws = _workspace(n, dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().plx_requantize(
             _lib.ptr(lat), rows, cols, _MODES[mode or _nn_mode], _lib.ptr(sigma), _lib.ptr(idx),
             _lib.ptr(packed), _lib.ptr(w), _lib.ptr(ws), ws.numel(), _lib.stream_of(dev),
@@ -448,7 +448,7 @@ def requantize_h24_many(
     total = sum(o["indices"].numel() for o in outs)
     ws = _workspace(total, dev)
     arr = (_lib.RequantizeItem * len(items))(*items)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().plx_requantize_batch(arr, len(items), _MODES[mode or _nn_mode], _lib.ptr(ws), ws.numel(),
                                              _lib.stream_of(dev))
     _lib.check(st, "requantize_h24_many")
@@ -462,7 +462,7 @@ def sigma16_pack(weight: torch.Tensor) -> torch.Tensor:
     _lib.require_device(weight, "sigma16_pack input")
     w = weight.detach().float().contiguous()
     out = torch.empty(w.shape[0], dtype=torch.float16, device=w.device)
-    with torch.cuda.device(w.device):
+    with _lib.on_device(w.device):
         st = _lib.lib().plx_sigma16_pack(_lib.ptr(w), w.shape[0], w.shape[1], _lib.ptr(out), _lib.stream_of(w.device))
     _lib.check(st, "sigma16_pack")
     return out

@@ -106,7 +106,7 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     w = weight.detach().contiguous()
     y = torch.empty_like(xx)
     d = xx.shape[-1]
-    with torch.cuda.device(xx.device):
+    with _lib.on_device(xx.device):
         st = _lib.lib().plx_rms_norm(_lib.ptr(xx), _lib.ptr(w), _lib.ptr(y), xx.numel() // d if d else 0, d,
                                      float(eps), _lib.stream_of(xx.device))
     _lib.check(st, "rms_norm")
@@ -126,7 +126,7 @@ def argmax_rows(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tenso
         out = torch.empty(x.shape[:-1], dtype=torch.long, device=x.device)
     if out.dtype != torch.long or out.numel() != xx.shape[0] or not out.is_contiguous() or out.device != x.device:
         raise ValueError("argmax_rows: out must be a contiguous int64 tensor with one element per row")
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         st = _lib.lib().plx_argmax_rows(_lib.ptr(xx), xx.shape[0], cols, _lib.ptr(out), _lib.stream_of(x.device))
     _lib.check(st, "argmax_rows")
     return out
@@ -169,7 +169,7 @@ def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_ln: RM
     heads = c // H24_DIM
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     qq, kk, vv, stride = _qkv_rows(q, k, v)
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         st = _lib.lib().plx_decode_attention(
             _lib.ptr(qq), _lib.ptr(kk), _lib.ptr(vv), stride, _lib.ptr(q_ln.weight.detach()),
             _lib.ptr(k_ln.weight.detach()), float(q_ln.eps), _lib.ptr(k_cache), _lib.ptr(v_cache), _lib.ptr(pos),
@@ -190,7 +190,7 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_ln: R
     heads = c // H24_DIM
     out = torch.empty(b, t, c, dtype=torch.float32, device=q.device)
     qq, kk, vv, stride = _qkv_rows(q, k, v)
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         st = _lib.lib().plx_prefill_attention(
             _lib.ptr(qq), _lib.ptr(kk), _lib.ptr(vv), stride, _lib.ptr(q_ln.weight.detach()),
             _lib.ptr(k_ln.weight.detach()), float(q_ln.eps), _lib.ptr(k_cache), _lib.ptr(v_cache), b, heads, t,

@@ -128,7 +128,7 @@ def pollux_h24_step_(
     norm = torch.zeros((), dtype=torch.float32, device=dev)  # an empty parameter's norm is 0 (not written)
     nws = int(_lib.lib().plx_pollux_step_workspace_bytes(rows, cols))
     ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().plx_pollux_step_h24(
             _lib.ptr(g), _lib.ptr(m), _lib.ptr(v), _lib.ptr(latent), rows, cols, _lib.ptr(scal),
             _castor._MODES[mode or _castor._nn_mode], _lib.ptr(sigma), _lib.ptr(idx), _lib.ptr(packed), _lib.ptr(w),
@@ -202,7 +202,7 @@ def pollux_h24_step_many_(
     arr = (_lib.PolluxStepItem * len(items))(*items)
     nws = int(_lib.lib().plx_pollux_step_batch_workspace_bytes(arr, len(items)))
     ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().plx_pollux_step_h24_batch(arr, len(items), _lib.ptr(scal),
                                                   _castor._MODES[mode or _castor._nn_mode], _lib.ptr(ws), nws,
                                                   _lib.stream_of(dev))

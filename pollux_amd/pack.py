@@ -54,7 +54,7 @@ def quantize_h24_layer(weight: torch.Tensor, *, return_indices: bool = False):
     else:
         idx = torch.empty(n, dtype=torch.int32, device=dev)
     if rows and cols:
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             lib = _lib.lib()
             if cols % H24_DIM == 0:
                 ws = _workspace(n, dev)
@@ -102,7 +102,7 @@ def quantize_int8_rows(weight: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor
     q = torch.empty(w.shape, dtype=torch.int8, device=w.device)
     mu = torch.empty(w.shape[:-1], dtype=torch.float16, device=w.device)
     if rows:
-        with torch.cuda.device(w.device):
+        with _lib.on_device(w.device):
             st = _lib.lib().plx_quantize_int8_rows(
                 _lib.ptr(w), rows, cols, _lib.ptr(q), _lib.ptr(mu), _lib.stream_of(w.device)
             )

@@ -32,7 +32,7 @@ def dequantize_h24(packed: torch.Tensor, sigma16: torch.Tensor, out_features: in
     if sg.numel() != out_features:
         raise ValueError(f"expected {out_features} sigma rows, got {sg.numel()}")
     out = torch.empty((out_features, in_features), dtype=torch.float16, device=pk.device)
-    with torch.cuda.device(pk.device):
+    with _lib.on_device(pk.device):
         st = _lib.lib().plx_dequant_f16(
             _lib.ptr(pk), pk.numel(), _lib.ptr(sg), out_features, in_features, _lib.ptr(out), _lib.stream_of(pk.device)
         )
@@ -59,7 +59,7 @@ def h24_plane_layout(packed: torch.Tensor, n_atoms: int) -> torch.Tensor:
     pk = packed.reshape(-1).contiguous()
     out = torch.empty(3 * n_atoms, dtype=torch.int16, device=pk.device)
     if n_atoms:
-        with torch.cuda.device(pk.device):
+        with _lib.on_device(pk.device):
             st = _lib.lib().plx_h24_plane_layout(_lib.ptr(pk), pk.numel(), n_atoms, _lib.ptr(out),
                                                  _lib.stream_of(pk.device))
         _lib.check(st, "h24_plane_layout")
@@ -96,22 +96,20 @@ def dequant_linear(
     assert_row_aligned_in_features(in_features)
     if x.shape[-1] != in_features:
         raise ValueError(f"x has {x.shape[-1]} features, layer expects {in_features}")
-    lead = x.shape[:-1]
-    xx = x.reshape(-1, in_features)
-    if xx.dtype not in (torch.bfloat16, torch.float32):
-        xx = xx.float()
+    xx = x if x.dtype in (torch.bfloat16, torch.float32) else x.float()
     xx = xx.contiguous()
-    pk = packed.reshape(-1).contiguous()
+    pk = packed.contiguous()
     if pk.data_ptr() % 16:
         pk = pk.clone()  # the kernel streams the packed bytes as aligned 16-byte vectors
     if xx.data_ptr() % 16:
         xx = xx.clone()
-    sg = sigma16.reshape(-1).contiguous()
-    y = torch.empty((xx.shape[0], out_features), dtype=torch.float32, device=pk.device)
+    m = xx.numel() // in_features
+    sg = sigma16.contiguous()
+    y = torch.empty((*x.shape[:-1], out_features), dtype=torch.float32, device=pk.device)
     flags = (DQL_X_F32 if xx.dtype == torch.float32 else 0) | (DQL_W_AS_X if weight_rounding == "as_x" else 0)
     src, nsrc = pk, pk.numel()
     n_atoms = out_features * (in_features // 24)
-    if planes is not None and plane_layout_takes(xx.shape[0], in_features) and 6 * n_atoms < 1 << 30:
+    if planes is not None and plane_layout_takes(m, in_features) and 6 * n_atoms < 1 << 30:
         if planes.dtype != torch.int16 or planes.numel() != 3 * n_atoms or planes.device != pk.device:
             raise ValueError("planes must be the weight's int16 plane layout (h24_plane_layout) on its device")
         src = planes.contiguous()
@@ -120,15 +118,15 @@ def dequant_linear(
         nsrc = 6 * n_atoms
         flags |= DQL_PLANES
     lib = _lib.lib()
-    nws = int(lib.plx_dequant_linear_workspace_bytes(out_features, in_features, xx.shape[0], flags))
+    nws = lib.plx_dequant_linear_workspace_bytes(out_features, in_features, m, flags)
     ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=pk.device) if nws else None
-    with torch.cuda.device(pk.device):
+    with _lib.on_device(pk.device):
         st = lib.plx_dequant_linear(
             _lib.ptr(src), nsrc, _lib.ptr(sg), out_features, in_features, _lib.ptr(xx),
-            flags, xx.shape[0], _lib.ptr(y), _lib.ptr(ws), nws, _lib.stream_of(pk.device),
+            flags, m, _lib.ptr(y), _lib.ptr(ws), nws, _lib.stream_of(pk.device),
         )
     _lib.check(st, "dequant_linear")
-    return y.reshape(*lead, out_features)
+    return y
 
 
 def dequant_linear_multi(
@@ -211,7 +209,7 @@ def dequant_linear_multi(
     lib = _lib.lib()
     nws = int(lib.plx_dequant_linear_multi_workspace_bytes(arr, len(weights), in_features, m, flags))
     ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=xx.device) if nws else None
-    with torch.cuda.device(xx.device):
+    with _lib.on_device(xx.device):
         st = lib.plx_dequant_linear_multi(arr, len(weights), in_features, _lib.ptr(xx), flags, m, _lib.ptr(nw), eps,
                                           _lib.ptr(ws), nws, _lib.stream_of(xx.device))
     _lib.check(st, "dequant_linear_multi")
@@ -398,7 +396,7 @@ def dequantize_int8_rows(q: torch.Tensor, mu16: torch.Tensor) -> torch.Tensor:
     mu = mu16.reshape(-1).contiguous()
     out = torch.empty(q.shape, dtype=torch.float16, device=q.device)
     if rows and cols:
-        with torch.cuda.device(q.device):
+        with _lib.on_device(q.device):
             st = _lib.lib().plx_dequant_int8_rows(
                 _lib.ptr(qq), _lib.ptr(mu), rows, cols, _lib.ptr(out), _lib.stream_of(q.device)
             )
@@ -436,7 +434,7 @@ def int8_linear(q: torch.Tensor, mu16: torch.Tensor, x: torch.Tensor, *,
     y = torch.empty((m, rows), dtype=torch.float32, device=x.device)
     n = int(_lib.lib().plx_int8_linear_workspace_bytes(rows, cols, m))
     ws = torch.empty(n, dtype=torch.uint8, device=x.device) if n else None
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         st = _lib.lib().plx_int8_linear_ws(_lib.ptr(qq), _lib.ptr(mu16.contiguous()), rows, cols, _lib.ptr(xx), m,
                                            _lib.ptr(nw), eps, _lib.ptr(y), _lib.ptr(ws), n,
                                            _lib.stream_of(x.device))
@@ -489,7 +487,7 @@ def int8_linear_argmax(q: torch.Tensor, mu16: torch.Tensor, x: torch.Tensor, ids
     if workspace is None:
         workspace = int8_linear_argmax_workspace(rows, m, x.device)
     y = torch.empty((m, rows), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         st = _lib.lib().plx_int8_linear_argmax(
             _lib.ptr(q.contiguous()), _lib.ptr(mu16.contiguous()), rows, cols, _lib.ptr(xx), m, _lib.ptr(nw), eps,
             _lib.ptr(y), _lib.ptr(ids), _lib.ptr(history), 0 if history is None else history.shape[1], _lib.ptr(pos),
@@ -520,7 +518,7 @@ def int8_embed(q: torch.Tensor, mu16: torch.Tensor, ids: torch.Tensor, *, pos_we
     if pos0 is not None:
         p0 = pos0.reshape(()).to(torch.int64)
     out = torch.empty((*ii.shape, cols), dtype=torch.float32, device=ids.device)
-    with torch.cuda.device(ids.device):
+    with _lib.on_device(ids.device):
         st = _lib.lib().plx_int8_embed(_lib.ptr(q.contiguous()), _lib.ptr(mu16.contiguous()), vocab, cols, _lib.ptr(ii),
                                        ii.shape[0], ii.shape[1], _lib.ptr(pw), 0 if pw is None else pw.shape[0],
                                        _lib.ptr(p0), _lib.ptr(out), _lib.stream_of(ids.device))
