@@ -266,6 +266,10 @@ int plx_dequant_f16(const uint8_t *packed, int64_t n_packed_bytes, const uint16_
                               plx_dequant_linear_multi); taken for one token
                               (rows of at most 320 atoms) and for batches above
                               4 tokens, with the same results */
+#define PLX_DQL_Y_BF16 32  /* plx_dequant_linear with bf16 x only: y is bf16, the
+                              fp32 results rounded once (RNE); more than 2
+                              tokens, or one from the plane layout; not with
+                              PLX_DQL_GELU */
 
 /* The plane layout of a packed weight: per atom 3 little-endian uint16
  * records (6 bytes, atom order), one per 8-coordinate plane: a 13-bit index

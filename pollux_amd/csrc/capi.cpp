@@ -438,8 +438,11 @@ int plx_dequant_linear(const uint8_t *packed, int64_t n_packed_bytes, const uint
   PLX_REQUIRE(rows >= 0 && cols > 0 && cols % kDim == 0, "plx_dequant_linear: bad shape (%lld, %lld)",
               static_cast<long long>(rows), static_cast<long long>(cols));
   PLX_REQUIRE(m_rows >= 0, "plx_dequant_linear: negative batch");
-  PLX_REQUIRE((flags & ~(PLX_DQL_X_F32 | PLX_DQL_W_AS_X | PLX_DQL_GELU | PLX_DQL_PLANES)) == 0,
+  PLX_REQUIRE((flags & ~(PLX_DQL_X_F32 | PLX_DQL_W_AS_X | PLX_DQL_GELU | PLX_DQL_PLANES | PLX_DQL_Y_BF16)) == 0,
               "plx_dequant_linear: unknown flags 0x%x", flags);
+  PLX_REQUIRE(!(flags & PLX_DQL_Y_BF16) ||
+                  (!(flags & (PLX_DQL_X_F32 | PLX_DQL_GELU)) && (m_rows > 2 || (m_rows <= 1 && (flags & PLX_DQL_PLANES)))),
+              "plx_dequant_linear: bf16 y takes bf16 x, more than 2 tokens or one from the plane layout, and no GELU");
   const int64_t n_atoms = rows * (cols / kDim);
   if (flags & PLX_DQL_PLANES) {
     PLX_REQUIRE(n_packed_bytes == 6 * n_atoms, "plx_dequant_linear: plane layout of %lld bytes does not match %lld atoms",

@@ -151,6 +151,10 @@ namespace {
 // L lanes share a row and stride over its atoms; a block is NT threads.
 // ---------------------------------------------------------------------------
 
+__device__ __forceinline__ uint16_t bf16_of(float v) {  // RNE
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v));
+}
+
 // Output epilogue of the dequant-linear kernels: GELU in torch's erf form
 // (F.gelu: x * 0.5 * (1 + erf(x * sqrt(1/2))), pollux.py:645) and / or a
 // residual added after it (x + linear(h), pollux.py:660-661).
@@ -652,7 +656,7 @@ template <int L, bool PL>
 __global__ __launch_bounds__(512) void dqgemv1_kernel(const uint8_t *__restrict__ packed, int packed_bytes,
                                                       const uint16_t *__restrict__ sigma16, int rows, int apr,
                                                       const uint16_t *__restrict__ x, const uint2 *__restrict__ kp_half,
-                                                      const uint4 *__restrict__ gv_tab, int round_w,
+                                                      const uint4 *__restrict__ gv_tab, int round_w, int y16,
                                                       float *__restrict__ y) {
   constexpr int NT = 512, R = NT / L, G = kG1Atoms;
   constexpr int VPT = PL ? 2 : 1;   // staged 16-byte vectors of the block's atom bytes per thread
@@ -799,7 +803,13 @@ __global__ __launch_bounds__(512) void dqgemv1_kernel(const uint8_t *__restrict_
       dq_value(1 + (sub & 3), sig, __uint_as_float(kSLatticeBits)))));
   const float mk = round_w ? bf16_bits_to_float(bf16_rne_bits(vk)) : vk;
   const float m1 = dpp_f32<0x00>(mk), m2 = dpp_f32<0x55>(mk), m3 = dpp_f32<0xAA>(mk), m4 = dpp_f32<0xFF>(mk);
-  if (sub == 0 && row < rows) y[row] = m4 * (acc[0] * 0.25f) + m2 * (acc[1] * 0.5f) + m1 * acc[2] - m3 * acc[3];
+  if (sub == 0 && row < rows) {
+    const float v = m4 * (acc[0] * 0.25f) + m2 * (acc[1] * 0.5f) + m1 * acc[2] - m3 * acc[3];
+    if (y16)
+      reinterpret_cast<uint16_t *>(y)[row] = bf16_of(v);
+    else
+      y[row] = v;
+  }
 }
 
 // packed 18-bit indices -> the plane layout: per atom the 3 records of its code
@@ -820,7 +830,7 @@ __global__ __launch_bounds__(256) void plane_layout_kernel(const uint8_t *__rest
 // length as in launch_dql; rows of more than 320 atoms are refused (the packed stream takes them).
 template <int L>
 int launch_gemv1_planes_l(const uint8_t *planes, const uint16_t *sigma16, int64_t rows, int64_t apr, const void *x,
-                          const DeviceTables *tab, int round_w, float *y, hipStream_t s) {
+                          const DeviceTables *tab, int round_w, int y16, float *y, hipStream_t s) {
   constexpr int NT = 512, R = NT / L;
   const int64_t blocks = (rows + R - 1) / R;
   const int64_t nvec_max = (6 * R * apr + 31) / 16;
@@ -832,20 +842,20 @@ int launch_gemv1_planes_l(const uint8_t *planes, const uint16_t *sigma16, int64_
   hipLaunchKernelGGL((dqgemv1_kernel<L, true>), dim3(static_cast<unsigned>(blocks)), dim3(NT),
                      static_cast<size_t>(NT) * (32 + 32 + 32), s, planes, static_cast<int>(6 * rows * apr), sigma16,
                      static_cast<int>(rows), static_cast<int>(apr), static_cast<const uint16_t *>(x),
-                     static_cast<const uint2 *>(nullptr), tab->gv_tab, round_w, y);
+                     static_cast<const uint2 *>(nullptr), tab->gv_tab, round_w, y16, y);
   return check_launch("dqgemv1_kernel");
 }
 
 int launch_gemv1_planes(const uint8_t *planes, const uint16_t *sigma16, int64_t rows, int64_t apr, const void *x,
-                        const DeviceTables *tab, int round_w, float *y, hipStream_t s) {
-  if (apr >= 160) return launch_gemv1_planes_l<64>(planes, sigma16, rows, apr, x, tab, round_w, y, s);
+                        const DeviceTables *tab, int round_w, int y16, float *y, hipStream_t s) {
+  if (apr >= 160) return launch_gemv1_planes_l<64>(planes, sigma16, rows, apr, x, tab, round_w, y16, y, s);
   // 16 lanes (32 rows per block) only while a lane's share is at most kG1Atoms atoms and the
   // block's records fit its 2 vectors per thread
   if (apr >= 16)
     return (rows + 31) / 32 < 192 || apr > static_cast<int64_t>(kG1Atoms) * 16 || 6 * 32 * apr + 31 > 16 * 2 * 512
-               ? launch_gemv1_planes_l<32>(planes, sigma16, rows, apr, x, tab, round_w, y, s)
-               : launch_gemv1_planes_l<16>(planes, sigma16, rows, apr, x, tab, round_w, y, s);
-  return launch_gemv1_planes_l<8>(planes, sigma16, rows, apr, x, tab, round_w, y, s);
+               ? launch_gemv1_planes_l<32>(planes, sigma16, rows, apr, x, tab, round_w, y16, y, s)
+               : launch_gemv1_planes_l<16>(planes, sigma16, rows, apr, x, tab, round_w, y16, y, s);
+  return launch_gemv1_planes_l<8>(planes, sigma16, rows, apr, x, tab, round_w, y16, y, s);
 }
 
 // t.norm_w (fp32 x only): x is normalised in the kernel when its rows fit in
@@ -896,7 +906,7 @@ int launch_dql(DqlTargets t, int64_t apr, const void *x, int64_t m, const uint4 
       hipLaunchKernelGGL((dqgemv1_kernel<L, false>), g, dim3(NT), static_cast<size_t>(NT) * (16 + 32 + 16), s,
                          t.packed[0], static_cast<int>(t.packed_bytes[0]), t.sigma16[0], static_cast<int>(t.rows[0]),
                          static_cast<int>(apr), static_cast<const uint16_t *>(x), dtab->kp_half, dtab->gv_tab, round_w,
-                         t.y[0]);
+                         0, t.y[0]);
       return check_launch("dqgemv1_kernel");
     }
   }
@@ -982,6 +992,9 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
+// what the last kernel of a batched call does to the sums: GELU; bf16 outputs (bf16 x), a launch and 6 bytes of
+// traffic per output less than a conversion after the call
+constexpr int kEpiGelu = 1, kEpiBf16 = 2;
 constexpr int kMmRows = 32;             // output rows per block
 constexpr int kMmMaxApb = 128;          // atoms of a row per block (kp_dq tile: 32 x 388 words = 49.7 KB)
 constexpr int kMmTargetBlocks = 192;    // K is split until the grid holds about this many blocks,
@@ -1285,7 +1298,7 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
     const uint8_t *__restrict__ packed, int64_t packed_bytes, const uint16_t *__restrict__ sigma16, int64_t rows,
     int64_t atoms_per_row, const uint4 *__restrict__ xf, int64_t n_quads_row, int64_t m_total, int splits, int apb,
     const uint32_t *__restrict__ kp_dq, const uint32_t *__restrict__ pl_ids, int pl_vecs, float *__restrict__ y,
-    float *__restrict__ partial, const float *__restrict__ residual, const float *__restrict__ tscale, int gelu) {
+    float *__restrict__ partial, const float *__restrict__ residual, const float *__restrict__ tscale, int epi) {
   extern __shared__ __align__(16) uint8_t smem[];
   constexpr bool F16 = XP == 2;
   static_assert(!F16 || (EXACT && !XD), "fp32 x: exact weights, from the copy");
@@ -1607,7 +1620,19 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
     if (splits == 1) {  // the final output: epilogue here (with a K split, in dqmm_reduce_kernel)
 #pragma unroll
       for (int c = 0; c < 4; ++c)
-        if (row + c < rows) sum[c] = dql_epilogue(sum[c], residual, (tok0 + tl) * rows + row + c, gelu);
+        if (row + c < rows) sum[c] = dql_epilogue(sum[c], residual, (tok0 + tl) * rows + row + c, epi & kEpiGelu);
+      if constexpr (XP == 1) {
+        if (epi & kEpiBf16) {
+          uint16_t *d16 = reinterpret_cast<uint16_t *>(y) + (tok0 + tl) * rows + row;
+          if (vec) {
+            *reinterpret_cast<uint2 *>(d16) = make_uint2(bf16_of(sum[0]) | static_cast<uint32_t>(bf16_of(sum[1])) << 16,
+                                                         bf16_of(sum[2]) | static_cast<uint32_t>(bf16_of(sum[3])) << 16);
+          } else {
+            for (int c = 0; c < 4 && row + c < rows; ++c) d16[c] = bf16_of(sum[c]);
+          }
+          continue;
+        }
+      }
     }
     if (vec) {
       *reinterpret_cast<f32x4_t *>(d) = sum;
@@ -1622,7 +1647,7 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
 template <bool VEC>
 __global__ __launch_bounds__(256) void dqmm_reduce_kernel(const float *__restrict__ partial, int splits, int64_t rows,
                                                           int64_t m_total, float *__restrict__ y,
-                                                          const float *__restrict__ residual, int gelu) {
+                                                          const float *__restrict__ residual, int epi) {
   constexpr int W = VEC ? 4 : 1;
   const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * W;
   if (i >= m_total * rows) return;
@@ -1630,7 +1655,6 @@ __global__ __launch_bounds__(256) void dqmm_reduce_kernel(const float *__restric
   const int64_t slab = tok / 64, tl = tok - slab * 64;
   const int64_t stride = 64 * rows;
   const float *p = partial + (slab * splits) * stride + tl * rows + row;
-  typedef float f4 __attribute__((ext_vector_type(4)));
   typedef float fw __attribute__((ext_vector_type(W)));
   fw s = {};
   int k = 0;
@@ -1643,9 +1667,16 @@ __global__ __launch_bounds__(256) void dqmm_reduce_kernel(const float *__restric
   }
   for (; k < splits; ++k) s += *reinterpret_cast<const fw *>(p + static_cast<int64_t>(k) * stride);
 #pragma unroll
-  for (int c = 0; c < W; ++c) s[c] = dql_epilogue(s[c], residual, i + c, gelu);
+  for (int c = 0; c < W; ++c) s[c] = dql_epilogue(s[c], residual, i + c, epi & kEpiGelu);
+  if (epi & kEpiBf16) {
+    typedef uint16_t hw __attribute__((ext_vector_type(W)));
+    hw h;
+#pragma unroll
+    for (int c = 0; c < W; ++c) h[c] = bf16_of(s[c]);
+    *reinterpret_cast<hw *>(reinterpret_cast<uint16_t *>(y) + i) = h;
+    return;
+  }
   *reinterpret_cast<fw *>(y + i) = s;
-  (void)sizeof(f4);
 }
 
 struct MmPlan {
@@ -1670,7 +1701,7 @@ MmPlan mm_plan(int64_t rows, int64_t apr) {
 template <int MT, int WV, int PD, bool EXACT, int XP, bool XD>
 int launch_dqmm_t(const uint8_t *packed, int64_t pb, const uint16_t *sigma16, int64_t rows, int64_t apr,
                   const uint4 *xf, int64_t m, float *y, float *partial, const MmPlan &pl, const uint32_t *kp_dq,
-                  const uint32_t *pl_ids, int pl_vecs, const float *residual, const float *tscale, int gelu,
+                  const uint32_t *pl_ids, int pl_vecs, const float *residual, const float *tscale, int epi,
                   hipStream_t s) {
   const int64_t row_blocks = (rows + kMmRows - 1) / kMmRows;
   const int64_t slabs = (m + 63) / 64;
@@ -1685,11 +1716,11 @@ int launch_dqmm_t(const uint8_t *packed, int64_t pb, const uint16_t *sigma16, in
   if (pl_ids)
     hipLaunchKernelGGL((dqmm_kernel<MT, WV, PD, EXACT, XP, XD, true>), g, dim3(64 * WV), shm, s, packed, pb, sigma16,
                        rows, apr, xf, nq, m, pl.splits, pl.apb, kp_dq, pl_ids, pl_vecs, y, partial, residual, tscale,
-                       gelu);
+                       epi);
   else
     hipLaunchKernelGGL((dqmm_kernel<MT, WV, PD, EXACT, XP, XD, false>), g, dim3(64 * WV), shm, s, packed, pb, sigma16,
                        rows, apr, xf, nq, m, pl.splits, pl.apb, kp_dq, pl_ids, pl_vecs, y, partial, residual, tscale,
-                       gelu);
+                       epi);
   return check_launch("dqmm_kernel");
 }
 
@@ -1697,13 +1728,13 @@ template <int MT>
 int launch_dqmm(const uint8_t *packed, int64_t pb, const uint16_t *sigma16, int64_t rows, int64_t apr,
                 const uint4 *xf, const float *tscale, int64_t m, float *y, float *partial, const MmPlan &pl,
                 const uint32_t *kp_dq, const uint32_t *pl_ids, int pl_vecs, bool exact, bool x_f32, bool direct,
-                const float *residual, int gelu, hipStream_t s) {
+                const float *residual, int epi, hipStream_t s) {
   // 8 waves (two per SIMD cover each other's load latency), one quad of x in
   // flight per wave; 4 waves with 2 quads in flight measured within 3%.
   // `direct`: bf16 x read in place (xf = x), else the fragment-order copy.
   auto go = [&](auto exact_, auto parts, auto direct_) {
     return launch_dqmm_t<MT, 8, 1, decltype(exact_)::value, decltype(parts)::value, decltype(direct_)::value>(
-        packed, pb, sigma16, rows, apr, xf, m, y, partial, pl, kp_dq, pl_ids, pl_vecs, residual, tscale, gelu, s);
+        packed, pb, sigma16, rows, apr, xf, m, y, partial, pl, kp_dq, pl_ids, pl_vecs, residual, tscale, epi, s);
   };
   using T = std::true_type;
   using F = std::false_type;
@@ -2013,15 +2044,15 @@ size_t bg_partial_bytes(const BgPlan &p, int64_t rows, int64_t m) {
   return p.splits > 1 ? static_cast<size_t>((m + 63) / 64) * p.splits * 64 * static_cast<size_t>(rows) * sizeof(float) : 0;
 }
 
-int launch_reduce(const float *partial, int splits, int64_t rows, int64_t m, float *y, const float *residual, int gelu,
+int launch_reduce(const float *partial, int splits, int64_t rows, int64_t m, float *y, const float *residual, int epi,
                   hipStream_t s) {
   const int64_t cnt = m * rows;
   if (rows % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0)
     hipLaunchKernelGGL((dqmm_reduce_kernel<true>), dim3(static_cast<unsigned>((cnt / 4 + 255) / 256)), dim3(256), 0, s,
-                       partial, splits, rows, m, y, residual, gelu);
+                       partial, splits, rows, m, y, residual, epi);
   else
     hipLaunchKernelGGL((dqmm_reduce_kernel<false>), dim3(static_cast<unsigned>((cnt + 255) / 256)), dim3(256), 0, s,
-                       partial, splits, rows, m, y, residual, gelu);
+                       partial, splits, rows, m, y, residual, epi);
   return check_launch("dqmm_reduce_kernel");
 }
 
@@ -2157,6 +2188,7 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
   const int x_is_f32 = flags & PLX_DQL_X_F32;
   const int round_w = !x_is_f32 && (flags & PLX_DQL_W_AS_X) ? 1 : 0;  // W.to(fp32) is exact
   const int gelu = (flags & PLX_DQL_GELU) ? 1 : 0;
+  const int epi = (gelu ? kEpiGelu : 0) | ((flags & PLX_DQL_Y_BF16) ? kEpiBf16 : 0);
   const bool norm = (flags & PLX_DQL_RMS_NORM) != 0;
   if (norm != (norm_w != nullptr))
     return fail(PLX_EINVAL, "dequant_linear: PLX_DQL_RMS_NORM and a norm weight go together");
@@ -2213,15 +2245,15 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
       const int64_t pb = ((t.rows * apr + 3) / 4) * 9;  // packed stream length
       st = m > 32 ? launch_dqmm<4>(t.packed, planes ? 6 * t.rows * apr : pb, t.sigma16, t.rows, apr, xf, tscale, m, t.y,
                                    part, pl, tab->kp_dq, planes ? tab->pl_ids : nullptr, pl_vecs, !round_w, x_is_f32,
-                                   !copy, t.residual, gelu, s)
+                                   !copy, t.residual, epi, s)
                   : m > 16 ? launch_dqmm<2>(t.packed, planes ? 6 * t.rows * apr : pb, t.sigma16, t.rows, apr, xf, tscale, m,
                                             t.y, part, pl, tab->kp_dq, planes ? tab->pl_ids : nullptr, pl_vecs,
-                                            !round_w, x_is_f32, !copy, t.residual, gelu, s)
+                                            !round_w, x_is_f32, !copy, t.residual, epi, s)
                            : launch_dqmm<1>(t.packed, planes ? 6 * t.rows * apr : pb, t.sigma16, t.rows, apr, xf, tscale, m,
                                             t.y, part, pl, tab->kp_dq, planes ? tab->pl_ids : nullptr, pl_vecs,
-                                            !round_w, x_is_f32, !copy, t.residual, gelu, s);
+                                            !round_w, x_is_f32, !copy, t.residual, epi, s);
       if (st != PLX_OK || pl.splits == 1) continue;
-      st = launch_reduce(part, pl.splits, t.rows, m, t.y, t.residual, gelu, s);
+      st = launch_reduce(part, pl.splits, t.rows, m, t.y, t.residual, epi, s);
     }
     return st;
   }
@@ -2232,7 +2264,7 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
     if (n == 1 && !x_is_f32 && !norm && !gelu && !targets[0].residual) {  // the plain bf16 call
       if (targets[0].rows <= 0) return PLX_OK;
       return launch_gemv1_planes(targets[0].packed, targets[0].sigma16, targets[0].rows, apr, x, tab, round_w,
-                                 targets[0].y, s);
+                                 flags & PLX_DQL_Y_BF16, targets[0].y, s);
     }
     if (apr > 320)
       return fail(PLX_EINVAL, "dequant_linear: the plane layout takes rows of at most 320 atoms at one token (got %lld)",

@@ -40,7 +40,7 @@ def dequantize_h24(packed: torch.Tensor, sigma16: torch.Tensor, out_features: in
     return out
 
 
-DQL_X_F32, DQL_W_AS_X, DQL_GELU, DQL_RMS_NORM, DQL_PLANES = 1, 2, 4, 8, 16  # plx_dequant_linear flags (include/pollux_amd.h)
+DQL_X_F32, DQL_W_AS_X, DQL_GELU, DQL_RMS_NORM, DQL_PLANES, DQL_Y_BF16 = 1, 2, 4, 8, 16, 32  # plx_dequant_linear flags (include/pollux_amd.h)
 
 
 def h24_plane_layout(packed: torch.Tensor, n_atoms: int) -> torch.Tensor:
@@ -75,7 +75,7 @@ def plane_layout_takes(m: int, in_features: int) -> bool:
 
 def dequant_linear(
     packed: torch.Tensor, sigma16: torch.Tensor, out_features: int, in_features: int, x: torch.Tensor,
-    weight_rounding: str = "exact", planes: torch.Tensor | None = None,
+    weight_rounding: str = "exact", planes: torch.Tensor | None = None, y_as_x: bool = False,
 ) -> torch.Tensor:
     """y = x @ W.T in fp32 without materialising W (pollux.py:491-507).
 
@@ -87,6 +87,8 @@ def dequant_linear(
     x: [..., in] bf16 or fp32 (other float dtypes are cast to fp32); returns fp32 [..., out].
     planes: the weight's h24_plane_layout, used for the batches plane_layout_takes
     names (same results, no per-atom table gathers); else the packed stream.
+    y_as_x: the result in x's dtype, rounded once from the fp32 sums (for bf16 x
+    mostly by the kernel that makes them).
     """
     _lib.require_device(packed, "dequant_linear packed input")
     if packed.dtype != torch.uint8 or sigma16.dtype != torch.float16:
@@ -105,7 +107,6 @@ def dequant_linear(
         xx = xx.clone()
     m = xx.numel() // in_features
     sg = sigma16.contiguous()
-    y = torch.empty((*x.shape[:-1], out_features), dtype=torch.float32, device=pk.device)
     flags = (DQL_X_F32 if xx.dtype == torch.float32 else 0) | (DQL_W_AS_X if weight_rounding == "as_x" else 0)
     src, nsrc = pk, pk.numel()
     n_atoms = out_features * (in_features // 24)
@@ -117,6 +118,10 @@ def dequant_linear(
             src = src.clone()
         nsrc = 6 * n_atoms
         flags |= DQL_PLANES
+    y16 = y_as_x and x.dtype == torch.bfloat16 and (m > 2 or (m == 1 and flags & DQL_PLANES))
+    if y16:
+        flags |= DQL_Y_BF16
+    y = torch.empty((*x.shape[:-1], out_features), dtype=torch.bfloat16 if y16 else torch.float32, device=pk.device)
     lib = _lib.lib()
     nws = lib.plx_dequant_linear_workspace_bytes(out_features, in_features, m, flags)
     ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=pk.device) if nws else None
@@ -126,7 +131,7 @@ def dequant_linear(
             flags, m, _lib.ptr(y), _lib.ptr(ws), nws, _lib.stream_of(pk.device),
         )
     _lib.check(st, "dequant_linear")
-    return y
+    return y.to(x.dtype) if y_as_x else y
 
 
 def dequant_linear_multi(
@@ -376,7 +381,7 @@ class PackedH24Linear(nn.Module):
             takes = self.use_plane_layout and plane_layout_takes(m, self.in_features)
             planes = self.plane_layout() if takes else None
             y = dequant_linear(self.packed_weights, self.sigma_rows, self.out_features, self.in_features, x,
-                               weight_rounding=self.weight_rounding, planes=planes).to(x.dtype)
+                               weight_rounding=self.weight_rounding, planes=planes, y_as_x=True)
             return y if self.bias is None else y + self.bias.to(x.dtype)
         return F.linear(x, self.weight.to(dtype=x.dtype), self.bias)
 
