@@ -410,7 +410,8 @@ int plx_dequant_int8_rows(const int8_t *q, const uint16_t *mu16, int64_t rows, i
  * kernel reads them once per 64 tokens (both exact products, fp32 sums; with a
  * norm the MFMA kernel scales each token's sums by the rsqrt at the end).
  * plx_int8_linear_ws: the same with a workspace (the size below, 16-byte
- * aligned; nothing needs clearing; null: as plx_int8_linear).  From 5 tokens x
+ * aligned; nothing needs clearing; 0 where the products are too small for it
+ * to pay; null: as plx_int8_linear).  From 5 tokens x
  * is then normalised and split once, into two fp16 parts per row scaled by a
  * power of two (x to its last fp32 bit; elements below 2^-28 of their row's
  * largest to 2^-52 of that), and the products are exact. */

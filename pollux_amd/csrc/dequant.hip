@@ -993,7 +993,8 @@ typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 // what the last kernel of a batched call does to the sums: GELU; bf16 outputs (bf16 x), a launch and 6 bytes of
-// traffic per output less than a conversion after the call
+// traffic per output less than a conversion after the call (per call from Python, one token 7680x1920 19.8 -> 14.7 us,
+// 64 tokens 1920x7680 27.9 -> 22.7)
 constexpr int kEpiGelu = 1, kEpiBf16 = 2;
 constexpr int kMmRows = 32;             // output rows per block
 constexpr int kMmMaxApb = 128;          // atoms of a row per block (kp_dq tile: 32 x 388 words = 49.7 KB)

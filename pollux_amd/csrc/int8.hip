@@ -45,6 +45,7 @@
 //   the position advances); an id or position out of range yields a NaN row.
 
 #include <algorithm>
+#include <type_traits>
 #include <hip/hip_fp16.h>
 
 #include "plx_device.h"
@@ -355,11 +356,12 @@ __device__ __forceinline__ void int8x8_hilo(uint32_t d0, uint32_t d1, __half2 s2
   lo = __builtin_bit_cast(bf16x8_i8, u4{pl[0], pl[1], pl[2], pl[3]});
 }
 
-// x split by every block (no workspace): the form of a call without one.
-template <int MT, bool NORM>
+// x split by every block: the form of small products and of calls without a workspace.
+template <int MT, bool NORM, bool ARG>
 __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8mm_kernel(
     const int8_t *__restrict__ q, const uint16_t *__restrict__ mu16, int64_t rows, int cols,
-    const float *__restrict__ x, int64_t m_total, const float *__restrict__ norm_w, float eps, float *__restrict__ y) {
+    const float *__restrict__ x, int64_t m_total, const float *__restrict__ norm_w, float eps, float *__restrict__ y,
+    uint64_t *__restrict__ keys) {
   constexpr int TOK = 16 * MT;
   __shared__ __align__(16) float red[kI8mmWaves][TOK][kI8mmRedStride];
   __shared__ float sq[kI8mmWaves][TOK];
@@ -518,6 +520,7 @@ __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8mm_kernel(
     for (int w = 1; w < kI8mmWaves; ++w) t2 += sq[w][tl];
     rs = 1.0f / sqrtf(t2 / static_cast<float>(cols) + eps);
   }
+  uint64_t kb = 0;
 #pragma unroll
   for (int i = 0; i < kRpt; ++i) {
     const int rr = part + kTpt * i;
@@ -526,7 +529,21 @@ __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8mm_kernel(
     for (int w = 1; w < kI8mmWaves; ++w) sum += red[w][tl][rr];
     if constexpr (NORM) sum *= rs;
     const int64_t row = row0 + rr;
-    if (tok < m_total && row < rows) y[tok * rows + row] = sum;
+    if (tok < m_total && row < rows) {
+      y[tok * rows + row] = sum;
+      if constexpr (ARG) {
+        const uint64_t k = arg_key(sum, static_cast<uint32_t>(row));
+        kb = k > kb ? k : kb;
+      }
+    }
+  }
+  if constexpr (ARG) {
+#pragma unroll
+    for (int d = 1; d < kTpt; d <<= 1) {
+      const uint64_t o = shfl_xor_u64(kb, d);
+      kb = o > kb ? o : kb;
+    }
+    if (part == 0 && tok < m_total) keys[tok * gridDim.x + blockIdx.x] = kb;
   }
 }
 
@@ -824,22 +841,37 @@ int int8_linear_blocks(int64_t rows, int64_t *rows_per_wave) {
 
 // From this many tokens the MFMA kernels run: they read the weights once for up to 64 tokens, the GEMV once per 4
 // tokens.  Measured on the Pollux head (50,688 x 1,920): GEMV 20.8 / 25.8 / 47.4 / 79.2 us at 1 / 2 / 4 / 5 tokens,
-// int8parts_kernel 31 at 5..16 (the lower edge stays at 5: the graph prefill's padded lengths count on it).  With a
-// workspace int8parts_kernel runs, always the faster; int8mm_kernel is left for calls without one.
+// int8parts_kernel 31 at 5..16 (the lower edge stays at 5: the graph prefill's padded lengths count on it).
 constexpr int64_t kI8mmMinTokens = 5;
 
 int64_t int8mm_row_blocks(int64_t rows) { return (rows + kI8mmRows - 1) / kI8mmRows; }
 
 int launch_int8mm(const int8_t *q, const uint16_t *mu16, int64_t rows, int cols, const float *x, int64_t m,
-                  const float *norm_w, float eps, float *y, hipStream_t s) {
+                  const float *norm_w, float eps, float *y, uint64_t *keys, hipStream_t s) {
   const int mt = x_parts_tiles(m);
   const int64_t slabs = (m + 16 * mt - 1) / (16 * mt);
   if (slabs > 0xFFFFll) return fail(PLX_EINVAL, "int8_linear: %lld tokens", static_cast<long long>(m));
   const dim3 g(static_cast<unsigned>(int8mm_row_blocks(rows)), static_cast<unsigned>(slabs)), b(64 * kI8mmWaves);
-  auto k = norm_w ? (mt == 1 ? int8mm_kernel<1, true> : mt == 2 ? int8mm_kernel<2, true> : int8mm_kernel<4, true>)
-                  : (mt == 1 ? int8mm_kernel<1, false> : mt == 2 ? int8mm_kernel<2, false> : int8mm_kernel<4, false>);
-  hipLaunchKernelGGL(k, g, b, 0, s, q, mu16, rows, cols, x, m, norm_w, eps, y);
+  auto pick = [&](auto norm, auto arg) {
+    constexpr bool N = decltype(norm)::value, A = decltype(arg)::value;
+    return mt == 1 ? int8mm_kernel<1, N, A> : mt == 2 ? int8mm_kernel<2, N, A> : int8mm_kernel<4, N, A>;
+  };
+  auto k = norm_w ? (keys ? pick(std::true_type{}, std::true_type{}) : pick(std::true_type{}, std::false_type{}))
+                  : (keys ? pick(std::false_type{}, std::true_type{}) : pick(std::false_type{}, std::false_type{}));
+  hipLaunchKernelGGL(k, g, b, 0, s, q, mu16, rows, cols, x, m, norm_w, eps, y, keys);
   return check_launch("int8mm_kernel");
+}
+
+// Whether x is split in a launch of its own: where the blocks' own splits cost more than that launch (about 6 us of a
+// call).  A block's time goes with the row length and its token tiles; up to 240 blocks run at once, more in turns.
+// Measured per call from Python, by block / once: 64 tokens 480 x 480 12.5 / 16.8 us, 480 x 960 19.5 / 16.4,
+// 50,688 x 192 22.9 / 17.9; 32 tokens 2,016 x 960 14.3 / 17.5, 2,016 x 1,920 23.2 / 17.2; 16 tokens 2,016 x 1,920
+// 17.5 / 17.2, 50,688 x 480 16.2 / 17.5, 50,688 x 960 28.5 / 18.5.  (Rises with the row length: the argmax workspace,
+// sized without it, takes the longest.)
+bool splits_once(int64_t rows, int64_t cols, int64_t m) {
+  const int64_t blocks = int8mm_row_blocks(rows) * ((m + 63) / 64);
+  const int64_t least = m > 32 ? 600 : m > 16 ? 1200 : 2000;
+  return cols * std::max<int64_t>(240, blocks) >= 240 * least;
 }
 
 // Workspace of the MFMA path from `ws` (16-byte aligned): the split x, then the normalised x where the norm is a
@@ -885,8 +917,8 @@ int int8_linear(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t col
   if (rows > 0x7FFFFFFFll) return fail(PLX_EINVAL, "int8_linear: too many rows");
   if (m >= kI8mmMinTokens) {
     const int ci = static_cast<int>(cols);
-    return ws ? launch_int8parts(q, mu16, rows, ci, x, m, norm_w, eps, y, keys, ws, s)
-              : launch_int8mm(q, mu16, rows, ci, x, m, norm_w, eps, y, s);
+    return ws && splits_once(rows, cols, m) ? launch_int8parts(q, mu16, rows, ci, x, m, norm_w, eps, y, keys, ws, s)
+              : launch_int8mm(q, mu16, rows, ci, x, m, norm_w, eps, y, keys, s);
   }
   int64_t rpw = 0;
   const int blocks = int8_linear_blocks(rows, &rpw);
@@ -943,7 +975,7 @@ uint8_t *align16(uint8_t *p) { return reinterpret_cast<uint8_t *>((reinterpret_c
 }  // namespace
 
 size_t int8_linear_workspace_bytes(int64_t rows, int64_t cols, int64_t m) {
-  if (rows <= 0 || m < kI8mmMinTokens || cols <= 0 || cols > kI8MaxCols) return 0;
+  if (rows <= 0 || m < kI8mmMinTokens || cols <= 0 || cols > kI8MaxCols || !splits_once(rows, cols, m)) return 0;
   return int8parts_bytes(cols, m);
 }
 

@@ -8,11 +8,14 @@ from oracle import torch_ref
 
 pytestmark = pytest.mark.gpu
 
-# one and several double steps of 64 columns and their halves, a wave without a step, the last row length whose
-# norm is fused into the split (2,016) and the first that is not, the longest; 1, 2 and 4 token tiles, a partial
-# second slab; one row, a partial row block, row blocks that do not fill the eight XCDs' turns
-SHAPES = [(1, 16, 5), (63, 48, 16), (64, 64, 17), (65, 80, 32), (130, 96, 33), (513, 112, 64), (520, 1920, 65),
-          (77, 2016, 6), (77, 2032, 40), (200, 4096, 129)]
+# x split once: one row and partial row blocks, 1, 2 and 4 token tiles, partial slabs, rows of parts of a double step
+# of 64 columns, waves without a step (80 columns), the last row length whose norm is fused into the split (2,016) and
+# the first that is not, the longest, the least work of the rule at each token count
+ONCE = [(1, 1040, 33), (63, 624, 64), (130, 960, 65), (64, 4096, 5), (65, 2016, 16), (70, 2032, 17), (520, 1920, 32),
+        (513, 2016, 40), (77, 2032, 40), (200, 4096, 129), (40_000, 80, 300), (33_000, 112, 130), (70, 608, 33)]
+# split by every block: just below that work, and the smallest
+BLOCK = [(1, 16, 5), (63, 48, 16), (65, 80, 32), (513, 112, 64), (70, 592, 33), (70, 1184, 32), (200, 1984, 16)]
+SHAPES = [(*s, True) for s in ONCE] + [(*s, False) for s in BLOCK]
 
 
 def _inputs(dev, rows, cols, m):
@@ -43,10 +46,13 @@ def _direct(q, mu, x, norm):
     return y
 
 
-@pytest.mark.parametrize("rows,cols,m", SHAPES)
+@pytest.mark.parametrize("rows,cols,m,once", SHAPES)
 @pytest.mark.parametrize("normed", [False, True])
-def test_both_forms_against_float64(rows, cols, m, normed):
+def test_both_forms_against_float64(rows, cols, m, once, normed):
+    from pollux_amd import _lib
     from pollux_amd.packed import int8_linear
+
+    assert (_lib.lib().plx_int8_linear_workspace_bytes(rows, cols, m) > 0) == once
 
     dev = torch.device("cuda:0")
     q, mu, x = _inputs(dev, rows, cols, m)
@@ -62,10 +68,10 @@ def test_both_forms_against_float64(rows, cols, m, normed):
     # fp32 roundings of a sum, each at most 2^-23 of sum|x||w| (the MFMA rounds down): six MFMAs (two for the split
     # x) of a wave's share of the steps of 32 columns, three additions over the waves, two scales, the split's last
     # bit of x; the norm: the sum of squares (half of its 11 + cols / 64 roundings), root, quotient, two products
-    per_step = {"split once": 2, "split by block": 6}
     steps = 2 * ((cols + 255) // 256)
-    for name, y in (("split once", int8_linear(q, mu, x, norm=norm)), ("split by block", _direct(q, mu, x, norm))):
-        n = per_step[name] * steps + 6 + ((11 + cols // 64) // 2 + 5 if normed else 0)
+    for name, per_step, y in (("layer", 2 if once else 6, int8_linear(q, mu, x, norm=norm)),
+                              ("no workspace", 6, _direct(q, mu, x, norm))):
+        n = per_step * steps + 6 + ((11 + cols // 64) // 2 + 5 if normed else 0)
         err = (y.double().cpu() - ref).abs()
         # (beside it the split's floor, 2^-52 of a row's largest |x| per term, and the smallest fp32 values)
         bound = n * 2.0**-23 * scale + cols * 2.0**-52 * xd.abs().amax(1, keepdim=True) * w.abs().amax(1) + 2.0**-140
@@ -77,7 +83,7 @@ def test_split_once_inf_nan_and_argmax_route():
     from pollux_amd.packed import int8_linear, int8_linear_argmax
 
     dev = torch.device("cuda:0")
-    q, mu, x = _inputs(dev, 200, 112, 70)
+    q, mu, x = _inputs(dev, 200, 624, 70)
     x[10, 5], x[11, 6], mu[9] = float("inf"), float("nan"), float("nan")
     q[:, 5] = torch.where(q[:, 5] == 0, 1, q[:, 5])
     y = int8_linear(q, mu, x)
