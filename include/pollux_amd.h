@@ -298,13 +298,16 @@ size_t plx_dequant_linear_workspace_bytes(int64_t rows, int64_t cols, int64_t m_
 /* y[m, r] = sum_i x[m, i] * W[r, i] for m < m_rows, with W the fp16
  * materialisation of (packed, sigma16) above, never stored: x is bf16 or fp32
  * (PLX_DQL_X_F32) [m_rows, cols], y fp32 [m_rows, rows].  The products with
- * the fp16 weights are exact and accumulated in fp32: the numerics of
- * F.linear(x.float(), W.float()).  With PLX_DQL_W_AS_X and bf16 x the weights
+ * the fp16 weights are accumulated in fp32, the numerics of
+ * F.linear(x.float(), W.float()); they are exact but for the last bit of fp32 x
+ * above 4 tokens (below).  With PLX_DQL_W_AS_X and bf16 x the weights
  * are rounded to bf16 (RNE) first; with PLX_DQL_GELU, y = gelu(x W^T) (torch's
  * erf form).  Results are deterministic (fixed summation order).  Batches
- * above 4 tokens of fp32 x (as two fp16 parts of the row scaled by a power of
- * two: x to 2^-23, or 2^-52 of the row's largest) or above 2 of bf16 x run on
- * MFMA and need the workspace sized by
+ * above 4 tokens of fp32 x or above 2 of bf16 x run on MFMA.  There fp32 x is
+ * two fp16 parts of its row scaled by a power of two, each value to its last
+ * fp32 bit (2^-23 of the value); a row with values further below its largest
+ * than these can hold (2^-28 of it or less) is three bf16 parts, exactly.
+ * They need the workspace sized by
  * plx_dequant_linear_workspace_bytes (a fragment-order copy of x, plus split
  * partial tiles for narrow layers); cols <= 2^22.
  * Replaces PackedH24Linear.forward after materialize (pollux.py:506-507:
@@ -407,14 +410,14 @@ int plx_dequant_int8_rows(const int8_t *q, const uint16_t *mu16, int64_t rows, i
  * token (the final norm ln_f before the head, pollux.py:699-700).
  * cols % 16 == 0 and <= 4,096; q, x, norm_weight 16-byte aligned.  Up to 4
  * tokens a GEMV streams the INT8 rows once per 4 tokens; from 5 tokens an MFMA
- * kernel reads them once per 64 tokens (both exact products, fp32 sums; with a
+ * kernel reads them once per 64 tokens (exact products, fp32 sums; with a
  * norm the MFMA kernel scales each token's sums by the rsqrt at the end).
  * plx_int8_linear_ws: the same with a workspace (the size below, 16-byte
  * aligned; nothing needs clearing; 0 where the products are too small for it
  * to pay; null: as plx_int8_linear).  From 5 tokens x
- * is then normalised and split once, into two fp16 parts per row scaled by a
- * power of two (x to its last fp32 bit; elements below 2^-28 of their row's
- * largest to 2^-52 of that), and the products are exact. */
+ * is then normalised and split once, as plx_dequant_linear's (two fp16 parts,
+ * each value to its last fp32 bit; rows of too wide a range three bf16 parts,
+ * exactly), and the products of the parts are exact. */
 int plx_int8_linear(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x,
                     int64_t m_rows, const float *norm_weight, float norm_eps, float *y, void *stream);
 size_t plx_int8_linear_workspace_bytes(int64_t rows, int64_t cols, int64_t m_rows);

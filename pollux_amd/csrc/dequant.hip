@@ -960,18 +960,19 @@ int launch_dql(DqlTargets t, int64_t apr, const void *x, int64_t m, const uint4 
 // dqmm_reduce_kernel sums the split partial tiles in split order).
 //   prologue: decode the block's 32 x apb codes from the packed stream and
 //             fetch their kp_dq words (3 per code) into LDS; 32 lanes build
-//             the 8-entry bf16 byte tables (hi, and lo when EXACT) of the
-//             block's rows;
+//             the 8-entry byte tables of the block's rows (bf16 x: bf16 hi,
+//             and lo when EXACT; fp32 x: scaled fp16);
 //   k loop:   each wave takes a contiguous share of the block's atoms in
 //             quads of 4 (= 3 K steps of 32) and reads its activation
 //             fragments (up to 32 bf16 tokens: from x in place; otherwise
 //             from a fragment-order copy that a small kernel writes first,
-//             fp32 x as two fp16 parts; L2-resident either way: every block
-//             reads all of it), PD quads ahead in registers; per K step a
+//             fp32 x as two fp16 parts, or three bf16 parts for a row of too
+//             wide a range; L2-resident either way: every block reads all of
+//             it), PD quads ahead in registers; per K step a
 //             lane decodes its B fragments (8 weights of one row = one plane
 //             of one atom) from one LDS word with v_perm_b32 byte lookups and
-//             issues 2*MT MFMAs (4*MT when EXACT).  No block barrier inside
-//             the loop.
+//             issues 2*MT MFMAs (4*MT when EXACT or fp32 x).  No block
+//             barrier inside the loop.
 //   epilogue: the waves' fp32 tiles are summed through LDS in wave order.
 // When the copy is used, xfrag_kernel runs first and writes it into the
 // caller's workspace.
@@ -1061,13 +1062,21 @@ __device__ __forceinline__ void group_codes(uint32_t d0, uint32_t d1, uint32_t d
 //
 // fp32 x is two fp16 parts: the token's row is scaled by a power of two (its largest finite |x| into
 // [2^14, 2^15)), then h = fp16(x'), m = fp16(2^11 (x' - h)).  x' - h is exact and has at most 13 significant
-// bits, so h + 2^-11 m is x' up to its last fp32 bit, i.e. 2^-23 |x| (0.5 * 2^-23 |x| rms), where |x| is at
-// least 2^-28 of the row's largest; smaller elements keep 2^-52 of that largest.  fp16 weights need no split,
+// bits, so h + 2^-11 m is x' up to its last fp32 bit, i.e. 2^-23 |x| (0.5 * 2^-23 |x| rms), where |x'| is at
+// least kWideBelow.  fp16 weights need no split,
 // so the GEMM takes two MFMAs per tile where three bf16 parts against hi + lo took six; with a third of the
-// fp32 roundings its results are closer to float64 than the exact split's (a
-// decoder block's keys at 1,024 tokens: 2.3e-7 -> 1.8e-7 relative), its time a third less (183 -> 123 us for 1,024
-// tokens, 7680x1920 and its like).
+// fp32 roundings its results are closer to float64 than the exact split's (24 to 7,680 columns, 5 to 1,024 tokens:
+// 0.5 to 0.96 of its error), its time a third less (183 -> 123 us for 1,024 tokens, 7680x1920 and its like).
 // inf / nan go to h alone, as they are.  The scale's inverse per token goes to tscale.
+//
+// A row with elements below that (2^-28 of its largest or less: fp16 has no exponents left for them, and an output
+// whose weights are zero at the large elements is made of such elements alone) is stored as three bf16 parts
+// instead, x = h + m + l exactly while the parts stay normal (|x| >= ~2^-110; inf / nan in h alone), unscaled, and
+// marked by tscale = 0: the GEMMs form that token's outputs again from the three parts against the weights' hi + lo.
+// One such element among 7,680 normal values is one row in 10,000, which the second pass would cost up to 50 us of a
+// call; H24 weights never see it alone (every code but the origin has two or more nonzero coordinates in an atom,
+// equal ones where it has fewer than 24), so beside elements of at least kWideBelow its floor of 2^-36 is 2^-23 of
+// theirs, and their rule is two elements below the line, one of them not zero.  INT8 weights are zero anywhere: one.
 __device__ __forceinline__ float pow2f(int e) { return __uint_as_float(static_cast<uint32_t>(e + 127) << 23); }
 
 // exponent e such that |v| 2^e is in [2^14, 2^15) for the largest finite |v| of a row (|e| <= 126)
@@ -1090,6 +1099,31 @@ __device__ __forceinline__ uint32_t split_f16(float v, float sc) {
   return __half_as_ushort(h) | mb << 16;
 }
 
+constexpr int kXfParts = 3;             // parts stored per fp32 element (the third only of rows kept as bf16 parts)
+constexpr float kWideBelow = 0x1p-13f;  // of the scaled row
+
+// The largest finite |v| into top, the smallest nonzero |v| into low as its bits less 1, shifted left by 1 (a zero
+// becomes the largest word; from 0, ~0u).
+__device__ __forceinline__ void range_of(float4 v, float &top, uint32_t &low) {
+  const float a[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    top = fmaxf(top, finite_abs(a[e]));
+    low = min(low, (__float_as_uint(a[e]) << 1) - 1u);
+  }
+}
+
+// whether the smallest nonzero |v| is below the line in a row scaled by sc
+__device__ __forceinline__ bool has_below(uint32_t low, float sc) {
+  return low != ~0u && __uint_as_float((low + 1u) >> 1) * sc < kWideBelow;
+}
+
+// how many of v are below the line in a row scaled by sc (zeros too)
+__device__ __forceinline__ int below_line(float4 v, float sc) {
+  return (finite_abs(v.x) * sc < kWideBelow) + (finite_abs(v.y) * sc < kWideBelow) +
+         (finite_abs(v.z) * sc < kWideBelow) + (finite_abs(v.w) * sc < kWideBelow);
+}
+
 __global__ __launch_bounds__(256) void xfrag_kernel(const uint16_t *__restrict__ x, int64_t m_total, int64_t cols,
                                                     int64_t n_quads_row, int tiles, uint4 *__restrict__ xf) {
   constexpr int kQuadFrags = kXfQuadBytes / 16;  // 768 per part
@@ -1108,19 +1142,38 @@ __global__ __launch_bounds__(256) void xfrag_kernel(const uint16_t *__restrict__
   xf[static_cast<int64_t>(blockIdx.y) * per_slab + f] = v;
 }
 
-// the two fp16 parts of columns 4i .. 4i+3 of token (slab, t, tl) into the copy
-__device__ __forceinline__ void store_parts(uint2 *__restrict__ xf, int64_t slab, int64_t n_quads_row, int t, int tl,
-                                            int64_t i, const float *v, float sc) {
+// the fragment of columns 4i .. 4i+3 of token (slab, t, tl) in the copy's first part
+__device__ __forceinline__ uint2 *part_slot(uint2 *__restrict__ xf, int64_t slab, int64_t n_quads_row, int t, int tl,
+                                            int64_t i) {
   constexpr int kQuadFrags = kXfQuadBytes / 16;
   const int64_t qs = i >> 3, quad = qs / 3;  // K step of the row, its quad
   const int c8 = static_cast<int>(i >> 1) & 3;
-  uint32_t p[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) p[e] = split_f16(v[e], sc);
   const int64_t within = ((qs - 3 * quad) * 4 + t) * 64 + tl + 16 * c8;
-  uint2 *d = xf + 2 * ((slab * n_quads_row + quad) * 2 * kQuadFrags + within) + (i & 1);
+  return xf + 2 * ((slab * n_quads_row + quad) * kXfParts * kQuadFrags + within) + (i & 1);
+}
+
+// the two fp16 parts of v scaled by sc
+__device__ __forceinline__ void store_parts(uint2 *d, float4 v, float sc) {
+  const uint32_t p[4] = {split_f16(v.x, sc), split_f16(v.y, sc), split_f16(v.z, sc), split_f16(v.w, sc)};
   d[0] = make_uint2((p[0] & 0xFFFFu) | p[1] << 16, (p[2] & 0xFFFFu) | p[3] << 16);
-  d[2 * kQuadFrags] = make_uint2(p[0] >> 16 | (p[1] & 0xFFFF0000u), p[2] >> 16 | (p[3] & 0xFFFF0000u));
+  d[kXfQuadBytes / 8] = make_uint2(p[0] >> 16 | (p[1] & 0xFFFF0000u), p[2] >> 16 | (p[3] & 0xFFFF0000u));
+}
+
+// the three bf16 parts of v
+__device__ __forceinline__ void store_exact_parts(uint2 *d, float4 v) {
+  const float a[4] = {v.x, v.y, v.z, v.w};
+  uint32_t p[3][4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float r = a[e];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      p[k][e] = bf16_rne_bits(r);
+      r = fabsf(a[e]) <= 3.0e38f ? r - __uint_as_float(p[k][e] << 16) : 0.f;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) d[k * (kXfQuadBytes / 8)] = make_uint2(p[k][0] | p[k][1] << 16, p[k][2] | p[k][3] << 16);
 }
 
 // fp32 x, one block per token row of each slab's `tiles` token tiles; REG: rows of up to 8,192 columns are read
@@ -1128,9 +1181,10 @@ __device__ __forceinline__ void store_parts(uint2 *__restrict__ xf, int64_t slab
 constexpr int kXsVec = 8;
 template <bool REG>
 __global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x, int64_t m_total, int64_t cols,
-                                                     int64_t n_quads_row, int tiles, uint2 *__restrict__ xf,
-                                                     float *__restrict__ tscale) {
-  __shared__ float red[4];
+                                                     int64_t n_quads_row, int tiles, int wide_from,
+                                                     uint2 *__restrict__ xf, float *__restrict__ tscale) {
+  __shared__ float red[2][4];
+  __shared__ int below;
   const int tid = threadIdx.x;
   const int per_slab = 16 * tiles;
   const int64_t slab = blockIdx.x / static_cast<unsigned>(per_slab);
@@ -1140,10 +1194,8 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x
   const int64_t n4 = live ? cols >> 2 : 0, n_pad = n_quads_row * 24;  // float4s of the row, with the last quad's padding
   const float4 *xr = reinterpret_cast<const float4 *>(x + (live ? tok : 0) * cols);
   float4 v[REG ? kXsVec : 1];
-  float mx[1] = {0.f};
-  auto top = [&](float4 a) {
-    mx[0] = fmaxf(fmaxf(fmaxf(mx[0], finite_abs(a.x)), finite_abs(a.y)), fmaxf(finite_abs(a.z), finite_abs(a.w)));
-  };
+  float top = 0.f;
+  uint32_t low = ~0u;
   if constexpr (REG) {
 #pragma unroll
     for (int k = 0; k < kXsVec; ++k) {
@@ -1151,29 +1203,49 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x
       v[k] = i < n4 ? xr[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
 #pragma unroll
-    for (int k = 0; k < kXsVec; ++k) top(v[k]);
+    for (int k = 0; k < kXsVec; ++k) range_of(v[k], top, low);
   } else {
-    for (int64_t i = tid; i < n4; i += 256) top(xr[i]);
+    for (int64_t i = tid; i < n4; i += 256) range_of(xr[i], top, low);
   }
+  float mx[2] = {top, low == ~0u ? -__builtin_inff() : -__uint_as_float((low + 1u) >> 1)};
   group_reduce<64, true>(mx);
-  if ((tid & 63) == 0) red[tid >> 6] = mx[0];
+  if ((tid & 63) == 0) {
+    red[0][tid >> 6] = mx[0];
+    red[1][tid >> 6] = mx[1];
+  }
   __syncthreads();
-  const int e = row_exponent(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+#pragma unroll
+  for (int i = 0; i < 2; ++i) mx[i] = fmaxf(fmaxf(red[i][0], red[i][1]), fmaxf(red[i][2], red[i][3]));
+  const int e = row_exponent(mx[0]);
   const float sc = pow2f(e);
+  if (__builtin_expect(mx[1] * sc > -kWideBelow, 0)) {  // (block-uniform)
+    bool wide = true;
+    if (wide_from > 1) {
+      if (tid == 0) below = 0;
+      __syncthreads();
+      int n = 0;
+      for (int64_t i = tid; i < n4; i += 256) n += below_line(xr[i], sc);
+      if (n) atomicAdd(&below, n);
+      __syncthreads();
+      wide = below >= wide_from;
+    }
+    if (wide) {
+      if (tid == 0) tscale[tok] = 0.f;
+      for (int64_t i = tid; i < n_pad; i += 256)
+        store_exact_parts(part_slot(xf, slab, n_quads_row, t, tl, i), i < n4 ? xr[i] : make_float4(0.f, 0.f, 0.f, 0.f));
+      return;
+    }
+  }
   if (tid == 0) tscale[tok] = pow2f(-e);
   if constexpr (REG) {
 #pragma unroll
     for (int k = 0; k < kXsVec; ++k) {
       const int64_t i = tid + 256 * k;
-      const float a[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-      if (i < n_pad) store_parts(xf, slab, n_quads_row, t, tl, i, a, sc);
+      if (i < n_pad) store_parts(part_slot(xf, slab, n_quads_row, t, tl, i), v[k], sc);
     }
   } else {
-    for (int64_t i = tid; i < n_pad; i += 256) {
-      const float4 u = i < n4 ? xr[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-      const float a[4] = {u.x, u.y, u.z, u.w};
-      store_parts(xf, slab, n_quads_row, t, tl, i, a, sc);
-    }
+    for (int64_t i = tid; i < n_pad; i += 256)
+      store_parts(part_slot(xf, slab, n_quads_row, t, tl, i), i < n4 ? xr[i] : make_float4(0.f, 0.f, 0.f, 0.f), sc);
   }
 }
 
@@ -1185,7 +1257,8 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x
 constexpr int kNfVec = 8;
 __global__ __launch_bounds__(256) void normfrag_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                        int64_t m_total, int cols, int64_t n_quads_row, int tiles,
-                                                       float eps, uint2 *__restrict__ xf, float *__restrict__ tscale) {
+                                                       int wide_from, float eps, uint2 *__restrict__ xf,
+                                                       float *__restrict__ tscale) {
   const int lane = threadIdx.x & 63;
   const int64_t tok = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   const int64_t slab = tok >> 6;
@@ -1213,22 +1286,41 @@ __global__ __launch_bounds__(256) void normfrag_kernel(const float *__restrict__
   ss = wave_reduce_sum(ss);
   const float r = 1.0f / sqrtf(ss / static_cast<float>(cols) + eps);
   float mx[1] = {0.f};
+  uint32_t low = ~0u;
 #pragma unroll
   for (int k = 0; k < kNfVec; ++k) {
     v[k] = live ? make_float4(v[k].x * r * g[k].x, v[k].y * r * g[k].y, v[k].z * r * g[k].z, v[k].w * r * g[k].w)
                 : make_float4(0.f, 0.f, 0.f, 0.f);
-    mx[0] = fmaxf(fmaxf(fmaxf(mx[0], finite_abs(v[k].x)), finite_abs(v[k].y)),
-                  fmaxf(finite_abs(v[k].z), finite_abs(v[k].w)));
+    range_of(v[k], mx[0], low);
   }
   group_reduce<64, true>(mx);
   const int e = row_exponent(mx[0]);
   const float sc = pow2f(e);
+  if (__builtin_expect(__any(has_below(low, sc)), 0)) {
+    bool wide = true;
+    if (wide_from > 1) {
+      float n[1] = {0.f};
+#pragma unroll
+      for (int k = 0; k < kNfVec; ++k)
+        if (lane + 64 * k < n4) n[0] += static_cast<float>(below_line(v[k], sc));
+      group_reduce<64>(n);
+      wide = n[0] >= static_cast<float>(wide_from);
+    }
+    if (wide) {
+      if (lane == 0) tscale[tok] = 0.f;
+#pragma unroll
+      for (int k = 0; k < kNfVec; ++k) {
+        const int i = lane + 64 * k;
+        if (i < n_quads_row * 24) store_exact_parts(part_slot(xf, slab, n_quads_row, t, tl, i), v[k]);
+      }
+      return;
+    }
+  }
   if (lane == 0) tscale[tok] = pow2f(-e);
 #pragma unroll
   for (int k = 0; k < kNfVec; ++k) {
     const int i = lane + 64 * k;
-    const float a[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-    if (i < n_quads_row * 24) store_parts(xf, slab, n_quads_row, t, tl, i, a, sc);
+    if (i < n_quads_row * 24) store_parts(part_slot(xf, slab, n_quads_row, t, tl, i), v[k], sc);
   }
 }
 
@@ -1289,9 +1381,19 @@ __device__ __forceinline__ f16x8_t times_2m11(f16x8_t w) {
   return w * f16x8_t{c, c, c, c, c, c, c, c};
 }
 
+// scaled fp16 weights times inv (the row's scale taken back: exact) as bf16 hi + lo (hi alone for inf / nan)
+__device__ __forceinline__ void hi_lo_of(f16x8_t w, float inv, bf16x8_t &hi, bf16x8_t &lo) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float v = static_cast<float>(w[e]) * inv;
+    hi[e] = static_cast<__bf16>(v);
+    lo[e] = static_cast<__bf16>(fabsf(v) <= 65504.f ? v - static_cast<float>(hi[e]) : 0.f);
+  }
+}
+
 // token tiles of 16; waves per block; quads of x in flight per wave; exact fp16 weights (hi + lo);
 // parts per activation (1: bf16 x; 2: fp32 x as two fp16 parts against the scaled fp16 weights and them times
-// 2^-11, see xsplit_kernel)
+// 2^-11, and the tokens stored as three bf16 parts once more from those, see xfrag_kernel)
 // PLN: `packed` is the plane layout (3 uint16 records per atom); the value-id
 // words come from the plane table, staged in LDS, instead of kp_dq gathers.
 template <int MT, int WV, int PD, bool EXACT, int XP, bool XD, bool PLN>
@@ -1305,6 +1407,7 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
   static_assert(!F16 || (EXACT && !XD), "fp32 x: exact weights, from the copy");
   constexpr int NT = 64 * WV;
   constexpr int TOK = 16 * MT;
+  constexpr int XS = F16 ? kXfParts : XP;  // parts a quad of the copy holds
   const int ws = mm_row_words(apb);
   constexpr int TPT = 3;  // PLN: plane-table vectors per thread (the host checks pl_vecs <= TPT * NT)
   const int region = max(kMmRows * ws + (PLN ? TPT * NT * 4 : 0), WV * TOK * kMmRedStride) * 4;
@@ -1342,13 +1445,13 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
   const int64_t cols = atoms_per_row * kDim;
   const int slab_bytes =
       XD ? static_cast<int>(min(static_cast<int64_t>(64), m_total - tok0) * cols * 2)
-         : static_cast<int>(n_quads_row * XP * kXfQuadBytes);
+         : static_cast<int>(n_quads_row * XS * kXfQuadBytes);
   const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
       XD ? const_cast<uint8_t *>(reinterpret_cast<const uint8_t *>(xf) + tok0 * cols * 2)
          : reinterpret_cast<uint8_t *>(const_cast<uint4 *>(xf + static_cast<int64_t>(blockIdx.y) * (slab_bytes / 16))),
       static_cast<short>(0), slab_bytes, kBufferFlags);
   const int xbase = XD ? static_cast<int>(j * cols * 2 + 16 * q)
-                       : static_cast<int>(a_begin / 4 + wq0) * XP * kXfQuadBytes + 16 * lane;
+                       : static_cast<int>(a_begin / 4 + wq0) * XS * kXfQuadBytes + 16 * lane;
   const int xcol0 = static_cast<int>(96 * (a_begin / 4 + wq0)) + 8 * q;  // XD: this lane's first column
   auto load_quad = [&](uint4 (&xa)[3][XP][MT], int qd) {
 #pragma unroll
@@ -1363,7 +1466,7 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
             off = qd < wqn && col < cols ? xbase + t * static_cast<int>(16 * cols * 2) + 2 * (col - 8 * q)
                                          : kBufferOutOfRange;
           } else {
-            off = qd < wqn ? xbase + (qd * XP + pp) * kXfQuadBytes + (4 * s + t) * 1024 : kBufferOutOfRange;
+            off = qd < wqn ? xbase + (qd * XS + pp) * kXfQuadBytes + (4 * s + t) * 1024 : kBufferOutOfRange;
           }
           asm("" : "+v"(off));  // one unconditional load (not one per select outcome under branches)
           xa[s][pp][t] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0));
@@ -1371,6 +1474,12 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
       }
     }
   };
+  float tsl = 1.f;  // F16: the scale of token tok0 + lane
+  if constexpr (F16) {
+    const __amdgpu_buffer_rsrc_t trs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(tscale + tok0),
+                                                                         static_cast<short>(0), TOK * 4, kBufferFlags);
+    tsl = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(trs, 4 * lane, 0, 0));
+  }
   uint4 xa[PD][3][XP][MT];
 #pragma unroll
   for (int u = 0; u < PD; ++u) load_quad(xa[u], u);  // in flight during the prologue
@@ -1592,6 +1701,50 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
   for (int u = 0; u < PD - 1; ++u)
     if (qd + u < wqn) compute_quad(xa[u], qd + u);
 
+  if constexpr (F16) {
+    // tokens stored as three bf16 parts: their outputs over this wave's quads, from the parts against the weights'
+    // hi + lo, in the place of what the fp16 products above made of their bits (other tokens never see those)
+    const uint64_t wide = __ballot(lane < TOK && tsl == 0.f);
+    if (__builtin_expect(wide != 0ull, 0)) {
+      const float inv0 = rscale[j], inv1 = rscale[16 + j];
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        if (((wide >> (16 * t)) & 0xFFFFull) == 0ull) continue;  // (wave-uniform)
+        f32x4_t c0 = {0.f, 0.f, 0.f, 0.f}, c1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int k = 0; k < wqn; ++k) {
+#pragma unroll
+          for (int s = 0; s < 3; ++s) {
+            bf16x8_t av[kXfParts];
+#pragma unroll
+            for (int pp = 0; pp < kXfParts; ++pp)
+              av[pp] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                        xrs, xbase + (k * XS + pp) * kXfQuadBytes + (4 * s + t) * 1024, 0, 0));
+            bf16x8_t h0, l0, h1, l1;
+            hi_lo_of(__builtin_bit_cast(f16x8_t, perm_decode(wrow0[12 * k + 4 * s], ta0.x, ta0.y, ta0.z, ta0.w)), inv0, h0, l0);
+            hi_lo_of(__builtin_bit_cast(f16x8_t, perm_decode(wrow1[12 * k + 4 * s], ta1.x, ta1.y, ta1.z, ta1.w)), inv1, h1, l1);
+#pragma unroll
+            for (int pp = 0; pp < kXfParts; ++pp) {
+              c0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[pp], h0, c0, 0, 0, 0);
+              c1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[pp], h1, c1, 0, 0, 0);
+            }
+#pragma unroll
+            for (int pp = 0; pp < kXfParts; ++pp) {
+              c0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[pp], l0, c0, 0, 0, 0);
+              c1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[pp], l1, c1, 0, 0, 0);
+            }
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if ((wide >> (16 * t + 4 * q + e)) & 1ull) {
+            acc[t][0][e] = c0[e];
+            acc[t][1][e] = c1[e];
+          }
+      }
+    }
+  }
+
   // ---- epilogue: the waves' tiles summed in wave order; C[token 16t + 4q + e][row 16rt + j] ----
   __syncthreads();  // every wave is done with the kp_dq tile
   float *rw = red + wave * (TOK * kMmRedStride);
@@ -1612,10 +1765,10 @@ __global__ __launch_bounds__(64 * WV, WV <= 4 ? 2 : 1) void dqmm_kernel(
     for (int w = 1; w < WV; ++w) sum += *reinterpret_cast<const f32x4_t *>(red + (w * TOK + tl) * kMmRedStride + 4 * g);
     const int64_t row = row0 + 4 * g;
     if (tok0 + tl >= m_total || row >= rows) continue;
-    if constexpr (F16) {  // the scales back (powers of two)
+    if constexpr (F16) {  // the scales back (powers of two; the bf16 parts have none)
       const float ts = tscale[tok0 + tl];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) sum[c] = sum[c] * rscale[4 * g + c] * ts;
+      for (int c = 0; c < 4; ++c) sum[c] = ts == 0.f ? sum[c] : sum[c] * rscale[4 * g + c] * ts;
     }
     float *d = dst + (tok_base + tl) * rows + row;
     if (splits == 1) {  // the final output: epilogue here (with a K split, in dqmm_reduce_kernel)
@@ -1845,7 +1998,7 @@ __global__ __launch_bounds__(256, 2) void dgemm_kernel(const uint4 *__restrict__
   // A step's units of 1 KiB: x fragments (slab, part, token tile), then weights (row tile); wave w loads token tile
   // w of every slab and part, and row tiles w, w + 4.
   // Raw buffer loads: the compiler moves plain loads of read-only memory down to where their values are stored.
-  const int64_t slab_bytes = static_cast<int64_t>(n_quads_row) * 2 * kXfQuadBytes;
+  const int64_t slab_bytes = static_cast<int64_t>(n_quads_row) * kXfParts * kXfQuadBytes;
   const int64_t tile_bytes = static_cast<int64_t>(ksteps) * 1024;  // one row tile's weights
   auto rsrc = [](const void *p, int64_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), static_cast<short>(0), static_cast<int>(bytes),
@@ -1865,7 +2018,7 @@ __global__ __launch_bounds__(256, 2) void dgemm_kernel(const uint4 *__restrict__
 #pragma unroll
     for (int i = 0; i < XU; ++i)
       r[i] = __builtin_amdgcn_raw_buffer_load_b128(i < 2 ? xr0 : xr1, 16 * lane,
-                                                   (quad * 2 + i % 2) * kXfQuadBytes + s * 4096 + wave * 1024, 0);
+                                                   (quad * kXfParts + i % 2) * kXfQuadBytes + s * 4096 + wave * 1024, 0);
 #pragma unroll
     for (int i = 0; i < WU; ++i)
       r[XU + i] = __builtin_amdgcn_raw_buffer_load_b128(
@@ -1964,6 +2117,48 @@ __global__ __launch_bounds__(256, 2) void dgemm_kernel(const uint4 *__restrict__
     ts[i] = tscale[min(slab * 64 + 16 * i + j, m_total - 1)];
     rs[i] = *reinterpret_cast<const float4 *>(rscale + local0 + 16 * i + 4 * q);
   }
+  // tokens stored as three bf16 parts (tscale 0): their sums again, from the parts against the weights' hi + lo (a
+  // step's six products from zero, then added, as above)
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    if (__builtin_expect(!__any(ts[t] == 0.f), 1)) continue;
+    f32x4_t c[4];
+    float inv[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      c[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      inv[r] = rscale[local0 + 16 * r + j];
+    }
+#pragma unroll 1
+    for (int k = k0; k < k1; ++k) {
+      const int quad = k / 3, s = k - 3 * quad;
+      bf16x8_t xp[kXfParts];
+      f16x8_t w[4];
+#pragma unroll
+      for (int p = 0; p < kXfParts; ++p)
+        xp[p] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                 ws ? xr1 : xr0, 16 * lane,
+                                                 (quad * kXfParts + p) * kXfQuadBytes + s * 4096 + t * 1024, 0));
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        w[r] = __builtin_bit_cast(f16x8_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                               wsr, 16 * lane, (wr * 4 + r) * static_cast<int>(tile_bytes) + k * 1024, 0));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        bf16x8_t hi, lo;
+        hi_lo_of(w[r], (k & 1) ? -inv[r] : inv[r], hi, lo);
+        f32x4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = kXfParts - 1; p >= 0; --p) d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, xp[p], d, 0, 0, 0);
+#pragma unroll
+        for (int p = kXfParts - 1; p >= 0; --p) d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, xp[p], d, 0, 0, 0);
+        c[r] += d;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (ts[t] == 0.f) acc[r][t] = c[r];
+  }
   float *dst = splits == 1 ? y : partial + (slab * splits + split) * 64 * rows;
   const bool fin = splits == 1;  // the final output (with a K split the epilogue runs in dqmm_reduce_kernel)
   const bool vec = (rows & 3) == 0 && ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(residual)) & 15u) == 0;
@@ -1984,10 +2179,12 @@ __global__ __launch_bounds__(256, 2) void dgemm_kernel(const uint4 *__restrict__
       const int64_t row = row_base + local0 + 16 * r + 4 * q;
       if (row >= rows) continue;
       f32x4_t v = acc[r][t];
-      v[0] = v[0] * rs[r].x * ts[t];
-      v[1] = v[1] * rs[r].y * ts[t];
-      v[2] = v[2] * rs[r].z * ts[t];
-      v[3] = v[3] * rs[r].w * ts[t];
+      if (ts[t] != 0.f) {
+        v[0] = v[0] * rs[r].x * ts[t];
+        v[1] = v[1] * rs[r].y * ts[t];
+        v[2] = v[2] * rs[r].z * ts[t];
+        v[3] = v[3] * rs[r].w * ts[t];
+      }
       float *d = dst + (fin ? tok : tl) * rows + row;
       if (vec) {
         if (fin) {
@@ -2099,7 +2296,7 @@ bool mm_x_copy(bool x_f32, int64_t m) { return x_f32 || m > 32; }
 MmWorkspace mm_workspace(int64_t rows, int64_t cols, int64_t m, const MmPlan &pl, bool x_f32) {
   MmWorkspace w;
   const size_t slabs = static_cast<size_t>((m + 63) / 64);
-  if (mm_x_copy(x_f32, m)) w.xf = slabs * static_cast<size_t>((cols + 95) / 96) * kXfQuadBytes * (x_f32 ? 2 : 1);
+  if (mm_x_copy(x_f32, m)) w.xf = slabs * static_cast<size_t>((cols + 95) / 96) * kXfQuadBytes * (x_f32 ? kXfParts : 1);
   if (x_f32) w.tscale = slabs * 64 * sizeof(float);
   if (pl.splits > 1) w.partial = slabs * pl.splits * 64 * static_cast<size_t>(rows) * sizeof(float);
   return w;
@@ -2153,8 +2350,8 @@ size_t x_parts_bytes(int64_t cols, int64_t m) {
 
 bool x_parts_fuses_norm(int64_t cols) { return (cols + 95) / 96 * 24 <= 64 * kNfVec; }
 
-int launch_x_parts(const float *x, const float *norm_w, float norm_eps, int64_t m, int64_t cols, float *xnorm, void *ws,
-                   hipStream_t s) {
+int launch_x_parts(const float *x, const float *norm_w, float norm_eps, int64_t m, int64_t cols, int wide_from,
+                   float *xnorm, void *ws, hipStream_t s) {
   const int64_t slabs = (m + 63) / 64, nq = (cols + 95) / 96;
   const int tiles = x_parts_tiles(m);
   float *tscale = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + mm_workspace(1, cols, m, MmPlan{}, true).xf);
@@ -2162,7 +2359,7 @@ int launch_x_parts(const float *x, const float *norm_w, float norm_eps, int64_t 
   if (norm_w && x_parts_fuses_norm(cols)) {
     // the norm writes the fragment-order copy itself (rows that fit normfrag_kernel's registers)
     hipLaunchKernelGGL(normfrag_kernel, dim3(static_cast<unsigned>(slabs * 16)), dim3(256), 0, s, x, norm_w, m,
-                       static_cast<int>(cols), nq, tiles, norm_eps, xf, tscale);
+                       static_cast<int>(cols), nq, tiles, wide_from, norm_eps, xf, tscale);
     return check_launch("normfrag_kernel");
   }
   if (norm_w) {
@@ -2172,9 +2369,9 @@ int launch_x_parts(const float *x, const float *norm_w, float norm_eps, int64_t 
   }
   const dim3 gs(static_cast<unsigned>(slabs * 16 * tiles));
   if (nq * 24 <= 256 * kXsVec)
-    hipLaunchKernelGGL(xsplit_kernel<true>, gs, dim3(256), 0, s, x, m, cols, nq, tiles, xf, tscale);
+    hipLaunchKernelGGL(xsplit_kernel<true>, gs, dim3(256), 0, s, x, m, cols, nq, tiles, wide_from, xf, tscale);
   else
-    hipLaunchKernelGGL(xsplit_kernel<false>, gs, dim3(256), 0, s, x, m, cols, nq, tiles, xf, tscale);
+    hipLaunchKernelGGL(xsplit_kernel<false>, gs, dim3(256), 0, s, x, m, cols, nq, tiles, wide_from, xf, tscale);
   return check_launch("xsplit_kernel");
 }
 
@@ -2224,7 +2421,7 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
     const size_t xf_bytes = mm_workspace(1, cols, m, MmPlan{}, x_is_f32 != 0).xf;
     float *tscale = reinterpret_cast<float *>(wsb + xf_bytes);  // fp32 x only
     if (x_is_f32) {
-      st = launch_x_parts(static_cast<const float *>(x), norm_w, norm_eps, m, cols, xnorm, wsb, s);
+      st = launch_x_parts(static_cast<const float *>(x), norm_w, norm_eps, m, cols, 2, xnorm, wsb, s);
     } else if (copy) {
       const int tiles = m > 32 ? 4 : 2;  // token tiles per slab the GEMM reads (its MT below): the copy writes only these
       hipLaunchKernelGGL(xfrag_kernel, dim3(static_cast<unsigned>(nq * 3), static_cast<unsigned>(slabs)), dim3(256), 0, s,

@@ -25,7 +25,9 @@
 //   1152 gives q exactly, and one fp16 multiply by s16 rounds q * s16 once -
 //   the same value as fp16(fp32(q) * fp32(s16)), whose fp32 product is exact.
 //
-// int8mm_kernel: the same product for two or more tokens on MFMA.  A block
+// int8mm_kernel: the same product for five or more tokens on MFMA where it is
+//   too small to split x in a launch of its own (int8parts_kernel, below), or
+//   without a workspace.  A block
 //   owns 64 rows x 16*MT tokens and its 4 waves split K (each wave a
 //   contiguous run of 32-column steps).  Per step a lane decodes 8 weights of
 //   one row per row tile (the fp16 values above, split exactly into bf16
@@ -553,6 +555,8 @@ __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8mm_kernel(
 // times 2^-11) where three bf16 parts against hi + lo took six, no split arithmetic, and a third of the fp32
 // roundings.  A block owns 64 rows x 16 MT tokens, its 4 waves split K; blocks of one XCD take the token slabs of a
 // row block in turn, so its bytes come from that XCD's L2 after the first.
+// A token whose row the two parts cannot hold comes as three bf16 parts, marked by a scale of 0 (xfrag_kernel in
+// dequant.hip): its sums are taken again, the parts against the weights' hi + lo.
 // A lane loads 16 bytes of a row, the pieces 2 qd and 2 qd + 1 of 8 columns of a double step of 64; the MFMA's K
 // order is free, so the fragments of x are read in the order that fits (256 contiguous bytes per lane group).
 //   What bounds it, from counting: reads of x from L2 (each of 792 row blocks reads all of it: 1.5 GB at 256 tokens;
@@ -567,7 +571,7 @@ __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8parts_kernel(
     const uint8_t *__restrict__ xf, const float *__restrict__ tscale, int64_t m_total, int row_blocks, int slabs,
     float *__restrict__ y, uint64_t *__restrict__ keys) {
   constexpr int TOK = 16 * MT;
-  constexpr int kPart = 3 * 4 * 1024, kQuad = 2 * kPart;  // bytes of the copy per part and per 96 columns
+  constexpr int kPart = 3 * 4 * 1024, kQuad = 3 * kPart;  // bytes of the copy per part and per 96 columns
   __shared__ __align__(16) float red[kI8mmWaves][TOK][kI8mmRedStride];
   __shared__ float rinv[kI8mmRows];
   const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, qd = lane >> 4;
@@ -612,6 +616,12 @@ __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8parts_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[t][r] = f32x4_i8{0.f, 0.f, 0.f, 0.f};
 
+  float tsl = 1.f;  // the scale of token tok0 + lane
+  {
+    const __amdgpu_buffer_rsrc_t trs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(tscale + tok0),
+                                                                         static_cast<short>(0), TOK * 4, kBufferFlags);
+    tsl = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(trs, 4 * lane, 0, 0));
+  }
   uint4 wv[2][4], xv[2][2][MT];  // weights of two double steps, x (part, token tile) of two halves of one
   auto load_w = [&](int step, uint4 (&w)[4]) {
     const int k = 64 * step + 16 * qd;
@@ -674,6 +684,52 @@ __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8parts_kernel(
     }
   }
 
+  const uint64_t wide = __ballot(lane < TOK && tsl == 0.f);
+  if (__builtin_expect(wide != 0ull, 0)) {
+    // tokens stored as three bf16 parts: their sums over this wave's steps in the place of what the fp16 products
+    // made of their bits (other tokens never see those)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      if (((wide >> (16 * t)) & 0xFFFFull) == 0ull) continue;  // (wave-uniform)
+      f32x4_i8 c[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) c[r] = f32x4_i8{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int i = 0; i < sn; ++i) {
+        const int st = s0 + i, k = 64 * st + 16 * qd, s32 = 2 * st + (qd >> 1), quad = s32 / 3;
+        uint4 w[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          w[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                               wrs, k < cols ? (16 * r + j) * cols + k : kBufferOutOfRange, 0, 0));
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          bf16x8_i8 xp[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+            xp[p] = __builtin_bit_cast(bf16x8_i8, __builtin_amdgcn_raw_buffer_load_b128(
+                                                      xrs, quad * kQuad + (s32 - 3 * quad) * 4096 +
+                                                               16 * (j + 16 * ((2 * qd + half) & 3)),
+                                                      p * kPart + t * 1024, 0));
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            bf16x8_i8 hi, lo;
+            int8x8_hilo(half ? w[r].z : w[r].x, half ? w[r].w : w[r].y, s2[r], hi, lo);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) c[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[p], hi, c[r], 0, 0, 0);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) c[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[p], lo, c[r], 0, 0, 0);
+          }
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if ((wide >> (16 * t + 4 * qd + e)) & 1ull) acc[t][r][e] = c[r][e];
+    }
+  }
+
   // C[token 16t + 4qd + e][row 16r + j] of every wave into LDS, summed in wave order, the scales taken back
 #pragma unroll
   for (int t = 0; t < MT; ++t)
@@ -694,7 +750,7 @@ __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8parts_kernel(
     float sum = red[0][tl][rr];
 #pragma unroll
     for (int w = 1; w < kI8mmWaves; ++w) sum += red[w][tl][rr];
-    sum = sum * rinv[rr] * ts;
+    if (ts != 0.f) sum = sum * rinv[rr] * ts;  // (the bf16 parts have no scales)
     const int64_t row = row0 + rr;
     if (tok < m_total && row < rows) {
       y[tok * rows + row] = sum;
@@ -890,7 +946,7 @@ int launch_int8parts(const int8_t *q, const uint16_t *mu16, int64_t rows, int co
     return fail(PLX_EINVAL, "int8_linear: %lld tokens", static_cast<long long>(m));
   const size_t x_bytes = x_parts_bytes(cols, m), xf_bytes = x_bytes - static_cast<size_t>(slabs) * 64 * sizeof(float);
   float *xnorm = reinterpret_cast<float *>(ws + ((x_bytes + 255) & ~static_cast<size_t>(255)));
-  const int st = launch_x_parts(x, norm_w, eps, m, cols, xnorm, ws, s);
+  const int st = launch_x_parts(x, norm_w, eps, m, cols, 1, xnorm, ws, s);
   if (st != PLX_OK) return st;
   auto k = keys ? (mt == 1 ? int8parts_kernel<1, true> : mt == 2 ? int8parts_kernel<2, true> : int8parts_kernel<4, true>)
                 : (mt == 1 ? int8parts_kernel<1, false> : mt == 2 ? int8parts_kernel<2, false> : int8parts_kernel<4, false>);

@@ -167,14 +167,16 @@ int launch_gather(const int32_t *idx, int64_t n, int out_dtype, void *out, hipSt
 int launch_dequant_f16(const uint8_t *packed, const uint16_t *sigma16, int64_t rows, int64_t cols,
                        uint16_t *w16, hipStream_t s);
 // fp32 x (normalised first when norm_w is given) as two scaled fp16 parts per row in MFMA fragment order, followed
-// by the rows' inverse scales (dequant.hip, xsplit_kernel): slab of 64 tokens, 96 columns (zero-padded), part,
-// 32 columns, token tile of 16, lane: 16 bytes.  Only the first x_parts_tiles(m) token tiles of a slab are written.
+// by the rows' inverse scales (dequant.hip, xsplit_kernel): slab of 64 tokens, 96 columns (zero-padded), part (room
+// for three), 32 columns, token tile of 16, lane: 16 bytes.  Only the first x_parts_tiles(m) token tiles of a slab
+// are written.  A row of too wide a range for them is three bf16 parts instead, its inverse scale 0: one with
+// wide_from or more elements that far below its largest, not all of them 0.
 // xnorm: [m, cols] scratch, used when the norm is not fused into the copy.  cols % 4 == 0, x 16-byte aligned.
 constexpr int x_parts_tiles(int64_t m) { return m > 32 ? 4 : m > 16 ? 2 : 1; }
 size_t x_parts_bytes(int64_t cols, int64_t m);
 bool x_parts_fuses_norm(int64_t cols);
-int launch_x_parts(const float *x, const float *norm_w, float norm_eps, int64_t m, int64_t cols, float *xnorm, void *ws,
-                   hipStream_t s);
+int launch_x_parts(const float *x, const float *norm_w, float norm_eps, int64_t m, int64_t cols, int wide_from,
+                   float *xnorm, void *ws, hipStream_t s);
 // workspace may be null: the MFMA kernel that splits x itself
 int launch_int8_linear(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x, int64_t m,
                        const float *norm_w, float eps, float *y, void *workspace, size_t workspace_bytes, hipStream_t s);

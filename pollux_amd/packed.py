@@ -79,8 +79,9 @@ def dequant_linear(
 ) -> torch.Tensor:
     """y = x @ W.T in fp32 without materialising W (pollux.py:491-507).
 
-    weight_rounding="exact": products with the fp16 weights, exact, accumulated
-    in fp32 -- the numerics of F.linear(x.float(), materialize(W).float()).
+    weight_rounding="exact": products with the fp16 weights, accumulated in
+    fp32 -- the numerics of F.linear(x.float(), materialize(W).float()) -- and
+    exact, but for the last bit of fp32 x (2^-23 of each value) above 4 tokens.
     weight_rounding="as_x": the reference's literal F.linear(x, W.to(x.dtype)),
     i.e. with bf16 activations the fp16 weight is rounded to bf16 first (for
     fp32 activations the two are the same).
@@ -413,8 +414,8 @@ def int8_linear(q: torch.Tensor, mu16: torch.Tensor, x: torch.Tensor, *,
                 norm: tuple[torch.Tensor, float] | None = None) -> torch.Tensor:
     """fp32 [..., rows] = n(x) @ W.T with W = q * (mu / 127) in fp16 (never stored) (plx_int8_linear_ws).
 
-    Exact products, fp32 sums: F.linear(x, W.float()) up to summation order
-    (PackedInt8Linear.forward, pollux.py:562-563).  ``norm``: (weight, eps) of
+    fp32 sums of exact products, but for the last bit of x (2^-23 of each value) where it is split once per
+    call: F.linear(x, W.float()) up to summation order (PackedInt8Linear.forward, pollux.py:562-563).  ``norm``: (weight, eps) of
     an RMSNorm applied to x first, or None.  x fp32 with a multiple of 16 up to
     4,096 features.
     """

@@ -96,7 +96,7 @@ def test_gemv_bf16_small_batches(dev, shape, m):
                                      ((7680, 1920), 64), ((1920, 7680), 64), ((37, 1920), 33), ((64, 1176), 40),
                                      ((4608, 1152), 100), ((130, 24), 20), ((5, 73728), 1), ((3, 73728), 20)])
 def test_ragged_shapes_fp32_activations(dev, shape, m):
-    # m > 16 runs the MFMA GEMM with each fp32 activation split into three bf16 parts
+    # m > 4 runs the MFMA GEMM with each fp32 activation as two scaled fp16 parts
     out_f, in_f = shape
     idx, sig, packed, g = _layer(out_f, in_f, 7 * out_f + m)
     x = torch.randn(m, in_f, generator=g) * 3.0

@@ -73,8 +73,7 @@ def test_both_forms_against_float64(rows, cols, m, once, normed):
                               ("no workspace", 6, _direct(q, mu, x, norm))):
         n = per_step * steps + 6 + ((11 + cols // 64) // 2 + 5 if normed else 0)
         err = (y.double().cpu() - ref).abs()
-        # (beside it the split's floor, 2^-52 of a row's largest |x| per term, and the smallest fp32 values)
-        bound = n * 2.0**-23 * scale + cols * 2.0**-52 * xd.abs().amax(1, keepdim=True) * w.abs().amax(1) + 2.0**-140
+        bound = n * 2.0**-23 * scale + 2.0**-140  # (and the smallest fp32 values)
         print(f"[int8 parts] {rows}x{cols} m={m} norm={normed} {name}: err / bound {(err / bound).max():.2e}", flush=True)
         assert (err <= bound).all(), name
 
