@@ -1903,16 +1903,19 @@ int launch_dqmm(const uint8_t *packed, int64_t pb, const uint16_t *sigma16, int6
 // dequant-GEMM for large batches of fp32 x: the weights are decoded once per call into a fragment-order copy
 // (wfrag_kernel, a chunk of rows at a time) and a dense GEMM runs on the two copies (dgemm_kernel).
 // dqmm_kernel decodes its rows again for every 64 tokens and reads every x fragment for 32 rows: more than the
-// copy costs (2 bytes a weight, written and read: 11 us for 7680x1920) above 320 tokens.  Per call, us,
-// dqmm_kernel / this path: 7680x1920 58 / 59 at 257 tokens, 85 / 65 at 512, 152 / 96 at 1,024; 1920x7680 63 / 63,
-// 96 / 74, 176 / 117; 1920x1920 39 / 33, 59 / 37, 100 / 46; 5760x1920 47 / 48, 67 / 60, 124 / 88.  (bf16 x stays
-// with dqmm_kernel, where it is one part and not scaled: 7680x1920 48 us at 512 tokens, here 59; 5760x1920 at
-// 1,024 70, here 90.)
+// copy costs (2 bytes a weight, written and read: 11 us for 7680x1920) above 320 tokens and kBigWork products.  Per
+// call, us, dqmm_kernel / this path: 7680x1920 58 / 59 at 257 tokens, 85 / 65 at 512, 152 / 96 at 1,024; 1920x7680
+// 63 / 63, 96 / 74, 176 / 117; 1920x1920 39 / 33, 59 / 37, 100 / 46; 5760x1920 47 / 48, 67 / 60, 124 / 88.  (bf16 x
+// stays with dqmm_kernel, where it is one part and not scaled: 7680x1920 48 us at 512 tokens, here 59; 5760x1920 at
+// 1,024 70, here 90.)  Below kBigWork the launches of the copy and of a split sum are what counts: 24x1920 at 330
+// tokens 18 / 22, 960x96 at 1,024 (94 M) 16 / 18, 128x480 at 1,024 (63 M) 21 / 24; above it 128x1920 at 512 (126 M)
+// 28 / 25, 512x480 at 512 (126 M) 25 / 23, 256x1920 at 330 (162 M) 32 / 25, 1920x96 at 1,024 (189 M) 26 / 18.
 // wf[row tile of 16][K step of 32][lane]: lane (j, q) holds columns 8q .. 8q+7 of the step of row j as scaled fp16
 // (zero past the weight), 16 bytes.
 // ---------------------------------------------------------------------------
 constexpr int kBgRows = 128, kBgTok = 128;          // block tile
 constexpr int64_t kBigTokens = 321;
+constexpr int64_t kBigWork = 120'000'000;           // rows x columns x tokens
 constexpr int64_t kBgChunkWeights = 24 << 20;       // weights decoded per launch: a copy of 48 MB
 constexpr int64_t kBgMaxCols = 1 << 16;             // longer rows stay with dqmm_kernel (a chunk of 128 rows)
 
@@ -2233,7 +2236,9 @@ BgPlan bg_plan(int64_t rows, int64_t cols, int64_t m) {
   return p;
 }
 
-bool uses_big(int64_t cols, int64_t m, bool x_f32) { return x_f32 && m >= kBigTokens && cols <= kBgMaxCols; }
+bool uses_big(int64_t rows, int64_t cols, int64_t m, bool x_f32) {
+  return x_f32 && m >= kBigTokens && cols <= kBgMaxCols && rows * cols >= (kBigWork + m - 1) / m;
+}
 
 size_t bg_w_bytes(const BgPlan &p, int64_t cols) {  // the decoded chunk, then its row scales
   return static_cast<size_t>(p.chunk) * (static_cast<size_t>((cols / kDim + 3) / 4) * 96 * 2 + sizeof(float));
@@ -2321,7 +2326,7 @@ size_t mm_workspace_bytes_multi(const int64_t *rows, int n, int64_t cols, int64_
     if (rows[i] <= 0) continue;
     const MmWorkspace w = mm_workspace(rows[i], cols, m, mm_plan(rows[i], cols / kDim), (flags & PLX_DQL_X_F32) != 0);
     size_t rest = w.partial;
-    if (uses_big(cols, m, (flags & PLX_DQL_X_F32) != 0)) {
+    if (uses_big(rows[i], cols, m, (flags & PLX_DQL_X_F32) != 0)) {
       const BgPlan p = bg_plan(rows[i], cols, m);
       rest = bg_w_bytes(p, cols) + bg_partial_bytes(p, rows[i], m);
     }
@@ -2433,7 +2438,7 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
     for (int i = 0; i < n && st == PLX_OK; ++i) {
       const DqlTarget &t = targets[i];
       if (t.rows <= 0) continue;
-      if (uses_big(cols, m, x_is_f32 != 0)) {
+      if (uses_big(t.rows, cols, m, x_is_f32 != 0)) {
         st = launch_big(t, cols, m, xf, tscale, tab, planes,
                         wsb + mm_workspace(t.rows, cols, m, MmPlan{}, true).x_bytes(), gelu, s);
         continue;
