@@ -291,8 +291,8 @@ int plx_h24_plane_layout(const uint8_t *packed, int64_t n_packed_bytes, int64_t 
  * most `capacity` of them into ids (which may be NULL).  Needs no device. */
 int64_t plx_plane_table(uint32_t *ids, int64_t capacity);
 
-/* Workspace (device bytes, 16-byte aligned) plx_dequant_linear needs for
- * this shape, batch and flags (0 when none). */
+/* Workspace (device bytes, 16-byte aligned) of plx_dequant_linear for this
+ * shape, batch and flags (0 when none).  Not monotonic in m_rows. */
 size_t plx_dequant_linear_workspace_bytes(int64_t rows, int64_t cols, int64_t m_rows, int flags);
 
 /* y[m, r] = sum_i x[m, i] * W[r, i] for m < m_rows, with W the fp16
@@ -307,9 +307,14 @@ size_t plx_dequant_linear_workspace_bytes(int64_t rows, int64_t cols, int64_t m_
  * two fp16 parts of its row scaled by a power of two, each value to its last
  * fp32 bit (2^-23 of the value); a row with values further below its largest
  * than these can hold (2^-28 of it or less) is three bf16 parts, exactly.
- * They need the workspace sized by
- * plx_dequant_linear_workspace_bytes (a fragment-order copy of x, plus split
- * partial tiles for narrow layers); cols <= 2^22.
+ * They need the workspace sized by plx_dequant_linear_workspace_bytes for
+ * these rows, cols, m_rows and flags: a fragment-order copy of x, the partial
+ * tiles of split sums and, for fp32 x of more than 320 tokens and 120 M
+ * products (cols <= 65,536), a copy of the decoded weights (2 bytes each, at
+ * most 48 MB) that those batches run faster with.  A workspace of the size for
+ * a larger m_rows will do, also where it is smaller than that (the call then
+ * takes the kernels it has room for, with other summation orders); cols <=
+ * 2^22.
  * Replaces PackedH24Linear.forward after materialize (pollux.py:506-507:
  * F.linear(x, weight.to(x.dtype))). */
 int plx_dequant_linear(const uint8_t *packed, int64_t n_packed_bytes, const uint16_t *sigma16,

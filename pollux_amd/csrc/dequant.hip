@@ -28,6 +28,7 @@
 
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "plx_device.h"
@@ -2208,6 +2209,10 @@ __global__ __launch_bounds__(256, 2) void dgemm_kernel(const uint4 *__restrict__
 struct BgPlan {
   int64_t chunk = 0;
   int splits = 1, steps = 0;
+  void unsplit(int64_t cols) {
+    splits = 1;
+    steps = static_cast<int>((3 * ((cols / kDim + 3) / 4) + 1) & ~static_cast<int64_t>(1));
+  }
 };
 
 BgPlan bg_plan(int64_t rows, int64_t cols, int64_t m) {
@@ -2259,10 +2264,9 @@ int launch_reduce(const float *partial, int splits, int64_t rows, int64_t m, flo
   return check_launch("dqmm_reduce_kernel");
 }
 
-// One weight of a large batch; ws: bg_w_bytes, then the split partials.
-int launch_big(const DqlTarget &t, int64_t cols, int64_t m, const uint4 *xf, const float *tscale, const DeviceTables *tab,
-               bool planes, uint8_t *ws, int gelu, hipStream_t s) {
-  const BgPlan p = bg_plan(t.rows, cols, m);
+// One weight of a large batch; ws: bg_w_bytes, then the split partials (p: bg_plan's, or unsplit).
+int launch_big(const DqlTarget &t, int64_t cols, int64_t m, const BgPlan &p, const uint4 *xf, const float *tscale,
+               const DeviceTables *tab, bool planes, uint8_t *ws, int gelu, hipStream_t s) {
   const int64_t apr = cols / kDim;
   const int nq = static_cast<int>((apr + 3) / 4);
   uint4 *wf = reinterpret_cast<uint4 *>(ws);
@@ -2317,31 +2321,37 @@ bool uses_mfma(int flags, int64_t m) { return m > ((flags & PLX_DQL_X_F32) ? 4 :
 
 }  // namespace
 
-// MFMA part (fragment-order x + split partials) of the workspace
-size_t mm_workspace_bytes_multi(const int64_t *rows, int n, int64_t cols, int64_t m, int flags) {
-  if (!uses_mfma(flags, m)) return 0;
-  // one fragment-order copy of x for every target, one partial buffer reused by them in stream order
-  size_t xf = 0, partial = 0;
-  for (int i = 0; i < n; ++i) {
-    if (rows[i] <= 0) continue;
-    const MmWorkspace w = mm_workspace(rows[i], cols, m, mm_plan(rows[i], cols / kDim), (flags & PLX_DQL_X_F32) != 0);
-    size_t rest = w.partial;
-    if (uses_big(rows[i], cols, m, (flags & PLX_DQL_X_F32) != 0)) {
-      const BgPlan p = bg_plan(rows[i], cols, m);
-      rest = bg_w_bytes(p, cols) + bg_partial_bytes(p, rows[i], m);
-    }
-    xf = w.x_bytes();
-    partial = partial > rest ? partial : rest;
-  }
-  return xf + partial;
+// The workspace ahead of the per-target part: the copy of x (with the tokens' scales; whole 256 bytes), then the
+// normalised x (PLX_DQL_RMS_NORM; whole 32 bytes).
+size_t ws_head_bytes(int64_t cols, int64_t m, int flags) {
+  size_t n = uses_mfma(flags, m) ? mm_workspace(1, cols, m, MmPlan{}, (flags & PLX_DQL_X_F32) != 0).x_bytes() : 0;
+  if (flags & PLX_DQL_RMS_NORM) n += static_cast<size_t>(m * cols) * 4;
+  return n;
 }
 
-// Layout: [MFMA part | normalised x (PLX_DQL_RMS_NORM), 256-byte aligned]
+// The per-target part, reused by the targets in stream order: the least that a call runs with (split partials of
+// dqmm_kernel), or what its kernels of choice take (`full`: large batches with the decoded weights too).
+size_t ws_target_bytes(const int64_t *rows, int n, int64_t cols, int64_t m, int flags, bool full) {
+  if (!uses_mfma(flags, m)) return 0;
+  const bool x_f32 = (flags & PLX_DQL_X_F32) != 0;
+  size_t most = 0;
+  for (int i = 0; i < n; ++i) {
+    if (rows[i] <= 0) continue;
+    most = std::max(most, mm_workspace(rows[i], cols, m, mm_plan(rows[i], cols / kDim), x_f32).partial);
+    if (full && uses_big(rows[i], cols, m, x_f32)) {
+      const BgPlan p = bg_plan(rows[i], cols, m);
+      most = std::max(most, bg_w_bytes(p, cols) + bg_partial_bytes(p, rows[i], m));
+    }
+  }
+  return most;
+}
+
 size_t dequant_linear_workspace_bytes_multi(const int64_t *rows, int n, int64_t cols, int64_t m, int flags) {
   if (cols <= 0 || n <= 0 || m <= 0) return 0;
-  size_t total = mm_workspace_bytes_multi(rows, n, cols, m, flags);
-  if (flags & PLX_DQL_RMS_NORM) total = ((total + 255) & ~static_cast<size_t>(255)) + static_cast<size_t>(m * cols) * 4;
-  return total;
+  bool any = false;
+  for (int i = 0; i < n; ++i) any |= rows[i] > 0;
+  if (!any) return (flags & PLX_DQL_RMS_NORM) ? static_cast<size_t>(m * cols) * 4 : 0;
+  return ws_head_bytes(cols, m, flags) + ws_target_bytes(rows, n, cols, m, flags, true);
 }
 
 size_t dequant_linear_workspace_bytes(int64_t rows, int64_t cols, int64_t m, int flags) {
@@ -2399,7 +2409,8 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
     return fail(PLX_EINVAL, "dequant_linear: the RMS norm takes fp32 x and a 16-byte aligned weight");
   int64_t rows_list[16];
   for (int i = 0; i < n; ++i) rows_list[i] = targets[i].rows;
-  const size_t need = dequant_linear_workspace_bytes_multi(rows_list, n, cols, m, flags);
+  // (a buffer sized for another batch may hold less than this one's kernels of choice take)
+  const size_t head = ws_head_bytes(cols, m, flags), need = head + ws_target_bytes(rows_list, n, cols, m, flags, false);
   if (workspace_bytes < need || (need && workspace == nullptr))
     return fail(PLX_EINVAL, "dequant_linear: workspace of %zu bytes is smaller than the %zu needed", workspace_bytes, need);
   if (need && (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0)
@@ -2410,10 +2421,8 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
   const int64_t apr = cols / kDim;
   const bool planes = (flags & PLX_DQL_PLANES) != 0;  // `packed` holds plane-layout records
   const int pl_vecs = static_cast<int>((plane_tables_host()->ids.size() + 3) / 4);
-  float *xnorm = norm ? reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) +
-                                                  ((mm_workspace_bytes_multi(rows_list, n, cols, m, flags) + 255) &
-                                                   ~static_cast<size_t>(255)))
-                      : nullptr;
+  const size_t x_bytes = ws_head_bytes(cols, m, flags & ~PLX_DQL_RMS_NORM);
+  float *xnorm = norm ? reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + x_bytes) : nullptr;
   if (uses_mfma(flags, m)) {
     // batches above 4 tokens: MFMA dequant-GEMM in slabs of 64 tokens, one launch (+ split sum) per target
     if (cols > kMmMaxCols)
@@ -2439,12 +2448,15 @@ int launch_dequant_linear_multi(const DqlTarget *targets, int n, int64_t cols, c
       const DqlTarget &t = targets[i];
       if (t.rows <= 0) continue;
       if (uses_big(t.rows, cols, m, x_is_f32 != 0)) {
-        st = launch_big(t, cols, m, xf, tscale, tab, planes,
-                        wsb + mm_workspace(t.rows, cols, m, MmPlan{}, true).x_bytes(), gelu, s);
-        continue;
+        BgPlan p = bg_plan(t.rows, cols, m);
+        if (workspace_bytes - head < bg_w_bytes(p, cols) + bg_partial_bytes(p, t.rows, m)) p.unsplit(cols);
+        if (workspace_bytes - head >= bg_w_bytes(p, cols)) {
+          st = launch_big(t, cols, m, p, xf, tscale, tab, planes, wsb + head, gelu, s);
+          continue;
+        }
       }
       const MmPlan pl = mm_plan(t.rows, apr);
-      float *part = reinterpret_cast<float *>(wsb + mm_workspace(t.rows, cols, m, pl, x_is_f32 != 0).x_bytes());
+      float *part = reinterpret_cast<float *>(wsb + head);
       const int64_t pb = ((t.rows * apr + 3) / 4) * 9;  // packed stream length
       st = m > 32 ? launch_dqmm<4>(t.packed, planes ? 6 * t.rows * apr : pb, t.sigma16, t.rows, apr, xf, tscale, m, t.y,
                                    part, pl, tab->kp_dq, planes ? tab->pl_ids : nullptr, pl_vecs, !round_w, x_is_f32,

@@ -6,10 +6,11 @@ A call that does sums in another order than one of up to 320 tokens, so its bits
 import pytest
 import torch
 
-from pollux_amd import castor
+from pollux_amd import _lib, castor
 from pollux_amd.packed import dequant_linear, dequantize_h24
 
 pytestmark = pytest.mark.gpu
+X_F32 = 1
 
 
 def _weight(dev, rows, cols, seed):
@@ -37,3 +38,33 @@ def test_both_sides_of_the_rule(dev, rows, cols, m, big):
     y = dequant_linear(pk, sg, rows, cols, x)
     assert torch.equal(y, _in_small_batches(pk, sg, rows, cols, x)) != big
     assert ((y.double() - x.double() @ w.T).abs() <= _bar(x.double(), w, cols)).all()
+
+
+def _call(pk, sg, rows, cols, x, ws, nbytes):
+    y = torch.empty(x.shape[0], rows, device=x.device)
+    st = _lib.lib().plx_dequant_linear(_lib.ptr(pk), pk.numel(), _lib.ptr(sg), rows, cols, _lib.ptr(x), X_F32, x.shape[0],
+                                       _lib.ptr(y), _lib.ptr(ws), nbytes, _lib.stream_of(x.device))
+    return st, y
+
+
+# a buffer sized once for the largest batch of a program serves the smaller ones; room for nothing but the sums that
+# the kernel of small batches splits is enough, less is refused
+@pytest.mark.parametrize("rows,cols,top", [(1920, 1920, 4000), (700, 7680, 2048), (7680, 480, 1500)])
+def test_smaller_workspaces(dev, rows, cols, top):
+    pk, sg = _weight(dev, rows, cols, 1)
+    w = dequantize_h24(pk, sg, rows, cols).double()
+    size = _lib.lib().plx_dequant_linear_workspace_bytes
+    full = size(rows, cols, top, X_F32)
+    ws = torch.empty(full, dtype=torch.uint8, device=dev)
+    for m in (5, 64, 320, 321, 500, 1000):
+        x = torch.randn(m, cols, generator=torch.Generator(device=dev).manual_seed(m), device=dev)
+        ref = x.double() @ w.T
+        head = (m + 63) // 64 * ((cols + 95) // 96 * 3 * 12288 + 256)
+        slab = size(rows, cols, 64, X_F32) - ((cols + 95) // 96 * 3 * 12288 + 256)  # the partials of a slab
+        least = head + (m + 63) // 64 * slab
+        copy = (rows + 127) // 128 * 128 * ((cols + 95) // 96 * 192 + 4)  # (one chunk)
+        for n in (full, size(rows, cols, m, X_F32), max(least, head + copy), least):
+            st, y = _call(pk, sg, rows, cols, x, ws, min(n, full))
+            _lib.check(st, "plx_dequant_linear")
+            assert ((y.double() - ref).abs() <= _bar(x.double(), w, cols)).all(), (m, n)
+        assert _call(pk, sg, rows, cols, x, ws, least - 1)[0] != 0
