@@ -440,7 +440,10 @@ int plx_int8_linear_ws(const int8_t *q, const uint16_t *mu16, int64_t rows, int6
  * advance of a greedy decode step.  Each block of the GEMV keeps its best
  * (value, index) per token in the workspace (the size below, 8-byte
  * aligned; nothing needs clearing) and one more block picks the winner: two
- * launches instead of the GEMV, an argmax and the bookkeeping. */
+ * launches instead of the GEMV, an argmax and the bookkeeping.  From 5 tokens
+ * the size also has room for the split x of any row length; a workspace for
+ * the keys alone (8 * m_rows * ceil(rows / 64) bytes) is taken too, every
+ * block then splitting x itself. */
 size_t plx_int8_linear_argmax_workspace_bytes(int64_t rows, int64_t m_rows);
 int plx_int8_linear_argmax(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x,
                            int64_t m_rows, const float *norm_weight, float norm_eps, float *y, int64_t *ids,

@@ -926,6 +926,7 @@ int launch_int8mm(const int8_t *q, const uint16_t *mu16, int64_t rows, int cols,
 // sized without it, takes the longest.)
 bool splits_once(int64_t rows, int64_t cols, int64_t m) {
   const int64_t blocks = int8mm_row_blocks(rows) * ((m + 63) / 64);
+  if (blocks >= int64_t{1} << 23) return false;  // (a grid of one dimension holds 2^24 of its blocks)
   const int64_t least = m > 32 ? 600 : m > 16 ? 1200 : 2000;
   return cols * std::max<int64_t>(240, blocks) >= 240 * least;
 }
@@ -1049,11 +1050,14 @@ int launch_int8_linear_argmax(const int8_t *q, const uint16_t *mu16, int64_t row
   if (m == 0) return PLX_OK;
   if (rows <= 0 || rows > 0x7FFFFFFFll) return fail(PLX_EINVAL, "int8_linear_argmax: %lld rows", static_cast<long long>(rows));
   const int64_t parts = int8_linear_parts(rows, m);
-  const size_t keys_bytes = int8_keys_bytes(rows, m), need = keys_bytes + int8_linear_workspace_bytes(rows, cols, m);
+  const size_t need = static_cast<size_t>(m) * static_cast<size_t>(parts) * sizeof(uint64_t);
   if (workspace == nullptr || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 7u) != 0)
     return fail(PLX_EINVAL, "int8_linear_argmax: workspace of %zu bytes (8-byte aligned) needed", need);
   uint64_t *keys = static_cast<uint64_t *>(workspace);
-  uint8_t *ws = align16(static_cast<uint8_t *>(workspace) + static_cast<size_t>(m) * static_cast<size_t>(parts) * 8);
+  // (with room for the keys alone every block splits x itself)
+  uint8_t *ws = workspace_bytes >= int8_keys_bytes(rows, m) + int8_linear_workspace_bytes(rows, cols, m)
+                    ? align16(static_cast<uint8_t *>(workspace) + need)
+                    : nullptr;
   const int st = int8_linear(q, mu16, rows, cols, x, m, norm_w, eps, y, keys, ws, s);
   if (st != PLX_OK) return st;
   int rsh = 0;

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from pollux_amd import _lib, castor
-from pollux_amd.packed import dequant_linear, dequantize_h24
+from pollux_amd.packed import dequant_linear, dequantize_h24, int8_linear
 
 pytestmark = pytest.mark.gpu
 X_F32 = 1
@@ -68,3 +68,25 @@ def test_smaller_workspaces(dev, rows, cols, top):
             _lib.check(st, "plx_dequant_linear")
             assert ((y.double() - ref).abs() <= _bar(x.double(), w, cols)).all(), (m, n)
         assert _call(pk, sg, rows, cols, x, ws, least - 1)[0] != 0
+
+
+@pytest.mark.parametrize("rows,cols,m", [(50_688, 1920, 16), (130, 4096, 70)])
+def test_argmax_with_room_for_the_keys_alone(dev, rows, cols, m):
+    g = torch.Generator(device=dev).manual_seed(m)
+    q = torch.randint(-127, 128, (rows, cols), generator=g, device=dev, dtype=torch.int8)
+    mu = (torch.rand(rows, generator=g, device=dev) * 0.1 + 0.01).half()
+    x = torch.randn(m, cols, generator=g, device=dev)
+    keys = 8 * m * ((rows + 63) // 64)
+    ws = torch.empty(keys, dtype=torch.uint8, device=dev)
+    y, ids = torch.empty(m, rows, device=dev), torch.empty(m, dtype=torch.long, device=dev)
+
+    def call(n):
+        return _lib.lib().plx_int8_linear_argmax(_lib.ptr(q), _lib.ptr(mu), rows, cols, _lib.ptr(x), m, None, 0.0,
+                                                 _lib.ptr(y), _lib.ptr(ids), None, 0, None, _lib.ptr(ws), n,
+                                                 _lib.stream_of(dev))
+
+    assert call(keys - 1) != 0
+    _lib.check(call(keys), "plx_int8_linear_argmax")
+    assert torch.equal(ids, torch.argmax(y, -1))
+    ref = int8_linear(q, mu, x)
+    assert (y - ref).norm() <= 1e-6 * ref.norm()
