@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from pollux_amd import _lib, castor
-from pollux_amd.packed import dequant_linear, dequantize_h24, int8_linear
+from pollux_amd.packed import dequant_linear, dequant_linear_multi, dequantize_h24, int8_linear
 
 pytestmark = pytest.mark.gpu
 X_F32 = 1
@@ -90,3 +90,43 @@ def test_argmax_with_room_for_the_keys_alone(dev, rows, cols, m):
     assert torch.equal(ids, torch.argmax(y, -1))
     ref = int8_linear(q, mu, x)
     assert (y - ref).norm() <= 1e-6 * ref.norm()
+
+
+def _splits(rows, cols, m):
+    """The plan's chunks of rows and K splits (bg_plan)."""
+    nq, blocks = (cols + 95) // 96, (rows + 127) // 128
+    fit = max(1, (24 << 20) // (nq * 96) // 128)
+    chunks = (blocks + fit - 1) // fit
+    per, steps, best = (blocks + chunks - 1) // chunks, 3 * nq, None
+    for sp in range(1, max(1, min(16, steps // 8)) + 1):
+        each = (steps + sp - 1) // sp + 1 & ~1
+        cost = (per * ((m + 127) // 128) * sp + 511) // 512 * each + (
+            3.0 + (2 * sp + 1) * (m * rows) * 1e-6 / chunks if sp > 1 else 0.0)
+        if best is None or cost < best[0]:
+            best = cost, (steps + each - 1) // each
+    return chunks, best[1]
+
+
+# several chunks of decoded rows (the last with a partial block), with and without K splits; residuals added by the
+# GEMM itself (no K split: vector stores, and scalar ones for rows no multiple of 4) and by the split sum; GELU
+@pytest.mark.parametrize("rows,cols,m,chunks,split", [
+    (16_500, 1920, 330, 2, True), (16_500, 1920, 1100, 2, False), (33_333, 960, 400, 2, False), (640, 480, 400, 1, False),
+    (641, 480, 400, 1, False), (1283, 336, 321, 1, False), (1283, 1920, 321, 1, True), (960, 960, 330, 1, True)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_chunks_and_epilogues(dev, rows, cols, m, chunks, split, gelu):
+    n, splits = _splits(rows, cols, m)
+    assert n == chunks and (splits > 1) == split
+    pk, sg = _weight(dev, rows, cols, rows)
+    g = torch.Generator(device=dev).manual_seed(m)
+    x, res = torch.randn(m, cols, generator=g, device=dev), torch.randn(m, rows, generator=g, device=dev)
+    w = dequantize_h24(pk, sg, rows, cols).double()
+    z = x.double() @ w.T
+    bar = _bar(x.double(), w, cols)
+    del w
+    for r in (None, res):
+        y, = dequant_linear_multi([(pk, sg, rows)], cols, x, residuals=[r], gelu=gelu)
+        ref = torch.nn.functional.gelu(z) if gelu else z
+        ref = ref if r is None else ref + r.double()
+        # (GELU's slope is below 1.13; its own fp32 steps and the residual's sum: 2^-22 of their size)
+        tol = 1.13 * bar + 2.0 ** -22 * (z.abs() + res.double().abs())
+        assert ((y.double() - ref).abs() <= tol).all()
