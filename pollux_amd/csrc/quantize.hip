@@ -1001,6 +1001,8 @@ constexpr int kT2StageVecs = kT2StageBytes / 16;   // 384
 constexpr int kT2Cap = 384;                        // candidate entries per wave (4 bytes each)
 constexpr int kT2Surv = 256;                       // survivor entries per wave (4 bytes each)
 constexpr uint32_t kNonFinite = 0xFFFFFFFFu;       // pair key of an atom with a NaN or infinite coordinate
+constexpr float kMaxSum = 0x1p120f;                // NN-P: sum |x| up to which no value of the scorers
+                                                   // overflows (the largest: a raised coordinate, 10 max |x|)
 constexpr uint32_t kRowMask = (1u << kRowBits) - 1u;
 constexpr float kC1 = 1.4140625f;                  // bf16(4s)
 constexpr float kC2 = 0.70703125f;                 // bf16(2s)
@@ -1170,9 +1172,9 @@ __global__ __launch_bounds__(kThreads, MODE == kModeP ? 3 : 4) void t12_kernel(u
   float mg[AT], v1[AT];
   uint32_t m1b[AT];  // the best type-1 key (0: below the origin's bound)
   float s1v[P ? AT : 1];    // NN-P: its score
-  uint32_t nonfinite = 0u;  // bit at: the atom has a NaN or infinite coordinate, or sum |x| overflows fp32
-                            // (NN-P: or sum |x| >= 2^96; pick_kernel scans every code for such an atom)
-  uint32_t snap = 0u;       // NN-P, bit at: |x| < 1e-8, the origin whatever the scores
+  uint32_t nonfinite = 0u;  // bit at: the atom has a NaN or infinite coordinate, or sum |x| overflows fp32 (NN-P:
+                            // is above kMaxSum; pick_kernel scans every code for such an atom)
+  uint32_t snap = 0u;       // bit at: the origin whatever the scores (NN-P: |x| < 1e-8 or a NaN coordinate)
   typedef typename std::conditional<P, const float *, const uint32_t *>::type atom_t;
   auto atom_of = [&](int al) { return reinterpret_cast<atom_t>(xw[wave][al]); };
 #pragma unroll
@@ -1229,9 +1231,11 @@ __global__ __launch_bounds__(kThreads, MODE == kModeP ? 3 : 4) void t12_kernel(u
         snap |= (sqrt(n2) < static_cast<double>(__uint_as_float(kEpsBits)) ? 1u : 0u) << at;
       }
     }
-    // sum |x| is NaN or infinite exactly when a coordinate is (or the sum overflows fp32): such an atom
-    // goes to the origin
-    nonfinite |= (ax <= (P ? 0x1p96f : 3.402823466e38f) ? 0u : 1u) << at;
+    // sum |x| is NaN or infinite exactly when a coordinate is (or the sum overflows fp32): under NN-B / NN-T such
+    // an atom goes to the origin
+    const bool out = !(ax <= (P ? kMaxSum : 3.402823466e38f));
+    nonfinite |= (out ? 1u : 0u) << at;
+    if constexpr (P) snap |= (ax != ax ? 1u : 0u) << at;  // NaN times any coordinate of a code is NaN
     const float s1 = t1 * kC1 + t2 * kC1;  // (NN-B / NN-T: exact products, one rounding)
     m1b[at] = sel::key_or_0(s1);
     if constexpr (P) {
@@ -1241,6 +1245,7 @@ __global__ __launch_bounds__(kThreads, MODE == kModeP ? 3 : 4) void t12_kernel(u
     v1[at] = t1;
     // the margin for the MFMA's fp32 summation order of U (NN-P: and for the rounding of its operand)
     mg[at] = ax * kC2 * 0x1p-14f + (P ? loss * kC2 : 0.f);
+    if (P && out) mg[at] = __builtin_nanf("");  // (no candidates)
   }
   for (int i = lane; i < NA; i += 64) st_r[wave][i] = 0xFFFFFFFFu;
   if constexpr (P)
@@ -1625,8 +1630,8 @@ __global__ __launch_bounds__(kThreads, MODE == kModeP ? 3 : 4) void t12_kernel(u
       // (a non-finite atom: the marker kNonFinite, which pick_kernel maps to the origin as the dense sweep
       // does; as a pair key it gives t3_kernel a NaN threshold, hence no candidates.  An atom whose
       // type-3 floor is above its best pair key: the floor without a row, as t3_kernel's starting best,
-      // which its type-3 best reaches, so pick_kernel takes t3_kernel's row.  NN-P: the marker's second word
-      // is 0 for the origin, 1 for an atom that pick_kernel scans)
+      // which its type-3 best reaches, so pick_kernel takes t3_kernel's row.  NN-P: the marker's second
+      // word is 0 for the origin, 1 for an atom that pick_kernel scans)
       reinterpret_cast<uint2 *>(&keys[a])[1] =
           ((nonfinite | snap) >> at) & 1u ? make_uint2(kNonFinite, P && ((snap >> at) & 1u) == 0u ? 1u : 0u)
           : !pair_can_win(M, F)           ? make_uint2(sel::store(F), 0xFFFFFFFFu)
@@ -2057,13 +2062,14 @@ __device__ __forceinline__ double row_score(const float *__restrict__ x, const i
 // neither reaches its bound or the atom has a NaN or infinite coordinate; then
 // the int32 index and, optionally, the packed 9-byte groups.
 // NN-P (x: the atoms): two keys closer than their fp32 sums can be trusted are
-// compared by the rows' fp64 scores, and the block scans all codes in fp64 for
-// an atom that the scorers left out (an infinite or NaN coordinate, or one so
-// large that an fp32 score could overflow): the lowest row of the highest
-// score that is a number, else the origin.
+// compared by the rows' fp64 scores.  NN-P: the block scans all codes in
+// fp64 for an atom that the scorers left out (one so large that their fp32
+// values could overflow, or an infinite coordinate): the lowest row of the
+// highest score that is a number, else the origin.  About 50 us an atom (one infinity: 1).
 template <int MODE>
 __global__ __launch_bounds__(256) void pick_kernel(const uint4 *__restrict__ keys, int64_t n_atoms,
-                                                   const float *__restrict__ x, const int8_t *__restrict__ cb_raw,
+                                                   const float *__restrict__ x,
+                                                   const int8_t *__restrict__ cb_raw,
                                                    int32_t *__restrict__ idx_out, uint8_t *__restrict__ packed_out) {
   typedef Sel<MODE> sel;
   constexpr bool P = MODE == kModeP;
@@ -2102,15 +2108,20 @@ __global__ __launch_bounds__(256) void pick_kernel(const uint4 *__restrict__ key
       __syncthreads();
       for (int al = 0; al < 256; ++al) {
         if (ids[al] == 0) continue;  // (block-uniform)
-        const float *xa = x + (a0 + al) * kDim;
         double bd = -__builtin_inf();
         uint32_t br = 0u;
-        for (uint32_t r = 1u + static_cast<uint32_t>(tid); r <= static_cast<uint32_t>(kKissing); r += 256u) {
-          const double d = row_score(xa, cb_raw, r);
-          if (d > bd) {
-            bd = d;
-            br = r;
+        bool ends = false;  // a score may be infinite: the first rows that have one end the scan
+        for (int i = 0; i < kDim; ++i) ends |= isinf(x[(a0 + al) * kDim + i]);
+        for (uint32_t r0 = 1u; r0 <= static_cast<uint32_t>(kKissing); r0 += 256u) {
+          const uint32_t r = r0 + static_cast<uint32_t>(tid);
+          if (r <= static_cast<uint32_t>(kKissing)) {
+            const double d = row_score(x + (a0 + al) * kDim, cb_raw, r);
+            if (d > bd) {
+              bd = d;
+              br = r;
+            }
           }
+          if (ends && __syncthreads_or(isinf(bd) && bd > 0.0)) break;  // (`ends`: block-uniform)
         }
         best_d[tid] = bd;
         best_r[tid] = br;
@@ -2274,8 +2285,8 @@ int resolve_launch(const uint4 *keys, int64_t n_atoms, const uint4 *xb, const De
 }
 
 template <int MODE>
-int pick_launch(const uint4 *keys, int64_t n_atoms, const float *x, const DeviceTables *tab, int32_t *idx_out,
-                uint8_t *packed_out, hipStream_t s) {
+int pick_launch(const uint4 *keys, int64_t n_atoms, const float *x, const DeviceTables *tab,
+                int32_t *idx_out, uint8_t *packed_out, hipStream_t s) {
   hipLaunchKernelGGL(pick_kernel<MODE>, dim3(static_cast<unsigned>((n_atoms + 255) / 256)), dim3(256), 0, s, keys,
                      n_atoms, x, tab->cb_raw, idx_out, packed_out);
   return check_launch("pick_kernel");
