@@ -1001,7 +1001,7 @@ constexpr int kT2StageVecs = kT2StageBytes / 16;   // 384
 constexpr int kT2Cap = 384;                        // candidate entries per wave (4 bytes each)
 constexpr int kT2Surv = 256;                       // survivor entries per wave (4 bytes each)
 constexpr uint32_t kNonFinite = 0xFFFFFFFFu;       // pair key of an atom with a NaN or infinite coordinate
-constexpr float kMaxSum = 0x1p120f;                // NN-P: sum |x| up to which no value of the scorers
+constexpr float kMaxSum = 0x1p120f;                // NN-T / NN-P: sum |x| up to which no value of the scorers
                                                    // overflows (the largest: a raised coordinate, 10 max |x|)
 constexpr uint32_t kRowMask = (1u << kRowBits) - 1u;
 constexpr float kC1 = 1.4140625f;                  // bf16(4s)
@@ -1172,9 +1172,10 @@ __global__ __launch_bounds__(kThreads, MODE == kModeP ? 3 : 4) void t12_kernel(u
   float mg[AT], v1[AT];
   uint32_t m1b[AT];  // the best type-1 key (0: below the origin's bound)
   float s1v[P ? AT : 1];    // NN-P: its score
-  uint32_t nonfinite = 0u;  // bit at: the atom has a NaN or infinite coordinate, or sum |x| overflows fp32 (NN-P:
-                            // is above kMaxSum; pick_kernel scans every code for such an atom)
-  uint32_t snap = 0u;       // bit at: the origin whatever the scores (NN-P: |x| < 1e-8 or a NaN coordinate)
+  uint32_t nonfinite = 0u;  // bit at: the atom has a NaN or infinite coordinate, or sum |x| overflows fp32 (NN-T /
+                            // NN-P: is above kMaxSum; pick_kernel scans every code for such an atom)
+  uint32_t snap = 0u;       // bit at: the origin whatever the scores (NN-P: |x| < 1e-8 or a NaN coordinate; NN-T: a
+                            // NaN or infinite one)
   typedef typename std::conditional<P, const float *, const uint32_t *>::type atom_t;
   auto atom_of = [&](int al) { return reinterpret_cast<atom_t>(xw[wave][al]); };
 #pragma unroll
@@ -1231,11 +1232,24 @@ __global__ __launch_bounds__(kThreads, MODE == kModeP ? 3 : 4) void t12_kernel(u
         snap |= (sqrt(n2) < static_cast<double>(__uint_as_float(kEpsBits)) ? 1u : 0u) << at;
       }
     }
-    // sum |x| is NaN or infinite exactly when a coordinate is (or the sum overflows fp32): under NN-B / NN-T such
-    // an atom goes to the origin
-    const bool out = !(ax <= (P ? kMaxSum : 3.402823466e38f));
+    // sum |x| is NaN or infinite exactly when a coordinate is (or the sum overflows fp32): under NN-B such an
+    // atom goes to the origin
+    const bool out = !(ax <= (MODE == kModeB ? 3.402823466e38f : kMaxSum));
     nonfinite |= (out ? 1u : 0u) << at;
-    if constexpr (P) snap |= (ax != ax ? 1u : 0u) << at;  // NaN times any coordinate of a code is NaN
+    if constexpr (MODE != kModeB) {
+      if (__ballot(out) != 0ull) {
+        bool bad = ax != ax;  // NN-P: NaN times any coordinate of a code is NaN
+        if constexpr (!P) {
+          for (int e = 0; e < 4; ++e)
+            bad |= (ww[e] & 0x7F80u) == 0x7F80u || (ww[e] & 0x7F800000u) == 0x7F800000u;
+          uint32_t any = bad ? 1u : 0u;
+          any |= __shfl_xor(any, 16, 64);
+          any |= __shfl_xor(any, 32, 64);
+          bad = any != 0u;
+        }
+        snap |= (out && bad ? 1u : 0u) << at;
+      }
+    }
     const float s1 = t1 * kC1 + t2 * kC1;  // (NN-B / NN-T: exact products, one rounding)
     m1b[at] = sel::key_or_0(s1);
     if constexpr (P) {
@@ -1245,7 +1259,7 @@ __global__ __launch_bounds__(kThreads, MODE == kModeP ? 3 : 4) void t12_kernel(u
     v1[at] = t1;
     // the margin for the MFMA's fp32 summation order of U (NN-P: and for the rounding of its operand)
     mg[at] = ax * kC2 * 0x1p-14f + (P ? loss * kC2 : 0.f);
-    if (P && out) mg[at] = __builtin_nanf("");  // (no candidates)
+    if (MODE != kModeB && out) mg[at] = __builtin_nanf("");  // (no candidates)
   }
   for (int i = lane; i < NA; i += 64) st_r[wave][i] = 0xFFFFFFFFu;
   if constexpr (P)
@@ -1630,10 +1644,10 @@ __global__ __launch_bounds__(kThreads, MODE == kModeP ? 3 : 4) void t12_kernel(u
       // (a non-finite atom: the marker kNonFinite, which pick_kernel maps to the origin as the dense sweep
       // does; as a pair key it gives t3_kernel a NaN threshold, hence no candidates.  An atom whose
       // type-3 floor is above its best pair key: the floor without a row, as t3_kernel's starting best,
-      // which its type-3 best reaches, so pick_kernel takes t3_kernel's row.  NN-P: the marker's second
+      // which its type-3 best reaches, so pick_kernel takes t3_kernel's row.  NN-T / NN-P: the marker's second
       // word is 0 for the origin, 1 for an atom that pick_kernel scans)
       reinterpret_cast<uint2 *>(&keys[a])[1] =
-          ((nonfinite | snap) >> at) & 1u ? make_uint2(kNonFinite, P && ((snap >> at) & 1u) == 0u ? 1u : 0u)
+          ((nonfinite | snap) >> at) & 1u ? make_uint2(kNonFinite, MODE != kModeB && ((snap >> at) & 1u) == 0u ? 1u : 0u)
           : !pair_can_win(M, F)           ? make_uint2(sel::store(F), 0xFFFFFFFFu)
           : M >= sel::kMin && r != 0xFFFFFFFFu ? make_uint2(sel::store(M), r & kRowMask)
                                                : make_uint2(0u, 0u);
@@ -2057,18 +2071,33 @@ __device__ __forceinline__ double row_score(const float *__restrict__ x, const i
   return exact_score(x, [&](int i) { return static_cast<int>(c[i]); });
 }
 
+// The bf16 codebook row's score of bf16 atom xb (NN-T) in fp64 (exact), rounded to fp32; one that overflows is
+// infinite, as the fp32 sums are.
+__device__ __forceinline__ double row_score16(const uint16_t *__restrict__ xb, const int8_t *__restrict__ cb_raw,
+                                              uint32_t row) {
+  const int8_t *c = cb_raw + static_cast<size_t>(row) * kDim;
+  double d = 0.0;
+#pragma unroll 4
+  for (int i = 0; i < kDim; ++i) {
+    const int k = c[i], m = k < 0 ? -k : k;
+    const float v = m == 0 ? 0.f : m == 1 ? kT3S : m == 2 ? kC2 : m == 3 ? kT3Alpha - kT3S : kC1;
+    d = fma(static_cast<double>(bf16_bits_to_float(xb[i])), static_cast<double>(k < 0 ? -v : v), d);
+  }
+  return static_cast<double>(static_cast<float>(d));
+}
+
 // The structured scorers' answer: the higher of the pair key (t12_kernel) and
 // the type-3 key (t3_kernel), the lower row on equal keys, the origin when
 // neither reaches its bound or the atom has a NaN or infinite coordinate; then
 // the int32 index and, optionally, the packed 9-byte groups.
 // NN-P (x: the atoms): two keys closer than their fp32 sums can be trusted are
-// compared by the rows' fp64 scores.  NN-P: the block scans all codes in
+// compared by the rows' fp64 scores.  NN-T / NN-P: the block scans all codes in
 // fp64 for an atom that the scorers left out (one so large that their fp32
-// values could overflow, or an infinite coordinate): the lowest row of the
+// values could overflow; NN-P: an infinite coordinate): the lowest row of the
 // highest score that is a number, else the origin.  About 50 us an atom (one infinity: 1).
 template <int MODE>
 __global__ __launch_bounds__(256) void pick_kernel(const uint4 *__restrict__ keys, int64_t n_atoms,
-                                                   const float *__restrict__ x,
+                                                   const float *__restrict__ x, const uint4 *__restrict__ xb,
                                                    const int8_t *__restrict__ cb_raw,
                                                    int32_t *__restrict__ idx_out, uint8_t *__restrict__ packed_out) {
   typedef Sel<MODE> sel;
@@ -2098,9 +2127,9 @@ __global__ __launch_bounds__(256) void pick_kernel(const uint4 *__restrict__ key
       if (t2) row = min(row, k.w);
     }
     id = row == kNone ? 0 : static_cast<int32_t>(row);
-    if constexpr (P) scan = k.z == kNonFinite && k.w == 1u;
+    if constexpr (MODE != kModeB) scan = k.z == kNonFinite && k.w == 1u;
   }
-  if constexpr (P) {
+  if constexpr (MODE != kModeB) {
     if (__syncthreads_or(scan)) {
       __shared__ double best_d[256];
       __shared__ uint32_t best_r[256];
@@ -2110,12 +2139,18 @@ __global__ __launch_bounds__(256) void pick_kernel(const uint4 *__restrict__ key
         if (ids[al] == 0) continue;  // (block-uniform)
         double bd = -__builtin_inf();
         uint32_t br = 0u;
-        bool ends = false;  // a score may be infinite: the first rows that have one end the scan
-        for (int i = 0; i < kDim; ++i) ends |= isinf(x[(a0 + al) * kDim + i]);
+        bool ends = !P;  // a score may be infinite: the first rows that have one end the scan
+        if constexpr (P) {
+          for (int i = 0; i < kDim; ++i) ends |= isinf(x[(a0 + al) * kDim + i]);
+        }
         for (uint32_t r0 = 1u; r0 <= static_cast<uint32_t>(kKissing); r0 += 256u) {
           const uint32_t r = r0 + static_cast<uint32_t>(tid);
           if (r <= static_cast<uint32_t>(kKissing)) {
-            const double d = row_score(x + (a0 + al) * kDim, cb_raw, r);
+            double d;
+            if constexpr (P)
+              d = row_score(x + (a0 + al) * kDim, cb_raw, r);
+            else
+              d = row_score16(reinterpret_cast<const uint16_t *>(xb + (a0 + al) * 3), cb_raw, r);
             if (d > bd) {
               bd = d;
               br = r;
@@ -2285,10 +2320,10 @@ int resolve_launch(const uint4 *keys, int64_t n_atoms, const uint4 *xb, const De
 }
 
 template <int MODE>
-int pick_launch(const uint4 *keys, int64_t n_atoms, const float *x, const DeviceTables *tab,
+int pick_launch(const uint4 *keys, int64_t n_atoms, const float *x, const uint4 *xb, const DeviceTables *tab,
                 int32_t *idx_out, uint8_t *packed_out, hipStream_t s) {
   hipLaunchKernelGGL(pick_kernel<MODE>, dim3(static_cast<unsigned>((n_atoms + 255) / 256)), dim3(256), 0, s, keys,
-                     n_atoms, x, tab->cb_raw, idx_out, packed_out);
+                     n_atoms, x, xb, tab->cb_raw, idx_out, packed_out);
   return check_launch("pick_kernel");
 }
 
@@ -2303,7 +2338,7 @@ int structured_launch(uint4 *xb, const float *src, const float *sigma, int64_t a
   if ((st = t12_launch_load<LOAD, MODE>(xb, src, sigma, apr, n_atoms, tab, keys, rec, s, rows_by_sweep)) != PLX_OK)
     return st;
   if ((st = t3_launch<MODE>(xb, src, n_atoms, tab, keys, rec, s, rows_by_sweep)) != PLX_OK) return st;
-  return pick_launch<MODE>(keys, n_atoms, src, tab, idx_out, packed_out, s);
+  return pick_launch<MODE>(keys, n_atoms, src, xb, tab, idx_out, packed_out, s);
 }
 
 // workspace = per-atom keys, the dense sweep's pair records (the structured scorers: t3_kernel's set-up
@@ -2458,7 +2493,7 @@ int launch_batch_mode(const RequantItem *items, int n_items, const DeviceTables 
     const int64_t apr = it.cols / kDim, n = it.rows * apr;
     if (n == 0) continue;
     if constexpr (!DENSE)
-      st = pick_launch<MODE>(keys + off, n, nullptr, tab, it.idx, it.packed, s);
+      st = pick_launch<MODE>(keys + off, n, nullptr, xb + off * 3, tab, it.idx, it.packed, s);
     else
       st = resolve_launch(keys + off, n, xb + off * 3, tab, recs + off, n_slices - s0, total, it.idx, it.packed, s);
     if (st != PLX_OK) return st;

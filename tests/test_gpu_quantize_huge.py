@@ -1,6 +1,7 @@
-"""NN-P on atoms near fp32's largest values and with NaN, against every code's exact score in float64.
+"""NN-T and NN-P on atoms near fp32's largest values and with NaN, against every code's exact score in float64.
 
-Expected: the lowest row of the highest score.  An atom whose runner-up lies within 24 * 2^-24 * 2 (|x|_2 |c|_2) of the best may differ (the bound on two fp32 sums).
+Expected: the lowest row of the highest score; under NN-T the scores are fp32, so all that overflow tie.  An atom
+whose runner-up lies within 24 * 2^-24 * 2 (|x|_2 |c|_2) of the best may differ (the bound on two fp32 sums).
 """
 
 import pytest
@@ -33,7 +34,7 @@ def _atoms(dev, n, scale):
 
 # sums of |x| up to the scorers' limit (2^120, crossed by atoms of 5e34), past it, past fp32 (1.5e37), where the best
 # scores overflow (1e38)
-@pytest.mark.parametrize("mode", ["pack"])
+@pytest.mark.parametrize("mode", ["fp32", "pack"])
 @pytest.mark.parametrize("scale", [2.0 ** 90, 1e33, 5e34, 7e34, 1e36, 1.5e37, 4e37, 1e38])
 def test_huge_atoms(dev, mode, scale):
     x = _atoms(dev, 500, scale)
@@ -44,7 +45,16 @@ def test_huge_atoms(dev, mode, scale):
     assert near.float().mean() < 0.05 and not bad.any()
 
 
-@pytest.mark.parametrize("mode", ["pack"])
+def test_huge_atoms_in_a_batch(dev):
+    # the batched requantize under NN-T: a row scaled by its own size has coordinates of a few units
+    g = torch.Generator(device=dev).manual_seed(3)
+    mats = [torch.randn(r, 48, generator=g, device=dev) * s for r, s in ((40, 1.0), (30, 1e18), (50, 1e-3))]
+    one = [castor.requantize_h24(w, mode="fp32") for w in mats]
+    many = castor.requantize_h24_many(mats, mode="fp32")
+    assert all(torch.equal(a["indices"], b["indices"]) for a, b in zip(one, many))
+
+
+@pytest.mark.parametrize("mode", ["fp32", "pack"])
 def test_blocks_of_nan_atoms(dev, mode):
     x = _atoms(dev, 5000, 1.0)
     ref = castor.quantize_indices(x, mode=mode)
@@ -65,7 +75,7 @@ def test_infinite_coordinates_under_pack(dev, n):
     x.scatter_(1, at, sign * float("inf"))
     x[500:, 0] = float("inf")
     want = []
-    c = torch.from_numpy(cb.codebook_int8()[1:]).to(dev).float()
+    c = torch.from_numpy(cb.codebook_int8()[1:].copy()).to(dev).float()
     for a in x.split(50):
         s = torch.where(a.isinf(), a.sign(), torch.zeros_like(a))
         ok = (s @ c.sign().T) == a.isinf().sum(1, keepdim=True)
