@@ -276,7 +276,9 @@ __global__ __launch_bounds__(kAttnThreads, 5) void decode_attention_kernel(
 // keys 4 g + r without any exchange between lanes; its A operand is V^T from LDS (one 16-byte read per lane
 // for 4 steps), in two tiles of dims (0-15; 16-23, then a row of ones that sums the probabilities).
 // Online softmax per query: the maximum over the tile's 64 keys, exchanged between the four lanes of a query
-// once per tile; the accumulators are rescaled only in tiles where some maximum of the wave rose.
+// once per tile; the accumulators are rescaled only in tiles where some maximum of the wave rose.  The maximum is
+// taken off before the scale: a rounded product of it would be common to a tile's keys, and beside scores of 2^31 (norm
+// weights of 1e4 and more) larger than the exponents that 2^x has.
 //   Error: scores in two chains of three MFMAs, a tile's sums from zero and then added: 1.9e-7 from float64 at 1,024
 // positions (one chain through the running sums 3.4e-7; the VALU form 1.9e-7).
 //   A V row that is not finite must not reach the queries before it (0 * inf): the tile that holds both
@@ -434,7 +436,6 @@ __global__ __launch_bounds__(kAttnThreads, 4) void prefill_attention_kernel(
       }
       m = mn;
     }
-    const float mc = m * scale_log2;
     // the tile's sums from zero, added to the running ones on the VALU: one rounding of those per tile
     f32x4 t0 = {0.f, 0.f, 0.f, 0.f}, t1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -442,7 +443,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void prefill_attention_kernel(
       if (kt >= live) continue;  // (wave-uniform)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        sc[kt][r] = __builtin_amdgcn_exp2f(fmaf(sc[kt][r], scale_log2, -mc));  // (a masked key: 2^-inf = 0)
+        sc[kt][r] = __builtin_amdgcn_exp2f((sc[kt][r] - m) * scale_log2);  // (a masked key: 2^-inf = 0)
       if (!own || all_finite) {
         const float4 a = *reinterpret_cast<const float4 *>(&vt[buf][vrow0 + 16 * kt]);
         const float4 b = *reinterpret_cast<const float4 *>(&vt[buf][vrow1 + 16 * kt]);

@@ -72,3 +72,28 @@ def test_a_bad_row_reaches_no_earlier_query(dev, bad, row):
     tol = 64 * 2.0 ** -24 * ref.abs().max().item()
     assert ((out[1, :row] - ref[1, :row]).abs() <= tol).all()
     assert not torch.isfinite(out[1, row:, 3]).any() and torch.isnan(out[1, row:, 24:]).all()
+
+
+@pytest.mark.parametrize("size", [30.0, 1e3, 1e5, 1e9])
+def test_scores_of_any_size(dev, size):
+    # norm weights far from 1 (scores up to 24 size^2): where one key's score leads by more than the fp32 roundings of
+    # the two (24 * 2^-24 of the products' sizes each) and the softmax's own width, the output is its value
+    b, heads, t, p0 = 1, 3, 200, 70
+    q, k, v, kc, vc, q_ln, k_ln = _case(dev, b, heads, t, p0, 300, 8)
+    with torch.no_grad():
+        q_ln.weight.mul_(size)
+        k_ln.weight.mul_(size)
+        kc.mul_(size)
+        out = prefill_attention(q, k, v, q_ln, k_ln, kc.clone(), vc.clone(), p0)
+        qn, kn = _norm(_heads(q, heads), q_ln.weight.double()), _norm(_heads(k, heads), k_ln.weight.double())
+        keys = torch.cat([kc[:, :, :p0].double(), kn], 2)
+        vals = torch.cat([vc[:, :, :p0].double(), _heads(v, heads)], 2)
+        mask = ~torch.ones(t, p0 + t, dtype=torch.bool, device=dev).tril(p0)
+        s = (qn @ keys.transpose(-1, -2).contiguous() / math.sqrt(24)).masked_fill(mask, -math.inf)
+        unsure = 24 * 2.0 ** -24 * (qn.abs() @ keys.abs().transpose(-1, -2).contiguous()).max(-1).values / math.sqrt(24)
+        top = s.topk(2, -1)
+        lead = top.values[..., 0] - top.values[..., 1] > 2 * unsure + 30
+        want = vals.gather(2, top.indices[..., :1].expand(-1, -1, -1, 24))
+    got = _heads(out, heads)
+    assert torch.isfinite(out).all() and lead.float().mean() > 0.3
+    assert ((got - want)[lead].abs() <= 1e-6 * vals.abs().max()).all()
