@@ -422,7 +422,9 @@ int plx_dequant_int8_rows(const int8_t *q, const uint16_t *mu16, int64_t rows, i
  * to pay; null: as plx_int8_linear).  From 5 tokens x
  * is then normalised and split once, as plx_dequant_linear's (two fp16 parts,
  * each value to its last fp32 bit; rows of too wide a range three bf16 parts,
- * exactly), and the products of the parts are exact. */
+ * exactly), and the products of the parts are exact.  Which form runs depends
+ * on rows, cols and m_rows, so a token's sums may differ in their last bits
+ * from one batch size to another. */
 int plx_int8_linear(const int8_t *q, const uint16_t *mu16, int64_t rows, int64_t cols, const float *x,
                     int64_t m_rows, const float *norm_weight, float norm_eps, float *y, void *stream);
 size_t plx_int8_linear_workspace_bytes(int64_t rows, int64_t cols, int64_t m_rows);

@@ -41,6 +41,8 @@ from .packed import (
 )
 from .plx import check_fingerprint, load_plx
 
+_BATCH_TOKENS = 320  # the dequant-linear's large-batch path starts above (kBigTokens, dequant.hip)
+
 # pollux.py:258-278: the config fields and their aliases
 CONFIG_FIELDS = (
     "n_layers", "n_heads", "d_head", "n_embd", "tokenizer_vocab_size", "vocab_size", "batch_size",
@@ -476,8 +478,8 @@ class GraphDecoder:
         """Prefill of ``idx`` [batch, t] from position 0; returns the logits of its last position.
 
         Replayed from a graph captured per padded length (4, then powers of
-        two from 16, at most the cache length; captured on first use): the prompt is
-        padded at its end, which causal attention makes exact -- no real
+        two from 16, at most the cache length, and the last length of 320 tokens
+        in all; captured on first use): the prompt is padded at its end, which causal attention makes exact -- no real
         position sees the padding, the logits come from position t - 1, and
         the padding's cache rows are overwritten by the decode steps before
         they are read.
@@ -487,9 +489,14 @@ class GraphDecoder:
             raise ValueError(f"prefill of {b} sequences for a decoder of batch {self.ids.shape[0]}")
         if not 1 <= t <= self.max_len:
             raise ValueError(f"a prompt of {t} tokens does not fit the cache's {self.max_len} positions")
-        # 4, then 16, 32, 64, ...: the edge at 4 is the dequant-linear's GEMV / GEMM switch, so the real
-        # tokens take the same kernels as without padding
-        T = min(4 if t <= 4 else max(16, 1 << (t - 1).bit_length()), self.max_len)
+        # 4, then 16, 32, 64, ...: the dequant-linear switches kernels above 4 tokens and above 320 (_BATCH_TOKENS) in
+        # all, so the real tokens take the same kernels as without padding, but for batches whose padding crosses
+        # the first edge; above the second, its K splits depend on the count, and results differ from an unpadded
+        # prefill's by their summation order
+        T = 4 if t <= 4 else max(16, 1 << (t - 1).bit_length())
+        if b * t <= _BATCH_TOKENS < b * T:
+            T = _BATCH_TOKENS // b
+        T = min(T, self.max_len)
         entry = self._prefills.get(T)
         if entry is None:
             entry = self._prefills[T] = self._capture_prefill(T)

@@ -244,3 +244,29 @@ def test_graph_prefill_buckets_match_eager(dev, tmp_path):
     assert sorted(dec._prefills) == [4, 16, 32, 64]
     with pytest.raises(ValueError):
         dec.prefill(torch.zeros(1, 65, dtype=torch.long, device=dev))
+
+
+def test_graph_prefill_keeps_the_kernels_of_320_tokens(dev):
+    # 16 prompts of 18 tokens (288 in all) stay on the side of 320 tokens where the unpadded prefill is: the same bits
+    from pollux_amd import castor
+    from pollux_amd.model import GraphDecoder
+
+    cfg = PolluxConfig(n_layers=1, n_heads=20, n_embd=480, vocab_size=96, tokenizer_vocab_size=96, seq_len=64)
+    g = torch.Generator(device=dev).manual_seed(1)
+    with torch.device(dev):
+        model = PackedPolluxModel(cfg).eval()
+    for name, buf in model.named_buffers():
+        if name.endswith("packed_weights"):
+            n = buf.numel() // 9 * 4
+            buf.copy_(castor.pack_indices(torch.randint(0, 196561, (n,), generator=g, device=dev)))
+        elif buf.dtype == torch.int8:
+            buf.copy_(torch.randint(-127, 128, buf.shape, generator=g, device=dev, dtype=torch.int8))
+        elif buf.dtype == torch.float16:
+            buf.copy_((torch.rand(buf.shape, generator=g, device=dev) * 0.045 + 0.005).half())
+    dec = GraphDecoder(model, batch=16)
+    for t in (17, 18, 20):
+        idx = torch.randint(0, 96, (16, t), generator=g, device=dev)
+        with torch.inference_mode():
+            want = model.prefill(idx, model.new_cache(16), last_only=True)[:, -1]
+            assert torch.equal(dec.prefill(idx), want), t
+    assert sorted(dec._prefills) == [20]
