@@ -48,14 +48,14 @@ ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
 METRIC = "atoms/sec Leech NN quantize (+MFMA util %); dequant-GEMV GB/s at d=1920"
-# The dense sweep (NN-T, NN-P, and NN-B with the dense type-3 sweep): every code scored,
+# The dense sweep (NN-B with every code scored, the structured scorers' baseline):
 # 2 * 24 * 196,560 = 9,434,880 flops per atom (origin free, K padding not counted).
 FLOP_PER_ATOM = 2 * 24 * 196_560
 # MFMA flops the dense sweep issues per atom: 9,216 tiles of 16 codes (the 98,304
 # type-3 codes, one representative per antipodal pair of the others, padding)
 # at K = 32 (24 coordinates + 8 zeros) -- 9,437,184.
 MFMA_FLOP_ISSUED_PER_ATOM = 2 * 32 * 9216 * 16
-# NN-B's default path, the structured scorers: t12_kernel scores the 98,256 type-1 / type-2
+# The structured scorers, every rule's path: t12_kernel scores the 98,256 type-1 / type-2
 # codes from the 759 octad sums of |x| (2 * 24 * 759 = 36,432 algorithmic MFMA flops per
 # atom, issued as 48 tiles at K = 32: 49,152) and t3_kernel the 98,304 type-3 codes from
 # the 2,048 representative Golay sign-pattern sums (2 * 24 * 2,048 = 98,304 flops per atom,
@@ -477,16 +477,23 @@ def optim_extras(device, mats, iters=9, sets=3):
 def pack_time_extras(mats, iters=5):
     """Pack-time NN-P quantizer (pack.py:139-180) on the config-2 weights: atoms/s.
 
-    NN-P scores fp32 atoms exactly (three bf16 MFMA parts per tile) and
-    rescans its candidates in fp64, so it does ~3x the MFMA work of NN-B.
+    NN-P runs the structured scorers: their MFMA bounds from the rounded
+    atoms, the candidates from the fp32 ones, those near the best in fp64.
     """
     from pollux_amd import pack
 
-    t = time_gpu(lambda: [pack.quantize_h24_layer(w) for w in mats], iters, 2)
+    def step():
+        for w in mats:
+            pack.quantize_h24_layer(w)
+
+    t = time_gpu(step, iters, 2)
+    _, kms = _scorer_profiled(step, iters)
     n = sum(w.numel() for w in mats) // 24
-    return {"atoms_per_s": n / t, "ms_per_layer": t * 1e3,
-            "mfma_issue_frac_of_bf16_peak": 3 * MFMA_FLOP_ISSUED_PER_ATOM * n / t / PEAK_BF16_FLOPS,
-            "note": "quantize_h24_layer (NN-P + sigma16 + 18-bit pack) on the four config-2 weights"}
+    issued = T12_MFMA_ISSUED_PER_ATOM + T3_MFMA_ISSUED_PER_ATOM
+    return {"atoms_per_s": n / t, "ms_per_layer": t * 1e3, **kms,
+            "mfma_issue_frac_of_bf16_peak": issued * n / t / PEAK_BF16_FLOPS,
+            "note": "quantize_h24_layer (NN-P + sigma16 + 18-bit pack) on the four config-2 weights; kernel times: the "
+                    "average over the four launches"}
 
 
 def json_from_profiles(name):
@@ -546,15 +553,15 @@ def _profiled(fn, iters, kernel=0, warmup=0, rounds=1, warm_s=0.0):
 
 def _scorer_profiled(fn, iters, mode="bf16", warmup=0):
     """(seconds per call, {kernel: ms per launch}) of fn over iters calls, the scoring kernels timed by HIP events:
-    NN-B's structured scorers (t3_kernel, t12_kernel), or nn_kernel (the dense sweep of the other modes)."""
+    the structured scorers (t3_kernel, t12_kernel), or nn_kernel (the dense sweep, "bf16-dense")."""
     from pollux_amd import _lib
 
-    if mode == "bf16":
-        t, t3 = _profiled(fn, iters, _lib.PROF_T3, warmup=warmup)
-        _, t12 = _profiled(fn, iters, _lib.PROF_T12)
-        return t, {"t3_kernel_ms_avg": t3, "t12_kernel_ms_avg": t12}
-    t, nn = _profiled(fn, iters, _lib.PROF_NN, warmup=warmup)
-    return t, {"nn_kernel_ms_avg": nn}
+    if mode == "bf16-dense":
+        t, nn = _profiled(fn, iters, _lib.PROF_NN, warmup=warmup)
+        return t, {"nn_kernel_ms_avg": nn}
+    t, t3 = _profiled(fn, iters, _lib.PROF_T3, warmup=warmup)
+    _, t12 = _profiled(fn, iters, _lib.PROF_T12)
+    return t, {"t3_kernel_ms_avg": t3, "t12_kernel_ms_avg": t12}
 
 
 def sweep_extras(device, mode="bf16", steps=10):
@@ -728,6 +735,13 @@ def decode_extras(device, prompt_len=64, new_tokens=128):
         e1.synchronize()
         return e0.elapsed_time(e1) / 1e3 / n
 
+    def median_call(fn, n=21):
+        """Median seconds of n calls, each timed alone (a pause of the allocator or the collector meets one of them),
+        after three untimed ones (library kernels load their code on first use)."""
+        for _ in range(3):
+            fn()
+        return sorted(timed(lambda _: fn(), 1) for _ in range(n))[n // 2]
+
     out = {}
     with torch.inference_mode():
         dec = GraphDecoder(model, batch=1)
@@ -770,12 +784,10 @@ def decode_extras(device, prompt_len=64, new_tokens=128):
         t_prefill_graph = timed(lambda n: [pdec.prefill(prompt) for _ in range(n)], 8)
         del pdec
         seq = torch.cat([prompt, prompt[:, :1]], dim=1)
-        model(seq)  # untimed: first use of each shape (library kernels load their code on first use)
-        t_recompute = timed(lambda n: [model(seq)[:, -1].argmax(-1) for _ in range(n)], 4)
+        t_recompute = median_call(lambda: model(seq)[:, -1].argmax(-1))
         del cache
         dense = PackedPolluxModel.from_packed_checkpoint(payload, device, materialize=True)
-        dense(seq)  # untimed, as above (hipBLASLt's first call per GEMM shape)
-        t_dense = timed(lambda n: [dense(seq)[:, -1].argmax(-1) for _ in range(n)], 4)
+        t_dense = median_call(lambda: dense(seq)[:, -1].argmax(-1))
         del dense
         # last: the batch-16 decoder's cache (4.5 GB) and graph pools stay with the allocator afterwards
         prompts16 = torch.randint(0, 50257, (16, prompt_len), generator=g, device=device)
@@ -804,7 +816,8 @@ def decode_extras(device, prompt_len=64, new_tokens=128):
                    f"step); prefill: the prompt into the "
                    f"cache with the last position's logits (time to first token), replayed from GraphDecoder's "
                    f"graph for the padded length or run eagerly into a new cache; recompute rows at a "
-                   f"{prompt_len + 1}-token prefix; random packed weights (valid indices), fp32 activations")
+                   f"{prompt_len + 1}-token prefix, the median of 21 calls; random packed weights (valid "
+                   f"indices), fp32 activations")
     return out
 
 
@@ -1030,7 +1043,7 @@ def main() -> int:
     for _ in range(args.warmup):
         idx = step()
     torch.cuda.synchronize()
-    structured = args.mode == "bf16"
+    structured, nn_b = args.mode != "bf16-dense", args.mode == "bf16"
     # the dominant kernel's launches are timed by HIP events on their stream inside the timed region
     _lib.check(lib.plx_profile_select(_lib.PROF_T3 if structured else _lib.PROF_NN), "plx_profile_select")
     _lib.check(lib.plx_profile_begin(), "plx_profile_begin")
@@ -1054,14 +1067,15 @@ def main() -> int:
     fpa = T3_FLOP_PER_ATOM if structured else FLOP_PER_ATOM
     issued = T3_MFMA_ISSUED_PER_ATOM if structured else MFMA_FLOP_ISSUED_PER_ATOM
     achieved = fpa * atoms * args.steps / kernel_s if kernel_s > 0 else 0.0
-    counters = json_from_profiles("quantize_c4_counters.json") if structured else {}
+    counters = json_from_profiles("quantize_c4_counters.json") if nn_b else {}
     roofline = {
         "bound": "mfma",
         "achieved": achieved / 1e12,
         "peak": PEAK_BF16_FLOPS / 1e12,
         "unit": "TFLOP/s",
         "frac": achieved / PEAK_BF16_FLOPS,
-        "traffic": traffic_from_profiles("t3_kernel_c4_traffic.json" if structured else "nn_kernel_c4_dense_traffic.json"),
+        "traffic": None if args.mode == "fp32" else
+        traffic_from_profiles("t3_kernel_c4_traffic.json" if nn_b else "nn_kernel_c4_dense_traffic.json"),
         "kernel": "t3_kernel (structured type-3 scorer: 128 Golay sign-pattern tiles on bf16 16x16x32 MFMA, the "
         "candidate words' 24 positions on the VALU)" if structured else
         "nn_kernel (bf16 16x16x32 MFMA scoring + running max over 9,216 tiles)",
@@ -1071,7 +1085,7 @@ def main() -> int:
         "flop_per_launch": fpa * atoms,
         "mfma_issue_frac": issued * atoms * args.steps / kernel_s / PEAK_BF16_FLOPS if kernel_s > 0 else 0.0,
     }
-    if structured:
+    if nn_b:
         # the type-1/2 scorer, and the dense sweep the two structured scorers replace
         _, t12_ms = _profiled(step, 3, _lib.PROF_T12)
         t_d, nn_d = _profiled(lambda: castor.quantize_indices(x, mode="bf16-dense"), 3, _lib.PROF_NN, warmup=1)
@@ -1129,7 +1143,7 @@ def main() -> int:
         },
         "roofline": roofline,
     }
-    if structured:
+    if nn_b:
         result["dense_sweep_baseline"] = result_dense
     log("[bench] dequant-GEMV / GEMM at config 5")
     gemv = gemv_extras(dev)
