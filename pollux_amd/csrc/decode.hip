@@ -283,9 +283,10 @@ __global__ __launch_bounds__(kAttnThreads, 5) void decode_attention_kernel(
 // positions (one chain through the running sums 3.4e-7; the VALU form 1.9e-7).
 //   A V row that is not finite must not reach the queries before it (0 * inf): the tile that holds both
 // (the block's own) then adds its keys one by one, each to the queries at or after it.
-//   What bounds it: the fp32 matrix rate (56 MFMAs of 32 cycles per 16 queries x 64 keys; 25% of the second
-// dims tile is padding).  1,024 tokens x 80 heads: 889 -> 119 us against a thread row of 16 lanes per query on the
-// VALU in four launches of 256 positions.
+//   What bounds it: the chain within a tile (barrier, LDS, dependent MFMAs, exchanges, exponentials), which four waves
+// per SIMD do not cover.  Counters at 1,024 tokens x 80 heads: matrix cores 24% busy (56 MFMAs of 32 cycles per 16
+// queries x 64 keys; 25% of the second dims tile is padding), VALU issue 18%, bank conflicts 4%.  There 889 -> 119 us
+// against a thread row of 16 lanes per query on the VALU in four launches of 256 positions.
 constexpr int kPfTile = 64;               // queries per block, keys per tile
 constexpr int kPfK = 26;                  // floats between keys in LDS (K)
 constexpr int kPfV = 68;                  // floats between dims in LDS (V^T)

@@ -559,8 +559,9 @@ __global__ __launch_bounds__(64 * kI8mmWaves, 2) void int8mm_kernel(
 // dequant.hip): its sums are taken again, the parts against the weights' hi + lo.
 // A lane loads 16 bytes of a row, the pieces 2 qd and 2 qd + 1 of 8 columns of a double step of 64; the MFMA's K
 // order is free, so the fragments of x are read in the order that fits (256 contiguous bytes per lane group).
-//   What bounds it, from counting: reads of x from L2 (each of 792 row blocks reads all of it: 1.5 GB at 256 tokens;
-// the MFMAs take about 40 us of the 141), at up to 16 tokens the weights' 97 MB.  50,688 x 1,920 with the norm, split
+//   What bounds it: reads from L2 (at 256 tokens each of 792 row blocks reads all of x, 1.56 GB, and the weights come
+// once per 64 tokens, 0.39 GB: 18.1 M requests counted, 13 TB/s; matrix cores 31% busy, VALU issue 32%), at up to 16
+// tokens the weights' 97 MB.  50,688 x 1,920 with the norm, split
 // launch included, against int8mm_kernel: 5-16 tokens 56 -> 31 us, 32 73 -> 39, 64 112 -> 52, 128 194 -> 81, 256
 // 361 -> 141; error against float64 at 256 tokens 3.2e-7 -> 2.1e-7.
 typedef _Float16 f16x8_i8 __attribute__((ext_vector_type(8)));
