@@ -1177,10 +1177,10 @@ __device__ __forceinline__ void store_exact_parts(uint2 *d, float4 v) {
   for (int k = 0; k < 3; ++k) d[k * (kXfQuadBytes / 8)] = make_uint2(p[k][0] | p[k][1] << 16, p[k][2] | p[k][3] << 16);
 }
 
-// fp32 x, one block per token row of each slab's `tiles` token tiles; REG: rows of up to 8,192 columns are read
-// once, into registers.
+// fp32 x, one block per token row of each slab's `tiles` token tiles; VEC: rows of up to 1,024 VEC columns are read
+// once, into registers (0: any length, read twice).
 constexpr int kXsVec = 8;
-template <bool REG>
+template <int VEC>
 __global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x, int64_t m_total, int64_t cols,
                                                      int64_t n_quads_row, int tiles, int wide_from,
                                                      uint2 *__restrict__ xf, float *__restrict__ tscale) {
@@ -1194,17 +1194,17 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x
   const bool live = tok < m_total;
   const int64_t n4 = live ? cols >> 2 : 0, n_pad = n_quads_row * 24;  // float4s of the row, with the last quad's padding
   const float4 *xr = reinterpret_cast<const float4 *>(x + (live ? tok : 0) * cols);
-  float4 v[REG ? kXsVec : 1];
+  float4 v[VEC ? VEC : 1];
   float top = 0.f;
   uint32_t low = ~0u;
-  if constexpr (REG) {
+  if constexpr (VEC != 0) {
 #pragma unroll
-    for (int k = 0; k < kXsVec; ++k) {
+    for (int k = 0; k < VEC; ++k) {
       const int64_t i = tid + 256 * k;
       v[k] = i < n4 ? xr[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
 #pragma unroll
-    for (int k = 0; k < kXsVec; ++k) range_of(v[k], top, low);
+    for (int k = 0; k < VEC; ++k) range_of(v[k], top, low);
   } else {
     for (int64_t i = tid; i < n4; i += 256) range_of(xr[i], top, low);
   }
@@ -1238,9 +1238,9 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x
     }
   }
   if (tid == 0) tscale[tok] = pow2f(-e);
-  if constexpr (REG) {
+  if constexpr (VEC != 0) {
 #pragma unroll
-    for (int k = 0; k < kXsVec; ++k) {
+    for (int k = 0; k < VEC; ++k) {
       const int64_t i = tid + 256 * k;
       if (i < n_pad) store_parts(part_slot(xf, slab, n_quads_row, t, tl, i), v[k], sc);
     }
@@ -1254,8 +1254,9 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float *__restrict__ x
 // xsplit_kernel in one launch, with the same values (the sum of squares in rmsnorm_kernel's order: lane l holds
 // float4 l + 64k of the row, fmaf over k and the four components, then the wave sum).  One wave per token row of
 // each 64-token slab; rows >= m write zeros, rows of token tiles the GEMM does not read (t >= tiles) nothing.
-// Rows of up to 64 * kNfVec float4s (padding of the last quad included).
+// Rows of up to 64 VEC float4s (padding of the last quad included).
 constexpr int kNfVec = 8;
+template <int VEC>
 __global__ __launch_bounds__(256) void normfrag_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                        int64_t m_total, int cols, int64_t n_quads_row, int tiles,
                                                        int wide_from, float eps, uint2 *__restrict__ xf,
@@ -1269,16 +1270,16 @@ __global__ __launch_bounds__(256) void normfrag_kernel(const float *__restrict__
   const bool live = tok < m_total;
   const float4 *xr = reinterpret_cast<const float4 *>(x + (live ? tok : 0) * static_cast<int64_t>(cols));
   const float4 *wr = reinterpret_cast<const float4 *>(w);
-  float4 v[kNfVec], g[kNfVec];
+  float4 v[VEC], g[VEC];
 #pragma unroll
-  for (int k = 0; k < kNfVec; ++k) {
+  for (int k = 0; k < VEC; ++k) {
     const int i = lane + 64 * k;
     v[k] = live && i < n4 ? xr[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     g[k] = i < n4 ? wr[i] : make_float4(0.f, 0.f, 0.f, 0.f);
   }
   float ss = 0.f;
 #pragma unroll
-  for (int k = 0; k < kNfVec; ++k) {
+  for (int k = 0; k < VEC; ++k) {
     ss = fmaf(v[k].x, v[k].x, ss);
     ss = fmaf(v[k].y, v[k].y, ss);
     ss = fmaf(v[k].z, v[k].z, ss);
@@ -1289,7 +1290,7 @@ __global__ __launch_bounds__(256) void normfrag_kernel(const float *__restrict__
   float mx[1] = {0.f};
   uint32_t low = ~0u;
 #pragma unroll
-  for (int k = 0; k < kNfVec; ++k) {
+  for (int k = 0; k < VEC; ++k) {
     v[k] = live ? make_float4(v[k].x * r * g[k].x, v[k].y * r * g[k].y, v[k].z * r * g[k].z, v[k].w * r * g[k].w)
                 : make_float4(0.f, 0.f, 0.f, 0.f);
     range_of(v[k], mx[0], low);
@@ -1302,7 +1303,7 @@ __global__ __launch_bounds__(256) void normfrag_kernel(const float *__restrict__
     if (wide_from > 1) {
       float n[1] = {0.f};
 #pragma unroll
-      for (int k = 0; k < kNfVec; ++k)
+      for (int k = 0; k < VEC; ++k)
         if (lane + 64 * k < n4) n[0] += static_cast<float>(below_line(v[k], sc));
       group_reduce<64>(n);
       wide = n[0] >= static_cast<float>(wide_from);
@@ -1310,7 +1311,7 @@ __global__ __launch_bounds__(256) void normfrag_kernel(const float *__restrict__
     if (wide) {
       if (lane == 0) tscale[tok] = 0.f;
 #pragma unroll
-      for (int k = 0; k < kNfVec; ++k) {
+      for (int k = 0; k < VEC; ++k) {
         const int i = lane + 64 * k;
         if (i < n_quads_row * 24) store_exact_parts(part_slot(xf, slab, n_quads_row, t, tl, i), v[k]);
       }
@@ -1319,7 +1320,7 @@ __global__ __launch_bounds__(256) void normfrag_kernel(const float *__restrict__
   }
   if (lane == 0) tscale[tok] = pow2f(-e);
 #pragma unroll
-  for (int k = 0; k < kNfVec; ++k) {
+  for (int k = 0; k < VEC; ++k) {
     const int i = lane + 64 * k;
     if (i < n_quads_row * 24) store_parts(part_slot(xf, slab, n_quads_row, t, tl, i), v[k], sc);
   }
@@ -2374,7 +2375,8 @@ int launch_x_parts(const float *x, const float *norm_w, float norm_eps, int64_t 
   uint2 *xf = static_cast<uint2 *>(ws);
   if (norm_w && x_parts_fuses_norm(cols)) {
     // the norm writes the fragment-order copy itself (rows that fit normfrag_kernel's registers)
-    hipLaunchKernelGGL(normfrag_kernel, dim3(static_cast<unsigned>(slabs * 16)), dim3(256), 0, s, x, norm_w, m,
+    auto k = nq * 24 <= 64 * 2 ? normfrag_kernel<2> : nq * 24 <= 64 * 4 ? normfrag_kernel<4> : normfrag_kernel<kNfVec>;
+    hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(slabs * 16)), dim3(256), 0, s, x, norm_w, m,
                        static_cast<int>(cols), nq, tiles, wide_from, norm_eps, xf, tscale);
     return check_launch("normfrag_kernel");
   }
@@ -2383,11 +2385,10 @@ int launch_x_parts(const float *x, const float *norm_w, float norm_eps, int64_t 
     if (st != PLX_OK) return st;
     x = xnorm;
   }
-  const dim3 gs(static_cast<unsigned>(slabs * 16 * tiles));
-  if (nq * 24 <= 256 * kXsVec)
-    hipLaunchKernelGGL(xsplit_kernel<true>, gs, dim3(256), 0, s, x, m, cols, nq, tiles, wide_from, xf, tscale);
-  else
-    hipLaunchKernelGGL(xsplit_kernel<false>, gs, dim3(256), 0, s, x, m, cols, nq, tiles, wide_from, xf, tscale);
+  // (registers for no more than the row: 12 rows of 432 columns, the norm's copies among them, 0.2 us a copy faster)
+  auto k = nq * 24 <= 256 * 2 ? xsplit_kernel<2> : nq * 24 <= 256 * kXsVec ? xsplit_kernel<kXsVec> : xsplit_kernel<0>;
+  hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(slabs * 16 * tiles)), dim3(256), 0, s, x, m, cols, nq, tiles, wide_from,
+                     xf, tscale);
   return check_launch("xsplit_kernel");
 }
 

@@ -81,7 +81,8 @@ def test_wide_rows(dev, rows, cols, m, kind):
     assert torch.equal(y[~wide], dequant_linear(pk, sg, rows, cols, calm)[~wide])
 
 
-@pytest.mark.parametrize("cols,m", [(960, 12), (960, 330), (2400, 40), (2400, 330)])  # norm fused into the copy; not
+# the norm fused into the copy, a row in 2, 4 and 8 registers a lane; not fused
+@pytest.mark.parametrize("cols,m", [(480, 20), (504, 33), (960, 12), (960, 330), (984, 70), (2016, 40), (2400, 40), (2400, 330)])
 def test_wide_rows_with_norm_and_epilogues(dev, cols, m):
     shapes = (130, 961)
     ws = [_weight(dev, r, cols, r) for r in shapes]
